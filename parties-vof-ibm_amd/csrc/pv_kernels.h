@@ -288,7 +288,6 @@ typedef struct pvk_mglev {
 } pvk_mglev;
 typedef struct pvk_mg {
     int nlev, c0, nu, fp32;           /* levels, first in-LDS level, sweeps per side, FP32 V-cycle */
-    int topf;                         /* faces of level c0 copied to LDS too (when they fit) */
     int wmask;                        /* in-LDS levels (bit l) with two coarse corrections (a W there) */
     int sh0;                          /* level-0 tile shape: 0 = 64 x 16, 1 = 32 x 16, 2 = 32 x 8,
                                          -1 = by width as the other levels */
@@ -305,7 +304,6 @@ typedef struct pvk_mg {
 /* faces of every level; with bottom != 0 also the bottom matrix P G P */
 void pvk_mg_setup(const pvk_mg *m, const double *bx0, const double *by0, int pf, int bottom, hipStream_t s);
 int  pvk_mg_nrz(const pvk_mg *m);
-size_t pvk_mg_lds_bytes(const pvk_mg *m);
 void pvk_mg_pre(const pvk_mg *m, int l, pvk_scal *sc, const pvk_pcg *w, int n, double tol, int maxit,
                 hipStream_t s);
 void pvk_mg_coarse(const pvk_mg *m, const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w, int n, double tol,

@@ -792,370 +792,487 @@ template <typename T> __global__ void __launch_bounds__(NTH) k_mg_bottom_proj(in
 }
 
 // ---------------------------------------------------------------------------
-// Levels c0 .. nlev-1 in one workgroup of 1024 threads.  x and f of every
-// level live in LDS, and the faces of every level below c0; those of level
-// c0 are copied too when they fit (topf), else read from its arrays.  The
-// kernel runs on one CU, so its time is instruction issue: each thread reads
-// the coefficients and neighbour indices of its cells once per level and
-// pass into registers, and a Gauss-Seidel update is then four LDS reads, the
-// weighted sum and one store.
+// Levels c0 .. nlev-1 in one workgroup.  The kernel runs on one CU, so its
+// time is a chain of barrier-separated half-sweeps; what a half-sweep costs
+// is instruction issue and LDS round trips.
+//
+// A thread owns 2 x 2 blocks of cells (one coarse cell each): two blocks of
+// level c0, one of each level below.  It keeps their faces, 1 / diagonal, f
+// and x in registers for the whole kernel; LDS holds only x, one array per
+// colour (so neighbouring lanes read neighbouring words), and the coarse
+// right-hand sides.  A half-sweep of a block is then four LDS reads (the
+// neighbours outside the block), two updates and two writes, the restricted
+// residual of a block is its owner's own sum, and every LDS address is an
+// offset from the one dynamic array, so the accesses are LDS instructions.
+// Reading the level descriptors (with their pointers) from LDS instead, as
+// an earlier form did, made every access a flat one, and each pass reloaded
+// the coefficients: at 1024^2 (64^2, 32^2 and the 16^2 bottom, W on both,
+// FP32) 53.5 us a launch against 33 now; FP64, V at 96^2, 26 against 15.
 // ---------------------------------------------------------------------------
-#define CT 1024
-#define MG_LOW PVK_MG_LOW   // 4096 -> 1024 -> 256 -> 64 cells
-static_assert(PVK_MG_LDS_CELLS <= 4 * CT, "level c0 is loaded as at most 4 cells a thread");
+#define CT 512
+static_assert(PVK_MG_LDS_CELLS <= 8 * CT, "level c0 has at most two 2 x 2 blocks a thread");
+static_assert(PVK_MG_LOW <= 3, "k_mg_coarse is instantiated for up to three smoothing levels");
 
-template <typename T> struct LdsLev {
-    int nx, ny, fp;         // cells; pitch of bx, by
-    int lnx;                // log2(nx) if nx is a power of two, else -1
-    T *x, *f;               // LDS, compact
-    const T *bx, *by;       // LDS (pitch nx) or the level's arrays
-};
-
-// q / n and q % n, by shift and mask when n = 2^l (l >= 0)
-__device__ __forceinline__ void divmod(int q, int n, int l, int &d, int &r)
-{
-    d = (l >= 0) ? (q >> l) : q / n;
-    r = q - d * n;
-}
 __device__ __forceinline__ int ilog2_or_neg(int n) { return (n > 0 && (n & (n - 1)) == 0) ? __ffs(n) - 1 : -1; }
 
-// a / b of the Gauss-Seidel update: FP64 divides; FP32 multiplies by the
-// hardware reciprocal (1 ulp), which keeps the V-cycle a fixed symmetric
-// operator (both sweep directions use the same value)
-template <typename T> __device__ __forceinline__ T gs_div(T a, T b) { return a / b; }
-template <> __device__ __forceinline__ float gs_div<float>(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
+// 1 / b of the Gauss-Seidel update: FP64 divides; FP32 takes the hardware
+// reciprocal (1 ulp), which keeps the V-cycle a fixed symmetric operator
+// (both sweep directions use the same value)
+template <typename T> __device__ __forceinline__ T gs_rcp(T b) { return T(1) / b; }
+template <> __device__ __forceinline__ float gs_rcp<float>(float b) { return __builtin_amdgcn_rcpf(b); }
 
-// A cell of an in-LDS level as one thread smooths it: the LDS indices of the
-// cell and of its four neighbours, the faces, 1 / (their sum) and f, read
-// once per level and pass and kept in registers for all the half-sweeps of
-// that pass.  A neighbour beyond a y wall has face 0 and is pointed at the
-// neighbour on the other side (a smoothing level has at least two rows):
-// a cell of the other colour, so already written when it is read (a cell of
-// the same colour may still hold stale LDS, and 0 * NaN is NaN).
-template <typename T> struct GsCell {
-    int s, e, w, n, so;
-    T ce, cw, cn, cs, id, f;
+// In-LDS layout, in units of T and at fixed places (the most a level can
+// need), so an access is an index register and an immediate offset: smoothing
+// level K's red and black x (row j, pair I at j hx + I: cells 2 I and 2 I + 1
+// of a row are one red, (i + j) even, and one black) and, below c0, its f;
+// the bottom's x; then in doubles the bottom's f and partial sums.
+template <int K> struct CLds {
+    static constexpr int N = PVK_MG_LDS_CELLS >> (2 * K);                 // cells at most
+    static constexpr int R = K ? CLds<(K ? K - 1 : 0)>::END : 0, B = R + N / 2, F = R + N, END = F + (K ? N : 0);
+};
+#define MG_BX CLds<2>::END                          // the bottom's x
+#define MG_BD (MG_BX + PVK_MG_BOTTOM)               // end of the T part
+#define MG_BF (PVK_MG_BOTTOM + 8)                   // the bottom's f
+static_assert(MG_BD % 2 == 0, "the doubles start on 8 bytes");
+template <typename T> static constexpr size_t coarse_lds_bytes()
+{
+    return MG_BD * sizeof(T) + sizeof(double) * (MG_BF + 3 * PVK_MG_BOTTOM);
+}
+static_assert(coarse_lds_bytes<double>() <= 65536, "a launch gets 64 KiB without asking for more");
+
+struct CGeo {
+    int nx, ny, hx, nblk;           // cells, blocks a row, blocks
 };
 
-template <typename T> __device__ __forceinline__ void gs_cell(const LdsLev<T> &L, int i, int j, GsCell<T> &c)
-{
-    const int nx = L.nx, fp = L.fp, ie = (i + 1 == nx) ? 0 : i + 1, iw = (i == 0) ? nx - 1 : i - 1;
-    c.s = j * nx + i;
-    c.e = j * nx + ie;
-    c.w = j * nx + iw;
-    c.n = (j + 1 < L.ny) ? c.s + nx : c.s - nx;
-    c.so = (j > 0) ? c.s - nx : c.s + nx;
-    c.ce = L.bx[j * fp + i];
-    c.cw = L.bx[j * fp + iw];
-    c.cn = (j + 1 < L.ny) ? L.by[j * fp + i] : T(0);
-    c.cs = (j > 0) ? L.by[(j - 1) * fp + i] : T(0);
-    c.id = gs_div(T(1), c.ce + c.cw + c.cn + c.cs);
-    c.f = L.f[c.s];
-}
-
-// Gauss-Seidel update of the cell from its neighbours' current x
-template <typename T> __device__ __forceinline__ void gs_update(T *x, const GsCell<T> &c)
-{
-    x[c.s] = (c.ce * x[c.e] + c.cw * x[c.w] + c.cn * x[c.n] + c.cs * x[c.so] - c.f) * c.id;
-}
-
-// residual f - A x at the cell
-template <typename T> __device__ __forceinline__ T gs_res(const T *x, const GsCell<T> &c)
-{
-    const T x0 = x[c.s];
-    return c.f - (c.ce * (x[c.e] - x0) - c.cw * (x0 - x[c.w]) + c.cn * (x[c.n] - x0) - c.cs * (x0 - x[c.so]));
-}
-
-// The cells of in-LDS level L pair along x: pair p = (ip, j) holds cells
-// 2 ip and 2 ip + 1 of row j, one red ((i + j) even) and one black.  Thread
-// t owns pairs t and t + CT (a level has at most 2 CT pairs).
-template <typename T> struct GsPairs {
-    GsCell<T> r[2], b[2];
-    int p[2];        // pair index, or -1
+// a 2 x 2 block: cells a (2I, 2J) and d (2I+1, 2J+1) are red, b (2I+1, 2J)
+// and c (2I, 2J+1) black; faces between them, to the left (la, lc), right
+// (br, dr), south (sa, sb) and north (nc, nd), 0 at a wall
+template <typename T> struct Blk {
+    T ab, cd, la, lc, br, dr, ac, bd, sa, sb, nc, nd;
+    T ia, ib, ic, id, fa, fb, fc, fd, a, b, c, d;
+    int s, l, r, up, dn;            // slots of row 2J: own, left, right block; of rows 2J+2 and 2J-1
+    int I, J;
+    bool on;
 };
 
-template <typename T> __device__ __forceinline__ void gs_pairs(const LdsLev<T> &L, GsPairs<T> &P)
+// The blocks' positions.  A neighbour beyond a wall has face 0; its slot is
+// the block's own (finite once the level has been swept, and 0 times it is 0).
+template <typename T, int NB> __device__ __forceinline__ void blk_place(const CGeo &g, Blk<T> (&k)[NB])
 {
-    const int hx = L.nx >> 1, npair = hx * L.ny, lhx = (L.lnx > 0) ? L.lnx - 1 : -1;
+    const int lhx = ilog2_or_neg(g.hx);
 #pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const int q = threadIdx.x + k * CT;
-        P.p[k] = -1;
-        if (q < npair) {
-            int j, ip;
-            divmod(q, hx, lhx, j, ip);
-            P.p[k] = q;
-            gs_cell(L, 2 * ip + (j & 1), j, P.r[k]);
-            gs_cell(L, 2 * ip + 1 - (j & 1), j, P.b[k]);
+    for (int u = 0; u < NB; u++) {
+        const int q = threadIdx.x + u * CT, hx = g.hx, hy = g.ny >> 1;
+        k[u].on = q < g.nblk;
+        const int qq = k[u].on ? q : 0;
+        const int j = (lhx >= 0) ? (qq >> lhx) : qq / hx, i = qq - j * hx;
+        k[u].I = i;
+        k[u].J = j;
+        k[u].s = 2 * j * hx + i;
+        k[u].l = k[u].s + ((i == 0) ? hx - 1 : -1);
+        k[u].r = k[u].s + ((i + 1 == hx) ? 1 - hx : 1);
+        k[u].dn = (j == 0) ? k[u].s : k[u].s - hx;
+        k[u].up = (j + 1 == hy) ? k[u].s : k[u].s + 2 * hx;
+    }
+}
+
+// Two values of a row from column 2 I on, in one load: a smoothing level's
+// width and pitch are even and its arrays start on two values.
+template <typename T> __device__ __forceinline__ void ld2(const T *a, int pitch, int i, int j, T &v0, T &v1)
+{
+    typedef T T2 __attribute__((ext_vector_type(2)));
+    const T2 v = *(const T2 *)(a + (ptrdiff_t)j * pitch + i);
+    v0 = v.x;
+    v1 = v.y;
+}
+
+template <typename T> __device__ __forceinline__ void st2(T *a, int pitch, int i, int j, T v0, T v1)
+{
+    typedef T T2 __attribute__((ext_vector_type(2)));
+    T2 v;
+    v.x = v0;
+    v.y = v1;
+    *(T2 *)(a + (ptrdiff_t)j * pitch + i) = v;
+}
+
+// faces of the blocks: every load unconditional, from clamped positions; the
+// wall faces are masked in blk_diag
+template <typename T, int NB> __device__ __forceinline__ void blk_faces(const Lev<T> &L, Blk<T> (&k)[NB])
+{
+#pragma unroll
+    for (int u = 0; u < NB; u++) {
+        const int i = 2 * k[u].I, j = 2 * k[u].J, iw = (i == 0) ? L.nx - 1 : i - 1, p = L.pitch;
+        ld2(L.bx, p, i, j, k[u].ab, k[u].br);
+        ld2(L.bx, p, i, j + 1, k[u].cd, k[u].dr);
+        ld2(L.by, p, i, max(j - 1, 0), k[u].sa, k[u].sb);
+        ld2(L.by, p, i, j, k[u].ac, k[u].bd);
+        ld2(L.by, p, i, j + 1, k[u].nc, k[u].nd);
+        k[u].la = ld(L.bx, p, iw, j);
+        k[u].lc = ld(L.bx, p, iw, j + 1);
+    }
+}
+template <typename T, int NB> __device__ __forceinline__ void blk_diag(const CGeo &g, Blk<T> (&k)[NB])
+{
+#pragma unroll
+    for (int u = 0; u < NB; u++) {
+        if (k[u].J == 0) k[u].sa = k[u].sb = T(0);
+        if (k[u].J + 1 == (g.ny >> 1)) k[u].nc = k[u].nd = T(0);
+        k[u].ia = gs_rcp(k[u].ab + k[u].la + k[u].ac + k[u].sa);
+        k[u].ib = gs_rcp(k[u].br + k[u].ab + k[u].bd + k[u].sb);
+        k[u].ic = gs_rcp(k[u].cd + k[u].lc + k[u].nc + k[u].ac);
+        k[u].id = gs_rcp(k[u].dr + k[u].cd + k[u].nd + k[u].bd);
+    }
+}
+
+// A barrier that orders LDS alone: loads from memory stay in flight across it.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// half-sweeps; each ends with a barrier (a colour's cells read only the other
+// colour, whose last writes a barrier has already ordered)
+template <int K, typename T, int NB> __device__ __forceinline__ void sweep_red0(const CGeo &g, T *x, Blk<T> (&k)[NB])
+{
+#pragma unroll
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            x[CLds<K>::R + k[u].s] = k[u].a = -k[u].fa * k[u].ia;
+            x[CLds<K>::R + k[u].s + g.hx] = k[u].d = -k[u].fd * k[u].id;
         }
-    }
+    lds_barrier();
 }
-
-// Pre-smoothing of in-LDS level L (red, from x = 0 when zero, black, then
-// nu - 1 more red-black pairs) and restriction: C.f = the sum of the four
-// fine residuals, through rs (one residual sum per fine pair).
-template <typename T> __device__ void lds_pre(const LdsLev<T> &L, const LdsLev<T> &C, T *rs, int nu, bool zero)
+template <int K, typename T, int NB> __device__ __forceinline__ void sweep_red(const CGeo &g, T *x, Blk<T> (&k)[NB])
 {
-    GsPairs<T> P;
-    gs_pairs(L, P);
-    // From x = 0 the first red update is -f / diag.  Otherwise (the second
-    // correction of a W) it is left out: the post-smoothing just ended with
-    // a red half-sweep and no black cell has changed since, so it would
-    // reproduce the same red values.
-    if (zero) {
+    const T *B = x + CLds<K>::B;
+    T w[NB], s[NB], e[NB], n[NB];
 #pragma unroll
-        for (int k = 0; k < 2; k++)
-            if (P.p[k] >= 0) L.x[P.r[k].s] = -P.r[k].f * P.r[k].id;
-        __syncthreads();
-    }
-#pragma unroll
-    for (int k = 0; k < 2; k++)
-        if (P.p[k] >= 0) gs_update(L.x, P.b[k]);
-    __syncthreads();
-    for (int sw = 1; sw < nu; sw++) {
-#pragma unroll
-        for (int k = 0; k < 2; k++)
-            if (P.p[k] >= 0) gs_update(L.x, P.r[k]);
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < 2; k++)
-            if (P.p[k] >= 0) gs_update(L.x, P.b[k]);
-        __syncthreads();
-    }
-#pragma unroll
-    for (int k = 0; k < 2; k++)
-        if (P.p[k] >= 0) rs[P.p[k]] = gs_res(L.x, P.r[k]) + gs_res(L.x, P.b[k]);
-    __syncthreads();
-    const int hx = L.nx >> 1;
-    for (int q = threadIdx.x; q < C.nx * C.ny; q += CT) {
-        int J, I;
-        divmod(q, C.nx, C.lnx, J, I);
-        C.f[q] = rs[2 * J * hx + I] + rs[(2 * J + 1) * hx + I];
-    }
-    __syncthreads();
-}
-
-// parent (coarse cell) of the cell at LDS index q of level L
-template <typename T> __device__ __forceinline__ int gs_parent(const LdsLev<T> &L, const LdsLev<T> &C, int q)
-{
-    int j, i;
-    divmod(q, L.nx, L.lnx, j, i);
-    return (j >> 1) * C.nx + (i >> 1);
-}
-
-// Coarse correction x += xc(parent) and post-smoothing (black first) of
-// in-LDS level L; C holds the coarse result.  The correction rides in the
-// first black half-sweep: its red neighbours are read as x + xc(their
-// parent), the value the separate correction would have stored; the red
-// cells themselves need not be corrected, the red half-sweep that follows
-// overwrites them from the updated black ones.
-template <typename T> __device__ void lds_post(const LdsLev<T> &L, const LdsLev<T> &C, int nu)
-{
-    GsPairs<T> P;
-    gs_pairs(L, P);
-#pragma unroll
-    for (int k = 0; k < 2; k++)
-        if (P.p[k] >= 0) {
-            const GsCell<T> &c = P.b[k];
-            const T *x = L.x, *xc = C.x;
-            const T xe = x[c.e] + xc[gs_parent(L, C, c.e)], xw = x[c.w] + xc[gs_parent(L, C, c.w)];
-            const T xn = x[c.n] + xc[gs_parent(L, C, c.n)], xs = x[c.so] + xc[gs_parent(L, C, c.so)];
-            L.x[c.s] = (c.ce * xe + c.cw * xw + c.cn * xn + c.cs * xs - c.f) * c.id;
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            w[u] = B[k[u].l];
+            s[u] = B[k[u].dn];
+            e[u] = B[k[u].r + g.hx];
+            n[u] = B[k[u].up];
         }
-    __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 2; k++)
-        if (P.p[k] >= 0) gs_update(L.x, P.r[k]);
-    __syncthreads();
-    for (int sw = 1; sw < nu; sw++) {
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            k[u].a = (k[u].ab * k[u].b + k[u].la * w[u] + k[u].ac * k[u].c + k[u].sa * s[u] - k[u].fa) * k[u].ia;
+            k[u].d = (k[u].dr * e[u] + k[u].cd * k[u].c + k[u].nd * n[u] + k[u].bd * k[u].b - k[u].fd) * k[u].id;
+            x[CLds<K>::R + k[u].s] = k[u].a;
+            x[CLds<K>::R + k[u].s + g.hx] = k[u].d;
+        }
+    lds_barrier();
+}
+template <int K, typename T, int NB> __device__ __forceinline__ void sweep_black(const CGeo &g, T *x, Blk<T> (&k)[NB])
+{
+    const T *R = x + CLds<K>::R;
+    T e[NB], s[NB], w[NB], n[NB];
 #pragma unroll
-        for (int k = 0; k < 2; k++)
-            if (P.p[k] >= 0) gs_update(L.x, P.b[k]);
-        __syncthreads();
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            e[u] = R[k[u].r];
+            s[u] = R[k[u].dn];
+            w[u] = R[k[u].l + g.hx];
+            n[u] = R[k[u].up];
+        }
 #pragma unroll
-        for (int k = 0; k < 2; k++)
-            if (P.p[k] >= 0) gs_update(L.x, P.r[k]);
-        __syncthreads();
-    }
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            k[u].b = (k[u].br * e[u] + k[u].ab * k[u].a + k[u].bd * k[u].d + k[u].sb * s[u] - k[u].fb) * k[u].ib;
+            k[u].c = (k[u].cd * k[u].d + k[u].lc * w[u] + k[u].nc * n[u] + k[u].ac * k[u].a - k[u].fc) * k[u].ic;
+            x[CLds<K>::B + k[u].s] = k[u].b;
+            x[CLds<K>::B + k[u].s + g.hx] = k[u].c;
+        }
+    lds_barrier();
+}
+// the first black half-sweep after the coarse correction: the red neighbours
+// are read as x + x_coarse(their parent); the red cells themselves need not be
+// corrected, the red half-sweep that follows overwrites them
+template <int K, bool BOT, typename T, int NB>
+__device__ __forceinline__ void sweep_black_corr(const CGeo &g, T *x, Blk<T> (&k)[NB])
+{
+    // x of the coarse cell (i, j)
+    auto px = [&](int i, int j) {
+        if constexpr (BOT) return x[MG_BX + j * g.hx + i];
+        else return x[CLds<K + 1>::R + (((i + j) & 1) ? CLds<K + 1>::N / 2 : 0) + j * (g.hx >> 1) + (i >> 1)];
+    };
+    const T *R = x + CLds<K>::R;
+    T e[NB], s[NB], w[NB], n[NB], pc[NB];
+#pragma unroll
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            const int i = k[u].I, j = k[u].J, d = k[u].dn != k[u].s, h = k[u].up != k[u].s;
+            e[u] = R[k[u].r] + px(i + k[u].r - k[u].s, j);
+            s[u] = R[k[u].dn] + px(i, j - d);
+            w[u] = R[k[u].l + g.hx] + px(i + k[u].l - k[u].s, j);
+            n[u] = R[k[u].up] + px(i, j + h);
+            pc[u] = px(i, j);
+        }
+#pragma unroll
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            const T a = k[u].a + pc[u], d = k[u].d + pc[u];
+            k[u].b = (k[u].br * e[u] + k[u].ab * a + k[u].bd * d + k[u].sb * s[u] - k[u].fb) * k[u].ib;
+            k[u].c = (k[u].cd * d + k[u].lc * w[u] + k[u].nc * n[u] + k[u].ac * a - k[u].fc) * k[u].ic;
+            x[CLds<K>::B + k[u].s] = k[u].b;
+            x[CLds<K>::B + k[u].s + g.hx] = k[u].c;
+        }
+    lds_barrier();
 }
 
-// in-LDS level l: x, f, bx, by (level c0 without topf: x, f)
-template <typename T> __device__ __forceinline__ LdsLev<T> lds_level(const pvk_mg &m, T *lds, int l)
+// Residual of the blocks, summed over each block: the coarse cell's f (with
+// row sums first, as (red + black) of row 2J plus (red + black) of row 2J+1),
+// to the next smoothing level's f, or to the bottom's in FP64
+template <int K, bool BOT, typename T, int NB>
+__device__ __forceinline__ void restrict_res(const CGeo &g, T *x, const Blk<T> (&k)[NB], double *bf)
 {
-    T *q = lds;
-    for (int k = m.c0; k < l; k++) q += ((k == m.c0 && !m.topf) ? 2 : 4) * m.L[k].nx * m.L[k].ny;
-    const int nc = m.L[l].nx * m.L[l].ny;
-    LdsLev<T> v;
-    v.nx = m.L[l].nx;
-    v.ny = m.L[l].ny;
-    v.lnx = ilog2_or_neg(v.nx);
-    v.x = q;
-    v.f = q + nc;
-    if (l == m.c0 && !m.topf) {
-        v.fp = m.L[l].pitch;
-        v.bx = (const T *)m.L[l].bx;
-        v.by = (const T *)m.L[l].by;
+    const T *R = x + CLds<K>::R, *B = x + CLds<K>::B;
+#pragma unroll
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            const T a = k[u].a, b = k[u].b, c = k[u].c, d = k[u].d;
+            const T ra = k[u].fa - (k[u].ab * (b - a) - k[u].la * (a - B[k[u].l]) + k[u].ac * (c - a) - k[u].sa * (a - B[k[u].dn]));
+            const T rd = k[u].fd - (k[u].dr * (B[k[u].r + g.hx] - d) - k[u].cd * (d - c) + k[u].nd * (B[k[u].up] - d) - k[u].bd * (d - b));
+            const T rb = k[u].fb - (k[u].br * (R[k[u].r] - b) - k[u].ab * (b - a) + k[u].bd * (d - b) - k[u].sb * (b - R[k[u].dn]));
+            const T rc = k[u].fc - (k[u].cd * (d - c) - k[u].lc * (c - R[k[u].l + g.hx]) + k[u].nc * (R[k[u].up] - c) - k[u].ac * (c - a));
+            const T v = (ra + rb) + (rd + rc);
+            const int q = threadIdx.x + u * CT;
+            if constexpr (BOT) bf[q] = (double)v;
+            else x[CLds<K + 1>::F + q] = v;
+        }
+    lds_barrier();
+}
+
+// Bottom level, x = -H f (H = P G P, symmetric, in the cycle's type), in
+// FP64.  Thread (q, r) = (threadIdx / 128, threadIdx % 128) sums a quarter of
+// the columns for rows 2 r and 2 r + 1 (each f from LDS serves two products),
+// reading H[c][2r], H[c][2r+1] = H[2r][c], H[2r+1][c]; the four quarters are
+// added in order through LDS.  H comes from the L2 through one CU (256 KiB or
+// 512 KiB a visit), so the loads are what it costs: they go out in chunks of
+// PF columns, one chunk ahead of the sums and the first one before the
+// residual that the solve waits for.  One load a column in the sums' loop,
+// as an earlier form had, left 12 us a visit, of the 1.7 us (FP32) the bytes
+// take.
+template <typename T> struct HChunk {
+    static constexpr int PF = sizeof(T) == 4 ? 8 : 4;
+    T h[PF][2];
+};
+template <typename T> __device__ __forceinline__ void bottom_load(int n, const T *H, int c, HChunk<T> &k)
+{
+    typedef T T2 __attribute__((ext_vector_type(2)));
+    const int r = min(2 * ((int)threadIdx.x & 127), n - 1);
+    const unsigned last = (unsigned)(n - 1) * n;
+    if ((n & 1) == 0) {                                            // rows 2r, 2r + 1 in one aligned load
+#pragma unroll
+        for (int u = 0; u < HChunk<T>::PF; u++) {
+            const T2 v = *(const T2 *)(H + (min((unsigned)(c + u) * n, last) + (r & ~1)));
+            k.h[u][0] = v.x;
+            k.h[u][1] = v.y;
+        }
     } else {
-        v.fp = v.nx;
-        v.bx = q + 2 * nc;
-        v.by = q + 3 * nc;
+        const int r1 = min(r + 1, n - 1);
+#pragma unroll
+        for (int u = 0; u < HChunk<T>::PF; u++) {
+            const unsigned o = min((unsigned)(c + u) * n, last);      // past the end: a value that is not used
+            k.h[u][0] = H[o + r];
+            k.h[u][1] = H[o + r1];
+        }
     }
-    return v;
 }
+// v - h f: fused where the product is exact in FP64 (FP32 entries), which rounds alike
+__device__ __forceinline__ double bottom_acc(float h, double f, double v) { return __builtin_fma(-(double)h, f, v); }
+__device__ __forceinline__ double bottom_acc(double h, double f, double v) { return v - h * f; }
+__device__ __forceinline__ int bottom_col0(int n) { return (threadIdx.x >> 7) * ((n + 3) / 4); }
 
-// residual sums of the restriction (one per fine pair of the largest
-// smoothing level, c0), after the levels
-template <typename T> __device__ __forceinline__ T *lds_scratch(const pvk_mg &m, T *lds)
+template <typename T>
+__device__ __forceinline__ void bottom_solve(int n, const T *H, HChunk<T> &k, const double *bf, double *part, T *X)
 {
-    T *q = lds;
-    for (int k = m.c0; k < m.nlev; k++) q += ((k == m.c0 && !m.topf) ? 2 : 4) * m.L[k].nx * m.L[k].ny;
-    return q;
-}
-
-// the bottom solve's partial sums (4 PVK_MG_BOTTOM doubles) after the
-// restriction scratch, 8-byte aligned
-template <typename T> __device__ __forceinline__ double *lds_bottom(const pvk_mg &m, T *lds)
-{
-    T *q = lds_scratch(m, lds);
-    if (m.nlev > m.c0 + 1) q += (m.L[m.c0].nx / 2) * m.L[m.c0].ny;
-    return (double *)(((uintptr_t)q + 7) & ~(uintptr_t)7);
-}
-
-// bottom level, x = -H f (H = P G P, symmetric, in the cycle's type: the
-// FP32 cycle reads half the bytes), H read from memory (up to 512 KiB; the
-// one workgroup streams it through one CU, so many loads are kept in
-// flight).  Thread (q, r) = (threadIdx / 256, threadIdx % 256) sums a
-// quarter of the columns for row r, in FP64, reading H[c][r] = H[r][c]:
-// consecutive threads read consecutive entries of row c.  The four quarters
-// are added in order through LDS.
-template <typename T> __device__ __forceinline__ void bottom_solve(const LdsLev<T> &B, const T *H, double *part)
-{
-    static_assert(CT == 4 * PVK_MG_BOTTOM, "four quarters of the bottom's columns, one row a thread");
-    const int n = B.nx * B.ny, r = threadIdx.x % PVK_MG_BOTTOM, q = threadIdx.x / PVK_MG_BOTTOM;
-    const int qn = (n + 3) / 4, c0 = q * qn, c1 = min(n, c0 + qn);
-    double v = 0.0;
-    if (r < n) {
-#pragma unroll 16
-        for (int c = c0; c < c1; c++) v -= (double)H[(size_t)c * n + r] * (double)B.f[c];
+    static_assert(CT == 2 * PVK_MG_BOTTOM, "four quarters of the bottom's columns, two rows a thread");
+    constexpr int PF = HChunk<T>::PF;
+    const int r = 2 * (threadIdx.x & 127), q = threadIdx.x >> 7, c0 = bottom_col0(n), nq = min((n + 3) / 4, n - c0);
+    double v0 = 0.0, v1 = 0.0;
+    for (int c = 0; c < nq; c += PF) {
+        HChunk<T> nx;
+        bottom_load(n, H, c0 + c + PF, nx);
+        const double *f = bf + c0 + c;
+        if (c + PF <= nq) {
+#pragma unroll
+            for (int u = 0; u < PF; u++) {
+                v0 = bottom_acc(k.h[u][0], f[u], v0);
+                v1 = bottom_acc(k.h[u][1], f[u], v1);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < PF; u++)
+                if (c + u < nq) {
+                    v0 = bottom_acc(k.h[u][0], f[u], v0);
+                    v1 = bottom_acc(k.h[u][1], f[u], v1);
+                }
+        }
+        k = nx;
     }
-    part[threadIdx.x] = v;
-    __syncthreads();
-    if (q == 0 && r < n)
-        B.x[r] = (T)(((part[r] + part[PVK_MG_BOTTOM + r]) + part[2 * PVK_MG_BOTTOM + r]) + part[3 * PVK_MG_BOTTOM + r]);
-    __syncthreads();
+    if (q > 0) {
+        part[(q - 1) * PVK_MG_BOTTOM + r] = v0;
+        part[(q - 1) * PVK_MG_BOTTOM + r + 1] = v1;
+    }
+    lds_barrier();
+    if (q == 0) {
+        if (r < n) X[r] = (T)(((v0 + part[r]) + part[PVK_MG_BOTTOM + r]) + part[2 * PVK_MG_BOTTOM + r]);
+        if (r + 1 < n)
+            X[r + 1] = (T)(((v1 + part[r + 1]) + part[PVK_MG_BOTTOM + r + 1]) + part[2 * PVK_MG_BOTTOM + r + 1]);
+    }
+    lds_barrier();
 }
 
-template <typename T> __global__ void __launch_bounds__(CT) k_mg_coarse(pvk_mg m, pvk_scal *sc)
+// everything a thread keeps: its blocks of each smoothing level
+template <typename T, int NL> struct CState {
+    CGeo g[NL + 1];                 // smoothing levels and the bottom
+    Blk<T> k0[2], k1[1], k2[1];
+    HChunk<T> h;                    // the bottom solve's first columns
+    T *x;
+    double *bf, *part;
+};
+
+// One visit of smoothing level K: a V, or with the level's bit in wmask two
+// coarse corrections with smoothing between them (pre-smooth, correct,
+// post-smooth, pre-smooth, correct, post-smooth: the error propagation
+// S^T C S S^T C S stays symmetric in the energy inner product).  From x = 0
+// the first red update is -f / diag; the second pre-smoothing leaves its red
+// half-sweep out: the post-smoothing just ended with one and no black cell
+// has changed since, so it would reproduce the same values.
+template <int K, typename T, int NL> __device__ __forceinline__ void cycle(const pvk_mg &m, CState<T, NL> &S);
+template <int K, int NB, typename T, int NL>
+__device__ __forceinline__ void cycle_level(const pvk_mg &m, CState<T, NL> &S, Blk<T> (&k)[NB])
+{
+    constexpr bool BOT = (K + 1 == NL);
+    const CGeo g = S.g[K];
+    T *x = S.x;
+    if constexpr (K > 0) {
+#pragma unroll
+        for (int u = 0; u < NB; u++)
+            if (k[u].on) {
+                const T *f = x + CLds<K>::F + 2 * k[u].J * g.nx + 2 * k[u].I;
+                k[u].fa = f[0];
+                k[u].fb = f[1];
+                k[u].fc = f[g.nx];
+                k[u].fd = f[g.nx + 1];
+            }
+    }
+    const int visits = 1 + ((m.wmask >> (m.c0 + K)) & 1);
+    for (int v = 0; v < visits; v++) {
+        if (v == 0) sweep_red0<K>(g, x, k);
+        sweep_black<K>(g, x, k);
+        for (int sw = 1; sw < m.nu; sw++) {
+            sweep_red<K>(g, x, k);
+            sweep_black<K>(g, x, k);
+        }
+        if constexpr (BOT) {
+            const int n = S.g[NL].nx * S.g[NL].ny;
+            bottom_load(n, (const T *)m.H, bottom_col0(n), S.h);
+        }
+        restrict_res<K, BOT>(g, x, k, S.bf);
+        cycle<K + 1>(m, S);
+        sweep_black_corr<K, BOT>(g, x, k);
+        sweep_red<K>(g, x, k);
+        for (int sw = 1; sw < m.nu; sw++) {
+            sweep_black<K>(g, x, k);
+            sweep_red<K>(g, x, k);
+        }
+    }
+}
+template <int K, typename T, int NL> __device__ __forceinline__ void cycle(const pvk_mg &m, CState<T, NL> &S)
+{
+    if constexpr (K == NL) bottom_solve(S.g[NL].nx * S.g[NL].ny, (const T *)m.H, S.h, S.bf, S.part, S.x + MG_BX);
+    else if constexpr (K == 0) cycle_level<0>(m, S, S.k0);
+    else if constexpr (K == 1) cycle_level<1>(m, S, S.k1);
+    else cycle_level<2>(m, S, S.k2);
+}
+
+template <typename T, int NL> __global__ void __launch_bounds__(CT) k_mg_coarse(pvk_mg m, pvk_scal *sc)
 {
     extern __shared__ double lds_raw[];
-    __shared__ LdsLev<T> lv[PVK_MG_LOW + 1];      // levels c0 .. nb
-    T *lds = (T *)lds_raw;
-    const int nb = m.nlev - 1;
-    // The loads below are valid whatever the stop flag says, so they are
-    // issued before it is read: one memory round trip instead of two.
-    // f of level c0 (and its faces with topf), the faces of the levels below
-    // it: every global load of this thread is issued before the first LDS
-    // store, so the loads wait for memory once, not once per level and pass.
-    // Level c0 has at most 4 CT cells, each level below at most CT, and there
-    // are at most MG_LOW of those (pv_mg_create).
-    T f0[4], bx0[4], by0[4], lbx[MG_LOW], lby[MG_LOW];
-    const Lev<T> G0 = lev<T>(m.L[m.c0]);
-    const int n0 = G0.nx * G0.ny, l0 = ilog2_or_neg(G0.nx);
+    T *x = (T *)lds_raw;
+    CState<T, NL> S;
+    S.x = x;
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const int q = threadIdx.x + u * CT;
-        f0[u] = bx0[u] = by0[u] = T(0);
-        if (q < n0) {
-            int j, i;
-            divmod(q, G0.nx, l0, j, i);
-            f0[u] = (m.c0 == 0 && m.r0) ? (T)m.r0[(ptrdiff_t)j * m.p0 + i] : ld(G0.f, G0.pitch, i, j);
-            if (m.topf) {
-                bx0[u] = ld(G0.bx, G0.pitch, i, j);
-                by0[u] = ld(G0.by, G0.pitch, i, j);
+    for (int K = 0; K <= NL; K++) {
+        const pvk_mglev &L = m.L[m.c0 + K];
+        S.g[K].nx = L.nx;
+        S.g[K].ny = L.ny;
+        S.g[K].hx = L.nx >> 1;
+        S.g[K].nblk = (L.nx >> 1) * (L.ny >> 1);
+    }
+    S.bf = (double *)(x + MG_BD);
+    S.part = S.bf + MG_BF;
+    const int nbot = S.g[NL].nx * S.g[NL].ny;
+    // level 0 of the FP32 cycle: r in, z out in FP64
+    const Lev<T> G0 = lev<T>(m.L[m.c0]);
+    const bool ext = sizeof(T) == 4 && m.c0 == 0;
+    // The loads below are valid whatever the stop flag says, so they are
+    // issued before it is read, every one before the first use: one memory
+    // round trip.
+    if constexpr (NL > 0) {
+        blk_place(S.g[0], S.k0);
+        blk_faces(G0, S.k0);
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int i = 2 * S.k0[u].I, j = 2 * S.k0[u].J;
+            if (ext) {
+                double a, b, c, d;
+                ld2(m.r0, m.p0, i, j, a, b);
+                ld2(m.r0, m.p0, i, j + 1, c, d);
+                S.k0[u].fa = (T)a;
+                S.k0[u].fb = (T)b;
+                S.k0[u].fc = (T)c;
+                S.k0[u].fd = (T)d;
+            } else {
+                ld2(G0.f, G0.pitch, i, j, S.k0[u].fa, S.k0[u].fb);
+                ld2(G0.f, G0.pitch, i, j + 1, S.k0[u].fc, S.k0[u].fd);
             }
         }
+    } else {
+        for (int q = threadIdx.x; q < nbot; q += CT) {
+            const int j = q / G0.nx, i = q - j * G0.nx;
+            S.bf[q] = ext ? (double)(T)m.r0[(ptrdiff_t)j * m.p0 + i] : (double)ld(G0.f, G0.pitch, i, j);
+        }
     }
-#pragma unroll
-    for (int k = 0; k < MG_LOW; k++) {
-        const Lev<T> G = lev<T>(m.L[min(m.c0 + 1 + k, nb)]);
-        const bool in = (m.c0 + 1 + k <= nb) && (int)threadIdx.x < G.nx * G.ny;
-        lbx[k] = in ? G.bx[threadIdx.x] : T(0);      // levels below c0: pitch = width
-        lby[k] = in ? G.by[threadIdx.x] : T(0);
+    if constexpr (NL > 1) {
+        blk_place(S.g[1], S.k1);
+        blk_faces(lev<T>(m.L[m.c0 + 1]), S.k1);
     }
+    if constexpr (NL > 2) {
+        blk_place(S.g[2], S.k2);
+        blk_faces(lev<T>(m.L[m.c0 + 2]), S.k2);
+    }
+    if constexpr (NL == 0) bottom_load(nbot, (const T *)m.H, bottom_col0(nbot), S.h);
     if (sc->p_done) return;
-    // the level descriptors, formed once: the schedule below reads them from
-    // LDS instead of walking the kernel argument with a run-time index
-    if (threadIdx.x <= (unsigned)(nb - m.c0)) lv[threadIdx.x] = lds_level(m, lds, m.c0 + (int)threadIdx.x);
-    double *part = lds_bottom(m, lds);             // the bottom solve's partial sums
-    {
-        const LdsLev<T> L0 = lds_level(m, lds, m.c0);
+    if constexpr (NL > 0) blk_diag(S.g[0], S.k0);
+    if constexpr (NL > 1) blk_diag(S.g[1], S.k1);
+    if constexpr (NL > 2) blk_diag(S.g[2], S.k2);
+    __syncthreads();
+    cycle<0>(m, S);
+    if constexpr (NL == 0) {
+        for (int q = threadIdx.x; q < nbot; q += CT) {
+            const int j = q / G0.nx, i = q - j * G0.nx;
+            if (ext) m.z0[(ptrdiff_t)j * m.p0 + i] = (double)x[MG_BX + q];
+            else G0.x[(ptrdiff_t)j * G0.pitch + i] = x[MG_BX + q];
+        }
+    } else {
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int q = threadIdx.x + u * CT;
-            if (q < n0) {
-                L0.f[q] = f0[u];
-                if (m.topf) {
-                    ((T *)L0.bx)[q] = bx0[u];
-                    ((T *)L0.by)[q] = by0[u];
+        for (int u = 0; u < 2; u++)
+            if (S.k0[u].on) {
+                const int i = 2 * S.k0[u].I, j = 2 * S.k0[u].J;
+                if (ext) {
+                    st2(m.z0, m.p0, i, j, (double)S.k0[u].a, (double)S.k0[u].b);
+                    st2(m.z0, m.p0, i, j + 1, (double)S.k0[u].c, (double)S.k0[u].d);
+                } else {
+                    st2(G0.x, G0.pitch, i, j, S.k0[u].a, S.k0[u].b);
+                    st2(G0.x, G0.pitch, i, j + 1, S.k0[u].c, S.k0[u].d);
                 }
             }
-        }
-#pragma unroll
-        for (int k = 0; k < MG_LOW; k++) {
-            if (m.c0 + 1 + k > nb) break;
-            const LdsLev<T> Ll = lds_level(m, lds, m.c0 + 1 + k);
-            if ((int)threadIdx.x < Ll.nx * Ll.ny) {
-                ((T *)Ll.bx)[threadIdx.x] = lbx[k];
-                ((T *)Ll.by)[threadIdx.x] = lby[k];
-            }
-        }
-    }
-    __syncthreads();
-    T *rs = lds_scratch(m, lds);
-    // The in-LDS levels: a V-cycle, except that the levels in m.wmask take
-    // two coarse corrections, smoothing between them (pre-smooth, correct,
-    // post-smooth, pre-smooth, correct, post-smooth: the error propagation
-    // S^T C S S^T C S stays symmetric in the energy inner product).  One
-    // schedule for all threads: level l, going down or coming back up, and
-    // the levels whose second correction is under way.
-    int l = m.c0;
-    bool down = true;
-    unsigned second = 0u;
-    for (;;) {
-        if (l == nb) {
-            bottom_solve(lv[nb - m.c0], (const T *)m.H, part);
-            l--;
-            down = false;
-            if (l < m.c0) break;
-            continue;
-        }
-        const LdsLev<T> Ll = lv[l - m.c0], Lc = lv[l + 1 - m.c0];
-        if (down) {
-            lds_pre(Ll, Lc, rs, m.nu, true);
-            l++;
-            continue;
-        }
-        lds_post(Ll, Lc, m.nu);
-        if (((m.wmask >> l) & 1) && !((second >> l) & 1u)) {
-            second |= 1u << l;
-            lds_pre(Ll, Lc, rs, m.nu, false);
-            l++;
-            down = true;
-            continue;
-        }
-        second &= ~(1u << l);
-        if (l == m.c0) break;
-        l--;
-    }
-    {
-        const Lev<T> G = lev<T>(m.L[m.c0]);
-        const LdsLev<T> top = lds_level(m, lds, m.c0);
-        for (int q = threadIdx.x; q < G.nx * G.ny; q += CT) {
-            int j, i;
-            divmod(q, G.nx, top.lnx, j, i);
-            if (m.c0 == 0 && m.z0) m.z0[(ptrdiff_t)j * m.p0 + i] = (double)top.x[q];
-            else G.x[(ptrdiff_t)j * G.pitch + i] = top.x[q];
-        }
     }
 }
 
@@ -1251,16 +1368,6 @@ static dim3 tile_grid(const pvk_mg *m, int l)
     return dim3((L.nx + tx - 1) / tx, (L.ny + ty - 1) / ty);
 }
 static dim3 cell_grid(const pvk_mglev &L) { return dim3((L.nx + TXP - 1) / TXP, (L.ny + TYR - 1) / TYR); }
-
-// LDS bytes of the one-workgroup kernel
-extern "C" size_t pvk_mg_lds_bytes(const pvk_mg *m)
-{
-    size_t n = 0;
-    for (int l = m->c0; l < m->nlev; l++) n += ((l == m->c0 && !m->topf) ? 2 : 4) * (size_t)m->L[l].nx * m->L[l].ny;
-    if (m->nlev > m->c0 + 1) n += (size_t)(m->L[m->c0].nx / 2) * m->L[m->c0].ny;   // restriction scratch
-    // + the bottom solve's partial sums (FP64, 8-byte aligned)
-    return n * (m->fp32 ? sizeof(float) : sizeof(double)) + 8 + sizeof(double) * 4 * PVK_MG_BOTTOM;
-}
 
 extern "C" int pvk_mg_nrz(const pvk_mg *m)
 {
@@ -1408,32 +1515,23 @@ extern "C" void pvk_mg_pre(const pvk_mg *m, int l, pvk_scal *sc, const pvk_pcg *
     else pre_t<double>(m, l, sc, w, n, tol, maxit, s);
 }
 
+template <typename T> static void coarse_t(const pvk_mg *m, pvk_scal *sc, hipStream_t s)
+{
+    constexpr size_t need = coarse_lds_bytes<T>();
+    switch (m->nlev - 1 - m->c0) {
+    case 0: hipLaunchKernelGGL((k_mg_coarse<T, 0>), dim3(1), dim3(CT), need, s, *m, sc); break;
+    case 1: hipLaunchKernelGGL((k_mg_coarse<T, 1>), dim3(1), dim3(CT), need, s, *m, sc); break;
+    case 2: hipLaunchKernelGGL((k_mg_coarse<T, 2>), dim3(1), dim3(CT), need, s, *m, sc); break;
+    default: hipLaunchKernelGGL((k_mg_coarse<T, 3>), dim3(1), dim3(CT), need, s, *m, sc); break;
+    }
+}
+
 extern "C" void pvk_mg_coarse(const pvk_mg *m, const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w, int n,
                               double tol, int maxit, hipStream_t s)
 {
-    // above 64 KiB of dynamic LDS the kernel must be allowed it (gfx950: up to
-    // 160 KiB per workgroup).  Handles of any size may launch from several host
-    // threads at once, so the limit is raised once per device and kernel, to
-    // the whole 160 KiB, under a lock; a refusal leaves the launch to report
-    // the error.
-    static std::mutex mu;
-    static unsigned char raised[64][2];
-    const size_t need = pvk_mg_lds_bytes(m);
-    if (need > 65536) {
-        int dev = 0;
-        (void)hipGetDevice(&dev);
-        std::lock_guard<std::mutex> lk(mu);
-        if (dev >= 0 && dev < 64 && !raised[dev][m->fp32]) {
-            const void *k = m->fp32 ? (const void *)k_mg_coarse<float> : (const void *)k_mg_coarse<double>;
-            if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess)
-                raised[dev][m->fp32] = 1;
-            else
-                (void)hipGetLastError();
-        }
-    }
     if (m->c0 == 0) hipLaunchKernelGGL(k_mg_check, dim3(1), dim3(NTH), 0, s, sc, *w, n, tol, maxit);
-    if (m->fp32) hipLaunchKernelGGL(k_mg_coarse<float>, dim3(1), dim3(CT), need, s, *m, sc);
-    else hipLaunchKernelGGL(k_mg_coarse<double>, dim3(1), dim3(CT), need, s, *m, sc);
+    if (m->fp32) coarse_t<float>(m, sc, s);
+    else coarse_t<double>(m, sc, s);
     if (m->c0 == 0)
         hipLaunchKernelGGL(k_mg_dot, dim3(1), dim3(NTH), 0, s, (const pvk_scal *)sc, *w, *g, rz_slot(n));
 }

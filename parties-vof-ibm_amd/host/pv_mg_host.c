@@ -159,10 +159,6 @@ int pv_mg_create(pv_bag *b)
         w->rdct = 1;
         w->flex = 0;
     }
-    /* the faces of level c0 go to LDS too when the whole set fits in 144 KiB */
-    m->topf = mf->topf = 1;
-    if (pvk_mg_lds_bytes(m) > 144 * 1024) m->topf = 0;
-    if (pvk_mg_lds_bytes(mf) > 144 * 1024) mf->topf = 0;
     b->mgp = (b->prm.precision == PV_PREC_MIXED) ? mf : m;
     b->mg_ok = 1;
     return PV_OK;
