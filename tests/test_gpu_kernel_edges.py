@@ -1,0 +1,62 @@
+"""Kernels at the sizes where their shape can go wrong: the edges of what a
+block or thread owns, remainders, and the smallest and largest of a range.
+Each against the restatement the repository has for it."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import mg_ref
+import pvof
+from helpers import regions, relerr
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def lib(gpu):
+    return pvof.load_lib()
+
+
+def params(nx, ny, **kw):
+    base = dict(NXM=nx, NYM=ny, xmax=1.0, ymax=ny / nx, Re=100.0, We=200.0, rho1=1.0, rho2=1e-3, mu1=1.0, mu2=1e-2,
+                Cn=2.0 / nx, Pe_CH=nx / 2.0, cfl=0.2, default_dt=1e-4, max_dt=1e-3, ch_tol=1e-12, CG_ETOL=1e-9,
+                pressure_solver=pvof.PV_PSOLVE_MG_PCG, p_rel_tol=1e-10, p_max_iter=3000)
+    base.update(kw)
+    return pvof.default_params(**base)
+
+
+def canonical(p, a):
+    """Cell array [ny][nx] -> canonical layout, x-ghosts periodic, y-ghosts copied."""
+    return np.pad(np.pad(a, ((3, 4), (0, 0)), mode="edge"), ((0, 0), (3, 4)), mode="wrap")
+
+
+# in-workgroup levels: none but the bottom (16 x 16, 8 x 12); one with an odd
+# bottom (18 x 26 -> 9 x 13); two, blocks not filling the threads (44 x 36);
+# the most blocks (64 x 64) and rows that are no power of two (60 x 68); a
+# bottom 64 wide (128 x 32 -> 64 x 16 -> 32 x 8); three smoothing levels
+# down to rows of two (512 x 8 -> ... -> 64 x 1); a tiled level above them
+# with an odd number of coarse columns (88 x 56 -> 44 x 28 -> 22 x 14 -> 11 x 7)
+@pytest.mark.parametrize("nx,ny", [(16, 16), (8, 12), (18, 26), (44, 36), (64, 64), (60, 68), (128, 32), (512, 8),
+                                   (88, 56)])
+@pytest.mark.parametrize("nu,w", [(2, 0), (1, 1), (2, 3)])
+@pytest.mark.parametrize("fp32", [0, 1])
+def test_in_workgroup_levels(lib, nx, ny, nu, w, fp32):
+    p = params(nx, ny)
+    s = pvof.Solver(p, lib)
+    s.check(lib.pv_set_mg_sweeps(s.h, nu))
+    s.check(lib.pv_set_mg_precision(s.h, fp32))
+    s.check(lib.pv_set_mg_cycle(s.h, w))
+    rho = mg_ref.bubbles(nx, ny, seed=nx + ny, nb=6)
+    f = np.random.default_rng(nx * ny).standard_normal((ny, nx))
+    f -= f.mean()
+    s.set("RHO", canonical(p, rho))
+    s.set("P_RES", canonical(p, f))
+    s.call("mg_vcycle_apply")
+    z = s.get("SCRATCH0")[regions(p)["cell"]]
+    bx, by = mg_ref.faces(rho, float(nx * nx), float(nx * nx))
+    lv, G = mg_ref.build(bx, by)
+    sizes = mg_ref.level_sizes(nx, ny)
+    c0 = next(i for i, sz in enumerate(sizes) if sz[0] * sz[1] <= mg_ref.LDS_CELLS)
+    zr = mg_ref.vcycle(lv, G, f, nu, wl=tuple(range(c0, min(c0 + w, len(lv) - 1))))
+    assert relerr(z, zr) < (1e-5 if fp32 else 1e-11)
