@@ -227,17 +227,6 @@ void pvk_mcg_iter(const pvk_grid *g, const pvk_phys *ph, int stage, pvk_scal *sc
 void pvk_p_rhs2(const pvk_grid *g, int stage, const pvk_scal *sc, const double *u, const double *v,
                 const double *rho, double *rhs, double *M, hipStream_t s);
 void pvk_p_operator(const pvk_grid *g, const double *rho, const double *x, double *Ax, hipStream_t s);
-void pvk_p_cg_init2(const pvk_grid *g, const double *rhs, const double *M, double *phi, double *r, double *d,
-                    int use_M, int shift_mean, const pvk_scal *sc, const pvk_red *rd, hipStream_t s);
-void pvk_p_cg_apply(const pvk_grid *g, pvk_scal *sc, const double *rho, const double *d, double *Ad,
-                    const pvk_red *rd, hipStream_t s);
-void pvk_p_cg_update(const pvk_grid *g, pvk_scal *sc, double *phi, const double *d, double *r,
-                     const double *Ad, const double *M, int use_M, const pvk_red *rd,
-                     hipStream_t s);
-void pvk_p_cg_dupdate(const pvk_grid *g, pvk_scal *sc, const double *z, const double *M, int use_M,
-                      double *d, hipStream_t s);
-void pvk_p_scalar2(const pvk_grid *g, pvk_scal *sc, int which, int mode, int maxit, double tol,
-                   const pvk_red *rd, int nb, hipStream_t s);
 void pvk_dot(const pvk_grid *g, const double *a, const double *b, const pvk_red *rd, hipStream_t s);
 void pvk_dot_sc(const pvk_grid *g, const pvk_scal *sc, const double *a, const double *b,
                 const pvk_red *rd, hipStream_t s);
@@ -262,6 +251,12 @@ void pvk_pcg_clear_done(pvk_scal *sc, hipStream_t s);
 /* sc->red[slot] = sum of the <r, z> partials rz[rzs] */
 void pvk_pcg_gamma(pvk_scal *sc, const pvk_pcg *w, int rzs, int slot, hipStream_t s);
 void pvk_pcg_prep(const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w, hipStream_t s);
+/* Jacobi-PCG (psolve_cg.c:130-293), M the inverse diagonal: faces and start,
+ * then iterations n = 0, 1, ...: half 0 = stop test, direction and operator,
+ * half 1 = step and new residual */
+void pvk_jac_start(const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w, const double *M, hipStream_t s);
+void pvk_jac_iter(const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w, const double *M, int half, int n, double tol,
+                  int maxit, hipStream_t s);
 void pvk_pcg_apply(const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w, int n, hipStream_t s);
 
 /* ---- multigrid-preconditioned CG (csrc/pv_mg.hip) ----

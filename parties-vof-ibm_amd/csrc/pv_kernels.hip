@@ -722,162 +722,6 @@ extern "C" void pvk_p_operator(const pvk_grid *g, const double *rho, const doubl
     hipLaunchKernelGGL(k_p_operator, grid2d(g), dim3(BX, BY), 0, s, *g, rho, x, Ax);
 }
 
-// PCG start with x0 = 0 (psolve_cg.c:166-194): r = rhs - A 0 = rhs, z = M r,
-// d = z, partial <r, z>.  use_M = 0 leaves z = r (the FFT path overwrites d).
-__global__ void k_p_cg_init(pvk_grid g, const double *rhs, const double *M, double *phi, double *r, double *d,
-                            int use_M, double shift_mean_slot, const pvk_scal *sc, double *part, int nb)
-{
-    CELL_IJ
-    double vals[2] = {0.0, 0.0};
-    if (in) {
-        double rr = AT(rhs, i, j);
-        if (shift_mean_slot != 0.0) rr = rr - sc->p_mean;
-        double z = use_M ? rr * AT(M, i, j) : rr;
-        AT(phi, i, j) = 0.0;
-        AT(r, i, j) = rr;
-        AT(d, i, j) = z;
-        vals[0] = rr * z;
-        vals[1] = rr * rr;
-    }
-    block_partials<2>(vals, part, nb);
-}
-extern "C" void pvk_p_cg_init2(const pvk_grid *g, const double *rhs, const double *M, double *phi, double *r,
-                               double *d, int use_M, int shift_mean, const pvk_scal *sc, const pvk_red *rd,
-                               hipStream_t s)
-{
-    hipLaunchKernelGGL(k_p_cg_init, grid2d(g), dim3(BX, BY), 0, s, *g, rhs, M, phi, r, d, use_M,
-                       shift_mean ? 1.0 : 0.0, sc, rd->part, rd->nblocks);
-}
-
-// Ad = A d; partial <d, Ad> (psolve_cg.c:203-208)
-__global__ void k_p_cg_apply(pvk_grid g, const pvk_scal *sc, const double *rho, const double *d, double *Ad,
-                             double *part, int nb)
-{
-    if (sc->p_done) return;
-    CELL_IJ
-    double vals[1] = {0.0};
-    if (in) {
-        double ad = p_op(g, rho, d, i, j);
-        AT(Ad, i, j) = ad;
-        vals[0] = AT(d, i, j) * ad;
-    }
-    block_partials<1>(vals, part, nb);
-}
-extern "C" void pvk_p_cg_apply(const pvk_grid *g, pvk_scal *sc, const double *rho, const double *d, double *Ad,
-                               const pvk_red *rd, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_p_cg_apply, grid2d(g), dim3(BX, BY), 0, s, *g, sc, rho, d, Ad, rd->part, rd->nblocks);
-}
-
-// phi += alpha d; r -= alpha Ad; z = M r; partials <r, z>, <r, r> (:211-230)
-__global__ void k_p_cg_update(pvk_grid g, const pvk_scal *sc, double *phi, const double *d, double *r,
-                              const double *Ad, const double *M, int use_M, double *part, int nb)
-{
-    if (sc->p_done) return;
-    CELL_IJ
-    double vals[2] = {0.0, 0.0};
-    if (in) {
-        const double alpha = sc->p_alpha;
-        AT(phi, i, j) += alpha * AT(d, i, j);
-        double rr = AT(r, i, j) - alpha * AT(Ad, i, j);
-        AT(r, i, j) = rr;
-        double z = use_M ? rr * AT(M, i, j) : rr;
-        vals[0] = rr * z;
-        vals[1] = rr * rr;
-    }
-    block_partials<2>(vals, part, nb);
-}
-extern "C" void pvk_p_cg_update(const pvk_grid *g, pvk_scal *sc, double *phi, const double *d, double *r,
-                                const double *Ad, const double *M, int use_M, const pvk_red *rd, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_p_cg_update, grid2d(g), dim3(BX, BY), 0, s, *g, sc, phi, d, r, Ad, M, use_M, rd->part,
-                       rd->nblocks);
-}
-
-// d = z + beta d, z = M r (Jacobi) or z given (FFT preconditioner) (:238-246)
-__global__ void k_p_cg_dupdate(pvk_grid g, const pvk_scal *sc, const double *zr, const double *M, int use_M,
-                               double *d)
-{
-    if (sc->p_done) return;
-    CELL_IJ
-    if (in) {
-        double z = use_M ? AT(zr, i, j) * AT(M, i, j) : AT(zr, i, j);
-        AT(d, i, j) = z + sc->p_beta * AT(d, i, j);
-    }
-}
-extern "C" void pvk_p_cg_dupdate(const pvk_grid *g, pvk_scal *sc, const double *z, const double *M, int use_M,
-                                 double *d, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_p_cg_dupdate, grid2d(g), dim3(BX, BY), 0, s, *g, sc, z, M, use_M, d);
-}
-
-// Scalar logic.  mode 0 = Jacobi-PCG (sqrt(r.z) absolute stop, psolve_cg.c),
-// mode 1 = FFT-PCG (||r|| / ||b|| stop).  which: 0 start, 1 alpha, 2 stop/beta,
-// 3 gamma after a new preconditioned residual (FFT path).
-__global__ void k_p_scalar(pvk_scal *sc, int which, int mode, int maxit, double tol, const double *part, int nb)
-{
-    if (which == 0) {
-        double rz = final_sum(part, nb, 0, false);
-        double rr = final_sum(part, nb, 1, false);
-        if (threadIdx.x == 0) {
-            sc->p_gamma = rz;
-            sc->p_iter = 0;
-            sc->p_done = 0;
-            if (mode == 0) {
-                sc->p_res = sqrt(rz);
-                if (sqrt(rz) < tol) sc->p_done = 4;   // early return: no gauge (:182-185)
-            } else {
-                double bn = sqrt(rr);
-                sc->p_bnorm = (bn == 0.0) ? 1.0 : bn;
-                sc->p_res = sqrt(rr) / sc->p_bnorm;
-                if (sc->p_res <= tol) sc->p_done = 1;
-            }
-            if (maxit <= 0 && !sc->p_done) sc->p_done = 3;
-        }
-        return;
-    }
-    if (sc->p_done) return;
-    if (which == 1) {
-        double dAd = final_sum(part, nb, 0, false);
-        if (threadIdx.x == 0) {
-            sc->p_alpha = (mode == 0) ? sc->p_gamma / (dAd + 1e-30) : sc->p_gamma / dAd;
-            sc->p_iter += 1;
-        }
-        return;
-    }
-    if (which == 2) {
-        double rz = final_sum(part, nb, 0, false);
-        double rr = final_sum(part, nb, 1, false);
-        if (threadIdx.x == 0) {
-            if (mode == 0) {
-                sc->p_res = sqrt(rz);
-                if (sqrt(rz) < tol) { sc->p_done = 1; return; }
-                sc->p_beta = rz / (sc->p_gamma + 1e-30);
-                sc->p_gamma = rz;
-            } else {
-                sc->p_res = sqrt(rr) / sc->p_bnorm;
-                if (sc->p_res <= tol) { sc->p_done = 1; return; }
-            }
-            if (sc->p_iter >= maxit) sc->p_done = 3;
-        }
-        return;
-    }
-    // which == 3: gamma_new = <r, z> with z from the FFT preconditioner;
-    // which == 4: first gamma = <r, z>, beta = 0 (so d = z)
-    double rz = final_sum(part, nb, 0, false);
-    if (threadIdx.x == 0) {
-        sc->p_beta = (which == 4) ? 0.0 : rz / sc->p_gamma;
-        sc->p_gamma = rz;
-    }
-}
-extern "C" void pvk_p_scalar2(const pvk_grid *g, pvk_scal *sc, int which, int mode, int maxit, double tol,
-                              const pvk_red *rd, int nb, hipStream_t s)
-{
-    (void)g;
-    hipLaunchKernelGGL(k_p_scalar, dim3(1), dim3(256), 0, s, sc, which, mode, maxit, tol, rd->part,
-                       nb > 0 ? nb : rd->nblocks);
-}
-
 // partial <a, b> over cells (i < NXM, j < NYM)
 __global__ void k_dot(pvk_grid g, const double *a, const double *b, double *part, int nb)
 {

@@ -806,6 +806,128 @@ extern "C" void pvk_pcg_apply(const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w,
     hipLaunchKernelGGL(k_pcg_apply, dim3(g->NYM), dim3(NTH), 0, s, *g, sc, *w, n);
 }
 
+// ---------------------------------------------------------------------------
+// Jacobi-PCG (psolve_cg.c:130-293): the reference's recurrences, absolute
+// stop sqrt(<r, z>) < tol, its early return without iterations (flag 4) and
+// EPS = 1e-30 in both step lengths.  Two launches an iteration, one block a
+// row: the apply kernel takes the stop test and beta from the previous
+// partials and forms d_n = z + beta d_{n-1} at the stencil points, the
+// update kernel forms the step, r and z = M r.  A form with one launch for
+// each of the ghost fill, operator, update, direction and two scalar steps
+// took 23.7 us an iteration at 128 x 256, where each launch is ~3 us of
+// latency; this one takes 9.8 (two RK3 steps 109 -> 64 ms).
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(NTH) k_jac_start(pvk_grid g, pvk_scal *sc, pvk_pcg w, const double *__restrict__ M)
+{
+    __shared__ double sh[NTH];
+    const int P = g.P, NXM = g.NXM, j = blockIdx.x;
+    if (j == 0 && threadIdx.x == 0) { sc->p_done = 0; sc->p_iter = 0; }
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < NXM; i += NTH) {
+        const double r = AT(w.rhs, i, j), z = r * AT(M, i, j);
+        AT(w.phi, i, j) = 0.0;
+        AT(w.r, i, j) = r;
+        AT(w.z, i, j) = z;
+        acc += r * z;
+    }
+    block_store_partial(acc, w.rz[0], j, sh);
+}
+
+// ONE: rows of at most NTH cells, one a thread; its loads go out before the
+// scalar sums are waited for (wider rows would hold too many at once)
+template <bool ONE>
+__global__ void __launch_bounds__(NTH) k_jac_apply(pvk_grid g, pvk_scal *sc, pvk_pcg w, int n, double tol, int maxit)
+{
+    __shared__ double sh[2 * NTH];
+    const int P = g.P, NXM = g.NXM, NYM = g.NYM, j = xcd_band(blockIdx.x, gridDim.x);
+    const int jn = (j + 1 == NYM) ? j : j + 1, js = (j == 0) ? 0 : j - 1;
+    const double *__restrict__ z = w.z, *__restrict__ dold = w.d[(n + 1) & 1];
+    const double *__restrict__ bx = w.bx, *__restrict__ by = w.by;
+    double zv[5], dv[5], cv[4];
+    auto load = [&](int i) {
+        const int ie = (i + 1 == NXM) ? 0 : i + 1, iw = (i == 0) ? NXM - 1 : i - 1;
+        zv[0] = AT(z, i, j);  zv[1] = AT(z, ie, j); zv[2] = AT(z, iw, j); zv[3] = AT(z, i, jn); zv[4] = AT(z, i, js);
+        if (n > 0) {
+            dv[0] = AT(dold, i, j);  dv[1] = AT(dold, ie, j); dv[2] = AT(dold, iw, j);
+            dv[3] = AT(dold, i, jn); dv[4] = AT(dold, i, js);
+        }
+        cv[0] = AT(bx, i, j); cv[1] = AT(bx, i - 1, j); cv[2] = AT(by, i, j); cv[3] = AT(by, i, j - 1);
+    };
+    if (ONE) load(min((int)threadIdx.x, NXM - 1));
+    if (sc->p_done) return;
+    double rz, rzo = 0.0, beta = 0.0;
+    if (n > 0) block_sum2(w.rz[n & 1], w.nrz, w.rz[(n + 1) & 1], w.nrz, sh, rz, rzo);
+    else rz = block_sum(w.rz[0], w.nrz, sh);
+    const double res = sqrt(rz);
+    const int stop = (res < tol) ? (n == 0 ? 4 : 1) : (n >= maxit ? 3 : 0);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc->p_res = res;
+        sc->p_iter = n;
+        if (stop) sc->p_done = stop;
+    }
+    if (stop) return;
+    if (n > 0) beta = rz / (rzo + 1e-30);
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < NXM; i += NTH) {
+        if (!ONE) load(i);
+        double d[5];
+#pragma unroll
+        for (int k = 0; k < 5; k++) d[k] = (n > 0) ? zv[k] + beta * dv[k] : zv[k];
+        const double ad = cv[0] * (d[1] - d[0]) - cv[1] * (d[0] - d[2]) + cv[2] * (d[3] - d[0]) - cv[3] * (d[0] - d[4]);
+        AT(w.d[n & 1], i, j) = d[0];
+        AT(w.Ad, i, j) = ad;
+        acc += d[0] * ad;
+    }
+    block_store_partial(acc, w.dad[0], j, sh);
+}
+
+template <bool ONE>
+__global__ void __launch_bounds__(NTH) k_jac_update(pvk_grid g, const pvk_scal *sc, pvk_pcg w, const double *__restrict__ M,
+                                                    int n)
+{
+    __shared__ double sh[2 * NTH];
+    const int P = g.P, NXM = g.NXM, j = xcd_band(blockIdx.x, gridDim.x);
+    const double *__restrict__ d = w.d[n & 1], *__restrict__ Ad = w.Ad;
+    double ph, dd, rr, aa, mm;
+    auto load = [&](int i) {
+        ph = AT(w.phi, i, j); dd = AT(d, i, j); rr = AT(w.r, i, j); aa = AT(Ad, i, j); mm = AT(M, i, j);
+    };
+    if (ONE) load(min((int)threadIdx.x, NXM - 1));
+    if (sc->p_done) return;
+    double rz, dad;
+    block_sum2(w.rz[n & 1], w.nrz, w.dad[0], w.ndad, sh, rz, dad);
+    const double alpha = rz / (dad + 1e-30);
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < NXM; i += NTH) {
+        if (!ONE) load(i);
+        const double r = rr - alpha * aa, z = r * mm;
+        AT(w.phi, i, j) = ph + alpha * dd;
+        AT(w.r, i, j) = r;
+        AT(w.z, i, j) = z;
+        acc += r * z;
+    }
+    block_store_partial(acc, w.rz[(n + 1) & 1], j, sh);
+}
+
+extern "C" void pvk_jac_start(const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w, const double *M, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_pcg_faces, dim3(g->NYM + 1), dim3(NTH), 0, s, *g, *w);
+    hipLaunchKernelGGL(k_jac_start, dim3(g->NYM), dim3(NTH), 0, s, *g, sc, *w, M);
+}
+
+extern "C" void pvk_jac_iter(const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w, const double *M, int half, int n, double tol,
+                             int maxit, hipStream_t s)
+{
+    const dim3 gr(g->NYM);
+    if (half == 0) {
+        if (g->NXM <= NTH) hipLaunchKernelGGL(k_jac_apply<true>, gr, dim3(NTH), 0, s, *g, sc, *w, n, tol, maxit);
+        else hipLaunchKernelGGL(k_jac_apply<false>, gr, dim3(NTH), 0, s, *g, sc, *w, n, tol, maxit);
+    } else {
+        if (g->NXM <= NTH) hipLaunchKernelGGL(k_jac_update<true>, gr, dim3(NTH), 0, s, *g, (const pvk_scal *)sc, *w, M, n);
+        else hipLaunchKernelGGL(k_jac_update<false>, gr, dim3(NTH), 0, s, *g, (const pvk_scal *)sc, *w, M, n);
+    }
+}
+
 // stage: 0 = K1 apply, 1 = K2 update + forward rows, 2 = K3 check + transpose,
 // 3 = K4 column DCTs, 4 = K5 transpose back, 5 = K6 inverse rows + <r, z>,
 // 6 = K4' check + tridiagonal y solves in place (replaces 2..4 for the

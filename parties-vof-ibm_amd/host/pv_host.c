@@ -274,7 +274,8 @@ static int create_on_device(pv_bag *b, const pv_params *prm)
     }
 }
 
-/* Work sets of the fused biharmonic and momentum CG loops: one band of rows
+/* Work sets of the fused biharmonic, momentum and Jacobi pressure CG loops (the
+ * last with one block and partial a row): one band of rows
  * per 256-thread block (1 row for the biharmonic CG, 1, 2 or 4 rows for the
  * momentum CG: 2 unless pv_set_momentum_rows says otherwise), one
  * partial-sum slot per band and reduction (sized for one-row bands). */
@@ -285,7 +286,7 @@ int pv_cg_create(pv_bag *b)
     int nbc = (ny + band - 1) / band, nbu = ny, nbv = ny - 1, c;
     int npap = ((ny + 7) / 8) * ((nx + 127) / 128);
     int nt0 = ((ny + 15) / 16) * ((nx + 63) / 64), nbs = (nt0 > nbc) ? nt0 : nbc;   /* start partials */
-    size_t n = 2 * (size_t)nbs + (size_t)nbc + (size_t)npap + 4 * (size_t)nbu + 4 * (size_t)nbv;
+    size_t n = 2 * (size_t)nbs + (size_t)nbc + (size_t)npap + 4 * (size_t)nbu + 4 * (size_t)nbv + 3 * (size_t)ny;
     double *q;
     HIPCHK(hipMalloc((void **)&b->cgmem, sizeof(double) * n));
     HIPCHK(hipMemset(b->cgmem, 0, sizeof(double) * n));
@@ -299,6 +300,15 @@ int pv_cg_create(pv_bag *b)
     b->ccg.rr[1] = q; q += nbc;
     b->ccg.pap = q; q += npap;
     b->ccg.npap = npap;
+    memset(&b->jac, 0, sizeof b->jac);
+    b->jac.rz[0] = q; q += ny;
+    b->jac.rz[1] = q; q += ny;
+    b->jac.dad[0] = q; q += ny;
+    b->jac.nrz = b->jac.ndad = ny;
+    b->jac.phi = b->f[PV_F_PHI]; b->jac.r = b->f[PV_F_P_RES]; b->jac.z = b->f[PV_FI_Z];
+    b->jac.d[0] = b->f[PV_F_P_D]; b->jac.d[1] = b->f[PV_FI_D2]; b->jac.Ad = b->f[PV_F_P_AD];
+    b->jac.rhs = b->f[PV_F_P_RHS]; b->jac.rho = b->f[PV_F_RHO];
+    b->jac.bx = b->f[PV_FI_PBX]; b->jac.by = b->f[PV_FI_PBY];
     memset(&b->mcg, 0, sizeof b->mcg);
     b->mcg.band = mband;
     b->mcg.rho = b->f[PV_F_RHO]; b->mcg.mu = b->f[PV_F_MU];

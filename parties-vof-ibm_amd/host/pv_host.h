@@ -105,6 +105,7 @@ struct pv_bag {
     double *fftmem;
     pvk_pcg pcg;
     double *pcgmem;
+    pvk_pcg jac;                   /* CG work set of the Jacobi-PCG */
     pvk_mg mg, mgf;                /* multigrid preconditioner, FP64 and FP32 V-cycle (mg_ok) */
     pvk_mg *mgp;                   /* the one in use */
     pvk_pcg mgw;                   /* CG work set of the MG-PCG: fields + its own partials */

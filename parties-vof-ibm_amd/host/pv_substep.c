@@ -421,36 +421,33 @@ int pv_Pressure_apply_BCs(pv_bag *b, int field)
 /* Jacobi-PCG (psolve_cg.c:130-293); phi starts at zero. */
 static int p_solve_jacobi(pv_bag *b)
 {
-    double *phi = FD(b, PV_F_PHI), *rhs = FD(b, PV_F_P_RHS), *r = FD(b, PV_F_P_RES), *d = FD(b, PV_F_P_D);
-    double *Ad = FD(b, PV_F_P_AD), *M = FD(b, PV_F_M_INV);
-    int maxit = b->ph.P_CG_MAXIT, chunk = b->p_chunk, total = 0;
+    const double *M = FD(b, PV_F_M_INV);
+    int maxit = b->ph.P_CG_MAXIT, chunk = b->p_chunk, n = 0, last;
     double tol = b->ph.P_CG_ETOL;
-    pvk_p_cg_init2(G(b), rhs, M, phi, r, d, 1, 0, b->d_sc, &b->rd, S(b));
-    pvk_p_scalar2(G(b), b->d_sc, 0, 0, maxit, tol, &b->rd, 0, S(b));
+    pvk_jac_start(G(b), b->d_sc, &b->jac, M, S(b));
     for (;;) {
         int k;
-        for (k = 0; k < chunk; k++) {
-            pvk_p_bc(G(b), d, S(b));
+        for (k = 0; k < chunk; k++, n++) {
             pv_tbegin(b, PV_T_P_APPLY);
-            pvk_p_cg_apply(G(b), b->d_sc, FD(b, PV_F_RHO), d, Ad, &b->rd, S(b));
+            pvk_jac_iter(G(b), b->d_sc, &b->jac, M, 0, n, tol, maxit, S(b));
             pv_tend(b, PV_T_P_APPLY);
-            pvk_p_scalar2(G(b), b->d_sc, 1, 0, maxit, tol, &b->rd, 0, S(b));
             pv_tbegin(b, PV_T_P_UPDATE);
-            pvk_p_cg_update(G(b), b->d_sc, phi, d, r, Ad, M, 1, &b->rd, S(b));
+            pvk_jac_iter(G(b), b->d_sc, &b->jac, M, 1, n, tol, maxit, S(b));
             pv_tend(b, PV_T_P_UPDATE);
-            pvk_p_scalar2(G(b), b->d_sc, 2, 0, maxit, tol, &b->rd, 0, S(b));
-            pv_tbegin(b, PV_T_P_DUPDATE);
-            pvk_p_cg_dupdate(G(b), b->d_sc, r, M, 1, d, S(b));
-            pv_tend(b, PV_T_P_DUPDATE);
         }
         LAUNCHCHK();
-        total += chunk;
         RC(pv_read_scalars(b));
         if (b->h_sc->p_done) break;
-        if (total > maxit + 16) return pv_set_error(PV_EHIP, "pressure CG did not stop (device flag)");
+        if (n > maxit + 16) return pv_set_error(PV_EHIP, "pressure CG did not stop (device flag)");
         chunk = 4;
     }
     b->p_chunk = (b->h_sc->p_iter > 4) ? b->h_sc->p_iter - 2 : 4;
+    /* the public direction field holds the last direction (z without iterations) */
+    last = b->h_sc->p_iter - 1;
+    if (last < 0) pvk_learn_copy(G(b), b->jac.z, FD(b, PV_F_P_D), S(b));
+    else if (last & 1) pvk_learn_copy(G(b), b->jac.d[1], FD(b, PV_F_P_D), S(b));
+    pvk_p_bc(G(b), FD(b, PV_F_P_D), S(b));
+    LAUNCHCHK();
     return PV_OK;
 }
 
