@@ -166,6 +166,9 @@ void pvk_p_bc(const pvk_grid *g, double *f, hipStream_t s);          /* Pressure
 void pvk_ghost_multi(const pvk_grid *g, double *f0, double *f1, double *f2, double *f3, int nf, int kind,
                      hipStream_t s);
 void pvk_fill(double *f, size_t n, double val, hipStream_t s);
+/* rows j0 .. j0 + nrow - 1 of the NYM + 7 canonical rows of a field, to or from a compact buffer */
+void pvk_pack_rows(const pvk_grid *g, const double *f, int j0, int nrow, double *buf, hipStream_t s);
+void pvk_unpack_rows(const pvk_grid *g, double *f, int j0, int nrow, const double *buf, hipStream_t s);
 void pvk_copy(const pvk_grid *g, const double *src, double *dst, hipStream_t s);
 
 /* ---- Cahn-Hilliard ---- */

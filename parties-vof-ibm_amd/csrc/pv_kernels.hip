@@ -271,6 +271,37 @@ extern "C" void pvk_mom_warm(const pvk_grid *g, int mode, double scale, double *
     hipLaunchKernelGGL(k_mom_warm, gr, dim3(BX, BY), 0, s, *g, mode, scale, u, v, su, sv, du, dv);
 }
 
+// Rows j0 .. j0 + n / w - 1 (w = NXM + 7 values each) of a field, counted
+// from its first ghost row, to or from a compact buffer in pinned host memory:
+// consecutive lanes touch consecutive words of the buffer, so the transfer
+// over the bus is whole lines both ways.
+__global__ void __launch_bounds__(256) k_pack_rows(const double *__restrict__ f, int P, int w, unsigned n, double *__restrict__ buf)
+{
+    for (unsigned q = blockIdx.x * 256 + threadIdx.x; q < n; q += gridDim.x * 256) {
+        const unsigned j = q / (unsigned)w;
+        buf[q] = f[(size_t)j * P + (q - j * w)];
+    }
+}
+__global__ void __launch_bounds__(256) k_unpack_rows(double *__restrict__ f, int P, int w, unsigned n, const double *__restrict__ buf)
+{
+    for (unsigned q = blockIdx.x * 256 + threadIdx.x; q < n; q += gridDim.x * 256) {
+        const unsigned j = q / (unsigned)w;
+        f[(size_t)j * P + (q - j * w)] = buf[q];
+    }
+}
+extern "C" void pvk_pack_rows(const pvk_grid *g, const double *f, int j0, int nrow, double *buf, hipStream_t s)
+{
+    const unsigned w = g->NXM + 7, n = w * (unsigned)nrow, nb = (n + 255) / 256;
+    hipLaunchKernelGGL(k_pack_rows, dim3(nb < 1024 ? nb : 1024), dim3(256), 0, s, f + (ptrdiff_t)(j0 - 3) * g->P - 3, g->P,
+                       (int)w, n, buf);
+}
+extern "C" void pvk_unpack_rows(const pvk_grid *g, double *f, int j0, int nrow, const double *buf, hipStream_t s)
+{
+    const unsigned w = g->NXM + 7, n = w * (unsigned)nrow, nb = (n + 255) / 256;
+    hipLaunchKernelGGL(k_unpack_rows, dim3(nb < 1024 ? nb : 1024), dim3(256), 0, s, f + (ptrdiff_t)(j0 - 3) * g->P - 3, g->P,
+                       (int)w, n, buf);
+}
+
 __global__ void k_fill(double *f, size_t n, double val)
 {
     size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;

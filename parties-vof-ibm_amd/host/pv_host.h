@@ -85,6 +85,9 @@ struct pv_bag {
     pvk_scal *d_sc;                /* device scalars */
     pvk_scal *h_sc;                /* pinned host mirror */
     hipStream_t stream;
+    double *xfer[2];               /* pinned staging of field transfers (made at the first one) */
+    hipEvent_t xfer_ev[2];
+    unsigned xfer_k;
     /* host view of the time state */
     double time, dt, dt_old;
     int stage, ntime, time_nonzero;

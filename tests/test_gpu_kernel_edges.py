@@ -60,3 +60,23 @@ def test_in_workgroup_levels(lib, nx, ny, nu, w, fp32):
     c0 = next(i for i, sz in enumerate(sizes) if sz[0] * sz[1] <= mg_ref.LDS_CELLS)
     zr = mg_ref.vcycle(lv, G, f, nu, wl=tuple(range(c0, min(c0 + w, len(lv) - 1))))
     assert relerr(z, zr) < (1e-5 if fp32 else 1e-11)
+
+
+# one row of a buffer's worth left over, exactly one buffer (2048-value rows,
+# 128 of them), one row more, and many buffers
+@pytest.mark.parametrize("nx,ny", [(8, 8), (1000, 300), (2041, 121), (2041, 122), (3001, 700)])
+def test_field_transfers(lib, nx, ny):
+    """Fields set and read back through the staged transfers, ghosts
+    included, bit for bit; two sets in a row do not overtake each other, and
+    a missing array is an error."""
+    p = params(nx, ny, pressure_solver=pvof.PV_PSOLVE_JACOBI_PCG)
+    s = pvof.Solver(p, lib)
+    rng = np.random.default_rng(nx + ny)
+    a, b = rng.standard_normal(s.shape), rng.standard_normal(s.shape)
+    for _ in range(2):
+        s.set("U", a)
+        s.set("V", b)
+        assert np.array_equal(s.get("U"), a) and np.array_equal(s.get("V"), b)
+        a, b = b, a
+    null = C.POINTER(C.c_double)()
+    assert lib.pv_get_field(s.h, pvof.F["U"], null) != 0 and lib.pv_set_field(s.h, pvof.F["U"], null) != 0
