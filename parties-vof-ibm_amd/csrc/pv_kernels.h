@@ -74,10 +74,12 @@ typedef struct pvk_fft {
     const double *wx, *wy;    /* (cos, -sin)(2 pi t / M), t < M: exp(-2 pi i t / M) */
     double *spec;             /* NXM * NYM spectral scratch, row-major */
     /* tridiagonal solves along y on the columns of spec (csrc/pv_pcg.hip,
-     * k_tri_cols): row coefficients as_j, an_j (psolve_fft.c:467-591), the
-     * modified wavenumber of each halfcomplex column, and the launch shape
-     * (tri_kw columns x tri_s segments of tri_l rows per block) */
-    const double *tri_as, *tri_an, *tri_mw;
+     * k_tri_cols; coefficients of psolve_fft.c:467-591 on the uniform grid):
+     * q, K, q^NYM and 1 / (1 - q^(2 NYM)) of each halfcomplex column, 1 / c,
+     * and the launch shape (tri_kw columns x tri_s segments of tri_l rows per
+     * block) */
+    const double *tri_q, *tri_k, *tri_qn, *tri_den;
+    double tri_ic;
     int tri_kw, tri_lkw, tri_s, tri_l;
 } pvk_fft;
 

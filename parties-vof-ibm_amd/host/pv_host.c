@@ -556,9 +556,10 @@ static int xlen_ok(int n)
  * of rows rows per thread (at most 16, the registers a thread keeps per
  * row; 0 = 8) and cols columns per block (a power of two; 0 = 2, or more
  * where a block would hold less than a wavefront; halved while the block
- * would exceed 512 threads).  The kernel is latency-bound (a chain of FP64 divisions per
- * segment): short segments and many blocks (512 at 1024 columns) run
- * fastest -- 20.6 us at 1024^2 against 25.1 us for 16 rows and 8 columns.
+ * would exceed 512 threads).  Short segments and many blocks (512 at 1024
+ * columns) are near the fastest at every size tried: 10.2 us at 1024^2 (9.9 for
+ * 16 rows and 4 columns, 14.7 for 8 and 1, 12.2 for 4 and 4), 8.3 us at 768 x
+ * 491 (7.9, 9.1, 9.9) and 6.0 us at 128 x 256 (6.5, 6.3, 7.3).
  * The blocks of one XCD take neighbouring columns, so each row's cache lines
  * come from HBM once per XCD.  Nonzero if no shape fits. */
 static int tri_shape(pv_bag *b, int rows, int cols)
@@ -617,7 +618,7 @@ int pv_fft_create(pv_bag *b)
     n_rtx = 2 * (size_t)(nx / 2 + 1); n_rty = 2 * (size_t)(ny / 2 + 1);
     n_dct = 2 * (size_t)ny;
     n_wx = 2 * (size_t)(nx / 2); n_wy = 2 * (size_t)(ny / 2);
-    total = n_rtx + n_rty + n_dct + nx + ny + n_wx + n_wy + 2 * (size_t)ny + nx;
+    total = n_rtx + n_rty + n_dct + nx + ny + n_wx + n_wy + 4 * (size_t)nx;
     h = (double *)calloc(total, sizeof(double));
     if (!h) return pv_set_error(PV_ENOMEM, "FFT table allocation failed");
     q = h;
@@ -643,16 +644,22 @@ int pv_fft_create(pv_bag *b)
     q += n_wx;
     for (k = 0; k < ny / 2; k++) { double a = 2.0 * PI_ * k / (ny / 2); q[2 * k] = cos(a); q[2 * k + 1] = -sin(a); }
     q += n_wy;
-    /* y tridiagonals of psolve_fft.c:467-591 (Neumann walls: as_0 = 0,
-     * an_{NYM-1} = 0) and the modified wavenumber of each halfcomplex column
-     * (:577-583, idx = idx_u[0]) */
-    for (k = 0; k < ny; k++) q[k] = (k > 0) ? b->hm.idy_v[k + 3] * b->hm.idy_c[k + 2] : 0.0;
-    q += ny;
-    for (k = 0; k < ny; k++) q[k] = (k < ny - 1) ? b->hm.idy_v[k + 3] * b->hm.idy_c[k + 3] : 0.0;
-    q += ny;
-    for (k = 0; k < nx; k++) {
-        int wave = (k < nx / 2) ? k : (nx - k);
-        q[k] = 2.0 * (1 - cos(2. * PI_ * wave / (nx))) * (b->hm.idx_u[3] * b->hm.idx_u[3]);
+    /* y tridiagonals of psolve_fft.c:467-591 (Neumann walls) on the uniform
+     * grid, c = idy_v idy_c, with the modified wavenumber of each halfcomplex
+     * column (:577-583, idx = idx_u[0]): 2 cosh(theta) = 2 + mw / c, q =
+     * exp(-theta), q / (1 - q^2) = 1 / (2 sinh(theta)) */
+    {
+        const double c = b->hm.idy_v[3] * b->hm.idy_c[3];
+        for (k = 0; k < nx; k++) {
+            int wave = (k < nx / 2) ? k : (nx - k);
+            double m = 2.0 * (1 - cos(2. * PI_ * wave / (nx))) * (b->hm.idx_u[3] * b->hm.idx_u[3]) / c;
+            double th = 2.0 * asinh(0.5 * sqrt(m));
+            q[k] = exp(-th);
+            q[nx + k] = (k > 0) ? 1.0 / (2.0 * sinh(th)) / c : 0.0;      /* column 0: a case of its own */
+            q[2 * nx + k] = (k > 0) ? exp(-th * ny) : 0.0;
+            q[3 * nx + k] = (k > 0) ? -1.0 / expm1(-2.0 * th * ny) : 0.0;
+        }
+        b->fft.tri_ic = 1.0 / c;
     }
     if (tri_shape(b, 0, 0)) { free(h); return PV_OK; }
     if (hipMalloc((void **)&d, sizeof(double) * (total + (size_t)nx * ny)) != hipSuccess) {
@@ -706,9 +713,10 @@ int pv_fft_create(pv_bag *b)
     b->fft.lamy = q; q += ny;
     b->fft.wx = q; q += n_wx;
     b->fft.wy = q; q += n_wy;
-    b->fft.tri_as = q; q += ny;
-    b->fft.tri_an = q; q += ny;
-    b->fft.tri_mw = q; q += nx;
+    b->fft.tri_q = q; q += nx;
+    b->fft.tri_k = q; q += nx;
+    b->fft.tri_qn = q; q += nx;
+    b->fft.tri_den = q; q += nx;
     b->fft.spec = q;
     b->fft.ok = 1;
     return PV_OK;
