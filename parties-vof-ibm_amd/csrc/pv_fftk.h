@@ -21,6 +21,17 @@
 
 #define SK_SQRT_HALF 0.70710678118654752440
 
+// Where element i of a transform lies in LDS.  Flat: at i.  Padded: one slot
+// is left after every eight elements, so the stride-8 stores of the first
+// radix-8 pass (and the 64-element jumps of the second) spread over all banks
+// instead of one double in sixteen.
+struct SkFlat {
+    static __host__ __device__ __forceinline__ int at(int i) { return i; }
+};
+struct SkPad {
+    static __host__ __device__ __forceinline__ int at(int i) { return i + (i >> 3); }
+};
+
 // (x + i y) times -i (forward) or +i (inverse)
 template <bool INV>
 __host__ __device__ __forceinline__ void sk_rot(double &x, double &y)
@@ -83,7 +94,7 @@ __host__ __device__ __forceinline__ void sk_dft8(double *vr, double *vi)
 // Read butterfly bb of a radix-R pass (R = 2^LR), twiddle, DFT: v[0..R).
 // All sizes are powers of two and passed as base-2 logarithms, so index
 // arithmetic is shifts and masks.
-template <int LR, bool INV>
+template <int LR, bool INV, class IX = SkFlat>
 __host__ __device__ __forceinline__ void sk_load(const double *sr, const double *si, int bb, int logM, int logNs,
                                                  const double *tw, double *vr, double *vi)
 {
@@ -91,8 +102,8 @@ __host__ __device__ __forceinline__ void sk_load(const double *sr, const double 
     const int stride = 1 << (logM - LR), k = bb & ((1 << logNs) - 1), step = k << (logM - logNs - LR);
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        vr[r] = sr[bb + r * stride];
-        vi[r] = si[bb + r * stride];
+        vr[r] = sr[IX::at(bb + r * stride)];
+        vi[r] = si[IX::at(bb + r * stride)];
     }
     if (logNs > 0) {
 #pragma unroll
@@ -109,7 +120,7 @@ __host__ __device__ __forceinline__ void sk_load(const double *sr, const double 
     else sk_dft2<INV>(vr, vi, 0, 1);
 }
 
-template <int LR>
+template <int LR, class IX = SkFlat>
 __host__ __device__ __forceinline__ void sk_store(double *sr, double *si, int bb, int logNs, const double *vr,
                                                   const double *vi)
 {
@@ -118,14 +129,14 @@ __host__ __device__ __forceinline__ void sk_store(double *sr, double *si, int bb
     const int base = ((bb >> logNs) << (logNs + LR)) + (bb & (Ns - 1));
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        sr[base + r * Ns] = vr[r];
-        si[base + r * Ns] = vi[r];
+        sr[IX::at(base + r * Ns)] = vr[r];
+        si[IX::at(base + r * Ns)] = vi[r];
     }
 }
 
 // One radix-R pass over a transform whose T threads have lane ids 0..T-1;
 // every thread of the block calls it (barriers inside).  bb >= M / R idle.
-template <int LR, bool INV>
+template <int LR, bool INV, class IX = SkFlat>
 __device__ __forceinline__ void sk_pass(double *sr, double *si, int logM, int logNs, const double *tw, int lane,
                                         int T)
 {
@@ -135,13 +146,13 @@ __device__ __forceinline__ void sk_pass(double *sr, double *si, int logM, int lo
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const int bb = lane + u * T;
-        if (bb < nbf) sk_load<LR, INV>(sr, si, bb, logM, logNs, tw, vr + (u << LR), vi + (u << LR));
+        if (bb < nbf) sk_load<LR, INV, IX>(sr, si, bb, logM, logNs, tw, vr + (u << LR), vi + (u << LR));
     }
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const int bb = lane + u * T;
-        if (bb < nbf) sk_store<LR>(sr, si, bb, logNs, vr + (u << LR), vi + (u << LR));
+        if (bb < nbf) sk_store<LR, IX>(sr, si, bb, logNs, vr + (u << LR), vi + (u << LR));
     }
     __syncthreads();
 }
@@ -155,6 +166,21 @@ __device__ __forceinline__ void sk_fft(double *sr, double *si, int logM, const d
     for (; rem >= 3; rem -= 3, logNs += 3) sk_pass<3, INV>(sr, si, logM, logNs, tw, lane, T);
     if (rem == 2) sk_pass<2, INV>(sr, si, logM, logNs, tw, lane, T);
     else if (rem == 1) sk_pass<1, INV>(sr, si, logM, logNs, tw, lane, T);
+}
+
+// The same from a thread's eight values in registers, v[r] = x[lane + r T]: the
+// first radix-8 pass (no twiddles) needs no LDS read.  M >= 8.
+template <bool INV, class IX>
+__device__ __forceinline__ void sk_fft_regs(double *vr, double *vi, double *sr, double *si, int logM, const double *tw,
+                                            int lane, int T)
+{
+    sk_dft8<INV>(vr, vi);
+    sk_store<3, IX>(sr, si, lane, 0, vr, vi);
+    __syncthreads();
+    int logNs = 3, rem = logM - 3;
+    for (; rem >= 3; rem -= 3, logNs += 3) sk_pass<3, INV, IX>(sr, si, logM, logNs, tw, lane, T);
+    if (rem == 2) sk_pass<2, INV, IX>(sr, si, logM, logNs, tw, lane, T);
+    else if (rem == 1) sk_pass<1, INV, IX>(sr, si, logM, logNs, tw, lane, T);
 }
 
 // ---------------------------------------------------------------------------
@@ -181,15 +207,15 @@ __host__ __device__ __forceinline__ void sk_dft3(double *vr, double *vi)
     else     { vr[1] = tr + di; vi[1] = ti - dr; vr[2] = tr - di; vi[2] = ti + dr; }
 }
 
-template <int R, bool INV>
+template <int R, bool INV, class IX = SkFlat>
 __host__ __device__ __forceinline__ void sg_load(const double *sr, const double *si, int bb, int M, int Ns,
                                                  const double *tw, double *vr, double *vi)
 {
     const int stride = M / R, k = bb % Ns, step = (M / (Ns * R)) * k;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        vr[r] = sr[bb + r * stride];
-        vi[r] = si[bb + r * stride];
+        vr[r] = sr[IX::at(bb + r * stride)];
+        vi[r] = si[IX::at(bb + r * stride)];
     }
     if (Ns > 1) {
 #pragma unroll
@@ -207,19 +233,19 @@ __host__ __device__ __forceinline__ void sg_load(const double *sr, const double 
     else sk_dft2<INV>(vr, vi, 0, 1);
 }
 
-template <int R>
+template <int R, class IX = SkFlat>
 __host__ __device__ __forceinline__ void sg_store(double *sr, double *si, int bb, int Ns, const double *vr,
                                                   const double *vi)
 {
     const int k = bb % Ns, base = (bb / Ns) * Ns * R + k;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        sr[base + r * Ns] = vr[r];
-        si[base + r * Ns] = vi[r];
+        sr[IX::at(base + r * Ns)] = vr[r];
+        si[IX::at(base + r * Ns)] = vi[r];
     }
 }
 
-template <int R, bool INV>
+template <int R, bool INV, class IX = SkFlat>
 __device__ __forceinline__ void sg_pass(double *sr, double *si, int M, int Ns, const double *tw, int lane, int T,
                                         bool act)
 {
@@ -229,26 +255,30 @@ __device__ __forceinline__ void sg_pass(double *sr, double *si, int M, int Ns, c
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const int bb = lane + u * T;
-        if (act && bb < nbf) sg_load<R, INV>(sr, si, bb, M, Ns, tw, vr + u * R, vi + u * R);
+        if (act && bb < nbf) sg_load<R, INV, IX>(sr, si, bb, M, Ns, tw, vr + u * R, vi + u * R);
     }
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const int bb = lane + u * T;
-        if (act && bb < nbf) sg_store<R>(sr, si, bb, Ns, vr + u * R, vi + u * R);
+        if (act && bb < nbf) sg_store<R, IX>(sr, si, bb, Ns, vr + u * R, vi + u * R);
     }
     __syncthreads();
 }
 
-// Whole transform of length M = 2^a 3^b (8 | M)
-template <bool INV>
-__device__ __forceinline__ void sg_fft(double *sr, double *si, int M, const double *tw, int lane, int T, bool act)
+// Whole transform of length M = 2^a 3^b (8 | M), from registers as sk_fft_regs
+template <bool INV, class IX>
+__device__ __forceinline__ void sg_fft_regs(double *vr, double *vi, double *sr, double *si, int M, const double *tw, int lane,
+                                            int T, bool act)
 {
-    int Ns = 1, two = M;
-    while (two % 3 == 0) two /= 3;                   // the power-of-two part
-    for (; two % 8 == 0; two /= 8, Ns *= 8) sg_pass<8, INV>(sr, si, M, Ns, tw, lane, T, act);
-    if (two == 4) { sg_pass<4, INV>(sr, si, M, Ns, tw, lane, T, act); Ns *= 4; }
-    else if (two == 2) { sg_pass<2, INV>(sr, si, M, Ns, tw, lane, T, act); Ns *= 2; }
-    for (; Ns < M; Ns *= 3) sg_pass<3, INV>(sr, si, M, Ns, tw, lane, T, act);
+    int Ns = 8, two = M / 8;
+    while (two % 3 == 0) two /= 3;                   // the rest of the power-of-two part
+    sk_dft8<INV>(vr, vi);
+    if (act) sg_store<8, IX>(sr, si, lane, 1, vr, vi);
+    __syncthreads();
+    for (; two % 8 == 0; two /= 8, Ns *= 8) sg_pass<8, INV, IX>(sr, si, M, Ns, tw, lane, T, act);
+    if (two == 4) { sg_pass<4, INV, IX>(sr, si, M, Ns, tw, lane, T, act); Ns *= 4; }
+    else if (two == 2) { sg_pass<2, INV, IX>(sr, si, M, Ns, tw, lane, T, act); Ns *= 2; }
+    for (; Ns < M; Ns *= 3) sg_pass<3, INV, IX>(sr, si, M, Ns, tw, lane, T, act);
 }
 #endif

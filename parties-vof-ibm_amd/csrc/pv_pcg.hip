@@ -33,28 +33,30 @@ struct cplx2 { double x, y; };
 // (pv_fftk.h): M / 8 threads, at least one
 __device__ __forceinline__ int sk_logT(int logM) { return logM >= 3 ? logM - 3 : 0; }
 
-// X_k, k = 0..M, of a real length-2M sequence from Z = FFT_M(x_{2m} + i x_{2m+1})
-__device__ __forceinline__ cplx2 rpost(const double *sr, const double *si, int base, int M, int k, const double *rt)
+// X_k, k = 0..M, of a real length-2M sequence from Z = FFT_M(x_{2m} + i x_{2m+1}):
+// Z_k (k = M: Z_0), Z_{M-k} (k = 0, M: Z_0) and c, s = cos, sin of pi k / M
+__device__ __forceinline__ cplx2 rpost(double zr, double zi, double br, double bi, double c, double s)
 {
-    int ka = (k == M) ? 0 : k, kb = (k == 0 || k == M) ? 0 : M - k;
-    double zr = sr[base + ka], zi = si[base + ka];
-    double cr = sr[base + kb], ci = -si[base + kb];
+    double cr = br, ci = -bi;
     double er = 0.5 * (zr + cr), ei = 0.5 * (zi + ci);
     double dr = zr - cr, di = zi - ci;
     double or_ = 0.5 * di, oi = -0.5 * dr;
-    double c = rt[2 * k], s = rt[2 * k + 1];
     cplx2 X;
     X.x = er + (c * or_ + s * oi);
     X.y = ei + (c * oi - s * or_);
     return X;
 }
+__device__ __forceinline__ cplx2 rpost(const double *sr, const double *si, int base, int M, int k, const double *rt)
+{
+    const int ka = (k == M) ? 0 : k, kb = (k == 0 || k == M) ? 0 : M - k;
+    return rpost(sr[base + ka], si[base + ka], sr[base + kb], si[base + kb], rt[2 * k], rt[2 * k + 1]);
+}
 
 // Y_k from X_k and X_{M-k} for the half-length inverse
-__device__ __forceinline__ cplx2 rpre(cplx2 Xk, cplx2 Xmk, int k, const double *rt)
+__device__ __forceinline__ cplx2 rpre(cplx2 Xk, cplx2 Xmk, double c, double s)
 {
     double ar = Xk.x + Xmk.x, ai = Xk.y - Xmk.y;
     double dr = Xk.x - Xmk.x, di = Xk.y + Xmk.y;
-    double c = rt[2 * k], s = rt[2 * k + 1];
     double pr = dr * c - di * s, pi_ = dr * s + di * c;
     cplx2 Y;
     Y.x = ar - pi_;
@@ -62,38 +64,9 @@ __device__ __forceinline__ cplx2 rpre(cplx2 Xk, cplx2 Xmk, int k, const double *
     return Y;
 }
 
-__device__ __forceinline__ cplx2 hcget(const double *row, int N, int k)
-{
-    cplx2 X;
-    X.x = row[k];
-    X.y = (k == 0 || k == N / 2) ? 0.0 : row[N - k];
-    return X;
-}
-
-// row q and entry m of item t of a block's rows of M values
-__device__ __forceinline__ void row_split(int t, int M, int logM, bool p2, int &q, int &m)
-{
-    if (p2) { q = t >> logM; m = t & (M - 1); }
-    else { q = t / M; m = t - q * M; }
-}
-
-// the block's transforms of its R rows: power-of-two lengths by the
-// shift-indexed passes, 2^a 3^b lengths by the mixed-radix ones
-template <bool INV>
-__device__ __forceinline__ void rows_fft(double *sr, double *si, int M, int logM, bool p2, int R, const double *tw)
-{
-    if (p2) {
-        const int lT = sk_logT(logM), q = threadIdx.x >> lT;
-        sk_fft<INV>(sr + q * M, si + q * M, logM, tw, threadIdx.x & ((1 << lT) - 1), 1 << lT);
-    } else {
-        const int T = M >> 3, q = threadIdx.x / T;
-        sg_fft<INV>(sr + q * M, si + q * M, M, tw, threadIdx.x - q * T, T, q < R);
-    }
-}
-
-// Every FFT kernel handles R = 2048 / M rows of M complex points per block
+// The y transforms handle R = 2048 / M columns of M complex points per block
 // (T = M / 8 threads per transform, 256 threads), so each thread owns
-// IT = R * M / 256 = 8 items of the row sweeps; the sweeps load all of a
+// IT = R * M / 256 = 8 items of the sweeps; the sweeps load all of a
 // thread's items before storing any, so the loads are in flight together.
 #define IT 8
 #define CPT 4
@@ -186,111 +159,196 @@ __global__ void __launch_bounds__(NTH) k_pcg_apply(pvk_grid g, pvk_scal *sc, pvk
 // K2: alpha; phi, r update; <r,r>; forward real FFT of the r rows -> spec
 // (also the start kernel when n < 0: r = rhs - mean, phi = 0)
 // ---------------------------------------------------------------------------
-template <bool P2>
-__global__ void __launch_bounds__(NTH) k_pcg_update_fwd(pvk_grid g, pvk_fft F, pvk_scal *sc, pvk_pcg w, int n)
+//
+// The row kernels: T = M / 8 threads a row, each with the row's items lane +
+// u T, u < 8 (two cells an item, one 16-byte load), which are also what the
+// first radix-8 pass of its transform takes, so that pass runs on registers.
+// A block is NT threads: one wavefront (NT / T rows of it) where T <= 64, else
+// T.  Every load of the kernel (cells, twiddles, the split table) is
+// unconditional, from clamped places, and goes out before the stop flag and
+// the scalar sums are waited for; LDS is padded (SkPad).  With guarded loads,
+// the twiddles staged one by one and the split table read where it is used, a
+// chain of ~12 us of memory latency whatever the grid, the forward kernel
+// took 19.6 us and the inverse one 13.7 at 1024^2 (13.4 and 10.9 at 128 x 256);
+// now 15.0 and 8.7 (7.9 and 5.3).  One wavefront a block against 256 threads
+// (NT / T rows): 15.0 and 8.7 against 15.8 and 9.4 at 1024^2, 14.1 and 9.5
+// against 15.0 and 11.6 at 768 x 491, 7.9 and 5.3 against 9.9 and 7.0 at 128 x 256.
+#define RU 8
+#define TWK 8                    // twiddle pairs a thread stages: M <= 8 NT
+typedef double v2d __attribute__((ext_vector_type(2)));
+
+template <int NT> struct RowGeo {
+    int M, T, q, lane, j, LS;    // LS: LDS doubles of one row's real (or imaginary) part
+    bool act;
+};
+template <bool P2, int NT> __device__ __forceinline__ RowGeo<NT> row_geo(const pvk_grid &g, const pvk_fft &F, int R)
+{
+    RowGeo<NT> o;
+    o.M = F.mx;
+    o.T = o.M >> 3;
+    o.q = P2 ? (int)threadIdx.x >> (F.logmx - 3) : (int)threadIdx.x / o.T;
+    o.lane = threadIdx.x - o.q * o.T;
+    o.LS = o.M + (o.M >> 3);
+    const int j = blockIdx.x * R + o.q;
+    o.act = o.q < R && j < g.NYM;
+    o.j = min(j, g.NYM - 1);
+    o.q = min(o.q, R - 1);
+    return o;
+}
+// this thread's share of the twiddle table, on its way to LDS
+template <int NT> __device__ __forceinline__ void tw_load(int M, const double *tw, v2d *v)
+{
+#pragma unroll
+    for (int k = 0; k < TWK; k++) v[k] = *(const v2d *)(tw + 2 * min((int)threadIdx.x + k * NT, M - 1));
+}
+template <int NT> __device__ __forceinline__ void tw_stage(int M, const v2d *v, double *lds)
+{
+#pragma unroll
+    for (int k = 0; k < TWK; k++) {
+        const int t = threadIdx.x + k * NT;
+        if (t < M) *(v2d *)(lds + 2 * t) = v[k];
+    }
+}
+// Sums of partials by a block of NT threads, the same order in every block:
+// the loads (16 a thread and array in flight; more partials than that are
+// added in a loop) and, later, the sums.
+#define RPB 16
+template <int NT> struct RowSums { double a[RPB], b[RPB]; };
+template <int NT> __device__ __forceinline__ void row_sums_load(const double *pa, int na, const double *pb, int nb, RowSums<NT> &v)
+{
+#pragma unroll
+    for (int k = 0; k < RPB; k++) {
+        const int b = threadIdx.x + k * NT;
+        v.a[k] = (b < na) ? pa[b] : 0.0;
+        v.b[k] = (b < nb) ? pb[b] : 0.0;
+    }
+}
+template <int NT> __device__ __forceinline__ void row_sums(const double *pa, int na, const double *pb, int nb,
+                                                           const RowSums<NT> &v, double *sh, double &ra, double &rb)
+{
+    const int t = threadIdx.x;
+    double sa = 0.0, sb = 0.0;
+#pragma unroll
+    for (int k = 0; k < RPB; k++) { sa += v.a[k]; sb += v.b[k]; }
+    for (int b = t + RPB * NT; b < na; b += NT) sa += pa[b];
+    for (int b = t + RPB * NT; b < nb; b += NT) sb += pb[b];
+    sa = lane_first(wave_sum(sa));
+    sb = lane_first(wave_sum(sb));
+    if (NT > 64) {
+        if ((t & 63) == 0) { sh[t >> 6] = sa; sh[8 + (t >> 6)] = sb; }
+        __syncthreads();
+        sa = sh[0];
+        sb = sh[8];
+        for (int w = 1; w < NT / 64; w++) { sa += sh[w]; sb += sh[8 + w]; }
+        __syncthreads();
+    }
+    ra = sa;
+    rb = sb;
+}
+template <int NT> __device__ __forceinline__ void row_partial(double v, double *part, double *sh)
+{
+    const int t = threadIdx.x;
+    v = wave_sum(v);
+    if (NT > 64) {
+        if ((t & 63) == 0) sh[t >> 6] = v;
+        __syncthreads();
+        for (int w = 1; t == 0 && w < NT / 64; w++) v += sh[w];
+    }
+    if (t == 0) part[blockIdx.x] = v;
+}
+template <bool INV, bool P2>
+__device__ __forceinline__ void rows_fft(double *vr, double *vi, double *sr, double *si, int M, int logM, const double *tw,
+                                         int lane, int T, bool act)
+{
+    if (P2) sk_fft_regs<INV, SkPad>(vr, vi, sr, si, logM, tw, lane, T);
+    else sg_fft_regs<INV, SkPad>(vr, vi, sr, si, M, tw, lane, T, act);
+}
+
+// MODE: the step of iteration n, the start (r = rhs - mean, phi = 0), a warm
+// restart (r = rhs - mean - A phi0, in Ad) or the transform of r as it is
+enum { ROW_STEP, ROW_START, ROW_WARM, ROW_PLAIN };
+template <bool P2, int NT, int MODE>
+__global__ void __launch_bounds__(NT) k_pcg_update_fwd(pvk_grid g, pvk_fft F, pvk_scal *sc, pvk_pcg w, int n)
 {
     extern __shared__ double lds[];
-    __shared__ double sh[2 * NTH];
-    if (w.chb == 0.0 && sc->p_done) return;
-    const int P = g.P, N = g.NXM, logM = F.logmx, M = F.mx, R = w.rrow, RM = R * M;
-    constexpr bool p2 = P2;     // power-of-two rows: shift-indexed passes
-    double *sr = lds, *si = lds + RM;
-    double *tw = stage_twiddles(lds, RM, M, F.wx);
-    const double *__restrict__ d = (n >= 0) ? w.d[n & 1] : w.rhs;
-    const double *__restrict__ Ad = w.Ad, *__restrict__ rhs = w.rhs;
+    __shared__ double sh[16];
+    const int P = g.P, N = g.NXM, R = w.rrow;
+    const RowGeo<NT> o = row_geo<P2, NT>(g, F, R);
+    const int M = o.M, T = o.T, lane = o.lane, j = o.j;
+    double *tw = lds, *sr = lds + 2 * M + 2 * o.q * o.LS, *si = sr + o.LS;
+    const double *pa = (MODE == ROW_STEP) ? w.rz[n & 1] : w.mean, *pb = w.dad[n & 1];
+    const int na = (MODE == ROW_STEP) ? w.nrz : (MODE == ROW_PLAIN ? 0 : w.nmean), nb = (MODE == ROW_STEP) ? w.ndad : 0;
+    const double *__restrict__ d = w.d[n & 1], *__restrict__ Ad = w.Ad;
+    const double *__restrict__ src = (MODE == ROW_STEP || MODE == ROW_PLAIN) ? w.r : w.rhs;
     double *__restrict__ phi = w.phi, *__restrict__ r = w.r;
-    const int j0 = blockIdx.x * R;
-    // the rows' loads go out before the scalar sums, whose partials and
-    // barriers would otherwise hold them back; the arithmetic is unchanged
-    double xa[IT], xb[IT], ea[IT], eb[IT], ra[IT], rb[IT], qa[IT], qb[IT];
+    RowSums<NT> ps;
+    v2d x[RU], e[RU], rv[RU], a[RU], rt[RU], tv[TWK];
+#define ROW2(f, u) (*(const v2d *)&AT(f, 2 * (lane + (u) * T), j))
+    if (MODE != ROW_PLAIN) row_sums_load<NT>(pa, na, pb, nb, ps);
 #pragma unroll
-    for (int u = 0; u < IT; u++) {
-        const int t = threadIdx.x + u * NTH;
-        int q, m;
-        row_split(t, M, logM, p2, q, m);
-        const int j = j0 + q, i = 2 * m;
-        xa[u] = xb[u] = ea[u] = eb[u] = ra[u] = rb[u] = qa[u] = qb[u] = 0.0;
-        if (t < RM && j < g.NYM) {
-            if (n >= 0) {
-                xa[u] = AT(phi, i, j); xb[u] = AT(phi, i + 1, j);
-                ea[u] = AT(d, i, j);   eb[u] = AT(d, i + 1, j);
-                ra[u] = AT(r, i, j);   rb[u] = AT(r, i + 1, j);
-                qa[u] = AT(Ad, i, j);  qb[u] = AT(Ad, i + 1, j);
-            } else if (n == -3) {               // M_fft of the current r, no update
-                ra[u] = AT(r, i, j);
-                rb[u] = AT(r, i + 1, j);
-            } else if (n == -2) {               // warm restart: Ad holds A phi0
-                xa[u] = AT(phi, i, j); xb[u] = AT(phi, i + 1, j);
-                ra[u] = AT(rhs, i, j);     rb[u] = AT(rhs, i + 1, j);
-                qa[u] = AT(Ad, i, j);      qb[u] = AT(Ad, i + 1, j);
-            } else {
-                ra[u] = AT(rhs, i, j);
-                rb[u] = AT(rhs, i + 1, j);
-            }
+    for (int u = 0; u < RU; u++) {
+        rv[u] = ROW2(src, u);
+        if (MODE == ROW_STEP || MODE == ROW_WARM) a[u] = ROW2(Ad, u);
+    }
+    tw_load<NT>(M, F.wx, tv);
+#pragma unroll
+    for (int u = 0; u < RU; u++) {
+        if (MODE == ROW_STEP) { x[u] = ROW2(phi, u); e[u] = ROW2(d, u); }
+        rt[u] = *(const v2d *)(F.rtx + 2 * (lane + u * T));
+    }
+    const v2d rtM = *(const v2d *)(F.rtx + 2 * M);
+    if (w.chb == 0.0 && sc->p_done) return;
+    double alpha = 0.0, mean = 0.0, s0, s1;
+    if (MODE != ROW_PLAIN) row_sums<NT>(pa, na, pb, nb, ps, sh, s0, s1);
+    if (MODE == ROW_STEP) alpha = s0 / s1;
+    else if (MODE != ROW_PLAIN) mean = s0 / ((double)g.NXM * (double)g.NYM);
+    tw_stage<NT>(M, tv, tw);
+    double vr[RU], vi[RU], acc = 0.0;
+#pragma unroll
+    for (int u = 0; u < RU; u++) {
+        if (MODE == ROW_STEP) {
+            rv[u].x = rv[u].x - alpha * a[u].x;
+            rv[u].y = rv[u].y - alpha * a[u].y;
+        } else if (MODE == ROW_WARM) {
+            rv[u].x = rv[u].x - mean - a[u].x;
+            rv[u].y = rv[u].y - mean - a[u].y;
+        } else if (MODE == ROW_START) {
+            rv[u].x = rv[u].x - mean;
+            rv[u].y = rv[u].y - mean;
+        }
+        vr[u] = rv[u].x;
+        vi[u] = rv[u].y;
+        if (o.act) acc += rv[u].x * rv[u].x + rv[u].y * rv[u].y;
+    }
+    if (o.act && MODE != ROW_PLAIN) {
+#pragma unroll
+        for (int u = 0; u < RU; u++) {
+            v2d *pp = (v2d *)&AT(phi, 2 * (lane + u * T), j);
+            if (MODE == ROW_STEP) {
+                v2d t;
+                t.x = x[u].x + alpha * e[u].x;
+                t.y = x[u].y + alpha * e[u].y;
+                *pp = t;
+            } else if (MODE == ROW_START) *pp = (v2d){0.0, 0.0};
+            *(v2d *)&AT(r, 2 * (lane + u * T), j) = rv[u];
         }
     }
-    double alpha = 0.0, mean = 0.0;
-    if (n >= 0) {
-        double srz, sdad;
-        block_sum2(w.rz[n & 1], w.nrz, w.dad[n & 1], w.ndad, sh, srz, sdad);
-        alpha = srz / sdad;
-    } else if (n != -3)
-        mean = block_sum(w.mean, w.nmean, sh) / ((double)g.NXM * (double)g.NYM);
-#pragma unroll
-    for (int u = 0; u < IT; u++) {
-        const int t = threadIdx.x + u * NTH;
-        int q, m;
-        row_split(t, M, logM, p2, q, m);
-        if (!(t < RM && j0 + q < g.NYM)) continue;
-        if (n >= 0) {
-            ra[u] = ra[u] - alpha * qa[u];
-            rb[u] = rb[u] - alpha * qb[u];
-        } else if (n == -2) {
-            ra[u] = ra[u] - mean - qa[u];
-            rb[u] = rb[u] - mean - qb[u];
-        } else if (n != -3) {
-            ra[u] = ra[u] - mean;
-            rb[u] = rb[u] - mean;
-        }
-    }
-    double acc = 0.0;
-#pragma unroll
-    for (int u = 0; u < IT; u++) {
-        const int t = threadIdx.x + u * NTH;
-        int q, m;
-        row_split(t, M, logM, p2, q, m);
-        const int j = j0 + q, i = 2 * m;
-        if (t < RM && j < g.NYM && n != -3) {
-            AT(phi, i, j) = (n >= 0) ? xa[u] + alpha * ea[u] : (n == -2 ? xa[u] : 0.0);
-            AT(phi, i + 1, j) = (n >= 0) ? xb[u] + alpha * eb[u] : (n == -2 ? xb[u] : 0.0);
-            AT(r, i, j) = ra[u];
-            AT(r, i + 1, j) = rb[u];
-        }
-        if (t < RM && j < g.NYM) acc += ra[u] * ra[u] + rb[u] * rb[u];
-        if (t < RM) { sr[t] = ra[u]; si[t] = rb[u]; }
-    }
-    block_store_partial(acc, w.rr, blockIdx.x, sh);
-    rows_fft<false>(sr, si, M, logM, p2, R, tw);
+#undef ROW2
+    __syncthreads();                            // twiddles staged
+    rows_fft<false, P2>(vr, vi, sr, si, M, F.logmx, tw, lane, T, o.act);
+    row_partial<NT>(acc, w.rr, sh);
     const double scale = 1.0 / (double)N;
-    // X_k, k < M (and X_M for each row below): halfcomplex row of spec
+    // X_k, k < M (and X_M): halfcomplex row of spec
+    double *row = F.spec + (size_t)j * N;
+    if (!o.act) return;
 #pragma unroll
-    for (int u = 0; u < IT; u++) {
-        const int t = threadIdx.x + u * NTH;
-        int q, k;
-        row_split(t, M, logM, p2, q, k);
-        const int j = j0 + q;
-        if (t < RM && j < g.NYM) {
-            cplx2 X = rpost(sr, si, q * M, M, k, F.rtx);
-            double *row = F.spec + (size_t)j * N;
-            row[k] = X.x * scale;
-            if (k > 0) row[N - k] = X.y * scale;
-        }
+    for (int u = 0; u < RU; u++) {
+        const int k = lane + u * T, kb = (k == 0) ? 0 : M - k;
+        const cplx2 X = rpost(sr[SkPad::at(k)], si[SkPad::at(k)], sr[SkPad::at(kb)], si[SkPad::at(kb)], rt[u].x, rt[u].y);
+        row[k] = X.x * scale;
+        if (k > 0) row[N - k] = X.y * scale;
     }
-    if ((int)threadIdx.x < R && j0 + (int)threadIdx.x < g.NYM) {
-        const int q = threadIdx.x;
-        cplx2 X = rpost(sr, si, q * M, M, M, F.rtx);
-        F.spec[(size_t)(j0 + q) * N + M] = X.x * scale;
-    }
+    if (lane == 0) row[M] = rpost(sr[0], si[0], sr[0], si[0], rtM.x, rtM.y).x * scale;
 }
 
 // ---------------------------------------------------------------------------
@@ -414,8 +472,8 @@ __global__ void __launch_bounds__(NTH) k_dct_rows(pvk_grid g, pvk_fft F, pvk_sca
             Xp[h].x = c * Cp + s * CNp;
             Xp[h].y = s * Cp - c * CNp;
         }
-        ya = rpre(Xp[0], Xp[1], k, F.rty);
-        yb = rpre(Xp[1], Xp[0], M - k, F.rty);
+        ya = rpre(Xp[0], Xp[1], F.rty[2 * k], F.rty[2 * k + 1]);
+        yb = rpre(Xp[1], Xp[0], F.rty[2 * (M - k)], F.rty[2 * (M - k) + 1]);
     };
 #pragma unroll
     for (int u = 0; u < IT / 2; u++) {
@@ -467,8 +525,8 @@ __global__ void __launch_bounds__(NTH) k_dct_rows(pvk_grid g, pvk_fft F, pvk_sca
 // with powers of q.  q, K, q^N and 1 / (1 - q^{2N}) are tables (per column), so
 // the kernel has no division; the elimination it replaces (partitioned
 // Thomas, a pivot division a row and a cyclic reduction of the separators
-// with two divisions a step) took 16.6 us at 1024^2 against 10.2 now, and 13.2
-// at 768 x 491 against 8.3.
+// with two divisions a step) took 16.6 us at 1024^2 against 10.6 now, and 13.2
+// at 768 x 491 against 8.7.
 // Column 0 (m = 0, row 0 replaced by the pin x_0 = 0) is two running sums:
 // x_{j+1} - x_j = -sum_{i > j} f_i / c.  With mean removal (the PCG's
 // pseudo-inverse) it is shifted to zero mean afterwards.  In the PCG this
@@ -543,10 +601,14 @@ __global__ void __launch_bounds__(512) k_tri_cols(pvk_grid g, pvk_fft F, pvk_sca
 #pragma unroll
     for (int l = 0; l < TRI_LMAX; l++) f[l] = spec[(size_t)min(j0 + min(l, L - 1), NY - 1) * NX + cc];
     const double q = F.tri_q[cc], K = F.tri_k[cc], qN = F.tri_qn[cc], den = F.tri_den[cc];
-    double rr = 0.0;
-    if (n != -3)
-        for (int b = t; b < w.nrr; b += nt) rr += w.rr[b];
+    double rr = 0.0, rp[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) rp[k] = (n != -3 && t + k * nt < w.nrr) ? w.rr[t + k * nt] : 0.0;
     if (sc->p_done) return;
+#pragma unroll
+    for (int k = 0; k < 8; k++) rr += rp[k];
+    if (n != -3)
+        for (int b = t + 8 * nt; b < w.nrr; b += nt) rr += w.rr[b];
     if (n != -3) {                          // stop test of iteration n (as the transpose stage does)
         rr = wave_sum(rr);
         if (lane == 0) ts[wv] = rr;
@@ -636,66 +698,61 @@ __global__ void __launch_bounds__(512) k_tri_cols(pvk_grid g, pvk_fft F, pvk_sca
 // ---------------------------------------------------------------------------
 // K6: z = inverse real FFT of spec rows; partials <r, z> into rz[(n+1)&1]
 // ---------------------------------------------------------------------------
-template <bool P2>
-__global__ void __launch_bounds__(NTH) k_ifft_rows_dot(pvk_grid g, pvk_fft F, pvk_scal *sc, pvk_pcg w, int n)
+template <bool P2, int NT>
+__global__ void __launch_bounds__(NT) k_ifft_rows_dot(pvk_grid g, pvk_fft F, pvk_scal *sc, pvk_pcg w, int n)
 {
     extern __shared__ double lds[];
-    __shared__ double sh[NTH];
-    if (w.chb == 0.0 && sc->p_done) return;
-    const int P = g.P, N = g.NXM, logM = F.logmx, M = F.mx, R = w.rrow, RM = R * M;
-    constexpr bool p2 = P2;     // power-of-two rows: shift-indexed passes
-    double *sr = lds, *si = lds + RM;
-    double *tw = stage_twiddles(lds, RM, M, F.wx);
+    __shared__ double sh[16];
+    const int P = g.P, N = g.NXM, R = w.rrow;
+    const RowGeo<NT> o = row_geo<P2, NT>(g, F, R);
+    const int M = o.M, T = o.T, lane = o.lane, j = o.j;
+    double *tw = lds, *sr = lds + 2 * M + 2 * o.q * o.LS, *si = sr + o.LS;
     const double *__restrict__ r = w.r;
     double *__restrict__ z = w.z;
-    const int j0 = blockIdx.x * R;
-    {
-        cplx2 Y[IT];
+    const double *row = F.spec + (size_t)j * N;
+    v2d rt[RU], rv[RU], tv[TWK];
+    double xr[RU], xi[RU], mr[RU], mi[RU];
 #pragma unroll
-        for (int u = 0; u < IT; u++) {
-            const int t = threadIdx.x + u * NTH;
-        int q, k;
-        row_split(t, M, logM, p2, q, k);
-        const int j = j0 + q;
-            Y[u].x = 0.0; Y[u].y = 0.0;
-            if (t < RM && j < g.NYM) {
-                const double *row = F.spec + (size_t)j * N;
-                Y[u] = rpre(hcget(row, N, k), hcget(row, N, M - k), k, F.rtx);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < IT; u++) {
-            const int t = threadIdx.x + u * NTH;
-            if (t < RM) { sr[t] = Y[u].x; si[t] = Y[u].y; }
-        }
+    for (int u = 0; u < RU; u++) {              // X_k and X_{M-k}
+        const int k = lane + u * T;
+        xr[u] = row[k];
+        xi[u] = row[k > 0 ? N - k : 0];
+        mr[u] = row[M - k];
+        mi[u] = row[M + k];
     }
-    __syncthreads();
-    rows_fft<true>(sr, si, M, logM, p2, R, tw);
-    double ra[IT], rb[IT];
+    tw_load<NT>(M, F.wx, tv);
 #pragma unroll
-    for (int u = 0; u < IT; u++) {
-        const int t = threadIdx.x + u * NTH;
-        int q, m;
-        row_split(t, M, logM, p2, q, m);
-        const int j = j0 + q;
-        ra[u] = rb[u] = 0.0;
-        if (t < RM && j < g.NYM) { ra[u] = AT(r, 2 * m, j); rb[u] = AT(r, 2 * m + 1, j); }
+    for (int u = 0; u < RU; u++) rt[u] = *(const v2d *)(F.rtx + 2 * (lane + u * T));
+#pragma unroll
+    for (int u = 0; u < RU; u++) rv[u] = *(const v2d *)&AT(r, 2 * (lane + u * T), j);
+    if (w.chb == 0.0 && sc->p_done) return;
+    tw_stage<NT>(M, tv, tw);
+    double vr[RU], vi[RU], acc = 0.0;
+#pragma unroll
+    for (int u = 0; u < RU; u++) {
+        const int k = lane + u * T;
+        cplx2 a, b;
+        a.x = xr[u];
+        a.y = (k == 0) ? 0.0 : xi[u];
+        b.x = mr[u];
+        b.y = (k == 0) ? 0.0 : mi[u];
+        const cplx2 Y = rpre(a, b, rt[u].x, rt[u].y);
+        vr[u] = Y.x;
+        vi[u] = Y.y;
     }
-    double acc = 0.0;
+    __syncthreads();                            // twiddles staged
+    rows_fft<true, P2>(vr, vi, sr, si, M, F.logmx, tw, lane, T, o.act);
+    if (o.act)
 #pragma unroll
-    for (int u = 0; u < IT; u++) {
-        const int t = threadIdx.x + u * NTH;
-        int q, m;
-        row_split(t, M, logM, p2, q, m);
-        const int j = j0 + q;
-        if (t < RM && j < g.NYM) {
-            const double a = sr[t], b = si[t];
-            AT(z, 2 * m, j) = a;
-            AT(z, 2 * m + 1, j) = b;
-            acc += ra[u] * a + rb[u] * b;
+        for (int u = 0; u < RU; u++) {
+            const int m = lane + u * T;
+            v2d t;
+            t.x = sr[SkPad::at(m)];
+            t.y = si[SkPad::at(m)];
+            *(v2d *)&AT(z, 2 * m, j) = t;
+            acc += rv[u].x * t.x + rv[u].y * t.y;
         }
-    }
-    block_store_partial(acc, w.rz[(n < 0) ? 0 : ((n + 1) & 1)], blockIdx.x, sh);
+    row_partial<NT>(acc, w.rz[(n < 0) ? 0 : ((n + 1) & 1)], sh);
 }
 
 __global__ void k_pcg_clear_done(pvk_scal *sc) { sc->p_done = 0; }
@@ -756,17 +813,41 @@ __global__ void __launch_bounds__(NTH) k_pcg_mean(pvk_grid g, pvk_scal *sc, pvk_
     block_store_partial(acc, w.mean, blockIdx.x, sh);
 }
 
-// R rows of N/2 complex values + the N/2 complex twiddles
+// threads of a block of the row kernels, and its LDS: R padded rows of N/2
+// complex values + the N/2 complex twiddles
+extern "C" int pvk_fft_row_threads(int N) { return N / 16 <= 64 ? 64 : (N / 16 <= 128 ? 128 : 256); }
+static size_t lds_row(int R, int N)
+{
+    const size_t M = N / 2;
+    return (2 * M + 2 * (size_t)R * (M + M / 8)) * sizeof(double);
+}
+#define FWD_STEP(P2, NT) k_pcg_update_fwd<P2, NT, ROW_STEP>
+#define FWD_START(P2, NT) k_pcg_update_fwd<P2, NT, ROW_START>
+#define FWD_WARM(P2, NT) k_pcg_update_fwd<P2, NT, ROW_WARM>
+#define FWD_PLAIN(P2, NT) k_pcg_update_fwd<P2, NT, ROW_PLAIN>
+#define INV_DOT(P2, NT) k_ifft_rows_dot<P2, NT>
+#define ROWS(KERNEL, N)                                                                                                    \
+    do {                                                                                                                   \
+        const int nt = pvk_fft_row_threads(g->NXM), nrow = (g->NYM + w->rrow - 1) / w->rrow;                               \
+        const size_t l = lds_row(w->rrow, g->NXM);                                                                         \
+        const dim3 gr(nrow);                                                                                               \
+        if (F->pow2x && nt == 64) hipLaunchKernelGGL((KERNEL(true, 64)), gr, dim3(64), l, s, *g, *F, sc, *w, N);           \
+        else if (F->pow2x && nt == 128) hipLaunchKernelGGL((KERNEL(true, 128)), gr, dim3(128), l, s, *g, *F, sc, *w, N);   \
+        else if (F->pow2x) hipLaunchKernelGGL((KERNEL(true, 256)), gr, dim3(256), l, s, *g, *F, sc, *w, N);                \
+        else if (nt == 64) hipLaunchKernelGGL((KERNEL(false, 64)), gr, dim3(64), l, s, *g, *F, sc, *w, N);                 \
+        else if (nt == 128) hipLaunchKernelGGL((KERNEL(false, 128)), gr, dim3(128), l, s, *g, *F, sc, *w, N);              \
+        else hipLaunchKernelGGL((KERNEL(false, 256)), gr, dim3(256), l, s, *g, *F, sc, *w, N);                             \
+    } while (0)
+// R columns of N/2 complex values + the N/2 complex twiddles (y transforms)
 static size_t lds_rows(int R, int N) { return ((size_t)R * (size_t)(N / 2) * 2 + (size_t)N) * sizeof(double); }
 
 extern "C" void pvk_pcg_start(const pvk_grid *g, const pvk_fft *F, pvk_scal *sc, const pvk_pcg *w, double tol,
                               hipStream_t s)
 {
-    int nband = (g->NYM + w->band - 1) / w->band, nrow = (g->NYM + w->rrow - 1) / w->rrow;
+    int nband = (g->NYM + w->band - 1) / w->band;
     hipLaunchKernelGGL(k_pcg_faces, dim3(g->NYM + 1), dim3(NTH), 0, s, *g, *w);
     hipLaunchKernelGGL(k_pcg_mean, dim3(nband), dim3(NTH), 0, s, *g, sc, *w);
-    if (F->pow2x) hipLaunchKernelGGL(k_pcg_update_fwd<true>, dim3(nrow), dim3(NTH), lds_rows(w->rrow, g->NXM), s, *g, *F, sc, *w, -1);
-    else hipLaunchKernelGGL(k_pcg_update_fwd<false>, dim3(nrow), dim3(NTH), lds_rows(w->rrow, g->NXM), s, *g, *F, sc, *w, -1);
+    ROWS(FWD_START, -1);
     (void)tol;
 }
 
@@ -913,16 +994,15 @@ extern "C" void pvk_jac_iter(const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w, 
 extern "C" void pvk_pcg_stage(const pvk_grid *g, const pvk_fft *F, pvk_scal *sc, const pvk_pcg *w, int stage, int n,
                               double tol, int maxit, hipStream_t s)
 {
-    int nband = (g->NYM + w->band - 1) / w->band, nrow = (g->NYM + w->rrow - 1) / w->rrow;
     switch (stage) {
     case 0:
         hipLaunchKernelGGL(k_pcg_apply, dim3(g->NYM), dim3(NTH), 0, s, *g, sc, *w, n);
         break;
     case 1:
-        if (F->pow2x)
-            hipLaunchKernelGGL(k_pcg_update_fwd<true>, dim3(nrow), dim3(NTH), lds_rows(w->rrow, g->NXM), s, *g, *F, sc, *w, n);
-        else
-            hipLaunchKernelGGL(k_pcg_update_fwd<false>, dim3(nrow), dim3(NTH), lds_rows(w->rrow, g->NXM), s, *g, *F, sc, *w, n);
+        if (n >= 0) ROWS(FWD_STEP, n);
+        else if (n == -2) ROWS(FWD_WARM, n);
+        else if (n == -3) ROWS(FWD_PLAIN, n);
+        else ROWS(FWD_START, n);
         break;
     case 2:
         hipLaunchKernelGGL(k_transpose, dim3((g->NXM + 31) / 32, (g->NYM + 31) / 32), dim3(NTH), 0, s, sc, *w,
@@ -944,10 +1024,7 @@ extern "C" void pvk_pcg_stage(const pvk_grid *g, const pvk_fft *F, pvk_scal *sc,
             hipLaunchKernelGGL(k_tri_cols<16>, gr, nt, 0, s, *g, *F, sc, *w, n, tol, maxit);
     } break;
     default:
-        if (F->pow2x)
-            hipLaunchKernelGGL(k_ifft_rows_dot<true>, dim3(nrow), dim3(NTH), lds_rows(w->rrow, g->NXM), s, *g, *F, sc, *w, n);
-        else
-            hipLaunchKernelGGL(k_ifft_rows_dot<false>, dim3(nrow), dim3(NTH), lds_rows(w->rrow, g->NXM), s, *g, *F, sc, *w, n);
+        ROWS(INV_DOT, n);
         break;
     }
 }

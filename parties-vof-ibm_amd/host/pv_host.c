@@ -675,11 +675,11 @@ int pv_fft_create(pv_bag *b)
     q = d;
     /* fused PCG work set: spectrum transpose + five partial buffers */
     {
-        /* row transforms use M/8 threads each (M = N/2, Stockham radix 8) in
-         * 256-thread blocks: 256 / (M/8) rows per block, 32 KiB of LDS */
+        /* transforms use M/8 threads each (M = N/2, Stockham radix 8): rows in
+         * blocks of pvk_fft_row_threads, columns in blocks of 256 */
         int band = (ny >= 512) ? 2 : 1, rrow, rdct, nband, nrow, np;
         double *pm;
-        rrow = 256 / ((nx / 2 >= 8) ? nx / 16 : 1);
+        rrow = pvk_fft_row_threads(nx) / (nx / 16);
         rdct = 256 / ((ny / 2 >= 8) ? ny / 16 : 1);
         nband = (ny + band - 1) / band;
         nrow = (ny + rrow - 1) / rrow;

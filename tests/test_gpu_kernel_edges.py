@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import mg_ref
+import oracle_lib
 import pvof
 from helpers import regions, relerr
 
@@ -80,3 +81,24 @@ def test_field_transfers(lib, nx, ny):
         a, b = b, a
     null = C.POINTER(C.c_double)()
     assert lib.pv_get_field(s.h, pvof.F["U"], null) != 0 and lib.pv_set_field(s.h, pvof.F["U"], null) != 0
+
+
+# rows of one thread (16), of three (48: threads left over in a wavefront), of
+# a whole wavefront (1024) and of blocks of 128 and 256 threads (2048; 3072
+# and 4096), with rows left over in the last block, and column counts of one
+# segment, a short last segment and several wavefronts of segments
+@pytest.mark.parametrize("nx,ny", [(16, 130), (48, 43), (1024, 9), (1152, 21), (2048, 13), (3072, 10), (4096, 17),
+                                   (64, 1031)])
+def test_fft_rows_and_columns(lib, nx, ny):
+    p = pvof.default_params(NXM=nx, NYM=ny, ymax=ny / nx)
+    o, s = oracle_lib.Oracle(p), pvof.Solver(p, lib)
+    R = regions(p)["cell"]
+    rhs = np.zeros(o.shape)
+    rhs[R] = np.random.default_rng(nx + ny).standard_normal((ny, nx))
+    rhs[R] -= rhs[R].mean()
+    for x in (o, s):
+        x.set("SCRATCH0", rhs)
+        x.call("Pressure_solve_fft", pvof.F["SCRATCH0"], pvof.F["SCRATCH1"])
+    got, ref = s.get("SCRATCH1")[R], o.get("SCRATCH1")[R]
+    assert np.isfinite(got).all()
+    assert relerr(got, ref) < 1e-10
