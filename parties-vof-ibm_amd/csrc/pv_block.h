@@ -12,6 +12,14 @@
 
 #define NTH 256
 
+// A barrier that orders LDS alone: loads from memory stay in flight across it.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // This thread's shares of up to three partial sums: sa = sum of pa[b] over
 // b = t, t + NTH, ... < na in increasing b (likewise sb, sc).  The partials
 // are loaded in batches of PVB per array, all loads of a batch in flight

@@ -8,7 +8,7 @@
 //              stencil point through the ghost-fill index maps (so no ghost
 //              fill kernel runs); A p; partial <p, A p>.
 //   K2 update: alpha; x += alpha p; r -= alpha A p; partials of the next
-//              residual products.
+//              residual products.  (Momentum: the next K1 makes the x step.)
 // A scalar that an earlier kernel already formed (||b||, the previous <r,z>)
 // is stored by block 0 in a parity-indexed slot that only later kernels read,
 // so a kernel re-adds at most two partial sets.  The arithmetic of every
@@ -330,7 +330,7 @@ extern "C" void pvk_ccg_iter(const pvk_grid *g, const pvk_phys *ph, int stage, p
 // ghost rows -1 / NYM holding minus rows 0 / NYM-1; v is x periodic (cell
 // image) and its wall rows 0 and NYM are never written by the solve.
 struct mom_band {
-    int comp, band, j0, j1, i0, ncell;
+    int comp, band, j0, j1, i0, jlo;
 };
 __device__ __forceinline__ mom_band mom_locate(const pvk_grid &g, const pvk_mcg &w)
 {
@@ -338,178 +338,334 @@ __device__ __forceinline__ mom_band mom_locate(const pvk_grid &g, const pvk_mcg 
     const int vb = xcd_band(blockIdx.x, gridDim.x);
     m.comp = (vb < w.nb[0]) ? 0 : 1;
     m.band = m.comp ? vb - w.nb[0] : vb;
-    const int jlo = m.comp ? 1 : 0, jhi = g.NYM;     // rows [jlo, NYM)
-    m.j0 = jlo + m.band * w.band;
-    m.j1 = min(jhi, m.j0 + w.band);
+    m.jlo = m.comp ? 1 : 0;                          // unknown rows [jlo, NYM)
+    m.j0 = m.jlo + m.band * w.band;
+    m.j1 = min(g.NYM, m.j0 + w.band);
     m.i0 = m.comp ? 0 : 1;
-    m.ncell = (m.j1 - m.j0) * g.NXM;
     return m;
 }
+// The FP32 form keeps what is an FP32 value as one: A d, the diagonal.
+template <class R> __device__ __forceinline__ const R *mom_Ad(const pvk_mcg &w, int c)
+{
+    if constexpr (sizeof(R) == sizeof(float)) return w.Adf[c];
+    else return w.Ad[c];
+}
+template <class R> __device__ __forceinline__ const R *mom_dg(const pvk_mcg &w, int c)
+{
+    if constexpr (sizeof(R) == sizeof(float)) return w.dgf[c];
+    else return w.dg[c];
+}
+// the diagonal + EPS (the FP64 form stores the sum)
+__device__ __forceinline__ double mom_D(float d) { return (double)d + 1e-14; }
+__device__ __forceinline__ double mom_D(double d) { return d; }
 
-// r = rhs - A x; dg = diag + EPS; d = r / dg; partial <r, d> (msolve_cg.c:627-645)
+// A thread's cells of its band, row by row, each row in chunks of NTH columns
+// (the order of its sums): position and the next one.
+struct mom_walk {
+    int j, cb;
+    __device__ __forceinline__ void next(int NXM)
+    {
+        cb += NTH;
+        if (cb >= NXM) { cb = 0; j++; }
+    }
+};
+
+// r = rhs - A x; dg = diag + EPS; d = r / dg; partial <r, d>
+// (msolve_cg.c:627-645), and what the iterations read instead of rho and mu:
+// the FP32 form the five coefficients, the FP64 form the time factor and
+// the corner viscosity, so that an iteration divides nothing to form A d.
+// Two cells a thread are in flight at once, each component's code knows its
+// stencil (one harmonic mean for the operator, the diagonal and the
+// coefficients), and what the preconditioned start overwrites is not formed.
+// Bound by memory latency: 74 us at 1024^2 in the FP32 form with one cell in
+// flight and the means formed three times over, 38 now.
+template <class R, int COMP>
+__device__ __forceinline__ void mcg_init_rows(const pvk_grid &g, const pvk_phys &ph, double alpha_k, double dt,
+                                              const pvk_mcg &w, const mom_band &m, double *sh)
+{
+    constexpr bool F32 = sizeof(R) == sizeof(float);
+    constexpr int U = 2;
+    const int P = g.P, NXM = g.NXM, NYM = g.NYM, t = threadIdx.x;
+    const double *x = w.x[COMP], *rhs = w.rhs[COMP], *rho = w.rho, *mu = w.mu;
+    double *r = w.r[COMP], *d = w.d[COMP][0];
+    double acc = 0.0;
+    for (mom_walk p = {m.j0, 0}; p.j < m.j1;) {
+        double ad[U], rr[U], dgv[U];
+        float cc[U][5], df[U];
+        double ft[U], mc[U], mp[U];
+        int jj[U], ii[U];
+        bool ok[U];
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            const int j = min(p.j, m.j1 - 1), i = m.i0 + min(p.cb + t, NXM - 1);
+            jj[k] = j;
+            ii[k] = i;
+            ok[k] = p.j < m.j1 && p.cb + t < NXM;
+            p.next(NXM);
+            ad[k] = (double)mom_op_vals<R>(g, ph, alpha_k, dt, rho, mu, COMP, i, j, R(AT(x, i, j)), R(AT(x, i + 1, j)),
+                                           R(AT(x, i - 1, j)), R(AT(x, i, j + 1)), R(AT(x, i, j - 1)));
+            rr[k] = AT(rhs, i, j) - ad[k];
+            const R dr = mom_diag<R>(g, ph, alpha_k, dt, rho, mu, COMP, i, j);
+            dgv[k] = (double)dr + 1e-14;
+            if constexpr (F32) {
+                df[k] = dr;
+                mom_coeffs(g, ph, alpha_k, dt, rho, mu, COMP, i, j, cc[k]);
+            } else {
+                ft[k] = mom_time<R>(g, alpha_k, dt, rho, COMP, i, j);
+                mc[k] = mom_corner<R>(g, mu, COMP, i, j);
+                mp[k] = COMP ? mom_corner<R>(g, mu, 1, i + 1, j) : mom_corner<R>(g, mu, 0, i, j + 1);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            if (!ok[k]) continue;
+            const int i = ii[k], j = jj[k];
+            AT(r, i, j) = rr[k];
+            if constexpr (F32) {
+#pragma unroll
+                for (int q = 0; q < 5; q++) AT(w.cf[COMP][q], i, j) = cc[k][q];
+                AT(w.dgf[COMP], i, j) = df[k];
+            } else {
+                AT(w.dg[COMP], i, j) = dgv[k];
+                AT(w.ft[COMP], i, j) = ft[k];
+                AT(w.mc[COMP], i, j) = mc[k];
+                if (COMP == 0 && j == NYM - 1) AT(w.mc[0], i, NYM) = mp[k];      // the last face's
+                if (COMP == 1 && i == NXM - 1) AT(w.mc[1], NXM, j) = mp[k];
+            }
+            if (w.maxit <= 0) AT(w.Ad[COMP], i, j) = ad[k];                     // else every A d comes after it
+            if (!F32 || !w.pc) {
+                const double dd = rr[k] / dgv[k];
+                AT(d, i, j) = dd;
+                acc += rr[k] * dd;
+            }
+        }
+    }
+    if (!F32 || !w.pc) block_store_partial(acc, w.rz[COMP][0], m.band, sh);
+}
 template <class R>
 __global__ void __launch_bounds__(NTH) k_mcg_init(pvk_grid g, pvk_phys ph, int stage, pvk_scal *sc, pvk_mcg w)
 {
     __shared__ double sh[NTH];
-    const int P = g.P, NXM = g.NXM;
     const mom_band m = mom_locate(g, w);
-    const int comp = m.comp ? 'v' : 'u';
     if (m.band == 0 && threadIdx.x == 0) { sc->m_done[m.comp] = (w.maxit <= 0); sc->m_iter[m.comp] = 0; }
     const double alpha_k = c_BET[stage], dt = sc->dt;
-    const double *x = w.x[m.comp], *rhs = w.rhs[m.comp];
-    double *r = w.r[m.comp], *dg = w.dg[m.comp], *d = w.d[m.comp][0], *Ad = w.Ad[m.comp];
-    double acc = 0.0;
-    for (int j = m.j0; j < m.j1; j++)
-    for (int i = m.i0 + (int)threadIdx.x; i < m.i0 + NXM; i += NTH) {
-        double ad = (double)mom_op<R>(g, ph, alpha_k, dt, w.rho, w.mu, x, comp, i, j);
-        double rr = AT(rhs, i, j) - ad;
-        double dgv = (double)mom_diag<R>(g, ph, alpha_k, dt, w.rho, w.mu, comp, i, j) + 1e-14;
-        if constexpr (sizeof(R) == sizeof(float)) {     // the FP32 iterations read these instead of rho, mu
-            float cc[5];
-            mom_coeffs(g, ph, alpha_k, dt, w.rho, w.mu, m.comp, i, j, cc);
-#pragma unroll
-            for (int k = 0; k < 5; k++) AT(w.cf[m.comp][k], i, j) = cc[k];
-        }
-        double dd = rr / dgv;
-        AT(Ad, i, j) = ad;
-        AT(r, i, j) = rr;
-        AT(dg, i, j) = dgv;
-        AT(d, i, j) = dd;
-        acc += rr * dd;
-    }
-    block_store_partial(acc, w.rz[m.comp][0], m.band, sh);
+    if (m.comp) mcg_init_rows<R, 1>(g, ph, alpha_k, dt, w, m, sh);
+    else mcg_init_rows<R, 0>(g, ph, alpha_k, dt, w, m, sh);
 }
 
 // K1: stop test sqrt(r.r / N) < CG_ETOL (msolve_cg.c:691-704), beta =
 // rz_new / (rz + EPS) (w.exact: rz_new / rz, 0 when rz is 0),
-// d_n = r / dg + beta d_{n-1} (:705-713) evaluated at
-// the five operator points through the ghost maps; Ad = A d_n; partial <d, Ad>.
+// d_n = z + beta d_{n-1} (:705-713), z the preconditioned residual, evaluated
+// at the five operator points through the ghost maps; Ad = A d_n; partial
+// <d, Ad>.  The x step of iteration n - 1 (x += alpha d) is made here, where
+// d_{n-1} is read anyway, and by the blocks that find the solve stopped.
+//
+// A block walks its band in chunks of MCH columns, a thread one column: its
+// own rows and the rows above and below stay in registers (the south and
+// north values), east and west go through LDS.  The first chunk's loads are
+// issued before the sums that give beta.  Bound by memory: 72 bytes a cell and
+// component in the FP64 form (84 MB at 512 x 1024), 64 in the FP32 form (537
+// MB at 2048^2: 123 us, 4.4 TB/s).  With the harmonic means and the time
+// factor formed anew in each iteration, r / dg divided at every stencil point
+// and the x step in the update kernel, the two kernels of an iteration took
+// 20.7 + 11.5 us at 512 x 1024 in FP64 (16.7 + 9.7 now), 37 + 19 at 1024^2
+// (28 + 14.6), and 120 + 196 at 2048^2 in the FP32 form with the polynomial
+// preconditioner (123 + 118).
 #define MCH 256                                                  // columns per chunk of k_mcg_apply
-#define MSQ (((BAND + 2) * (MCH + 2) + NTH - 1) / NTH)     // staged values per thread
-template <class R, int BAND, bool PC>
-__global__ void __launch_bounds__(NTH) k_mcg_apply(pvk_grid g, pvk_phys ph, int stage, pvk_scal *sc, pvk_mcg w,
-                                                  int n)
+template <class R, int BAND, bool FIRST>
+__global__ void __launch_bounds__(NTH) k_mcg_apply(pvk_grid g, pvk_phys ph, pvk_scal *sc, pvk_mcg w, int n)
 {
-    __shared__ double sh[NTH];
-    __shared__ double sd[BAND + 2][MCH + 2];
+    constexpr bool F32 = sizeof(R) == sizeof(float);
+    __shared__ double sh[2 * NTH];
+    __shared__ double sd[2][BAND][MCH + 2];
     const mom_band m = mom_locate(g, w);
-    const int c = m.comp;
-    if (sc->m_done[c]) return;
-    const int P = g.P, NXM = g.NXM, NYM = g.NYM;
-    const double EPS = 1e-14;
-    const bool lead = (m.band == 0 && threadIdx.x == 0);
-    const double rz = block_sum(w.rz[c][n & 1], w.nb[c], sh);
-    double beta = 0.0;
-    if (n > 0) {
-        const double rr = block_sum(w.rr[c], w.nb[c], sh);
-        const double rms = sqrt(w.in_tot[c] * rr);
-        bool stop = rms < w.tol;
-        if (!stop) {
-            const double rzo = sc->m_rzb[c][(n + 1) & 1];
-            beta = w.exact ? (rzo != 0.0 ? rz / rzo : 0.0) : rz / (rzo + EPS);
-            stop = (n >= w.maxit);
+    const int c = m.comp, t = threadIdx.x;
+    const int was = sc->m_done[c], it = sc->m_iter[c];
+    if (was && (FIRST || it != n)) return;               // stopped, x complete
+    const int P = g.P, NXM = g.NXM, NYM = g.NYM, nrow = m.j1 - m.j0;
+    const bool lead = (m.band == 0 && t == 0);
+    const double *zc = FIRST ? w.d[c][0] : w.z[c], *dold = w.d[c][(n + 1) & 1], *dwall = w.d[c][0];
+    double *dnew = w.d[c][n & 1], *x = w.x[c];
+    R *Ad = const_cast<R *>(mom_Ad<R>(w, c));
+
+    // a chunk's values: z and d_{n-1} of rows j0 - 1 .. j0 + BAND, those of the
+    // ring column this thread sees to, x, and the operator's factors
+    double z[BAND + 2], o[BAND + 2], rz_, ro_, xv[BAND];
+    R cf[BAND][5];                                       // FP32: the coefficients; FP64: ft, xp, xm in 0..2
+    double yf[BAND + 1];                                 // FP64: the y face viscosities
+    auto ghost = [&](int b) { return b < m.jlo || b >= NYM; };
+    auto ncol = [&](int cb) { return min(MCH, NXM - cb); };
+    auto load = [&](int cb) {
+        const int i = m.i0 + cb + min(t, ncol(cb) - 1);
+#pragma unroll
+        for (int a = 0; a < BAND + 2; a++) {
+            const int b = m.j0 - 1 + a, bc = min(max(b, m.jlo), NYM - 1);
+            z[a] = (c && ghost(b)) ? AT(dwall, i, b < 1 ? 0 : NYM) : AT(zc, i, bc);
+            if (!FIRST) o[a] = AT(dold, i, bc);
         }
-        if (stop) {
+        if (t < 2 * BAND) {                              // thread 2 a + side: row j0 + a, west or east column
+            const int e = m.i0 + cb + ((t & 1) ? ncol(cb) : -1), b = min(m.j0 + (t >> 1), NYM - 1);
+            const int ie = c ? wrapc(e, NXM) : wrapu(e, NXM);
+            rz_ = AT(zc, ie, b);
+            if (!FIRST) ro_ = AT(dold, ie, b);
+        }
+#pragma unroll
+        for (int a = 0; a < BAND; a++) {
+            const int b = min(m.j0 + a, NYM - 1);
+            if (!FIRST) xv[a] = AT(x, i, b);
+            if constexpr (F32) {
+#pragma unroll
+                for (int k = 0; k < 5; k++) cf[a][k] = AT(w.cf[c][k], i, b);
+            } else {
+                cf[a][0] = AT(w.ft[c], i, b);
+                cf[a][1] = c ? AT(w.mc[1], i + 1, b) : AT(w.mu, i, b);
+                cf[a][2] = c ? AT(w.mc[1], i, b) : AT(w.mu, i - 1, b);
+            }
+        }
+        if constexpr (!F32) {
+#pragma unroll
+            for (int a = 0; a <= BAND; a++)
+                yf[a] = c ? AT(w.mu, i, min(m.j0 - 1 + a, NYM - 1)) : AT(w.mc[0], i, min(m.j0 + a, NYM));
+        }
+    };
+    load(0);
+
+    double beta = 0.0, alpha = 0.0;
+    if (FIRST) {
+        const double rz = block_sum(w.rz[c][0], w.nb[c], sh);
+        if (lead) sc->m_rzb[c][0] = rz;
+    } else {
+        double rz, rr;
+        block_sum2(w.rz[c][n & 1], w.nb[c], w.rr[c], w.nb[c], sh, rz, rr);
+        const double rms = sqrt(w.in_tot[c] * rr), rzo = sc->m_rzb[c][(n + 1) & 1];
+        alpha = sc->m_alpha[c];
+        if (rms < w.tol || n >= w.maxit) {
             if (lead) {
                 sc->m_rms[c] = rms;
                 sc->m_iter[c] = n;
                 sc->m_done[c] = (rms < w.tol) ? 1 : 3;
             }
+            // the last x step; the public fields of the last A d and residual
+            for (int j = m.j0; j < m.j1; j++)
+                for (int i = m.i0 + t; i < m.i0 + NXM; i += NTH) {
+                    AT(x, i, j) += alpha * AT(dold, i, j);
+                    if constexpr (F32) {
+                        AT(w.Ad[c], i, j) = (double)AT(Ad, i, j);
+                        if (w.pc && (n & 1)) AT(w.r[c], i, j) = AT(w.r2[c], i, j);
+                    }
+                }
             return;
         }
+        beta = w.exact ? (rzo != 0.0 ? rz / rzo : 0.0) : rz / (rzo + 1e-14);
+        if (lead) sc->m_rzb[c][n & 1] = rz;
     }
-    if (lead) sc->m_rzb[c][n & 1] = rz;
-    const double *r = w.r[c], *dg = w.dg[c], *dold = w.d[c][(n + 1) & 1], *dwall = w.d[c][0], *zc = w.z[c];
-    double *dnew = w.d[c][n & 1], *Ad = w.Ad[c];
-    const double alpha_k = c_BET[stage], dt = sc->dt;
-    // d at (a, b) after the CG-type ghost fill of the new direction
-    auto dv = [&](int a, int b) -> double {
-        if (c == 0) {
-            const int ia = wrapu(a, NXM);
-            const int jb = b < 0 ? 0 : (b >= NYM ? NYM - 1 : b);
-            double val = (n == 0) ? AT(dwall, ia, jb)
-                                  : (PC ? AT(zc, ia, jb) : AT(r, ia, jb) / AT(dg, ia, jb)) + beta * AT(dold, ia, jb);
-            return (b < 0 || b >= NYM) ? -val : val;
-        }
-        const int ia = wrapc(a, NXM);
-        if (b <= 0 || b >= NYM) return AT(dwall, ia, b);
-        return (n == 0) ? AT(dwall, ia, b)
-                        : (PC ? AT(zc, ia, b) : AT(r, ia, b) / AT(dg, ia, b)) + beta * AT(dold, ia, b);
-    };
-    // The band (w.band = BAND rows, the last one may have fewer) in chunks of MCH columns: d of the
-    // chunk and a one-cell ring is formed once into LDS (every value as dv
-    // forms it), then A d of the chunk reads its neighbours there.
-    const int nrow = m.j1 - m.j0;
+
     double acc = 0.0;
-    for (int cb = 0; cb < NXM; cb += MCH) {
-        double sv[MSQ];
+    int par = 0;
+    for (int cb = 0; cb < NXM; cb += MCH, par ^= 1) {
+        if (cb) load(cb);
+        const int nc = ncol(cb);
+        double dv[BAND + 2];
 #pragma unroll
-        for (int k = 0; k < MSQ; k++) {               // all loads of the stage in flight together
-            const int q = threadIdx.x + k * NTH, a = q / (MCH + 2), bb = q - a * (MCH + 2);
-            sv[k] = (a < nrow + 2) ? dv(m.i0 + cb - 1 + bb, m.j0 - 1 + a) : 0.0;
+        for (int a = 0; a < BAND + 2; a++) {
+            const double v = FIRST ? z[a] : z[a] + beta * o[a];
+            dv[a] = ghost(m.j0 - 1 + a) ? (c ? z[a] : -v) : v;
         }
+        if (t < nc) {
 #pragma unroll
-        for (int k = 0; k < MSQ; k++) {
-            const int q = threadIdx.x + k * NTH, a = q / (MCH + 2), bb = q - a * (MCH + 2);
-            if (a < BAND + 2) sd[a][bb] = sv[k];
+            for (int a = 0; a < BAND; a++) sd[par][a][t + 1] = dv[a + 1];
         }
+        if (t < 2 * BAND) sd[par][t >> 1][(t & 1) ? nc + 1 : 0] = FIRST ? rz_ : rz_ + beta * ro_;
         __syncthreads();
-        for (int q = threadIdx.x; q < nrow * MCH; q += NTH) {
-            const int a = q / MCH, bb = q - a * MCH, j = m.j0 + a, i = m.i0 + cb + bb;
-            if (cb + bb < NXM) {
-                const double dc = sd[a + 1][bb + 1];
-                double ad;
-                if constexpr (sizeof(R) == sizeof(float)) {
-                    float cc[5];
+        if (t < nc) {
+            const int i = m.i0 + cb + t;
 #pragma unroll
-                    for (int k = 0; k < 5; k++) cc[k] = AT(w.cf[c][k], i, j);
-                    ad = (double)mom_op_coeffs(cc, float(dc), float(sd[a + 1][bb + 2]), float(sd[a + 1][bb]),
-                                               float(sd[a + 2][bb + 1]), float(sd[a][bb + 1]));
-                } else {
-                    ad = (double)mom_op_vals<R>(g, ph, alpha_k, dt, w.rho, w.mu, c, i, j, R(dc), R(sd[a + 1][bb + 2]),
-                                                R(sd[a + 1][bb]), R(sd[a + 2][bb + 1]), R(sd[a][bb + 1]));
+            for (int a = 0; a < BAND; a++) {
+                if (a < nrow) {
+                    const int j = m.j0 + a;
+                    const double dc = dv[a + 1], dE = sd[par][a][t + 2], dW = sd[par][a][t];
+                    R ad;
+                    if constexpr (F32)
+                        ad = mom_op_coeffs(cf[a], float(dc), float(dE), float(dW), float(dv[a + 2]), float(dv[a]));
+                    else
+                        ad = mom_op_flux<R>(g, ph.iRe, c, i, j, cf[a][0], cf[a][1], cf[a][2], yf[a + 1], yf[a], dc, dE,
+                                            dW, dv[a + 2], dv[a]);
+                    if (!FIRST) {
+                        AT(x, i, j) = xv[a] + alpha * o[a + 1];
+                        AT(dnew, i, j) = dc;
+                    }
+                    AT(Ad, i, j) = ad;
+                    acc += dc * (double)ad;
                 }
-                if (n > 0) AT(dnew, i, j) = dc;
-                AT(Ad, i, j) = ad;
-                acc += dc * ad;
             }
         }
-        __syncthreads();
     }
     block_store_partial(acc, w.dad[c], m.band, sh);
 }
 
-// K2: alpha = rz / (dAd + EPS) (msolve_cg.c:674; w.exact: rz / dAd, 0 when
-// dAd is 0); x += alpha d; r -= alpha Ad;
-// partials of r^2 / dg and r^2 (:676-690).
+// the step of iteration n: alpha = rz / (dAd + EPS) (msolve_cg.c:674; w.exact:
+// rz / dAd, 0 when dAd is 0)
+__device__ __forceinline__ double mom_alpha(pvk_scal *sc, const pvk_mcg &w, const mom_band &m, int n, double *sh)
+{
+    const int c = m.comp;
+    const double dAd = block_sum(w.dad[c], w.nb[c], sh);
+    const double rzn = sc->m_rzb[c][n & 1];
+    const double alpha = w.exact ? (dAd != 0.0 ? rzn / dAd : 0.0) : rzn / (dAd + 1e-14);
+    if (m.band == 0 && threadIdx.x == 0) { sc->m_iter[c] = n + 1; sc->m_alpha[c] = alpha; }
+    return alpha;
+}
+
+// K2: alpha; r -= alpha Ad; z = r / dg; partials of r^2 / dg and r^2
+// (msolve_cg.c:676-690).  Four cells a thread in flight, the first four's
+// loads ahead of the sums.
+template <class R>
 __global__ void __launch_bounds__(NTH) k_mcg_update(pvk_grid g, pvk_scal *sc, pvk_mcg w, int n)
 {
     __shared__ double sh[NTH];
     const mom_band m = mom_locate(g, w);
-    const int c = m.comp;
+    const int c = m.comp, t = threadIdx.x;
     if (sc->m_done[c]) return;
     const int P = g.P, NXM = g.NXM;
-    const double EPS = 1e-14;
-    const double dAd = block_sum(w.dad[c], w.nb[c], sh);
-    const double rzn = sc->m_rzb[c][n & 1];
-    const double alpha = w.exact ? (dAd != 0.0 ? rzn / dAd : 0.0) : rzn / (dAd + EPS);
-    if (m.band == 0 && threadIdx.x == 0) sc->m_iter[c] = n + 1;
-    double *x = w.x[c], *r = w.r[c];
-    const double *d = w.d[c][n & 1], *Ad = w.Ad[c], *dg = w.dg[c];
+    double *r = w.r[c], *z = w.z[c];
+    const R *Ad = mom_Ad<R>(w, c), *dg = mom_dg<R>(w, c);
+    double rv[CPT];
+    R av[CPT], gv[CPT];
+    auto load = [&](mom_walk p) {
+#pragma unroll
+        for (int k = 0; k < CPT; k++) {
+            const int j = min(p.j, m.j1 - 1), i = m.i0 + min(p.cb + t, NXM - 1);
+            rv[k] = AT(r, i, j);
+            av[k] = AT(Ad, i, j);
+            gv[k] = AT(dg, i, j);
+            p.next(NXM);
+        }
+    };
+    mom_walk p = {m.j0, 0};
+    load(p);
+    const double alpha = mom_alpha(sc, w, m, n, sh);
     double a0 = 0.0, a1 = 0.0;
-    for (int j = m.j0; j < m.j1; j++)
-    for (int i = m.i0 + (int)threadIdx.x; i < m.i0 + NXM; i += NTH) {
-        AT(x, i, j) += alpha * AT(d, i, j);
-        double ri = AT(r, i, j) - alpha * AT(Ad, i, j);
-        AT(r, i, j) = ri;
-        a0 += ri * ri / AT(dg, i, j);
-        a1 += ri * ri;
+    while (p.j < m.j1) {
+        mom_walk q = p;
+#pragma unroll
+        for (int k = 0; k < CPT; k++) {
+            if (q.j < m.j1 && q.cb + t < NXM) {
+                const int j = q.j, i = m.i0 + q.cb + t;
+                const double ri = rv[k] - alpha * (double)av[k], D = mom_D(gv[k]);
+                AT(r, i, j) = ri;
+                AT(z, i, j) = ri / D;
+                a0 += ri * ri / D;
+                a1 += ri * ri;
+            }
+            q.next(NXM);
+        }
+        p = q;
+        if (p.j < m.j1) load(p);
     }
     block_store_partial(a0, w.rz[c][(n + 1) & 1], m.band, sh);
     block_store_partial(a1, w.rr[c], m.band, sh);
 }
 
-// Momentum preconditioner pc = 1, the first-order Neumann polynomial of
+// Momentum preconditioner pc = 1 (FP32 form), the first-order Neumann polynomial of
 // the Jacobi splitting A = D - N: z = D^-1 (r + N D^-1 r), i.e.
 // z_p = (r_p + sum_q c_pq r_q / D_q) / D_p over the unknown neighbours q of
 // p (periodic in x, no coupling across the walls), c_pq the FP32 operator
@@ -520,128 +676,114 @@ __global__ void __launch_bounds__(NTH) k_mcg_update(pvk_grid g, pvk_scal *sc, pv
 // iterations for one more stencil of r per iteration, which the update
 // kernel forms from r_n and A d_n at the neighbours (r is double-buffered:
 // r_{n+1} goes to the other buffer while neighbours read r_n).
-template <class RF>
-__device__ __forceinline__ double mom_pc_z(const pvk_grid &g, const pvk_mcg &w, int c, int i, int j, RF rv)
-{
-    const int P = g.P, NXM = g.NXM, NYM = g.NYM;
-    const double *dg = w.dg[c];
-    const int ie = c ? wrapc(i + 1, NXM) : wrapu(i + 1, NXM);
-    const int iw = c ? wrapc(i - 1, NXM) : wrapu(i - 1, NXM);
-    const int jlo = c ? 1 : 0;
-    double s = rv(i, j);
-    s += (double)AT(w.cf[c][1], i, j) * (rv(ie, j) / AT(dg, ie, j));
-    s += (double)AT(w.cf[c][2], i, j) * (rv(iw, j) / AT(dg, iw, j));
-    if (j + 1 < NYM) s += (double)AT(w.cf[c][3], i, j) * (rv(i, j + 1) / AT(dg, i, j + 1));
-    if (j - 1 >= jlo) s += (double)AT(w.cf[c][4], i, j) * (rv(i, j - 1) / AT(dg, i, j - 1));
-    return s / AT(dg, i, j);
-}
-
-// pc = 1 start: d_0 = z_0 = M r_0, partial <r_0, z_0> (replacing the Jacobi
-// ones of the start kernel)
-__global__ void __launch_bounds__(NTH) k_mcg_pc_start(pvk_grid g, pvk_mcg w)
-{
-    __shared__ double sh[NTH];
-    const int P = g.P, NXM = g.NXM;
-    const mom_band m = mom_locate(g, w);
-    const int c = m.comp;
-    const double *r = w.r[c];
-    double *d = w.d[c][0];
-    auto rv = [&](int a, int b) { return AT(r, a, b); };
-    double acc = 0.0;
-    for (int j = m.j0; j < m.j1; j++)
-    for (int i = m.i0 + (int)threadIdx.x; i < m.i0 + NXM; i += NTH) {
-        const double zz = mom_pc_z(g, w, c, i, j, rv);
-        AT(d, i, j) = zz;
-        acc += AT(r, i, j) * zz;
-    }
-    block_store_partial(acc, w.rz[c][0], m.band, sh);
-}
-
-// pc = 1 update: alpha as k_mcg_update; x += alpha d; r_{n+1} = r_n - alpha
-// A d_n into the other r buffer; z_{n+1} = M r_{n+1}; partials <r, z>, <r, r>
+//
+// START: d_0 = z_0 = M r_0, partial <r_0, z_0>.  Otherwise alpha as k_mcg_update,
+// r_{n+1} = r_n - alpha A d_n, z_{n+1} = M r_{n+1}, partials <r, z>, <r, r>.
+//
+// A thread's column: the quotients r / D of its own, the row above and the
+// row below it forms itself, east and west come through LDS (three divisions
+// a cell instead of five); the next chunk's loads are in flight over this one.
+// Bound by memory, 48 bytes a cell and component (80 with the x step here and
+// A d and the diagonal as doubles): 36 -> 23 us at 1024^2, 196 -> 118 at
+// 2048^2; the start 26 -> 18 and 162 -> 98.
+template <bool START>
 __global__ void __launch_bounds__(NTH) k_mcg_update_pc(pvk_grid g, pvk_scal *sc, pvk_mcg w, int n)
 {
     __shared__ double sh[NTH];
+    __shared__ double sq[2][NTH + 2];
     const mom_band m = mom_locate(g, w);
-    const int c = m.comp;
-    if (sc->m_done[c]) return;
-    const int P = g.P, NXM = g.NXM;
-    const double EPS = 1e-14;
-    const double dAd = block_sum(w.dad[c], w.nb[c], sh);
-    const double rzn = sc->m_rzb[c][n & 1];
-    const double alpha = w.exact ? (dAd != 0.0 ? rzn / dAd : 0.0) : rzn / (dAd + EPS);
-    if (m.band == 0 && threadIdx.x == 0) sc->m_iter[c] = n + 1;
-    double *x = w.x[c], *z = w.z[c];
+    const int c = m.comp, t = threadIdx.x;
+    if (!START && sc->m_done[c]) return;
+    const int P = g.P, NXM = g.NXM, NYM = g.NYM;
     const double *rold = (n & 1) ? w.r2[c] : w.r[c];
-    double *rnew = (n & 1) ? w.r[c] : w.r2[c];
-    const double *d = w.d[c][n & 1], *Ad = w.Ad[c];
-    auto rv = [&](int a, int b) { return AT(rold, a, b) - alpha * AT(Ad, a, b); };
+    double *rnew = (n & 1) ? w.r[c] : w.r2[c], *z = START ? w.d[c][0] : w.z[c];
+    const float *Ad = w.Adf[c], *dg = w.dgf[c];
+    struct cell { double r; float a, d; };
+    struct chunk { cell o, n, s, e; float c[4]; };
+    auto get = [&](cell &q, int i, int j) {
+        q.r = AT(rold, i, j);
+        if (!START) q.a = AT(Ad, i, j);
+        q.d = AT(dg, i, j);
+    };
+    auto load = [&](chunk &k, mom_walk p) {
+        const int nc = min(NTH, NXM - p.cb), i = m.i0 + p.cb + min(t, nc - 1);
+        get(k.o, i, p.j);
+        get(k.n, i, min(p.j + 1, NYM - 1));
+        get(k.s, i, max(p.j - 1, m.jlo));
+        if (t < 2) {                                    // the column west, east of the chunk
+            const int e = m.i0 + p.cb + (t ? nc : -1);
+            get(k.e, c ? wrapc(e, NXM) : wrapu(e, NXM), p.j);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) k.c[q] = AT(w.cf[c][1 + q], i, p.j);
+    };
+    chunk k;
+    mom_walk p = {m.j0, 0};
+    load(k, p);
+    const double alpha = START ? 0.0 : mom_alpha(sc, w, m, n, sh);
+    auto rv = [&](const cell &q) { return START ? q.r : q.r - alpha * (double)q.a; };
+    auto quo = [&](const cell &q) { return rv(q) / mom_D(q.d); };
     double a0 = 0.0, a1 = 0.0;
-    for (int j = m.j0; j < m.j1; j++)
-    for (int i = m.i0 + (int)threadIdx.x; i < m.i0 + NXM; i += NTH) {
-        AT(x, i, j) += alpha * AT(d, i, j);
-        const double ri = rv(i, j);
-        const double zz = mom_pc_z(g, w, c, i, j, rv);
-        AT(rnew, i, j) = ri;
-        AT(z, i, j) = zz;
-        a0 += ri * zz;
-        a1 += ri * ri;
+    for (int par = 0; p.j < m.j1; par ^= 1) {
+        const int nc = min(NTH, NXM - p.cb), i = m.i0 + p.cb + t, j = p.j;
+        const double ri = rv(k.o), qn = quo(k.n), qs = quo(k.s), D = mom_D(k.o.d);
+        const float cE = k.c[0], cW = k.c[1], cN = k.c[2], cS = k.c[3];
+        if (t < nc) sq[par][t + 1] = quo(k.o);
+        if (t < 2) sq[par][t ? nc + 1 : 0] = quo(k.e);
+        p.next(NXM);
+        if (p.j < m.j1) load(k, p);
+        lds_barrier();
+        if (t < nc) {
+            double s = ri;
+            s += (double)cE * sq[par][t + 2];
+            s += (double)cW * sq[par][t];
+            if (j + 1 < NYM) s += (double)cN * qn;
+            if (j - 1 >= m.jlo) s += (double)cS * qs;
+            const double zz = s / D;
+            if (!START) AT(rnew, i, j) = ri;
+            AT(z, i, j) = zz;
+            a0 += ri * zz;
+            a1 += ri * ri;
+        }
     }
-    block_store_partial(a0, w.rz[c][(n + 1) & 1], m.band, sh);
-    block_store_partial(a1, w.rr[c], m.band, sh);
-}
-
-// pc = 1, after the loop: a component that stopped after an odd number of
-// updates holds its residual in r2: copy it to r (the public field)
-__global__ void __launch_bounds__(NTH) k_mcg_pc_finish(pvk_grid g, const pvk_scal *sc, pvk_mcg w)
-{
-    const int P = g.P, NXM = g.NXM;
-    const mom_band m = mom_locate(g, w);
-    const int c = m.comp;
-    if (!(sc->m_iter[c] & 1)) return;
-    for (int j = m.j0; j < m.j1; j++)
-    for (int i = m.i0 + (int)threadIdx.x; i < m.i0 + NXM; i += NTH) AT(w.r[c], i, j) = AT(w.r2[c], i, j);
-}
-
-extern "C" void pvk_mcg_pc_start(const pvk_grid *g, const pvk_mcg *w, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_mcg_pc_start, dim3(w->nb[0] + w->nb[1]), dim3(NTH), 0, s, *g, *w);
-}
-
-extern "C" void pvk_mcg_pc_finish(const pvk_grid *g, const pvk_scal *sc, const pvk_mcg *w, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_mcg_pc_finish, dim3(w->nb[0] + w->nb[1]), dim3(NTH), 0, s, *g, sc, *w);
+    block_store_partial(a0, w.rz[c][START ? 0 : (n + 1) & 1], m.band, sh);
+    if (!START) block_store_partial(a1, w.rr[c], m.band, sh);
 }
 
 extern "C" void pvk_mcg_init(const pvk_grid *g, const pvk_phys *ph, int stage, pvk_scal *sc, const pvk_mcg *w,
                              hipStream_t s)
 {
-    if (ph->precision)
-        hipLaunchKernelGGL(k_mcg_init<float>, dim3(w->nb[0] + w->nb[1]), dim3(NTH), 0, s, *g, *ph, stage, sc, *w);
-    else
-        hipLaunchKernelGGL(k_mcg_init<double>, dim3(w->nb[0] + w->nb[1]), dim3(NTH), 0, s, *g, *ph, stage, sc, *w);
+    const dim3 gr(w->nb[0] + w->nb[1]);
+    if (ph->precision) {
+        hipLaunchKernelGGL(k_mcg_init<float>, gr, dim3(NTH), 0, s, *g, *ph, stage, sc, *w);
+        if (w->pc) hipLaunchKernelGGL(k_mcg_update_pc<true>, gr, dim3(NTH), 0, s, *g, sc, *w, 0);
+    } else
+        hipLaunchKernelGGL(k_mcg_init<double>, gr, dim3(NTH), 0, s, *g, *ph, stage, sc, *w);
 }
 
-extern "C" void pvk_mcg_iter(const pvk_grid *g, const pvk_phys *ph, int stage, pvk_scal *sc, const pvk_mcg *w,
-                             int half, int n, hipStream_t s)
+template <class R, bool FIRST>
+static void mcg_apply(const pvk_grid *g, const pvk_phys *ph, pvk_scal *sc, const pvk_mcg *w, int n, hipStream_t s)
 {
-#define MCG_APPLY(RT, B, PC) \
-    hipLaunchKernelGGL((k_mcg_apply<RT, B, PC>), dim3(w->nb[0] + w->nb[1]), dim3(NTH), 0, s, *g, *ph, stage, sc, *w, n)
-    if (half == 0 && ph->precision && w->pc) {      // the polynomial preconditioner: FP32 form only
-        if (w->band == 1) MCG_APPLY(float, 1, true);
-        else if (w->band == 2) MCG_APPLY(float, 2, true);
-        else MCG_APPLY(float, 4, true);
-    } else if (half == 0 && ph->precision) {
-        if (w->band == 1) MCG_APPLY(float, 1, false);
-        else if (w->band == 2) MCG_APPLY(float, 2, false);
-        else MCG_APPLY(float, 4, false);
+    const dim3 gr(w->nb[0] + w->nb[1]);
+    if (w->band == 1) hipLaunchKernelGGL((k_mcg_apply<R, 1, FIRST>), gr, dim3(NTH), 0, s, *g, *ph, sc, *w, n);
+    else if (w->band == 2) hipLaunchKernelGGL((k_mcg_apply<R, 2, FIRST>), gr, dim3(NTH), 0, s, *g, *ph, sc, *w, n);
+    else hipLaunchKernelGGL((k_mcg_apply<R, 4, FIRST>), gr, dim3(NTH), 0, s, *g, *ph, sc, *w, n);
+}
+
+extern "C" void pvk_mcg_iter(const pvk_grid *g, const pvk_phys *ph, pvk_scal *sc, const pvk_mcg *w, int half, int n,
+                             hipStream_t s)
+{
+    const dim3 gr(w->nb[0] + w->nb[1]);
+    if (half == 0 && ph->precision) {
+        if (n == 0) mcg_apply<float, true>(g, ph, sc, w, n, s);
+        else mcg_apply<float, false>(g, ph, sc, w, n, s);
     } else if (half == 0) {
-        if (w->band == 1) MCG_APPLY(double, 1, false);
-        else if (w->band == 2) MCG_APPLY(double, 2, false);
-        else MCG_APPLY(double, 4, false);
-    } else if (w->pc)
-#undef MCG_APPLY
-        hipLaunchKernelGGL(k_mcg_update_pc, dim3(w->nb[0] + w->nb[1]), dim3(NTH), 0, s, *g, sc, *w, n);
+        if (n == 0) mcg_apply<double, true>(g, ph, sc, w, n, s);
+        else mcg_apply<double, false>(g, ph, sc, w, n, s);
+    } else if (!ph->precision)
+        hipLaunchKernelGGL(k_mcg_update<double>, gr, dim3(NTH), 0, s, *g, sc, *w, n);
+    else if (w->pc)                                  // the polynomial preconditioner: FP32 form only
+        hipLaunchKernelGGL(k_mcg_update_pc<false>, gr, dim3(NTH), 0, s, *g, sc, *w, n);
     else
-        hipLaunchKernelGGL(k_mcg_update, dim3(w->nb[0] + w->nb[1]), dim3(NTH), 0, s, *g, sc, *w, n);
+        hipLaunchKernelGGL(k_mcg_update<float>, gr, dim3(NTH), 0, s, *g, sc, *w, n);
 }

@@ -27,6 +27,7 @@ typedef struct pvk_scal {
     /* momentum Jacobi-PCG per component 0 = u, 1 = v (msolve_cg.c:525-722) */
     double m_rzb[2][2];      /* [component][n & 1]: <r, z> of iterations n and n - 1 */
     double m_rms[2];
+    double m_alpha[2];       /* step of the last update */
     int    m_iter[2], m_done[2];
     /* pressure PCG (psolve_cg.c:130-293 or FFT-PCG) */
     double p_gamma, p_alpha, p_beta, p_res, p_bnorm, p_mean;
@@ -131,13 +132,16 @@ typedef struct pvk_mcg {             /* momentum Jacobi-PCG, [0] = u, [1] = v */
     int nb[2], band;                 /* nb[c] = 0 leaves component c out */
     int maxit;
     float *cf[2][5];                 /* FP32 form: operator coefficients (centre, E, W, N, S) of each
-                                        unknown, pitch P, formed by the start kernel */
+                                        unknown, pitch P, formed by the start kernel ... */
+    float *dgf[2], *Adf[2];          /* ... the diagonal before EPS is added, and A d */
+    double *ft[2], *mc[2];           /* FP64 form: face rho / (alpha dt) and corner viscosity of each
+                                        unknown, formed by the start kernel */
     int exact;                       /* 0: EPS = 1e-14 added to the step denominators (the
                                         reference); 1: the denominators as they are, a zero
                                         one giving a zero step */
     int pc;                          /* 0: Jacobi (the reference); 1: first-order Neumann
                                         polynomial of the Jacobi splitting (FP32 form) */
-    double *r2[2], *z[2];            /* pc = 1: r of odd iterations, preconditioned residual */
+    double *r2[2], *z[2];            /* pc = 1: r of odd iterations; preconditioned residual */
     double tol, in_tot[2];           /* CG_ETOL; 1 / number of unknowns */
 } pvk_mcg;
 
@@ -221,12 +225,11 @@ void pvk_mom_matvec(const pvk_grid *g, const pvk_phys *ph, int stage, const pvk_
 /* fused momentum Jacobi-PCG for the components with nb[c] > 0 */
 void pvk_mcg_init(const pvk_grid *g, const pvk_phys *ph, int stage, pvk_scal *sc, const pvk_mcg *w,
                   hipStream_t s);
-/* pc = 1: z_0 = M r_0 into d[c][0] and <r_0, z_0> after pvk_mcg_init; after the
- * loop, the final residual back into r[c] when it ended in r2[c] */
-void pvk_mcg_pc_start(const pvk_grid *g, const pvk_mcg *w, hipStream_t s);
-void pvk_mcg_pc_finish(const pvk_grid *g, const pvk_scal *sc, const pvk_mcg *w, hipStream_t s);
-void pvk_mcg_iter(const pvk_grid *g, const pvk_phys *ph, int stage, pvk_scal *sc, const pvk_mcg *w,
-                  int half, int n, hipStream_t s);
+/* half 0 of iteration n forms d_n and A d_n and makes the x step of iteration
+ * n - 1; half 1 makes the r step.  The half 0 that finds the solve stopped makes
+ * the last x step, so a solve ends with a half 0 (at n = maxit at the latest). */
+void pvk_mcg_iter(const pvk_grid *g, const pvk_phys *ph, pvk_scal *sc, const pvk_mcg *w, int half, int n,
+                  hipStream_t s);
 
 /* ---- pressure ---- */
 void pvk_p_rhs2(const pvk_grid *g, int stage, const pvk_scal *sc, const double *u, const double *v,

@@ -924,14 +924,6 @@ template <typename T, int NB> __device__ __forceinline__ void blk_diag(const CGe
     }
 }
 
-// A barrier that orders LDS alone: loads from memory stay in flight across it.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // half-sweeps; each ends with a barrier (a colour's cells read only the other
 // colour, whose last writes a barrier has already ordered)
 template <int K, typename T, int NB> __device__ __forceinline__ void sweep_red0(const CGeo &g, T *x, Blk<T> (&k)[NB])

@@ -192,50 +192,58 @@ __device__ __forceinline__ R harm(R a, R b) { return R(2.0) * (a) * (b) / ((a) +
 template <class R = double>
 __device__ __forceinline__ R avg2(R a, R b) { return R(0.5) * ((a) + (b)); }
 
+// Viscosity at corner (i, j), the lower left one of cell (i, j): for u the harmonic mean over y of
+// the means over x (msolve_cg.c:103-249), for v the harmonic mean over x of the means over y.
+template <class R = double>
+__device__ __forceinline__ R mom_corner(const pvk_grid &g, const double *mu, int comp, int i, int j)
+{
+    const int P = g.P;
+    const R c = R(AT(mu, i, j)), w = R(AT(mu, i - 1, j)), s = R(AT(mu, i, j - 1)), sw = R(AT(mu, i - 1, j - 1));
+    return comp == 0 ? harm<R>(avg2<R>(w, c), avg2<R>(sw, s)) : harm<R>(avg2<R>(s, c), avg2<R>(sw, w));
+}
+// rho at the face / (alpha_k dt)
+template <class R = double>
+__device__ __forceinline__ R mom_time(const pvk_grid &g, double alpha_k, double dt, const double *rho, int comp, int i,
+                                      int j)
+{
+    const int P = g.P;
+    const R rho_face = R(0.5) * (R(AT(rho, i, j)) + R(comp == 0 ? AT(rho, i - 1, j) : AT(rho, i, j - 1)));
+    return rho_face / (R(alpha_k) * R(dt));
+}
+
 // Jacobi diagonal (lsolver/msolve_cg.c:103-249) and operator (:255-493).
+// comp 0 = u, 1 = v.
 template <class R = double>
 __device__ __forceinline__ R mom_diag(const pvk_grid &g, const pvk_phys &ph, double alpha_k, double dt,
                                       const double *rho, const double *mu, int comp, int i, int j)
 {
     const int P = g.P;
     const R iRe = R(ph.iRe);
-    R rho_face, d_time, dx, dy;
-    if (comp == 'u') {
-        rho_face = R(0.5) * (R(AT(rho, i, j)) + R(AT(rho, i - 1, j)));
-        d_time = rho_face / (R(alpha_k) * R(dt));
+    const R d_time = mom_time<R>(g, alpha_k, dt, rho, comp, i, j);
+    R dx, dy;
+    if (comp == 0) {
         R mu_xp = R(AT(mu, i, j)), mu_xm = R(AT(mu, i - 1, j));
-        R mu_yp = harm<R>(avg2<R>(R(AT(mu, i - 1, j + 1)), R(AT(mu, i, j + 1))), avg2<R>(R(AT(mu, i - 1, j)), R(AT(mu, i, j))));
-        R mu_ym = harm<R>(avg2<R>(R(AT(mu, i - 1, j)), R(AT(mu, i, j))), avg2<R>(R(AT(mu, i - 1, j - 1)), R(AT(mu, i, j - 1))));
+        R mu_yp = mom_corner<R>(g, mu, 0, i, j + 1), mu_ym = mom_corner<R>(g, mu, 0, i, j);
         dx = iRe * ((mu_xp * R(g.idx_u[i]) + mu_xm * R(g.idx_u[i - 1])) * R(g.idx_c[i - 1]));
         dy = iRe * (mu_yp * R(g.idy_c[j]) + mu_ym * R(g.idy_c[j - 1])) * R(g.idy_v[j]);
     } else {
-        rho_face = R(0.5) * (R(AT(rho, i, j)) + R(AT(rho, i, j - 1)));
-        d_time = rho_face / (R(alpha_k) * R(dt));
         R mu_yp = R(AT(mu, i, j)), mu_ym = R(AT(mu, i, j - 1));
-        R mu_xp = harm<R>(avg2<R>(R(AT(mu, i + 1, j - 1)), R(AT(mu, i + 1, j))), avg2<R>(R(AT(mu, i, j - 1)), R(AT(mu, i, j))));
-        R mu_xm = harm<R>(avg2<R>(R(AT(mu, i, j - 1)), R(AT(mu, i, j))), avg2<R>(R(AT(mu, i - 1, j - 1)), R(AT(mu, i - 1, j))));
+        R mu_xp = mom_corner<R>(g, mu, 1, i + 1, j), mu_xm = mom_corner<R>(g, mu, 1, i, j);
         dx = iRe * ((mu_xp * R(g.idx_c[i]) + mu_xm * R(g.idx_c[i - 1])) * R(g.idx_u[i]));
         dy = iRe * (mu_yp * R(g.idy_v[j]) + mu_ym * R(g.idy_v[j - 1])) * R(g.idy_c[j - 1]);
     }
     return d_time + dx + dy + R(0.0) + R(0.0);
 }
 
-// The operator with the five x values supplied (centre, E, W, N, S).
+// The operator with the face factors (time, viscosities) and the five x
+// values supplied (centre, E, W, N, S).
 template <class R = double>
-__device__ __forceinline__ R mom_op_vals(const pvk_grid &g, const pvk_phys &ph, double alpha_k, double dt,
-                                         const double *rho, const double *mu, int comp, int i, int j, R xc, R xE,
-                                         R xW, R xN, R xS)
+__device__ __forceinline__ R mom_op_flux(const pvk_grid &g, R iRe, int comp, int i, int j, R factor_time, R mu_xp,
+                                         R mu_xm, R mu_yp, R mu_ym, R xc, R xE, R xW, R xN, R xS)
 {
-    const int P = g.P;
-    const R iRe = R(ph.iRe);
     R op = R(0.0);
+    R Ax_val = factor_time * xc;
     if (comp == 0) {
-        R rho_face = R(0.5) * (R(AT(rho, i, j)) + R(AT(rho, i - 1, j)));
-        R factor_time = rho_face / (R(alpha_k) * R(dt));
-        R Ax_val = factor_time * xc;
-        R mu_xp = R(AT(mu, i, j)), mu_xm = R(AT(mu, i - 1, j));
-        R mu_yp = harm<R>(avg2<R>(R(AT(mu, i - 1, j + 1)), R(AT(mu, i, j + 1))), avg2<R>(R(AT(mu, i - 1, j)), R(AT(mu, i, j))));
-        R mu_ym = harm<R>(avg2<R>(R(AT(mu, i - 1, j)), R(AT(mu, i, j))), avg2<R>(R(AT(mu, i - 1, j - 1)), R(AT(mu, i, j - 1))));
         R flux_xp = mu_xp * (xE - xc) * R(g.idx_u[i]);
         R flux_xm = mu_xm * (xc - xW) * R(g.idx_u[i - 1]);
         R flux_yp = mu_yp * (xN - xc) * R(g.idy_c[j]);
@@ -245,12 +253,6 @@ __device__ __forceinline__ R mom_op_vals(const pvk_grid &g, const pvk_phys &ph, 
         op += R(0.0);
         return Ax_val - op;
     }
-    R rho_face = R(0.5) * (R(AT(rho, i, j)) + R(AT(rho, i, j - 1)));
-    R factor_time = rho_face / (R(alpha_k) * R(dt));
-    R Ax_val = factor_time * xc;
-    R mu_yp = R(AT(mu, i, j)), mu_ym = R(AT(mu, i, j - 1));
-    R mu_xp = harm<R>(avg2<R>(R(AT(mu, i + 1, j - 1)), R(AT(mu, i + 1, j))), avg2<R>(R(AT(mu, i, j - 1)), R(AT(mu, i, j))));
-    R mu_xm = harm<R>(avg2<R>(R(AT(mu, i, j - 1)), R(AT(mu, i, j))), avg2<R>(R(AT(mu, i - 1, j - 1)), R(AT(mu, i - 1, j))));
     R flux_xp = mu_xp * (xE - xc) * R(g.idx_c[i]);
     R flux_xm = mu_xm * (xc - xW) * R(g.idx_c[i - 1]);
     R flux_yp = mu_yp * (xN - xc) * R(g.idy_v[j]);
@@ -258,6 +260,21 @@ __device__ __forceinline__ R mom_op_vals(const pvk_grid &g, const pvk_phys &ph, 
     op += iRe * ((flux_xp - flux_xm) * R(g.idx_u[i]));
     op += iRe * (flux_yp - flux_ym) * R(g.idy_c[j - 1]);
     return Ax_val - op;
+}
+
+// The same with the factors formed from rho and mu.
+template <class R = double>
+__device__ __forceinline__ R mom_op_vals(const pvk_grid &g, const pvk_phys &ph, double alpha_k, double dt,
+                                         const double *rho, const double *mu, int comp, int i, int j, R xc, R xE,
+                                         R xW, R xN, R xS)
+{
+    const int P = g.P;
+    const R ft = mom_time<R>(g, alpha_k, dt, rho, comp, i, j);
+    if (comp == 0)
+        return mom_op_flux<R>(g, R(ph.iRe), 0, i, j, ft, R(AT(mu, i, j)), R(AT(mu, i - 1, j)),
+                              mom_corner<R>(g, mu, 0, i, j + 1), mom_corner<R>(g, mu, 0, i, j), xc, xE, xW, xN, xS);
+    return mom_op_flux<R>(g, R(ph.iRe), 1, i, j, ft, mom_corner<R>(g, mu, 1, i + 1, j), mom_corner<R>(g, mu, 1, i, j),
+                          R(AT(mu, i, j)), R(AT(mu, i, j - 1)), xc, xE, xW, xN, xS);
 }
 
 // The operator's coefficients at (i, j) in FP32 (centre, E, W, N, S):
@@ -268,14 +285,10 @@ __device__ __forceinline__ void mom_coeffs(const pvk_grid &g, const pvk_phys &ph
 {
     const int P = g.P;
     const float iRe = float(ph.iRe);
+    c[0] = mom_time<float>(g, alpha_k, dt, rho, comp, i, j);
     if (comp == 0) {
-        const float rho_face = 0.5f * (float(AT(rho, i, j)) + float(AT(rho, i - 1, j)));
-        c[0] = rho_face / (float(alpha_k) * float(dt));
         const float mu_xp = float(AT(mu, i, j)), mu_xm = float(AT(mu, i - 1, j));
-        const float mu_yp = harm<float>(avg2<float>(float(AT(mu, i - 1, j + 1)), float(AT(mu, i, j + 1))),
-                                        avg2<float>(float(AT(mu, i - 1, j)), float(AT(mu, i, j))));
-        const float mu_ym = harm<float>(avg2<float>(float(AT(mu, i - 1, j)), float(AT(mu, i, j))),
-                                        avg2<float>(float(AT(mu, i - 1, j - 1)), float(AT(mu, i, j - 1))));
+        const float mu_yp = mom_corner<float>(g, mu, 0, i, j + 1), mu_ym = mom_corner<float>(g, mu, 0, i, j);
         const float sx = iRe * float(g.idx_c[i - 1]), sy = iRe * float(g.idy_v[j]);
         c[1] = sx * (mu_xp * float(g.idx_u[i]));
         c[2] = sx * (mu_xm * float(g.idx_u[i - 1]));
@@ -283,13 +296,8 @@ __device__ __forceinline__ void mom_coeffs(const pvk_grid &g, const pvk_phys &ph
         c[4] = sy * (mu_ym * float(g.idy_c[j - 1]));
         return;
     }
-    const float rho_face = 0.5f * (float(AT(rho, i, j)) + float(AT(rho, i, j - 1)));
-    c[0] = rho_face / (float(alpha_k) * float(dt));
     const float mu_yp = float(AT(mu, i, j)), mu_ym = float(AT(mu, i, j - 1));
-    const float mu_xp = harm<float>(avg2<float>(float(AT(mu, i + 1, j - 1)), float(AT(mu, i + 1, j))),
-                                    avg2<float>(float(AT(mu, i, j - 1)), float(AT(mu, i, j))));
-    const float mu_xm = harm<float>(avg2<float>(float(AT(mu, i, j - 1)), float(AT(mu, i, j))),
-                                    avg2<float>(float(AT(mu, i - 1, j - 1)), float(AT(mu, i - 1, j))));
+    const float mu_xp = mom_corner<float>(g, mu, 1, i + 1, j), mu_xm = mom_corner<float>(g, mu, 1, i, j);
     const float sx = iRe * float(g.idx_u[i]), sy = iRe * float(g.idy_c[j - 1]);
     c[1] = sx * (mu_xp * float(g.idx_c[i]));
     c[2] = sx * (mu_xm * float(g.idx_c[i - 1]));

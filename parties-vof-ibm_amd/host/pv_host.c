@@ -332,10 +332,16 @@ int pv_cg_create(pv_bag *b)
         b->mcg.dad[c] = q; q += nbk;
         b->mcg.rr[c] = q; q += nbk;
         b->mcg.nb[c] = (c ? ny - 1 + mband - 1 : ny + mband - 1) / mband;
-        /* coefficient k of component c: half (k & 1) of field MCF(3c + k / 2),
-         * each half NYM rows of pitch P floats from the field's cell (0, 0) */
+        /* FP32 form: coefficient k of component c is half (k & 1) of field
+         * MCF(3c + k / 2), each half NYM rows of pitch P floats from the field's
+         * cell (0, 0); the diagonal is the sixth half and A d takes the FP64
+         * diagonal's field.  FP64 form: two of the same fields */
         for (int k = 0; k < 5; k++)
             b->mcg.cf[c][k] = (float *)b->f[PV_FI_MCF0 + 3 * c + k / 2] + (size_t)(k & 1) * ny * b->g.P;
+        b->mcg.dgf[c] = (float *)b->f[PV_FI_MCF0 + 3 * c + 2] + (size_t)ny * b->g.P;
+        b->mcg.Adf[c] = (float *)b->f[c ? PV_FI_DG_V : PV_FI_DG_U];
+        b->mcg.ft[c] = b->f[PV_FI_MCF0 + 3 * c];
+        b->mcg.mc[c] = b->f[PV_FI_MCF0 + 3 * c + 1];
     }
     return PV_OK;
 }

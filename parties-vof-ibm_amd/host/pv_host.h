@@ -8,7 +8,7 @@
 
 /* device-only work arrays after the public fields */
 enum pv_internal_field {
-    PV_FI_DG_U = PV_NFIELDS,   /* Jacobi diagonal + EPS, u (msolve_cg.c:103-249) */
+    PV_FI_DG_U = PV_NFIELDS,   /* Jacobi diagonal + EPS, u (msolve_cg.c:103-249); FP32 form: A d */
     PV_FI_DG_V,                /* same, v */
     PV_FI_TMP,                 /* scratch */
     PV_FI_Z,                   /* preconditioned residual of the pressure PCG */
@@ -30,15 +30,15 @@ enum pv_internal_field {
     PV_FI_MV2,
     PV_FI_MUS,                 /* u and v before the momentum solve */
     PV_FI_MVS,
-    PV_FI_MCF0,                /* FP32 momentum operator coefficients, two arrays per field: */
-    PV_FI_MCF1,                /* u in MCF0..2, v in MCF3..5 (five used of six each) */
+    PV_FI_MCF0,                /* momentum operator coefficients, u in MCF0..2, v in MCF3..5: FP32 */
+    PV_FI_MCF1,                /* form two arrays per field (with the diagonal), FP64 form one */
     PV_FI_MCF2,
     PV_FI_MCF3,
     PV_FI_MCF4,
     PV_FI_MCF5,
-    PV_FI_MZU,                 /* momentum polynomial preconditioner: z of u and v ... */
+    PV_FI_MZU,                 /* momentum PCG: preconditioned residuals of u and v ... */
     PV_FI_MZV,
-    PV_FI_MRU2,                /* ... and the residuals of odd iterations */
+    PV_FI_MRU2,                /* ... and, polynomial preconditioner, the residuals of odd iterations */
     PV_FI_MRV2,
     PV_FI_END
 };

@@ -340,15 +340,14 @@ static int mom_solve(pv_bag *b, int mask)
     chunk = (mask & 1) ? b->mom_chunk[0] : b->mom_chunk[1];
     if ((mask & 2) && b->mom_chunk[1] > chunk) chunk = b->mom_chunk[1];
     pvk_mcg_init(G(b), &b->ph, st, b->d_sc, &w, S(b));
-    if (w.pc) pvk_mcg_pc_start(G(b), &w, S(b));
     for (;;) {
         int k, done = 1;
         for (k = 0; k < chunk && n <= maxn; k++, n++) {
             pv_tbegin(b, PV_T_MOM_APPLY);
-            pvk_mcg_iter(G(b), &b->ph, st, b->d_sc, &w, 0, n, S(b));
+            pvk_mcg_iter(G(b), &b->ph, b->d_sc, &w, 0, n, S(b));
             pv_tend(b, PV_T_MOM_APPLY);
             pv_tbegin(b, PV_T_MOM_UPDATE);
-            pvk_mcg_iter(G(b), &b->ph, st, b->d_sc, &w, 1, n, S(b));
+            pvk_mcg_iter(G(b), &b->ph, b->d_sc, &w, 1, n, S(b));
             pv_tend(b, PV_T_MOM_UPDATE);
         }
         LAUNCHCHK();
@@ -358,10 +357,6 @@ static int mom_solve(pv_bag *b, int mask)
         if (done) break;
         if (n > maxn) return pv_set_error(PV_EHIP, "momentum CG did not stop (device flag)");
         chunk = 2;
-    }
-    if (w.pc) {
-        pvk_mcg_pc_finish(G(b), b->d_sc, &w, S(b));
-        LAUNCHCHK();
     }
     for (c = 0; c < 2; c++) {
         if (!(mask & (1 << c))) continue;
@@ -1299,8 +1294,8 @@ static int mom_time(pv_bag *b, int iters, float *ms)
         hipEventRecord(e0, S(b));
         pvk_mcg_init(G(b), &b->ph, b->stage, b->d_sc, &w, S(b));
         for (n = 0; n <= iters; n++) {
-            pvk_mcg_iter(G(b), &b->ph, b->stage, b->d_sc, &w, 0, n, S(b));
-            pvk_mcg_iter(G(b), &b->ph, b->stage, b->d_sc, &w, 1, n, S(b));
+            pvk_mcg_iter(G(b), &b->ph, b->d_sc, &w, 0, n, S(b));
+            pvk_mcg_iter(G(b), &b->ph, b->d_sc, &w, 1, n, S(b));
         }
         hipEventRecord(e1, S(b));
         if (hipGetLastError() != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||

@@ -102,3 +102,49 @@ def test_fft_rows_and_columns(lib, nx, ny):
     got, ref = s.get("SCRATCH1")[R], o.get("SCRATCH1")[R]
     assert np.isfinite(got).all()
     assert relerr(got, ref) < 1e-10
+
+
+# columns: less than a chunk of 256, one short of one, exactly one, one over,
+# two and a remainder; rows: every remainder of the bands of 1, 2 and 4 rows
+# of u (NYM rows) and v (NYM - 1)
+@pytest.mark.parametrize("nx,ny", [(16, 8), (96, 11), (255, 9), (256, 8), (257, 13), (520, 10)])
+@pytest.mark.parametrize("rows", [1, 2, 4])
+@pytest.mark.parametrize("form", ["fp64", "mixed", "mixed_pc"])
+def test_momentum_cg(lib, nx, ny, rows, form):
+    """Five iterations from a random start over random densities and
+    viscosities: x against the oracle's, and in FP64, where the path is the
+    same to rounding, r and A d.  The polynomial preconditioner takes another
+    path, so it is solved out on both sides and the velocity compared.  The diagonal dominates (dt / dx^2 below 1), so
+    rounding is not amplified: FP64 order of sums 1e-11, FP32 operator 1e-5."""
+    pc = form == "mixed_pc"
+    kw = dict(CG_ETOL=1e-11, CG_MAXIT=200) if pc else dict(CG_ETOL=1e-30, CG_MAXIT=5)
+    p = params(nx, ny, pressure_solver=pvof.PV_PSOLVE_JACOBI_PCG, **kw)
+    pm = params(nx, ny, pressure_solver=pvof.PV_PSOLVE_JACOBI_PCG,
+                precision=pvof.PV_PREC_FP64 if form == "fp64" else pvof.PV_PREC_MIXED, **kw)
+    o, s = oracle_lib.Oracle(p), pvof.Solver(pm, lib)
+    rng = np.random.default_rng(nx * ny + rows)
+    fields = dict(RHO=canonical(p, rng.uniform(0.5, 1.0, (ny, nx))), MU=canonical(p, rng.uniform(0.1, 1.0, (ny, nx))))
+    for f in ("U", "V", "U_RHS", "V_RHS"):
+        fields[f] = rng.standard_normal(o.shape) * (1e4 if "RHS" in f else 1.0)
+    for x in (o, s):
+        for f, a in fields.items():
+            x.set(f, a)
+        x.call("set_time_state", 0.0, 2e-4, 2e-4, 2)
+    s.check(lib.pv_set_momentum_rows(s.h, rows))
+    if pc:
+        s.check(lib.pv_set_momentum_preconditioner(s.h, 1))
+        s.check(lib.pv_set_momentum_cg_steps(s.h, 1))
+        o.call("set_momentum_cg_steps", 1)
+    R = regions(p)
+    tol = 1e-11 if form == "fp64" else 1e-5
+    for c in ("u", "v"):
+        n, it = o.call("Velocity_solve_cg", ord(c)), C.c_int()
+        s.call("Velocity_solve_cg", ord(c), C.byref(it))
+        names = [c.upper()]
+        if not pc:
+            assert n == it.value == 5
+        if form == "fp64":
+            names += [c.upper() + q for q in ("_R", "_AD")]
+        for f in names:
+            assert np.isfinite(s.get(f)).all()
+            assert relerr(s.get(f)[R[c]], o.get(f)[R[c]]) < tol, (f, relerr(s.get(f)[R[c]], o.get(f)[R[c]]))
