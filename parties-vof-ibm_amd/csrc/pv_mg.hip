@@ -63,15 +63,6 @@ template <typename T> __device__ __forceinline__ T fget(const Lev<T> &L, const d
     return r0 ? (T)r0[(ptrdiff_t)j * p0 + i] : ld(L.f, L.pitch, i, j);
 }
 
-// the CG step of iteration n folded into the level-0 pre-smoothing:
-// r_{n+1} = r_n - alpha (A d_n - mean(A d_n)), phi += alpha d_n
-struct MgStep {
-    const double *Ad, *d;
-    double *phi, *rnew;
-    double alpha, mad;
-    bool on;
-};
-
 // stop test of CG iteration n on the <r, r> partials (as k_transpose):
 // n = -1 sets the reference norm, n = -2 keeps it (warm restart).  The
 // partials of r_{n+1} come from the level-0 pre-smoothing (rrt, per tile)
@@ -92,211 +83,231 @@ __device__ void mg_stop_test(pvk_scal *sc, const pvk_pcg &w, int n, double tol, 
 }
 
 // ---------------------------------------------------------------------------
+// 2 x 2 blocks of cells (one coarse cell each), what a thread of the smoothing
+// kernels owns: cells a (2I, 2J) and d (2I+1, 2J+1) are red, b (2I+1, 2J)
+// and c (2I, 2J+1) black; faces between them, to the left (la, lc), right
+// (br, dr), south (sa, sb) and north (nc, nd), 0 at a wall.  The faces, f,
+// 1 / diagonal and x stay in registers; LDS holds x, one array per colour
+// (row j, pair I at j hx + I: cells 2 I and 2 I + 1 of a row are one red,
+// (i + j) even, and one black), at offsets R and B of the array x.
+// ---------------------------------------------------------------------------
+template <typename T> struct Blk {
+    T ab, cd, la, lc, br, dr, ac, bd, sa, sb, nc, nd;
+    T ia, ib, ic, id, fa, fb, fc, fd, a, b, c, d;
+    int s, l, r, up, dn;            // slots of row 2J: own, left, right block; of rows 2J+2 and 2J-1
+    int I, J;
+    bool on;
+};
+
+// Two values of a row from column 2 I on, in one load: a smoothing level's
+// width and pitch are even and its arrays start on two values.
+template <typename T> __device__ __forceinline__ void ld2(const T *a, int pitch, int i, int j, T &v0, T &v1)
+{
+    typedef T T2 __attribute__((ext_vector_type(2)));
+    const T2 v = *(const T2 *)(a + (ptrdiff_t)j * pitch + i);
+    v0 = v.x;
+    v1 = v.y;
+}
+
+template <typename T> __device__ __forceinline__ void st2(T *a, int pitch, int i, int j, T v0, T v1)
+{
+    typedef T T2 __attribute__((ext_vector_type(2)));
+    T2 v;
+    v.x = v0;
+    v.y = v1;
+    *(T2 *)(a + (ptrdiff_t)j * pitch + i) = v;
+}
+
+// faces of the blocks: every load unconditional, from clamped positions; the
+// wall faces are masked in blk_diag
+template <typename T, int NB> __device__ __forceinline__ void blk_faces(const Lev<T> &L, Blk<T> (&k)[NB])
+{
+#pragma unroll
+    for (int u = 0; u < NB; u++) {
+        const int i = 2 * k[u].I, j = 2 * k[u].J, iw = (i == 0) ? L.nx - 1 : i - 1, p = L.pitch;
+        ld2(L.bx, p, i, j, k[u].ab, k[u].br);
+        ld2(L.bx, p, i, j + 1, k[u].cd, k[u].dr);
+        ld2(L.by, p, i, max(j - 1, 0), k[u].sa, k[u].sb);
+        ld2(L.by, p, i, j, k[u].ac, k[u].bd);
+        ld2(L.by, p, i, j + 1, k[u].nc, k[u].nd);
+        k[u].la = ld(L.bx, p, iw, j);
+        k[u].lc = ld(L.bx, p, iw, j + 1);
+    }
+}
+// 1 / b of the Gauss-Seidel update: FP64 divides; FP32 takes the hardware
+// reciprocal (1 ulp), which keeps the V-cycle a fixed symmetric operator
+// (both sweep directions use the same value)
+template <typename T> __device__ __forceinline__ T gs_rcp(T b) { return T(1) / b; }
+template <> __device__ __forceinline__ float gs_rcp<float>(float b) { return __builtin_amdgcn_rcpf(b); }
+
+// wall faces and 1 / diagonal (RCP: gs_rcp; else a division)
+template <bool RCP, typename T, int NB> __device__ __forceinline__ void blk_diag(int ny, Blk<T> (&k)[NB])
+{
+    auto inv = [](T b) { return RCP ? gs_rcp(b) : T(1) / b; };
+#pragma unroll
+    for (int u = 0; u < NB; u++) {
+        if (k[u].J == 0) k[u].sa = k[u].sb = T(0);
+        if (k[u].J + 1 == (ny >> 1)) k[u].nc = k[u].nd = T(0);
+        k[u].ia = inv(k[u].ab + k[u].la + k[u].ac + k[u].sa);
+        k[u].ib = inv(k[u].br + k[u].ab + k[u].bd + k[u].sb);
+        k[u].ic = inv(k[u].cd + k[u].lc + k[u].nc + k[u].ac);
+        k[u].id = inv(k[u].dr + k[u].cd + k[u].nd + k[u].bd);
+    }
+}
+
+// half-sweeps; each ends with a barrier (a colour's cells read only the other
+// colour, whose last writes a barrier has already ordered)
+template <int R, int B, typename T, int NB> __device__ __forceinline__ void sweep_red0(int hx, T *x, Blk<T> (&k)[NB])
+{
+#pragma unroll
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            x[R + k[u].s] = k[u].a = -k[u].fa * k[u].ia;
+            x[R + k[u].s + hx] = k[u].d = -k[u].fd * k[u].id;
+        }
+    lds_barrier();
+}
+template <int R, int B, typename T, int NB> __device__ __forceinline__ void sweep_red(int hx, T *x, Blk<T> (&k)[NB])
+{
+    const T *q = x + B;
+    T w[NB], s[NB], e[NB], n[NB];
+#pragma unroll
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            w[u] = q[k[u].l];
+            s[u] = q[k[u].dn];
+            e[u] = q[k[u].r + hx];
+            n[u] = q[k[u].up];
+        }
+#pragma unroll
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            k[u].a = (k[u].ab * k[u].b + k[u].la * w[u] + k[u].ac * k[u].c + k[u].sa * s[u] - k[u].fa) * k[u].ia;
+            k[u].d = (k[u].dr * e[u] + k[u].cd * k[u].c + k[u].nd * n[u] + k[u].bd * k[u].b - k[u].fd) * k[u].id;
+            x[R + k[u].s] = k[u].a;
+            x[R + k[u].s + hx] = k[u].d;
+        }
+    lds_barrier();
+}
+template <int R, int B, typename T, int NB> __device__ __forceinline__ void sweep_black(int hx, T *x, Blk<T> (&k)[NB])
+{
+    const T *q = x + R;
+    T e[NB], s[NB], w[NB], n[NB];
+#pragma unroll
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            e[u] = q[k[u].r];
+            s[u] = q[k[u].dn];
+            w[u] = q[k[u].l + hx];
+            n[u] = q[k[u].up];
+        }
+#pragma unroll
+    for (int u = 0; u < NB; u++)
+        if (k[u].on) {
+            k[u].b = (k[u].br * e[u] + k[u].ab * k[u].a + k[u].bd * k[u].d + k[u].sb * s[u] - k[u].fb) * k[u].ib;
+            k[u].c = (k[u].cd * k[u].d + k[u].lc * w[u] + k[u].nc * n[u] + k[u].ac * k[u].a - k[u].fc) * k[u].ic;
+            x[B + k[u].s] = k[u].b;
+            x[B + k[u].s + hx] = k[u].c;
+        }
+    lds_barrier();
+}
+// the four residuals f - A x of a block
+template <int R, int B, typename T>
+__device__ __forceinline__ void blk_residual(int hx, const T *x, const Blk<T> &k, T &ra, T &rb, T &rc, T &rd)
+{
+    const T a = k.a, b = k.b, c = k.c, d = k.d, *r = x + R, *q = x + B;
+    ra = k.fa - (k.ab * (b - a) - k.la * (a - q[k.l]) + k.ac * (c - a) - k.sa * (a - q[k.dn]));
+    rd = k.fd - (k.dr * (q[k.r + hx] - d) - k.cd * (d - c) + k.nd * (q[k.up] - d) - k.bd * (d - b));
+    rb = k.fb - (k.br * (r[k.r] - b) - k.ab * (b - a) + k.bd * (d - b) - k.sb * (b - r[k.dn]));
+    rc = k.fc - (k.cd * (d - c) - k.lc * (c - r[k.l + hx]) + k.nc * (r[k.up] - c) - k.ac * (c - a));
+}
+
+// ---------------------------------------------------------------------------
 // Fused smoothing of one level (levels with more than PVK_MG_LDS_CELLS cells).
-// A block owns a core tile of TX x TY cells (64 x 16 on levels wider than
-// 512, 32 x 16 up to 512, 32 x 8 up to 256: smaller tiles, more blocks, on
+// A workgroup owns a core tile of TX x TY cells (64 x 16 on levels wider than
+// 512, 32 x 16 up to 512, 32 x 8 up to 256: smaller tiles, more workgroups, on
 // the levels whose time is latency) and works on it extended by a halo of 2 nu
-// cells (periodic in x, cut at the walls in y): half-sweep k updates the
-// cells of its colour at distance >= k from the extended edge, so after
-// 2 nu half-sweeps the core (and the ring the residual needs) holds exactly
-// what sweeping the whole level would give.  f, the face coefficients and
-// 1 / (their sum) stay in registers, x in LDS.
+// cells (periodic in x, cut at the walls in y): half-sweep k is right on the
+// cells at distance >= k from the extended edge (the others read an own value
+// where a neighbour would be), so after 2 nu half-sweeps the core (and the ring
+// the residual needs) holds exactly what sweeping the whole level would give.
+//
+// A thread owns one 2 x 2 block of the extended tile, two on the widest tile.
+// What bounds these kernels on large levels is instruction issue.  With a
+// thread a cell (half the lanes idle in each half-sweep, four LDS reads an
+// update, five loads, a column modulo and a position a cell) a launch took,
+// pre and post, FP32, 21.7 and 15.4 us at 1024^2, 75 and 33 at 2048^2; with
+// blocks 14.7 and 10.9, 58 and 26: the rate of the memory they touch (62 and
+// 27 MB at 1024^2) within a factor of two, at 2048^2 4.2 TB/s.
 // ---------------------------------------------------------------------------
 template <int NU, int SH> struct MgTile {
     static constexpr int TX = (SH == 0) ? 64 : 32;    // core tile
     static constexpr int TY = (SH == 2) ? 8 : 16;
     static constexpr int H = 2 * NU;                  // halo
-    static constexpr int W = TX + 2 * H;              // extended width
-    static constexpr int HT = TY + 2 * H;          // extended height
-    static constexpr int NC = W * HT;
-    static constexpr int K = (NC + NTH - 1) / NTH;    // cells per thread
-    static constexpr int KC = (TX * TY + NTH - 1) / NTH; // core cells per thread
+    static constexpr int HX = (TX + 2 * H) / 2;       // blocks a row of the extended tile
+    static constexpr int HY = (TY + 2 * H) / 2;       // rows of blocks
+    static constexpr int NBLK = HX * HY;
+    static constexpr int NB = (NBLK + NTH - 1) / NTH; // blocks per thread
+    static constexpr int R = 0, B = 2 * NBLK;         // x by colour
+    static constexpr int KC = (TX * TY + NTH - 1) / NTH; // core cells per thread, row by row
 };
 
-// is extended-tile cell (lx, ly) in the core, and in the level (x0 + lx the
-// unwrapped column)?
-template <int NU, int SH> __device__ __forceinline__ bool tile_core(int lx, int ly, int x0, int gj, int nx, int ny)
-{
-    using TT = MgTile<NU, SH>;
-    return lx >= TT::H && lx < TT::H + TT::TX && ly >= TT::H && ly < TT::H + TT::TY && x0 + lx < nx && gj < ny;
-}
-
-// Column and row in the level of extended-tile cell c (clamped into the
-// tile and, for rows, into the level: a cell outside it is masked later).
-template <int NU, int SH>
-__device__ __forceinline__ void tile_cell(int c, int x0, int y0, int nx, int ny, int &gi, int &gj)
-{
-    using TT = MgTile<NU, SH>;
-    c = min(c, TT::NC - 1);
-    const int ly = c / TT::W, lx = c - ly * TT::W;
-    gj = min(max(y0 + ly, 0), ny - 1);
-    gi = (x0 + lx) % nx;
-    if (gi < 0) gi += nx;
-}
-
-// is extended-tile cell c a cell of the level?
-template <int NU, int SH> __device__ __forceinline__ bool tile_in(int c, int y0, int ny)
-{
-    using TT = MgTile<NU, SH>;
-    const int gj = y0 + c / TT::W;
-    return c < TT::NC && gj >= 0 && gj < ny;
-}
-
-// The raw faces of this thread's cells of the extended tile.  Every load is
-// unconditional, from indices clamped into the level (the face arrays hold
-// every row, wall rows included), so the loads issue back to back with no
-// wait between them; tile_mask zeroes what lies outside the level or on a
-// wall once they have arrived.
+// Positions of this thread's blocks: slots in the tile (at its edge and at a
+// wall the own slot: finite, and not used or times a face of 0), columns wrapped
+// into the level and rows clamped into it (off outside: those slots are never read).
+// The mask of blocks in the core: bit u.
 template <int NU, int SH, typename T>
-__device__ __forceinline__ void tile_faces(const Lev<T> &L, int x0, int y0, T *ce, T *cw, T *cn, T *cs)
+__device__ __forceinline__ int tile_place(int nx, int ny, int bx, int by, Blk<T> (&k)[MgTile<NU, SH>::NB])
 {
     using TT = MgTile<NU, SH>;
-    const int p = L.pitch;
+    const int hx = nx >> 1, hy = ny >> 1;
+    int core = 0;
 #pragma unroll
-    for (int u = 0; u < TT::K; u++) {
-        int gi, gj;
-        tile_cell<NU, SH>(threadIdx.x + u * NTH, x0, y0, L.nx, L.ny, gi, gj);
-        const int giw = (gi == 0) ? L.nx - 1 : gi - 1;
-        ce[u] = ld(L.bx, p, gi, gj);
-        cw[u] = ld(L.bx, p, giw, gj);
-        cn[u] = ld(L.by, p, gi, gj);
-        cs[u] = ld(L.by, p, gi, max(gj - 1, 0));
-    }
-}
-
-// The level's right-hand side of this thread's cells of the extended tile
-// (raw, unconditional loads as tile_faces).
-template <int NU, int SH, typename T>
-__device__ __forceinline__ void tile_rhs(const Lev<T> &L, const double *r0, int p0, int x0, int y0, T *f)
-{
-    using TT = MgTile<NU, SH>;
-    if (r0) {
-#pragma unroll
-        for (int u = 0; u < TT::K; u++) {
-            int gi, gj;
-            tile_cell<NU, SH>(threadIdx.x + u * NTH, x0, y0, L.nx, L.ny, gi, gj);
-            f[u] = (T)r0[(ptrdiff_t)gj * p0 + gi];
+    for (int u = 0; u < TT::NB; u++) {
+        const int q = min((int)threadIdx.x + u * NTH, TT::NBLK - 1), j = q / TT::HX, i = q - j * TT::HX;
+        const int gi = bx * (TT::TX / 2) + i - TT::H / 2, gj = by * (TT::TY / 2) + j - TT::H / 2;
+        int I = gi < 0 ? gi + hx : (gi >= hx ? gi - hx : gi);
+        if (hx < TT::HX) {                              // a level narrower than the tile: round it more than once
+            I %= hx;
+            if (I < 0) I += hx;
         }
-    } else {
+        k[u].on = (int)threadIdx.x + u * NTH < TT::NBLK && gj >= 0 && gj < hy;
+        k[u].I = I;
+        k[u].J = min(max(gj, 0), hy - 1);
+        k[u].s = 2 * j * TT::HX + i;
+        k[u].l = k[u].s - (i > 0);
+        k[u].r = k[u].s + (i + 1 < TT::HX);
+        k[u].dn = (j == 0 || gj <= 0) ? k[u].s : k[u].s - TT::HX;
+        k[u].up = (j + 1 == TT::HY || gj + 1 >= hy) ? k[u].s : k[u].s + 2 * TT::HX;
+        if (k[u].on && i >= TT::H / 2 && i < (TT::H + TT::TX) / 2 && j >= TT::H / 2 && j < (TT::H + TT::TY) / 2 && gi < hx)
+            core |= 1 << u;
+    }
+    return core;
+}
+
+// f of the blocks: the level's, or from the FP64 field r0
+template <typename T, int NB>
+__device__ __forceinline__ void blk_rhs(const Lev<T> &L, const double *r0, int p0, Blk<T> (&k)[NB])
+{
 #pragma unroll
-        for (int u = 0; u < TT::K; u++) {
-            int gi, gj;
-            tile_cell<NU, SH>(threadIdx.x + u * NTH, x0, y0, L.nx, L.ny, gi, gj);
-            f[u] = ld(L.f, L.pitch, gi, gj);
+    for (int u = 0; u < NB; u++) {
+        const int i = 2 * k[u].I, j = 2 * k[u].J;
+        if (r0) {
+            double a, b, c, d;
+            ld2(r0, p0, i, j, a, b);
+            ld2(r0, p0, i, j + 1, c, d);
+            k[u].fa = (T)a;
+            k[u].fb = (T)b;
+            k[u].fc = (T)c;
+            k[u].fd = (T)d;
+        } else {
+            ld2(L.f, L.pitch, i, j, k[u].fa, k[u].fb);
+            ld2(L.f, L.pitch, i, j + 1, k[u].fc, k[u].fd);
         }
     }
 }
 
-// Zero f and the faces outside the level and the wall faces, and form
-// 1 / (sum of the faces).
-template <int NU, int SH, typename T>
-__device__ __forceinline__ void tile_mask(int y0, int ny, T *f, T *ce, T *cw, T *cn, T *cs, T *id)
-{
-    using TT = MgTile<NU, SH>;
-#pragma unroll
-    for (int u = 0; u < TT::K; u++) {
-        const int c = threadIdx.x + u * NTH, gj = y0 + c / TT::W;
-        const bool in = tile_in<NU, SH>(c, y0, ny);
-        f[u] = in ? f[u] : T(0);
-        ce[u] = in ? ce[u] : T(0);
-        cw[u] = in ? cw[u] : T(0);
-        cn[u] = (in && gj + 1 < ny) ? cn[u] : T(0);
-        cs[u] = (in && gj > 0) ? cs[u] : T(0);
-        id[u] = in ? T(1) / (ce[u] + cw[u] + cn[u] + cs[u]) : T(0);
-    }
-}
-
-// The CG step's loads of the level-0 pre-smoothing: r_n and A d_n of this
-// thread's cells of the extended tile (ra, aa; before the step's scalars
-// are summed, in flight meanwhile), then d_n and phi of its cells of the core
-// (core cell q = threadIdx.x + k NTH, row-major in the core: dd, pp; in
-// flight while f is formed).  Every load is unconditional, from an index
-// clamped into the level (cells outside it are masked when the values are
-// used), so the loads issue back to back with no wait between them.
-template <int NU, int SH, typename T>
-__device__ __forceinline__ void tile_step_loads(const Lev<T> &L, const double *r0, int p0, const MgStep &st,
-                                                int x0, int y0, double *ra, double *aa)
-{
-    using TT = MgTile<NU, SH>;
-#pragma unroll
-    for (int u = 0; u < TT::K; u++) {
-        int gi, gj;
-        tile_cell<NU, SH>(threadIdx.x + u * NTH, x0, y0, L.nx, L.ny, gi, gj);
-        const size_t idx = (size_t)gj * p0 + gi;
-        ra[u] = r0[idx];
-        aa[u] = st.Ad[idx];
-    }
-}
-
-template <int NU, int SH, typename T>
-__device__ __forceinline__ void tile_step_core_loads(const Lev<T> &L, int p0, const MgStep &st, int bx, int by,
-                                                     double *dd, double *pp)
-{
-    using TT = MgTile<NU, SH>;
-#pragma unroll
-    for (int k = 0; k < TT::KC; k++) {
-        const int q = min(threadIdx.x + k * NTH, TT::TX * TT::TY - 1), ly = q / TT::TX, lx = q - ly * TT::TX;
-        const int gi = min(bx * TT::TX + lx, L.nx - 1), gj = min(by * TT::TY + ly, L.ny - 1);
-        const size_t idx = (size_t)gj * p0 + gi;
-        dd[k] = st.d[idx];
-        pp[k] = st.phi[idx];
-    }
-}
-
-// f = r_{n+1} = r_n - alpha (A d_n - mean) of this thread's cells of the
-// extended tile from the step's loads (tile_mask zeroes it outside the
-// level); the core cells' r_{n+1} also go to rl (FP64, row-major in the
-// core) for the core pass.
-template <int NU, int SH, typename T>
-__device__ __forceinline__ void tile_rhs_step(const Lev<T> &L, const MgStep &st, int x0, int y0, const double *ra,
-                                              const double *aa, T *f, double *rl)
-{
-    using TT = MgTile<NU, SH>;
-#pragma unroll
-    for (int u = 0; u < TT::K; u++) {
-        const int c = threadIdx.x + u * NTH, ly = c / TT::W, lx = c - ly * TT::W, gj = y0 + ly;
-        const double rn = ra[u] - st.alpha * (aa[u] - st.mad);
-        f[u] = (T)rn;
-        if (tile_in<NU, SH>(c, y0, L.ny) && tile_core<NU, SH>(lx, ly, x0, gj, L.nx, L.ny))
-            rl[(ly - TT::H) * TT::TX + lx - TT::H] = rn;
-    }
-}
-
-// the core pass of the CG step: r_{n+1} (from rl) to rnew, phi += alpha d_n,
-// and this thread's share of <r_{n+1}, r_{n+1}>
-template <int NU, int SH, typename T>
-__device__ __forceinline__ double tile_step_core(const Lev<T> &L, int p0, const MgStep &st, int bx, int by,
-                                                 const double *dd, const double *pp, const double *rl)
-{
-    using TT = MgTile<NU, SH>;
-    double acc = 0.0;
-#pragma unroll
-    for (int k = 0; k < TT::KC; k++) {
-        const int q = threadIdx.x + k * NTH, ly = q / TT::TX, lx = q - ly * TT::TX;
-        const int gi = bx * TT::TX + lx, gj = by * TT::TY + ly;
-        if (q < TT::TX * TT::TY && gi < L.nx && gj < L.ny) {
-            const size_t idx = (size_t)gj * p0 + gi;
-            const double rn = rl[q];
-            st.rnew[idx] = rn;
-            st.phi[idx] = pp[k] + st.alpha * dd[k];
-            acc += rn * rn;
-        }
-    }
-    return acc;
-}
-
-// f, faces and 1 / (their sum) of this thread's cells of the extended tile:
-// every global load of the smoothing is in this one batch.
-template <int NU, int SH, typename T>
-__device__ __forceinline__ void tile_coeffs(const Lev<T> &L, const double *r0, int p0, int x0, int y0, T *f,
-                                            T *ce, T *cw, T *cn, T *cs, T *id)
-{
-    tile_faces<NU, SH>(L, x0, y0, ce, cw, cn, cs);
-    tile_rhs<NU, SH>(L, r0, p0, x0, y0, f);
-    tile_mask<NU, SH>(y0, L.ny, f, ce, cw, cn, cs, id);
-}
-
-// tile of this block, XCD-aware (consecutive tiles of a run share an L2)
+// tile of this workgroup, XCD-aware (consecutive tiles of a run share an L2)
 __device__ __forceinline__ void tile_of(int &bx, int &by)
 {
     const int t = xcd_band(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
@@ -304,120 +315,126 @@ __device__ __forceinline__ void tile_of(int &bx, int &by)
     bx = t - by * gridDim.x;
 }
 
-// half-sweep k of colour col on the cells at distance >= k from the edge
-template <int NU, int SH, typename T>
-__device__ __forceinline__ void tile_sweep(T *xs, int x0, int y0, int ny, int k, int col, const T *f, const T *ce,
-                                           const T *cw, const T *cn, const T *cs, const T *id)
+// core cell q = threadIdx.x + m NTH, row by row: its place in the core and in
+// the level (clamped into it); is it a cell of the level?
+template <int NU, int SH>
+__device__ __forceinline__ bool core_cell(int m, int bx, int by, int nx, int ny, int &q, int &gi, int &gj)
 {
     using TT = MgTile<NU, SH>;
-    T v[TT::K];
-    bool act[TT::K];
-#pragma unroll
-    for (int u = 0; u < TT::K; u++) {
-        const int c = threadIdx.x + u * NTH, ly = c / TT::W, lx = c - ly * TT::W, gj = y0 + ly;
-        act[u] = c < TT::NC && gj >= 0 && gj < ny && (((x0 + lx + gj) & 1) == col) && lx >= k && lx < TT::W - k &&
-                 ly >= k && ly < TT::HT - k;
-        v[u] = T(0);
-        if (act[u]) {
-            const T xe = (k > 0) ? xs[c + 1] : T(0), xw = (k > 0) ? xs[c - 1] : T(0);
-            const T xn = (k > 0) ? xs[c + TT::W] : T(0), xq = (k > 0) ? xs[c - TT::W] : T(0);
-            v[u] = (ce[u] * xe + cw[u] * xw + cn[u] * xn + cs[u] * xq - f[u]) * id[u];
-        }
-    }
-    // a colour's cells read only the other colour: no barrier before writing
-#pragma unroll
-    for (int u = 0; u < TT::K; u++)
-        if (act[u]) xs[threadIdx.x + u * NTH] = v[u];
-    __syncthreads();
+    const int t = threadIdx.x + m * NTH;
+    q = min(t, TT::TX * TT::TY - 1);
+    const int ly = q / TT::TX, lx = q - ly * TT::TX, x = bx * TT::TX + lx, y = by * TT::TY + ly;
+    gi = min(x, nx - 1);
+    gj = min(y, ny - 1);
+    return t < TT::TX * TT::TY && x < nx && y < ny;
 }
 
 // pre-smoothing from x = 0 and restriction of the residual; the stop test of
 // iteration n in block (0, 0) (check: the kernel after the one that formed
 // the residual).  On level 0 with step (CG iteration n >= 0) the kernel
-// first does the CG step: f = r_{n+1} is formed on the fly from r_n = r0
-// (tile and halo), and the core writes r_{n+1} to rnew, phi += alpha d and
-// the partial <r_{n+1}, r_{n+1}> of the tile.
+// first does the CG step: f = r_{n+1} = r_n - alpha (A d_n - mean) is formed on
+// the fly from r_n = r0 (tile and halo), and the core writes r_{n+1} to rnew,
+// phi += alpha d and the partial <r_{n+1}, r_{n+1}> of the tile.  The red x of
+// the core goes to xp (the post kernel reads it with halos while it writes x;
+// its first half-sweep overwrites the black), row j of it holding the row's
+// reds side by side.
 template <int NU, int SH, typename T>
 __global__ void __launch_bounds__(NTH, sizeof(T) == 4 ? 4 : 3) k_mg_pre(Lev<T> L, Lev<T> C, const double *r0, double *rnew, int p0,
                                                pvk_scal *sc, pvk_pcg w, int n, double tol, int maxit, int check,
                                                int step, int ncell)
 {
     using TT = MgTile<NU, SH>;
-    __shared__ T xs[TT::NC];
-    __shared__ double rl[TT::TX * TT::TY];      // r_{n+1} of the core; then rs
+    constexpr int R = TT::R, B = TT::B, NB = TT::NB, KC = TT::KC;
+    __shared__ T x[4 * TT::NBLK];
+    __shared__ __align__(16) double rl[TT::TX * TT::TY];      // r_{n+1} of the core
     __shared__ double sh[3 * NTH];
-    T *rs = (T *)rl;                              // core residual, after the sweeps
     if (sc->p_done) return;
     if (check && n != -3 && blockIdx.x == 0 && blockIdx.y == 0) mg_stop_test(sc, w, n, tol, maxit, sh);
     int bx, by;
     tile_of(bx, by);
-    const int x0 = bx * TT::TX - TT::H, y0 = by * TT::TY - TT::H;
-    T f[TT::K], ce[TT::K], cw[TT::K], cn[TT::K], cs[TT::K], id[TT::K];
-    MgStep st;
-    st.on = step && n >= 0;
-    st.Ad = w.Ad;
-    st.d = w.d[n & 1];
-    st.phi = w.phi;
-    st.rnew = rnew;
-    st.alpha = st.mad = 0.0;
+    Blk<T> k[NB];
+    const int core = tile_place<NU, SH>(L.nx, L.ny, bx, by, k);
+    const bool on = step && n >= 0;
     double acc = 0.0;
-    if (st.on) {
+    blk_faces(L, k);
+    if (on) {
         // the tile's loads go out first and are in flight while the step's
-        // scalars are summed (the three sums' loads together); nothing
-        // waits on memory before the sums
-        double ra[TT::K], aa[TT::K], dd[TT::KC], pp[TT::KC];
-        tile_faces<NU, SH>(L, x0, y0, ce, cw, cn, cs);
-        tile_step_loads<NU, SH>(L, r0, p0, st, x0, y0, ra, aa);
+        // scalars are summed (the three sums' loads together), the core's
+        // d_n and phi while f is formed; every load is unconditional
+        double r[NB][4], a[NB][4], dd[KC], pp[KC];
+        const double *d = w.d[n & 1];
+        double *phi = w.phi;
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            const int i = 2 * k[u].I, j = 2 * k[u].J;
+            ld2(r0, p0, i, j, r[u][0], r[u][1]);
+            ld2(r0, p0, i, j + 1, r[u][2], r[u][3]);
+            ld2(w.Ad, p0, i, j, a[u][0], a[u][1]);
+            ld2(w.Ad, p0, i, j + 1, a[u][2], a[u][3]);
+        }
         double rz, dad, sad;
         block_sum3(w.rz[n & 1], w.nrz, w.dad[n & 1], w.ndad, w.sad, w.ndad, sh, rz, dad, sad);
-        st.alpha = rz / dad;
-        st.mad = sad / (double)ncell;
-        tile_step_core_loads<NU, SH>(L, p0, st, bx, by, dd, pp);
-        tile_rhs_step<NU, SH>(L, st, x0, y0, ra, aa, f, rl);
-        tile_mask<NU, SH>(y0, L.ny, f, ce, cw, cn, cs, id);
-        for (int c = threadIdx.x; c < TT::NC; c += NTH) xs[c] = T(0);
-        __syncthreads();
-        // (rs, on rl's memory, is written after the sweeps' barriers)
-        acc = tile_step_core<NU, SH>(L, p0, st, bx, by, dd, pp, rl);
+        const double alpha = rz / dad, mad = sad / (double)ncell;
+#pragma unroll
+        for (int m = 0; m < KC; m++) {
+            int q, gi, gj;
+            core_cell<NU, SH>(m, bx, by, L.nx, L.ny, q, gi, gj);
+            const size_t idx = (size_t)gj * p0 + gi;
+            dd[m] = d[idx];
+            pp[m] = phi[idx];
+        }
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) r[u][e] -= alpha * (a[u][e] - mad);
+            k[u].fa = (T)r[u][0];
+            k[u].fb = (T)r[u][1];
+            k[u].fc = (T)r[u][2];
+            k[u].fd = (T)r[u][3];
+            if (core >> u & 1) {
+                const int j = k[u].s / TT::HX - TT::H, i = 2 * (k[u].s % TT::HX) - TT::H;
+                st2(rl, TT::TX, i, j, r[u][0], r[u][1]);
+                st2(rl, TT::TX, i, j + 1, r[u][2], r[u][3]);
+            }
+        }
+        blk_diag<false>(L.ny, k);
+        sweep_red0<R, B>(TT::HX, x, k);         // its barrier orders rl too
+#pragma unroll
+        for (int m = 0; m < KC; m++) {
+            int q, gi, gj;
+            if (core_cell<NU, SH>(m, bx, by, L.nx, L.ny, q, gi, gj)) {
+                const size_t idx = (size_t)gj * p0 + gi;
+                const double rn = rl[q];
+                rnew[idx] = rn;
+                phi[idx] = pp[m] + alpha * dd[m];
+                acc += rn * rn;
+            }
+        }
     } else {
-        tile_coeffs<NU, SH>(L, r0, p0, x0, y0, f, ce, cw, cn, cs, id);
-        for (int c = threadIdx.x; c < TT::NC; c += NTH) xs[c] = T(0);
-        __syncthreads();
+        blk_rhs(L, r0, p0, k);
+        blk_diag<false>(L.ny, k);
+        sweep_red0<R, B>(TT::HX, x, k);
     }
-    for (int k = 0; k < 2 * NU; k++) tile_sweep<NU, SH>(xs, x0, y0, L.ny, k, k & 1, f, ce, cw, cn, cs, id);
-    // residual f - A x of each core cell from the registers (a wall face is
-    // 0 there) to rs, and the core of x for the post-smoothing (to xp: the
-    // post kernel reads it with halos while it writes x)
+    sweep_black<R, B>(TT::HX, x, k);
+    if constexpr (NU == 2) {
+        sweep_red<R, B>(TT::HX, x, k);
+        sweep_black<R, B>(TT::HX, x, k);
+    }
 #pragma unroll
-    for (int u = 0; u < TT::K; u++) {
-        const int c = threadIdx.x + u * NTH, ly = c / TT::W, lx = c - ly * TT::W, gj = y0 + ly;
-        if (c < TT::NC && gj >= 0 && tile_core<NU, SH>(lx, ly, x0, gj, L.nx, L.ny)) {
-            const T x0c = xs[c];
-            rs[(ly - TT::H) * TT::TX + lx - TT::H] =
-                f[u] - (ce[u] * (xs[c + 1] - x0c) - cw[u] * (x0c - xs[c - 1]) + cn[u] * (xs[c + TT::W] - x0c) -
-                        cs[u] * (x0c - xs[c - TT::W]));
-            L.xp[(ptrdiff_t)gj * L.pitch + x0 + lx] = x0c;
+    for (int u = 0; u < NB; u++)
+        if (core >> u & 1) {                    // a core block's coarse cell is its own
+            T ra, rb, rc, rd;
+            blk_residual<R, B>(TT::HX, x, k[u], ra, rb, rc, rd);
+            C.f[(ptrdiff_t)k[u].J * C.pitch + k[u].I] = ra + rb + rc + rd;
+            T *xp = L.xp + (ptrdiff_t)(2 * k[u].J) * L.pitch + k[u].I;
+            xp[0] = k[u].a;
+            xp[L.pitch] = k[u].d;
         }
-    }
-    __syncthreads();
-    // restriction: one coarse cell per thread (TT::TX/2 x TT::TY/2 <= NTH)
-    if ((int)threadIdx.x < (TT::TX / 2) * (TT::TY / 2)) {
-        const int I = threadIdx.x % (TT::TX / 2), J = threadIdx.x / (TT::TX / 2);
-        const int gI = bx * (TT::TX / 2) + I, gJ = by * (TT::TY / 2) + J;
-        if (gI < C.nx && gJ < C.ny) {
-            T s = T(0);
-#pragma unroll
-            for (int dj = 0; dj < 2; dj++)
-#pragma unroll
-                for (int di = 0; di < 2; di++) s += rs[(2 * J + dj) * TT::TX + 2 * I + di];
-            C.f[(ptrdiff_t)gJ * C.pitch + gI] = s;
-        }
-    }
-    if (st.on) block_store_partial(acc, w.rrt, by * gridDim.x + bx, sh);
+    if (on) block_store_partial(acc, w.rrt, by * gridDim.x + bx, sh);
 }
 
-// coarse correction xp + xc(parent) and post-smoothing (black first); the
-// result goes to x, or to the FP64 z0 on level 0 of the FP32 V-cycle.  The
+// coarse correction xp + xc(parent) and post-smoothing (black first, so only
+// the red xp is there); the result goes to x, or to the FP64 z0 on level 0 of the FP32 V-cycle.  The
 // input (xp) and the output are separate arrays: a block reads its halo from
 // the neighbouring tiles' cores, which their blocks overwrite, and when the
 // level has more tiles than the GPU holds at once those blocks may already
@@ -428,51 +445,59 @@ __global__ void __launch_bounds__(NTH, sizeof(T) == 4 ? 4 : 3) k_mg_post(Lev<T> 
                                                 const pvk_scal *sc, pvk_pcg w, int dot, int slot)
 {
     using TT = MgTile<NU, SH>;
-    __shared__ T xs[TT::NC];
+    constexpr int R = TT::R, B = TT::B, NB = TT::NB, KC = TT::KC;
+    __shared__ T x[4 * TT::NBLK];
     __shared__ double sh[NTH];
     if (sc->p_done) return;
     int bx, by;
     tile_of(bx, by);
-    const int x0 = bx * TT::TX - TT::H, y0 = by * TT::TY - TT::H;
-    T f[TT::K], ce[TT::K], cw[TT::K], cn[TT::K], cs[TT::K], id[TT::K], xa[TT::K], xb[TT::K];
-    double fd[TT::KC];
-    // every global load of the kernel first, unconditional (clamped indices)
-    tile_faces<NU, SH>(L, x0, y0, ce, cw, cn, cs);
-    tile_rhs<NU, SH>(L, r0, p0, x0, y0, f);
+    Blk<T> k[NB];
+    tile_place<NU, SH>(L.nx, L.ny, bx, by, k);
+    // every global load of the kernel first, unconditional (clamped positions)
+    T xc[NB];
+    double fd[KC];
+    blk_faces(L, k);
+    blk_rhs(L, r0, p0, k);
 #pragma unroll
-    for (int u = 0; u < TT::K; u++) {           // x = xp + the parent's correction
-        int gi, gj;
-        tile_cell<NU, SH>(threadIdx.x + u * NTH, x0, y0, L.nx, L.ny, gi, gj);
-        xa[u] = ld(L.xp, L.pitch, gi, gj);
-        xb[u] = ld(C.x, C.pitch, gi >> 1, gj >> 1);
+    for (int u = 0; u < NB; u++) {
+        const T *xp = L.xp + (ptrdiff_t)(2 * k[u].J) * L.pitch + k[u].I;
+        k[u].a = xp[0];
+        k[u].d = xp[L.pitch];
+        xc[u] = ld(C.x, C.pitch, k[u].I, k[u].J);
     }
 #pragma unroll
-    for (int k = 0; k < TT::KC; k++) {          // the core's f for the dot
-        fd[k] = 0.0;
+    for (int m = 0; m < KC; m++) {              // the core's f for the dot
+        fd[m] = 0.0;
         if (dot) {
-            const int q = min(threadIdx.x + k * NTH, TT::TX * TT::TY - 1), ly = q / TT::TX, lx = q - ly * TT::TX;
-            const int gi = min(bx * TT::TX + lx, L.nx - 1), gj = min(by * TT::TY + ly, L.ny - 1);
-            fd[k] = r0 ? r0[(ptrdiff_t)gj * p0 + gi] : (double)ld(L.f, L.pitch, gi, gj);
+            int q, gi, gj;
+            core_cell<NU, SH>(m, bx, by, L.nx, L.ny, q, gi, gj);
+            fd[m] = r0 ? r0[(ptrdiff_t)gj * p0 + gi] : (double)ld(L.f, L.pitch, gi, gj);
         }
     }
-    tile_mask<NU, SH>(y0, L.ny, f, ce, cw, cn, cs, id);
+    blk_diag<false>(L.ny, k);
 #pragma unroll
-    for (int u = 0; u < TT::K; u++) {
-        const int c = threadIdx.x + u * NTH;
-        if (c < TT::NC) xs[c] = tile_in<NU, SH>(c, y0, L.ny) ? xa[u] + xb[u] : T(0);
+    for (int u = 0; u < NB; u++)                // x = xp + the parent's correction
+        if (k[u].on) {
+            x[R + k[u].s] = k[u].a = k[u].a + xc[u];
+            x[R + k[u].s + TT::HX] = k[u].d = k[u].d + xc[u];
+        }
+    lds_barrier();
+    sweep_black<R, B>(TT::HX, x, k);
+    sweep_red<R, B>(TT::HX, x, k);
+    if constexpr (NU == 2) {
+        sweep_black<R, B>(TT::HX, x, k);
+        sweep_red<R, B>(TT::HX, x, k);
     }
-    __syncthreads();
-    for (int k = 1; k <= 2 * NU; k++) tile_sweep<NU, SH>(xs, x0, y0, L.ny, k, k & 1, f, ce, cw, cn, cs, id);
     double acc = 0.0;
 #pragma unroll
-    for (int k = 0; k < TT::KC; k++) {
-        const int c = threadIdx.x + k * NTH, ly = c / TT::TX, lx = c - ly * TT::TX;
-        const int gi = bx * TT::TX + lx, gj = by * TT::TY + ly;
-        if (c < TT::TX * TT::TY && gi < L.nx && gj < L.ny) {
-            const T v = xs[(ly + TT::H) * TT::W + lx + TT::H];
+    for (int m = 0; m < KC; m++) {
+        int q, gi, gj;
+        if (core_cell<NU, SH>(m, bx, by, L.nx, L.ny, q, gi, gj)) {
+            const int ly = q / TT::TX + TT::H, lx = q % TT::TX + TT::H;
+            const T v = x[(((lx + ly) & 1) ? B : R) + ly * TT::HX + (lx >> 1)];
             if (z0) z0[(ptrdiff_t)gj * p0 + gi] = (double)v;
             else L.x[(ptrdiff_t)gj * L.pitch + gi] = v;
-            if (dot) acc += fd[k] * (double)v;
+            if (dot) acc += fd[m] * (double)v;
         }
     }
     if (dot) block_store_partial(acc, w.rz[slot], by * gridDim.x + bx, sh);
@@ -815,12 +840,6 @@ static_assert(PVK_MG_LOW <= 3, "k_mg_coarse is instantiated for up to three smoo
 
 __device__ __forceinline__ int ilog2_or_neg(int n) { return (n > 0 && (n & (n - 1)) == 0) ? __ffs(n) - 1 : -1; }
 
-// 1 / b of the Gauss-Seidel update: FP64 divides; FP32 takes the hardware
-// reciprocal (1 ulp), which keeps the V-cycle a fixed symmetric operator
-// (both sweep directions use the same value)
-template <typename T> __device__ __forceinline__ T gs_rcp(T b) { return T(1) / b; }
-template <> __device__ __forceinline__ float gs_rcp<float>(float b) { return __builtin_amdgcn_rcpf(b); }
-
 // In-LDS layout, in units of T and at fixed places (the most a level can
 // need), so an access is an index register and an immediate offset: smoothing
 // level K's red and black x (row j, pair I at j hx + I: cells 2 I and 2 I + 1
@@ -844,17 +863,6 @@ struct CGeo {
     int nx, ny, hx, nblk;           // cells, blocks a row, blocks
 };
 
-// a 2 x 2 block: cells a (2I, 2J) and d (2I+1, 2J+1) are red, b (2I+1, 2J)
-// and c (2I, 2J+1) black; faces between them, to the left (la, lc), right
-// (br, dr), south (sa, sb) and north (nc, nd), 0 at a wall
-template <typename T> struct Blk {
-    T ab, cd, la, lc, br, dr, ac, bd, sa, sb, nc, nd;
-    T ia, ib, ic, id, fa, fb, fc, fd, a, b, c, d;
-    int s, l, r, up, dn;            // slots of row 2J: own, left, right block; of rows 2J+2 and 2J-1
-    int I, J;
-    bool on;
-};
-
 // The blocks' positions.  A neighbour beyond a wall has face 0; its slot is
 // the block's own (finite once the level has been swept, and 0 times it is 0).
 template <typename T, int NB> __device__ __forceinline__ void blk_place(const CGeo &g, Blk<T> (&k)[NB])
@@ -876,110 +884,6 @@ template <typename T, int NB> __device__ __forceinline__ void blk_place(const CG
     }
 }
 
-// Two values of a row from column 2 I on, in one load: a smoothing level's
-// width and pitch are even and its arrays start on two values.
-template <typename T> __device__ __forceinline__ void ld2(const T *a, int pitch, int i, int j, T &v0, T &v1)
-{
-    typedef T T2 __attribute__((ext_vector_type(2)));
-    const T2 v = *(const T2 *)(a + (ptrdiff_t)j * pitch + i);
-    v0 = v.x;
-    v1 = v.y;
-}
-
-template <typename T> __device__ __forceinline__ void st2(T *a, int pitch, int i, int j, T v0, T v1)
-{
-    typedef T T2 __attribute__((ext_vector_type(2)));
-    T2 v;
-    v.x = v0;
-    v.y = v1;
-    *(T2 *)(a + (ptrdiff_t)j * pitch + i) = v;
-}
-
-// faces of the blocks: every load unconditional, from clamped positions; the
-// wall faces are masked in blk_diag
-template <typename T, int NB> __device__ __forceinline__ void blk_faces(const Lev<T> &L, Blk<T> (&k)[NB])
-{
-#pragma unroll
-    for (int u = 0; u < NB; u++) {
-        const int i = 2 * k[u].I, j = 2 * k[u].J, iw = (i == 0) ? L.nx - 1 : i - 1, p = L.pitch;
-        ld2(L.bx, p, i, j, k[u].ab, k[u].br);
-        ld2(L.bx, p, i, j + 1, k[u].cd, k[u].dr);
-        ld2(L.by, p, i, max(j - 1, 0), k[u].sa, k[u].sb);
-        ld2(L.by, p, i, j, k[u].ac, k[u].bd);
-        ld2(L.by, p, i, j + 1, k[u].nc, k[u].nd);
-        k[u].la = ld(L.bx, p, iw, j);
-        k[u].lc = ld(L.bx, p, iw, j + 1);
-    }
-}
-template <typename T, int NB> __device__ __forceinline__ void blk_diag(const CGeo &g, Blk<T> (&k)[NB])
-{
-#pragma unroll
-    for (int u = 0; u < NB; u++) {
-        if (k[u].J == 0) k[u].sa = k[u].sb = T(0);
-        if (k[u].J + 1 == (g.ny >> 1)) k[u].nc = k[u].nd = T(0);
-        k[u].ia = gs_rcp(k[u].ab + k[u].la + k[u].ac + k[u].sa);
-        k[u].ib = gs_rcp(k[u].br + k[u].ab + k[u].bd + k[u].sb);
-        k[u].ic = gs_rcp(k[u].cd + k[u].lc + k[u].nc + k[u].ac);
-        k[u].id = gs_rcp(k[u].dr + k[u].cd + k[u].nd + k[u].bd);
-    }
-}
-
-// half-sweeps; each ends with a barrier (a colour's cells read only the other
-// colour, whose last writes a barrier has already ordered)
-template <int K, typename T, int NB> __device__ __forceinline__ void sweep_red0(const CGeo &g, T *x, Blk<T> (&k)[NB])
-{
-#pragma unroll
-    for (int u = 0; u < NB; u++)
-        if (k[u].on) {
-            x[CLds<K>::R + k[u].s] = k[u].a = -k[u].fa * k[u].ia;
-            x[CLds<K>::R + k[u].s + g.hx] = k[u].d = -k[u].fd * k[u].id;
-        }
-    lds_barrier();
-}
-template <int K, typename T, int NB> __device__ __forceinline__ void sweep_red(const CGeo &g, T *x, Blk<T> (&k)[NB])
-{
-    const T *B = x + CLds<K>::B;
-    T w[NB], s[NB], e[NB], n[NB];
-#pragma unroll
-    for (int u = 0; u < NB; u++)
-        if (k[u].on) {
-            w[u] = B[k[u].l];
-            s[u] = B[k[u].dn];
-            e[u] = B[k[u].r + g.hx];
-            n[u] = B[k[u].up];
-        }
-#pragma unroll
-    for (int u = 0; u < NB; u++)
-        if (k[u].on) {
-            k[u].a = (k[u].ab * k[u].b + k[u].la * w[u] + k[u].ac * k[u].c + k[u].sa * s[u] - k[u].fa) * k[u].ia;
-            k[u].d = (k[u].dr * e[u] + k[u].cd * k[u].c + k[u].nd * n[u] + k[u].bd * k[u].b - k[u].fd) * k[u].id;
-            x[CLds<K>::R + k[u].s] = k[u].a;
-            x[CLds<K>::R + k[u].s + g.hx] = k[u].d;
-        }
-    lds_barrier();
-}
-template <int K, typename T, int NB> __device__ __forceinline__ void sweep_black(const CGeo &g, T *x, Blk<T> (&k)[NB])
-{
-    const T *R = x + CLds<K>::R;
-    T e[NB], s[NB], w[NB], n[NB];
-#pragma unroll
-    for (int u = 0; u < NB; u++)
-        if (k[u].on) {
-            e[u] = R[k[u].r];
-            s[u] = R[k[u].dn];
-            w[u] = R[k[u].l + g.hx];
-            n[u] = R[k[u].up];
-        }
-#pragma unroll
-    for (int u = 0; u < NB; u++)
-        if (k[u].on) {
-            k[u].b = (k[u].br * e[u] + k[u].ab * k[u].a + k[u].bd * k[u].d + k[u].sb * s[u] - k[u].fb) * k[u].ib;
-            k[u].c = (k[u].cd * k[u].d + k[u].lc * w[u] + k[u].nc * n[u] + k[u].ac * k[u].a - k[u].fc) * k[u].ic;
-            x[CLds<K>::B + k[u].s] = k[u].b;
-            x[CLds<K>::B + k[u].s + g.hx] = k[u].c;
-        }
-    lds_barrier();
-}
 // the first black half-sweep after the coarse correction: the red neighbours
 // are read as x + x_coarse(their parent); the red cells themselves need not be
 // corrected, the red half-sweep that follows overwrites them
@@ -1021,15 +925,11 @@ __device__ __forceinline__ void sweep_black_corr(const CGeo &g, T *x, Blk<T> (&k
 template <int K, bool BOT, typename T, int NB>
 __device__ __forceinline__ void restrict_res(const CGeo &g, T *x, const Blk<T> (&k)[NB], double *bf)
 {
-    const T *R = x + CLds<K>::R, *B = x + CLds<K>::B;
 #pragma unroll
     for (int u = 0; u < NB; u++)
         if (k[u].on) {
-            const T a = k[u].a, b = k[u].b, c = k[u].c, d = k[u].d;
-            const T ra = k[u].fa - (k[u].ab * (b - a) - k[u].la * (a - B[k[u].l]) + k[u].ac * (c - a) - k[u].sa * (a - B[k[u].dn]));
-            const T rd = k[u].fd - (k[u].dr * (B[k[u].r + g.hx] - d) - k[u].cd * (d - c) + k[u].nd * (B[k[u].up] - d) - k[u].bd * (d - b));
-            const T rb = k[u].fb - (k[u].br * (R[k[u].r] - b) - k[u].ab * (b - a) + k[u].bd * (d - b) - k[u].sb * (b - R[k[u].dn]));
-            const T rc = k[u].fc - (k[u].cd * (d - c) - k[u].lc * (c - R[k[u].l + g.hx]) + k[u].nc * (R[k[u].up] - c) - k[u].ac * (c - a));
+            T ra, rb, rc, rd;
+            blk_residual<CLds<K>::R, CLds<K>::B>(g.hx, x, k[u], ra, rb, rc, rd);
             const T v = (ra + rb) + (rd + rc);
             const int q = threadIdx.x + u * CT;
             if constexpr (BOT) bf[q] = (double)v;
@@ -1155,11 +1055,11 @@ __device__ __forceinline__ void cycle_level(const pvk_mg &m, CState<T, NL> &S, B
     }
     const int visits = 1 + ((m.wmask >> (m.c0 + K)) & 1);
     for (int v = 0; v < visits; v++) {
-        if (v == 0) sweep_red0<K>(g, x, k);
-        sweep_black<K>(g, x, k);
+        if (v == 0) sweep_red0<CLds<K>::R, CLds<K>::B>(g.hx, x, k);
+        sweep_black<CLds<K>::R, CLds<K>::B>(g.hx, x, k);
         for (int sw = 1; sw < m.nu; sw++) {
-            sweep_red<K>(g, x, k);
-            sweep_black<K>(g, x, k);
+            sweep_red<CLds<K>::R, CLds<K>::B>(g.hx, x, k);
+            sweep_black<CLds<K>::R, CLds<K>::B>(g.hx, x, k);
         }
         if constexpr (BOT) {
             const int n = S.g[NL].nx * S.g[NL].ny;
@@ -1168,10 +1068,10 @@ __device__ __forceinline__ void cycle_level(const pvk_mg &m, CState<T, NL> &S, B
         restrict_res<K, BOT>(g, x, k, S.bf);
         cycle<K + 1>(m, S);
         sweep_black_corr<K, BOT>(g, x, k);
-        sweep_red<K>(g, x, k);
+        sweep_red<CLds<K>::R, CLds<K>::B>(g.hx, x, k);
         for (int sw = 1; sw < m.nu; sw++) {
-            sweep_black<K>(g, x, k);
-            sweep_red<K>(g, x, k);
+            sweep_black<CLds<K>::R, CLds<K>::B>(g.hx, x, k);
+            sweep_red<CLds<K>::R, CLds<K>::B>(g.hx, x, k);
         }
     }
 }
@@ -1241,9 +1141,9 @@ template <typename T, int NL> __global__ void __launch_bounds__(CT) k_mg_coarse(
     }
     if constexpr (NL == 0) bottom_load(nbot, (const T *)m.H, bottom_col0(nbot), S.h);
     if (sc->p_done) return;
-    if constexpr (NL > 0) blk_diag(S.g[0], S.k0);
-    if constexpr (NL > 1) blk_diag(S.g[1], S.k1);
-    if constexpr (NL > 2) blk_diag(S.g[2], S.k2);
+    if constexpr (NL > 0) blk_diag<true>(S.g[0].ny, S.k0);
+    if constexpr (NL > 1) blk_diag<true>(S.g[1].ny, S.k1);
+    if constexpr (NL > 2) blk_diag<true>(S.g[2].ny, S.k2);
     __syncthreads();
     cycle<0>(m, S);
     if constexpr (NL == 0) {

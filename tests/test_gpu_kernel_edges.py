@@ -148,3 +148,37 @@ def test_momentum_cg(lib, nx, ny, rows, form):
         for f in names:
             assert np.isfinite(s.get(f)).all()
             assert relerr(s.get(f)[R[c]], o.get(f)[R[c]]) < tol, (f, relerr(s.get(f)[R[c]], o.get(f)[R[c]]))
+
+
+# tiled levels: narrower than a tile, the halo going round more than once
+# (16 x 1024), tiles of 32 x 8 with a part left over (200 x 56), of 32 x 16 with
+# one in both directions (400 x 40), and of 64 x 16 down to 32 x 16 (1056 x 64:
+# 1056, 528 and 264 wide)
+@pytest.mark.parametrize("nx,ny", [(16, 1024), (200, 56), (400, 40), (1056, 64)])
+@pytest.mark.parametrize("nu", [1, 2])
+@pytest.mark.parametrize("fp32", [0, 1])
+def test_tiled_levels(lib, nx, ny, nu, fp32):
+    """The V-cycle against the restatement, and a solve (whose level-0 kernel
+    makes the CG step) against the system it solves, with the tolerances the
+    other sizes have."""
+    p = params(nx, ny)
+    s = pvof.Solver(p, lib)
+    s.check(lib.pv_set_mg_sweeps(s.h, nu))
+    s.check(lib.pv_set_mg_precision(s.h, fp32))
+    rho = mg_ref.bubbles(nx, ny, seed=nx + ny, nb=6)
+    f = np.random.default_rng(nx * ny).standard_normal((ny, nx))
+    f -= f.mean()
+    s.set("RHO", canonical(p, rho))
+    s.set("P_RES", canonical(p, f))
+    s.call("mg_vcycle_apply")
+    R = regions(p)["cell"]
+    z = s.get("SCRATCH0")[R]
+    bx, by = mg_ref.faces(rho, float(nx * nx), float(nx * nx))
+    lv, G = mg_ref.build(bx, by)
+    assert relerr(z, mg_ref.vcycle(lv, G, f, nu)) < (1e-5 if fp32 else 1e-11)
+    s.set("P_RHS", canonical(p, f))
+    it = C.c_int()
+    s.call("Pressure_solve_cg", C.byref(it))
+    phi = s.get("PHI")[R]
+    assert 0 < it.value < p.p_max_iter
+    assert np.linalg.norm(mg_ref.apply_a(bx, by, phi) - f) <= 1.05e-10 * np.linalg.norm(f)
