@@ -100,56 +100,86 @@ __global__ void __launch_bounds__(NTH) k_pcg_faces(pvk_grid g, pvk_pcg w)
 
 // ---------------------------------------------------------------------------
 // K1: d_n = z + beta d_{n-1}, Ad = A d_n, partial <d_n, Ad>.  One block per
-// row j: the y neighbours and row clamps are block-uniform.
+// row j: the y neighbours and row clamps are block-uniform.  A thread's CPT
+// columns of the three rows are loaded ahead of the sums that give beta (all
+// blocks of a grid this size run at once, so nothing else covers them); its
+// row's east and west values go through LDS.  Bound by memory, 48 bytes a
+// cell: 11.9 us at 1024^2 (50 MB; 14.9 with every stencil
+// value formed from its own loads after the sums), 50 at 2048^2 (73), 6.6 at
+// 768 x 491 (10.6).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(NTH) k_pcg_apply(pvk_grid g, pvk_scal *sc, pvk_pcg w, int n)
+template <bool FIRST>
+__global__ void __launch_bounds__(NTH, 4) k_pcg_apply(pvk_grid g, pvk_scal *sc, pvk_pcg w, int n)
 {
     __shared__ double sh[2 * NTH];
+    __shared__ double sd[2][NTH * CPT + 2];
     if (sc->p_done) return;
-    const int P = g.P, NXM = g.NXM, NYM = g.NYM;
-    double beta = 0.0, sa, sb;
-    if (n > 0 && w.flex) {    // flexible CG: A-orthogonal to the previous direction only
-        block_sum2(w.zad, w.nrz, w.dad[(n + 1) & 1], w.ndad, sh, sa, sb);
-        beta = -sa / sb;
-    } else if (n > 0) {       // Fletcher-Reeves: gamma_n / gamma_{n-1}
-        block_sum2(w.rz[n & 1], w.nrz, w.rz[(n + 1) & 1], w.nrz, sh, sa, sb);
-        beta = sa / sb;
-    }
+    const int P = g.P, NXM = g.NXM, NYM = g.NYM, t = threadIdx.x;
     const double *__restrict__ z = w.z;
     const double *__restrict__ dold = w.d[(n + 1) & 1];
     const double *__restrict__ bx = w.bx, *__restrict__ by = w.by;
     double *__restrict__ dnew = w.d[n & 1];
     double *__restrict__ Ad = w.Ad;
     const int j = xcd_band(blockIdx.x, gridDim.x);
-    const int jn = (j + 1 == NYM) ? j : j + 1, js = (j == 0) ? 0 : j - 1;
+    const int jr[3] = {j, (j + 1 == NYM) ? j : j + 1, (j == 0) ? 0 : j - 1};
+    double zv[CPT][3], ov[CPT][3], cx[CPT][2], cy[CPT][2], ze, oe;
+    auto load = [&](int base) {
+#pragma unroll
+        for (int u = 0; u < CPT; u++)
+            if (base + u * NTH < NXM) {
+                const int i = min(base + u * NTH + t, NXM - 1);
+#pragma unroll
+                for (int r = 0; r < 3; r++) {
+                    zv[u][r] = AT(z, i, jr[r]);
+                    if (!FIRST) ov[u][r] = AT(dold, i, jr[r]);
+                }
+                cx[u][0] = AT(bx, i, j);
+                cx[u][1] = AT(bx, i - 1, j);
+                cy[u][0] = AT(by, i, j);
+                cy[u][1] = AT(by, i, j - 1);
+            }
+        if (t < 2) {                                 // the columns west and east of the chunk
+            const int e = base + NTH * CPT, ie = t ? (e < NXM ? e : 0) : (base ? base - 1 : NXM - 1);
+            ze = AT(z, ie, j);
+            if (!FIRST) oe = AT(dold, ie, j);
+        }
+    };
+    load(0);
+    double beta = 0.0, sa, sb;
+    if (!FIRST && w.flex) {   // flexible CG: A-orthogonal to the previous direction only
+        block_sum2(w.zad, w.nrz, w.dad[(n + 1) & 1], w.ndad, sh, sa, sb);
+        beta = -sa / sb;
+    } else if (!FIRST) {      // Fletcher-Reeves: gamma_n / gamma_{n-1}
+        block_sum2(w.rz[n & 1], w.nrz, w.rz[(n + 1) & 1], w.nrz, sh, sa, sb);
+        beta = sa / sb;
+    }
+    auto dn = [&](double zz, double oo) { return FIRST ? zz : zz + beta * oo; };
     double acc = 0.0, sacc = 0.0;
-    for (int base = 0; base < NXM; base += NTH * CPT) {
-        double dc[CPT], ad[CPT];
+    int par = 0;
+    for (int base = 0; base < NXM; base += NTH * CPT, par ^= 1) {
+        const int nc = min(NTH * CPT, NXM - base);
+        double dc[CPT];
+        if (base) load(base);
 #pragma unroll
-        for (int u = 0; u < CPT; u++) {
-            const int i = base + u * NTH + (int)threadIdx.x;
-            dc[u] = 0.0; ad[u] = 0.0;
-            if (i < NXM) {
-                const int ie = (i + 1 == NXM) ? 0 : i + 1, iw = (i == 0) ? NXM - 1 : i - 1;
-#define DN(ii, jj) (n == 0 ? AT(z, ii, jj) : AT(z, ii, jj) + beta * AT(dold, ii, jj))
-                const double d0 = DN(i, j), dE = DN(ie, j), dW = DN(iw, j), dN = DN(i, jn), dS = DN(i, js);
-#undef DN
-                const double cxp = AT(bx, i, j), cxm = AT(bx, i - 1, j);
-                const double cyp = AT(by, i, j), cym = AT(by, i, j - 1);
-                dc[u] = d0;
-                ad[u] = cxp * (dE - d0) - cxm * (d0 - dW) + cyp * (dN - d0) - cym * (d0 - dS);
+        for (int u = 0; u < CPT; u++)
+            if (u * NTH < nc) {
+                dc[u] = dn(zv[u][0], ov[u][0]);
+                if (u * NTH + t < nc) sd[par][u * NTH + t + 1] = dc[u];
             }
-        }
+        if (t < 2) sd[par][t ? nc + 1 : 0] = dn(ze, oe);
+        __syncthreads();
 #pragma unroll
-        for (int u = 0; u < CPT; u++) {
-            const int i = base + u * NTH + (int)threadIdx.x;
-            if (i < NXM) {
-                AT(dnew, i, j) = dc[u];
-                AT(Ad, i, j) = ad[u];
-                acc += dc[u] * ad[u];
-                sacc += ad[u];
+        for (int u = 0; u < CPT; u++)
+            if (u * NTH + t < nc) {
+                const int b = u * NTH + t, i = base + b;
+                const double d0 = dc[u], dE = sd[par][b + 2], dW = sd[par][b];
+                const double dN = dn(zv[u][1], ov[u][1]), dS = dn(zv[u][2], ov[u][2]);
+                const double ad = cx[u][0] * (dE - d0) - cx[u][1] * (d0 - dW) + cy[u][0] * (dN - d0) - cy[u][1] * (d0 - dS);
+                AT(dnew, i, j) = d0;
+                AT(Ad, i, j) = ad;
+                acc += d0 * ad;
+                sacc += ad;
             }
-        }
     }
     block_store_partial(acc, w.dad[n & 1], j, sh);
     if (w.sad) block_store_partial(sacc, w.sad, j, sh);
@@ -862,7 +892,8 @@ extern "C" void pvk_pcg_prep(const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w, 
 // K1 alone (d_n = z + beta d_{n-1}, Ad, <d_n, Ad>), for any preconditioner
 extern "C" void pvk_pcg_apply(const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w, int n, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_pcg_apply, dim3(g->NYM), dim3(NTH), 0, s, *g, sc, *w, n);
+    if (n == 0) hipLaunchKernelGGL(k_pcg_apply<true>, dim3(g->NYM), dim3(NTH), 0, s, *g, sc, *w, n);
+    else hipLaunchKernelGGL(k_pcg_apply<false>, dim3(g->NYM), dim3(NTH), 0, s, *g, sc, *w, n);
 }
 
 // ---------------------------------------------------------------------------
@@ -996,7 +1027,7 @@ extern "C" void pvk_pcg_stage(const pvk_grid *g, const pvk_fft *F, pvk_scal *sc,
 {
     switch (stage) {
     case 0:
-        hipLaunchKernelGGL(k_pcg_apply, dim3(g->NYM), dim3(NTH), 0, s, *g, sc, *w, n);
+        pvk_pcg_apply(g, sc, w, n, s);
         break;
     case 1:
         if (n >= 0) ROWS(FWD_STEP, n);

@@ -182,3 +182,30 @@ def test_tiled_levels(lib, nx, ny, nu, fp32):
     phi = s.get("PHI")[R]
     assert 0 < it.value < p.p_max_iter
     assert np.linalg.norm(mg_ref.apply_a(bx, by, phi) - f) <= 1.05e-10 * np.linalg.norm(f)
+
+
+# rows of less than a block (48), exactly one thread a column (256), a chunk of
+# 1024 columns and a part (1152) and two chunks (2048)
+@pytest.mark.parametrize("nx,ny", [(48, 43), (256, 9), (1152, 21), (2048, 13)])
+def test_pressure_apply_rows(lib, nx, ny):
+    """A d of the FFT-PCG's last iteration (the first, the third: the second
+    direction buffer in between) against the operator on that d.  Both sides
+    round four products and their sum: at most eight ulp of |A| |d| a cell."""
+    R = regions(params(nx, ny))["cell"]
+    rho = mg_ref.bubbles(nx, ny, seed=nx, nb=6)
+    bx, by = mg_ref.faces(rho, float(nx * nx), float(nx * nx))
+    f = np.random.default_rng(ny).standard_normal((ny, nx))
+    f -= f.mean()
+    for its in (1, 3):
+        p = params(nx, ny, pressure_solver=pvof.PV_PSOLVE_FFT_PCG, p_max_iter=its, p_rel_tol=1e-14)
+        s = pvof.Solver(p, lib)
+        s.set("RHO", canonical(p, rho))
+        s.set("P_RHS", canonical(p, f))
+        it = C.c_int()
+        s.call("Pressure_solve_cg", C.byref(it))
+        assert it.value == its
+        d, ad = s.get("P_D")[R], s.get("P_AD")[R]
+        assert np.abs(d).max() > 0
+        big = 4 * max(bx.max(), by.max()) * np.abs(d).max()
+        assert np.abs(ad - mg_ref.apply_a(bx, by, d)).max() <= 8 * np.finfo(float).eps * big
+        s.close()
