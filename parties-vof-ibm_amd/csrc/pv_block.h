@@ -109,6 +109,20 @@ __device__ __forceinline__ double block_sum(const double *part, int n, double *s
     return r;
 }
 
+// The same in a workgroup of more than NTH threads: the first NTH add.
+__device__ __forceinline__ double block_sum_wide(const double *part, int n, double *sh)
+{
+    if (threadIdx.x < NTH) {
+        double s, u0, u1;
+        thread_sums(part, n, nullptr, 0, nullptr, 0, s, u0, u1);
+        sh[threadIdx.x] = s;
+    }
+    __syncthreads();
+    const double r = tree_sum(sh);
+    __syncthreads();
+    return r;
+}
+
 // Two sums of partials in one pass, each added in exactly block_sum's order;
 // sh holds 2 * NTH doubles.
 __device__ __forceinline__ void block_sum2(const double *pa, int na, const double *pb, int nb, double *sh,

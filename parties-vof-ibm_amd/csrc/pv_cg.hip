@@ -45,19 +45,6 @@ template <int W> __device__ __forceinline__ int chx(int i, int n)
 // them.  Their partial sums keep the order of 256 threads with four cells each.
 #define NTC 1024
 
-// block_sum in a workgroup of NTC threads: the first NTH add, in its order
-__device__ __forceinline__ double block_sum_c(const double *part, int n, double *sh)
-{
-    if (threadIdx.x < NTH) {
-        double s, u0, u1;
-        thread_sums(part, n, nullptr, 0, nullptr, 0, s, u0, u1);
-        sh[threadIdx.x] = s;
-    }
-    __syncthreads();
-    const double r = tree_sum(sh);
-    __syncthreads();
-    return r;
-}
 // block_store_partial of N values a cell, one cell a thread (sh: N NTC doubles)
 template <int N> __device__ __forceinline__ void cells_store_partial(const double (&v)[N], double *const (&part)[N], int slot, double *sh)
 {
@@ -310,10 +297,10 @@ __global__ void __launch_bounds__(NTC) k_ccg_apply(pvk_grid g, pvk_phys ph, int 
         rv[k] = AT(r, ia, jb);
         pv[k] = (n == 0) ? 0.0 : AT(pold, ia, jb);
     }
-    const double rr = 2.0 * block_sum_c(w.rr[n & 1], (n == 0) ? w.nt0 : w.nb, sh);   // start: one per tile
+    const double rr = 2.0 * block_sum_wide(w.rr[n & 1], (n == 0) ? w.nt0 : w.nb, sh);   // start: one per tile
     double bnorm;
     if (n == 0) {
-        bnorm = sqrt(2.0 * block_sum_c(w.bb, w.nt0, sh));
+        bnorm = sqrt(2.0 * block_sum_wide(w.bb, w.nt0, sh));
         if (bnorm < 1e-30) bnorm = 1.0;
         if (lead) sc->ch_bnorm = bnorm;
     } else {

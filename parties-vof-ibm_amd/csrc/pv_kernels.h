@@ -168,6 +168,8 @@ void pvk_halo_u(const pvk_grid *g, double *f, hipStream_t s);
  * ulike: u-type wrap (pnodes+1 layers below, image column 0 included) */
 void pvk_xwrap(const pvk_grid *g, double *f, int ulike, int pnodes, hipStream_t s);
 void pvk_vel_bc(const pvk_grid *g, double *f, int comp, int type, hipStream_t s);
+/* the NORMAL velocity fills of u and v, and the pressure fill of p (NULL: none) */
+void pvk_bc_uvp(const pvk_grid *g, double *u, double *v, double *p, hipStream_t s);
 void pvk_p_bc(const pvk_grid *g, double *f, hipStream_t s);          /* Pressure_apply_BCs + cell halo */
 void pvk_ghost_multi(const pvk_grid *g, double *f0, double *f1, double *f2, double *f3, int nf, int kind,
                      hipStream_t s);

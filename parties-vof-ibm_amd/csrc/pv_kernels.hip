@@ -105,15 +105,17 @@ __device__ double final_sum(const double *part, int nb, int k, bool is_max)
 //       4 = u velocity: -mirror row -1 / NYM + u-type halo (Velocity.c:2600-2682),
 //       5 = v velocity NORMAL: rows 0, NYM = 0 + cell halo (Velocity.c:2566-2644),
 //       6 = v velocity CG: cell halo only.
-__global__ void k_ghost(pvk_grid g, double *f0, double *f1, double *f2, double *f3, int nf, int kind)
+__host__ __device__ static int ghost_cells(const pvk_grid &g, int kind)
+{
+    return 6 * (g.NXM + 7) + ((kind == 3 || kind == 4) ? 7 : 6) * g.NYM;
+}
+// ghost cell t of a field
+__device__ __forceinline__ void ghost_put(const pvk_grid &g, double *f, int kind, int t)
 {
     const int P = g.P, NXM = g.NXM, NYM = g.NYM;
     const int nrow = NXM + 7;                       // i in [-3, NXM+3]
     const int nrowcells = 6 * nrow;                 // 3 ghost rows top and bottom
     const int ncol = (kind == 3 || kind == 4) ? 7 : 6;
-    const int ncolcells = ncol * NYM;
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nrowcells + ncolcells) return;
     int i, j;
     if (t < nrowcells) {
         int r = t / nrow;
@@ -125,50 +127,72 @@ __global__ void k_ghost(pvk_grid g, double *f0, double *f1, double *f2, double *
         if (ncol == 7) i = (c < 4) ? -c : NXM + 1 + (c - 4);
         else i = (c < 3) ? -1 - c : NXM + (c - 3);
     }
+    double val;
+    bool write = true;
+    switch (kind) {
+    case 0: {
+        if (i == NXM + 3 || j == NYM + 3) { write = false; val = 0.0; break; }
+        int ii = wrapc(i, NXM);
+        int jj = j < 0 ? 0 : (j >= NYM ? NYM - 1 : j);
+        val = AT(f, ii, jj);
+    } break;
+    case 1: {
+        if (i == NXM + 3) { write = false; val = 0.0; break; }
+        int ii = wrapc(i, NXM);
+        if (j == -1) val = AT(f, ii, 0);
+        else if (j == NYM) val = AT(f, ii, NYM - 1);
+        else if (j < -1 || j > NYM) { if (i >= 0 && i < NXM) { write = false; val = 0.0; break; } val = AT(f, ii, j); }
+        else val = AT(f, ii, j);
+    } break;
+    case 2: case 6: {
+        if (i >= 0 && i < NXM) { write = false; val = 0.0; break; }
+        if (i == NXM + 3) { write = false; val = 0.0; break; }
+        val = AT(f, wrapc(i, NXM), j);
+    } break;
+    case 3: {
+        if (i >= 1 && i <= NXM) { write = false; val = 0.0; break; }
+        val = AT(f, wrapu(i, NXM), j);
+    } break;
+    case 4: {
+        int ii = wrapu(i, NXM);
+        if (j == -1) val = -AT(f, ii, 0);
+        else if (j == NYM) val = -AT(f, ii, NYM - 1);
+        else if (i >= 1 && i <= NXM) { write = false; val = 0.0; }
+        else val = AT(f, ii, j);
+    } break;
+    case 5: default: {
+        if (i == NXM + 3) { write = false; val = 0.0; break; }
+        if (j == 0 || j == NYM) val = 0.0;
+        else if (i >= 0 && i < NXM) { write = false; val = 0.0; }
+        else val = AT(f, wrapc(i, NXM), j);
+    } break;
+    }
+    if (write) AT(f, i, j) = val;
+}
+__global__ void k_ghost(pvk_grid g, double *f0, double *f1, double *f2, double *f3, int nf, int kind)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= ghost_cells(g, kind)) return;
     double *fs[4] = {f0, f1, f2, f3};
-    for (int q = 0; q < nf; q++) {
-        double *f = fs[q];
-        double val;
-        bool write = true;
-        switch (kind) {
-        case 0: {
-            if (i == NXM + 3 || j == NYM + 3) { write = false; val = 0.0; break; }
-            int ii = wrapc(i, NXM);
-            int jj = j < 0 ? 0 : (j >= NYM ? NYM - 1 : j);
-            val = AT(f, ii, jj);
-        } break;
-        case 1: {
-            if (i == NXM + 3) { write = false; val = 0.0; break; }
-            int ii = wrapc(i, NXM);
-            if (j == -1) val = AT(f, ii, 0);
-            else if (j == NYM) val = AT(f, ii, NYM - 1);
-            else if (j < -1 || j > NYM) { if (i >= 0 && i < NXM) { write = false; val = 0.0; break; } val = AT(f, ii, j); }
-            else val = AT(f, ii, j);
-        } break;
-        case 2: case 6: {
-            if (i >= 0 && i < NXM) { write = false; val = 0.0; break; }
-            if (i == NXM + 3) { write = false; val = 0.0; break; }
-            val = AT(f, wrapc(i, NXM), j);
-        } break;
-        case 3: {
-            if (i >= 1 && i <= NXM) { write = false; val = 0.0; break; }
-            val = AT(f, wrapu(i, NXM), j);
-        } break;
-        case 4: {
-            int ii = wrapu(i, NXM);
-            if (j == -1) val = -AT(f, ii, 0);
-            else if (j == NYM) val = -AT(f, ii, NYM - 1);
-            else if (i >= 1 && i <= NXM) { write = false; val = 0.0; }
-            else val = AT(f, ii, j);
-        } break;
-        case 5: default: {
-            if (i == NXM + 3) { write = false; val = 0.0; break; }
-            if (j == 0 || j == NYM) val = 0.0;
-            else if (i >= 0 && i < NXM) { write = false; val = 0.0; }
-            else val = AT(f, wrapc(i, NXM), j);
-        } break;
-        }
-        if (write) AT(f, i, j) = val;
+    for (int q = 0; q < nf; q++) ghost_put(g, fs[q], kind, t);
+}
+
+// The NORMAL fills of u (kind 4) and v (kind 5, and row 0) and, p given, the
+// pressure's (kind 1) in one launch: workgroups [0, nu) take u, the next nv v
+// (its ghosts, then row 0), the rest p.  As four launches, 3 us and a gap each.
+__global__ void __launch_bounds__(256) k_bc_uvp(pvk_grid g, double *u, double *v, double *p, int nu, int nv)
+{
+    const int P = g.P, b = blockIdx.x, n5 = ghost_cells(g, 5);
+    if (b < nu) {
+        const int t = b * 256 + threadIdx.x;
+        if (t < ghost_cells(g, 4)) ghost_put(g, u, 4, t);
+    } else if (b < nu + nv) {
+        const int t = (b - nu) * 256 + threadIdx.x;
+        if (t < n5) ghost_put(g, v, 5, t);
+        else if (t < n5 + g.NXM + 7) AT(v, t - n5 - 3, 0) = 0.0;
+    } else {
+        const int t = (b - nu - nv) * 256 + threadIdx.x;
+        if (t < ghost_cells(g, 1)) ghost_put(g, p, 1, t);
     }
 }
 
@@ -185,8 +209,7 @@ __global__ void k_zero_row(pvk_grid g, double *f, int j)
 static void launch_ghost(const pvk_grid *g, double *f0, double *f1, double *f2, double *f3, int nf,
                          int kind, hipStream_t s)
 {
-    int ncol = (kind == 3 || kind == 4) ? 7 : 6;
-    int n = 6 * (g->NXM + 7) + ncol * g->NYM;
+    const int n = ghost_cells(*g, kind);
     hipLaunchKernelGGL(k_ghost, dim3((n + 255) / 256), dim3(256), 0, s, *g, f0, f1, f2, f3, nf, kind);
 }
 
@@ -208,6 +231,13 @@ extern "C" void pvk_vel_bc(const pvk_grid *g, double *f, int comp, int type, hip
     } else {
         launch_ghost(g, f, 0, 0, 0, 1, 6, s);
     }
+}
+
+extern "C" void pvk_bc_uvp(const pvk_grid *g, double *u, double *v, double *p, hipStream_t s)
+{
+    const int nu = (ghost_cells(*g, 4) + 255) / 256, nv = (ghost_cells(*g, 5) + g->NXM + 7 + 255) / 256;
+    const int np = p ? (ghost_cells(*g, 1) + 255) / 256 : 0;
+    hipLaunchKernelGGL(k_bc_uvp, dim3(nu + nv + np), dim3(256), 0, s, *g, u, v, p, nu, nv);
 }
 
 // Communication.c:146-295 on one rank that is its own x neighbour: thread

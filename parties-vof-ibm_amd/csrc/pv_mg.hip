@@ -67,10 +67,11 @@ template <typename T> __device__ __forceinline__ T fget(const Lev<T> &L, const d
 // n = -1 sets the reference norm, n = -2 keeps it (warm restart).  The
 // partials of r_{n+1} come from the level-0 pre-smoothing (rrt, per tile)
 // when it forms r_{n+1}, else from the start or update kernels (rr, per row).
-__device__ void mg_stop_test(pvk_scal *sc, const pvk_pcg &w, int n, double tol, int maxit, double *sh)
+// Returns whether the solve stops here.  (Any workgroup of at least NTH threads.)
+__device__ bool mg_stop_test(pvk_scal *sc, const pvk_pcg &w, int n, double tol, int maxit, double *sh)
 {
     const bool tiles = (n >= 0 && w.nrrt > 0);
-    const double rr = tiles ? block_sum(w.rrt, w.nrrt, sh) : block_sum(w.rr, w.nrr, sh);
+    const double rr = block_sum_wide(tiles ? w.rrt : w.rr, tiles ? w.nrrt : w.nrr, sh);
     const double bn = (n == -1) ? ((sqrt(rr) == 0.0) ? 1.0 : sqrt(rr)) : sc->p_bnorm;
     const double rel = sqrt(rr) / bn;
     const bool done = (rel <= tol) || (n + 1 >= maxit && n >= 0);
@@ -80,6 +81,7 @@ __device__ void mg_stop_test(pvk_scal *sc, const pvk_pcg &w, int n, double tol, 
         sc->p_iter = (n < 0) ? 0 : n + 1;
         if (done) sc->p_done = (rel <= tol) ? 1 : 3;
     }
+    return done;
 }
 
 // ---------------------------------------------------------------------------
@@ -1083,7 +1085,10 @@ template <int K, typename T, int NL> __device__ __forceinline__ void cycle(const
     else cycle_level<2>(m, S, S.k2);
 }
 
-template <typename T, int NL> __global__ void __launch_bounds__(CT) k_mg_coarse(pvk_mg m, pvk_scal *sc)
+// check: the stop test of iteration n first (grids with at most one tiled level;
+// as a launch of its own 2 us and a gap an iteration)
+template <typename T, int NL>
+__global__ void __launch_bounds__(CT) k_mg_coarse(pvk_mg m, pvk_scal *sc, pvk_pcg w, int n, double tol, int maxit, int check)
 {
     extern __shared__ double lds_raw[];
     T *x = (T *)lds_raw;
@@ -1141,6 +1146,7 @@ template <typename T, int NL> __global__ void __launch_bounds__(CT) k_mg_coarse(
     }
     if constexpr (NL == 0) bottom_load(nbot, (const T *)m.H, bottom_col0(nbot), S.h);
     if (sc->p_done) return;
+    if (check && mg_stop_test(sc, w, n, tol, maxit, S.bf + (NL > 0 ? 0 : MG_BF))) return;
     if constexpr (NL > 0) blk_diag<true>(S.g[0].ny, S.k0);
     if constexpr (NL > 1) blk_diag<true>(S.g[1].ny, S.k1);
     if constexpr (NL > 2) blk_diag<true>(S.g[2].ny, S.k2);
@@ -1383,9 +1389,6 @@ static void pre_t(const pvk_mg *m, int l, pvk_scal *sc, const pvk_pcg *w, int n,
     const int sh = tile_shape(m, l), chk = (l == 1), nc = m->L[0].nx * m->L[0].ny;
     if (m->nu == 1) MG_SHAPES(k_mg_pre, 1, L, C, r0, rnew, m->p0, sc, *w, n, tol, maxit, chk, step, nc);
     else MG_SHAPES(k_mg_pre, 2, L, C, r0, rnew, m->p0, sc, *w, n, tol, maxit, chk, step, nc);
-    // levels 0 .. 1 only: the stop test of the residual pre level 0 formed
-    if (l == 0 && m->c0 == 1 && n != -3)
-        hipLaunchKernelGGL(k_mg_check, dim3(1), dim3(NTH), 0, s, sc, *w, n, tol, maxit);
 }
 
 template <typename T> static void post_t(const pvk_mg *m, int l, pvk_scal *sc, const pvk_pcg *w, int n, hipStream_t s)
@@ -1407,23 +1410,26 @@ extern "C" void pvk_mg_pre(const pvk_mg *m, int l, pvk_scal *sc, const pvk_pcg *
     else pre_t<double>(m, l, sc, w, n, tol, maxit, s);
 }
 
-template <typename T> static void coarse_t(const pvk_mg *m, pvk_scal *sc, hipStream_t s)
+template <typename T>
+static void coarse_t(const pvk_mg *m, pvk_scal *sc, const pvk_pcg *w, int n, double tol, int maxit, hipStream_t s)
 {
     constexpr size_t need = coarse_lds_bytes<T>();
+    const int chk = m->c0 <= 1 && n != -3;
+#define MG_COARSE(NL) hipLaunchKernelGGL((k_mg_coarse<T, NL>), dim3(1), dim3(CT), need, s, *m, sc, *w, n, tol, maxit, chk)
     switch (m->nlev - 1 - m->c0) {
-    case 0: hipLaunchKernelGGL((k_mg_coarse<T, 0>), dim3(1), dim3(CT), need, s, *m, sc); break;
-    case 1: hipLaunchKernelGGL((k_mg_coarse<T, 1>), dim3(1), dim3(CT), need, s, *m, sc); break;
-    case 2: hipLaunchKernelGGL((k_mg_coarse<T, 2>), dim3(1), dim3(CT), need, s, *m, sc); break;
-    default: hipLaunchKernelGGL((k_mg_coarse<T, 3>), dim3(1), dim3(CT), need, s, *m, sc); break;
+    case 0: MG_COARSE(0); break;
+    case 1: MG_COARSE(1); break;
+    case 2: MG_COARSE(2); break;
+    default: MG_COARSE(3); break;
     }
+#undef MG_COARSE
 }
 
 extern "C" void pvk_mg_coarse(const pvk_mg *m, const pvk_grid *g, pvk_scal *sc, const pvk_pcg *w, int n,
                               double tol, int maxit, hipStream_t s)
 {
-    if (m->c0 == 0) hipLaunchKernelGGL(k_mg_check, dim3(1), dim3(NTH), 0, s, sc, *w, n, tol, maxit);
-    if (m->fp32) coarse_t<float>(m, sc, s);
-    else coarse_t<double>(m, sc, s);
+    if (m->fp32) coarse_t<float>(m, sc, w, n, tol, maxit, s);
+    else coarse_t<double>(m, sc, w, n, tol, maxit, s);
     if (m->c0 == 0)
         hipLaunchKernelGGL(k_mg_dot, dim3(1), dim3(NTH), 0, s, (const pvk_scal *)sc, *w, *g, rz_slot(n));
 }

@@ -983,8 +983,9 @@ static int p_solve_learned_fcg(pv_bag *b)
     return PV_OK;
 }
 
-/* Pressure_solve_cg + the mean-removal gauge (psolve_cg.c:255-279) */
-static int p_solve(pv_bag *b)
+/* Pressure_solve_cg + the mean-removal gauge (psolve_cg.c:255-279); ghosts = 0
+ * leaves phi's halo to the projection's fill, which writes all of it */
+static int p_solve(pv_bag *b, int ghosts)
 {
     if (b->prm.pressure_solver == PV_PSOLVE_FFT_PCG)
         RC((b->learn && b->learn->collecting) ? p_solve_collect(b) : p_solve_fft_pcg(b));
@@ -996,7 +997,7 @@ static int p_solve(pv_bag *b)
     if (b->h_sc->p_done != 4) {
         pvk_p_mean(G(b), FD(b, PV_F_PHI), &b->rd, S(b));
         pvk_p_mean_finalize(G(b), b->d_sc, &b->rd, S(b));
-        pvk_p_sub_mean(G(b), b->d_sc, FD(b, PV_F_PHI), 1, S(b));
+        pvk_p_sub_mean(G(b), b->d_sc, FD(b, PV_F_PHI), ghosts, S(b));
         LAUNCHCHK();
     }
     b->st.n_p[b->stage] += b->h_sc->p_iter;
@@ -1011,17 +1012,23 @@ static int p_solve(pv_bag *b)
 int pv_Pressure_solve_cg(pv_bag *b, int *iters)
 {
     RC(begin(b));
-    RC(p_solve(b));
+    RC(p_solve(b, 1));
     if (iters) *iters = b->h_sc->p_iter;
     return PV_OK;
+}
+
+/* the projection; the ghosts of P, u and v are the caller's */
+static void project(pv_bag *b)
+{
+    pvk_p_bc(G(b), FD(b, PV_F_PHI), S(b));
+    pvk_project(G(b), b->stage, b->d_sc, FD(b, PV_F_RHO), FD(b, PV_F_PHI), FD(b, PV_F_P), FD(b, PV_F_U),
+                FD(b, PV_F_V), S(b));
 }
 
 int pv_Pressure_project_velocity(pv_bag *b)
 {
     RC(begin(b));
-    pvk_p_bc(G(b), FD(b, PV_F_PHI), S(b));
-    pvk_project(G(b), b->stage, b->d_sc, FD(b, PV_F_RHO), FD(b, PV_F_PHI), FD(b, PV_F_P), FD(b, PV_F_U),
-                FD(b, PV_F_V), S(b));
+    project(b);
     pvk_p_bc(G(b), FD(b, PV_F_P), S(b));
     LAUNCHCHK();
     return PV_OK;
@@ -1089,10 +1096,10 @@ static int pressure_passes(pv_bag *b)
         pvk_p_rhs2(G(b), st, b->d_sc, FD(b, PV_F_U), FD(b, PV_F_V), FD(b, PV_F_RHO), FD(b, PV_F_P_RHS),
                    FD(b, PV_F_M_INV), S(b));
         LAUNCHCHK();
-        RC(p_solve(b));
-        RC(pv_Pressure_project_velocity(b));
-        pvk_vel_bc(G(b), FD(b, PV_F_U), 'u', PV_VEL_TYPE_NORMAL, S(b));
-        pvk_vel_bc(G(b), FD(b, PV_F_V), 'v', PV_VEL_TYPE_NORMAL, S(b));
+        RC(p_solve(b, 0));
+        project(b);
+        pvk_bc_uvp(G(b), FD(b, PV_F_U), FD(b, PV_F_V), FD(b, PV_F_P), S(b));
+        LAUNCHCHK();
         RC(pv_Pressure_compute_velocity_divergence(b, &div));
         passes++;
         if (passes > 10) {
@@ -1123,8 +1130,7 @@ int pv_Temporal_int_all_the_equations(pv_bag *b)
                      FD(b, PV_FI_MVS), FD(b, PV_FI_MU0 + st), FD(b, PV_FI_MV0 + st), S(b));
         /* the CG's first residual reads ghosts (periodic image, wall mirrors)
          * of the start: make them those of the shifted start */
-        pvk_vel_bc(G(b), FD(b, PV_F_U), 'u', PV_VEL_TYPE_NORMAL, S(b));
-        pvk_vel_bc(G(b), FD(b, PV_F_V), 'v', PV_VEL_TYPE_NORMAL, S(b));
+        pvk_bc_uvp(G(b), FD(b, PV_F_U), FD(b, PV_F_V), NULL, S(b));
     } else if (b->m_warm)
         pvk_mom_warm(G(b), 0, 0.0, FD(b, PV_F_U), FD(b, PV_F_V), FD(b, PV_FI_MUS), FD(b, PV_FI_MVS),
                      FD(b, PV_FI_MU0 + st), FD(b, PV_FI_MV0 + st), S(b));
@@ -1135,8 +1141,7 @@ int pv_Temporal_int_all_the_equations(pv_bag *b)
         b->have_mprev[st] = 1;
         b->mprev_dt[st] = b->dt;
     }
-    pvk_vel_bc(G(b), FD(b, PV_F_U), 'u', PV_VEL_TYPE_NORMAL, S(b));
-    pvk_vel_bc(G(b), FD(b, PV_F_V), 'v', PV_VEL_TYPE_NORMAL, S(b));
+    pvk_bc_uvp(G(b), FD(b, PV_F_U), FD(b, PV_F_V), NULL, S(b));
     LAUNCHCHK();
     RC(pressure_passes(b));
     b->st.clamp_delta[st] = b->h_sc->clamp_delta;

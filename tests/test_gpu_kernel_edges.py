@@ -236,3 +236,21 @@ def test_cahn_hilliard_tiles(lib, nx, ny, stage):
     assert relerr(s.get("CH_RHS_N")[R], o.get("CH_RHS_N")[R]) < 1e-12
     assert relerr(s.get("C_L")[R], o.get("C_L")[R]) < 1e-11
     assert abs(o.stats()["n_ch"][stage] - s.stats()["n_ch"][stage]) <= 1
+
+
+# one workgroup's worth of ghosts a field and several, with parts left over
+@pytest.mark.parametrize("nx,ny", [(8, 8), (33, 9), (300, 11), (16, 600)])
+def test_fused_boundary_fill(lib, nx, ny):
+    """After a substep the ghosts of u, v and p are what the fills of the
+    single fields leave, which the other tests hold against the oracle."""
+    p = params(nx, ny, pressure_solver=pvof.PV_PSOLVE_JACOBI_PCG, P_CG_ETOL=1e-8, P_CG_MAXIT=4000)
+    s = pvof.Solver(p, lib)
+    s.init_from_F(pvof.ic(lib, "bubbles", p, seed=3, nmin=2, nmax=3, rmin=0.02, rmax=0.04, gas_inside=1))
+    s.call("Temporal_int_all_the_equations")
+    got = {f: s.get(f).copy() for f in ("U", "V", "P")}
+    assert all(np.abs(a).max() > 0 for a in got.values())
+    for f in ("U", "V"):
+        s.call("Velocity_update_boundaries", pvof.F[f], pvof.PV_VEL_TYPE_NORMAL)
+    s.call("Pressure_apply_BCs", pvof.F["P"])
+    for f, a in got.items():
+        assert np.array_equal(s.get(f), a), f
