@@ -941,72 +941,93 @@ __device__ __forceinline__ void restrict_res(const CGeo &g, T *x, const Blk<T> (
 }
 
 // Bottom level, x = -H f (H = P G P, symmetric, in the cycle's type), in
-// FP64.  Thread (q, r) = (threadIdx / 128, threadIdx % 128) sums a quarter of
-// the columns for rows 2 r and 2 r + 1 (each f from LDS serves two products),
-// reading H[c][2r], H[c][2r+1] = H[2r][c], H[2r+1][c]; the four quarters are
-// added in order through LDS.  H comes from the L2 through one CU (256 KiB or
+// FP64.  Wavefronts 2 q and 2 q + 1 sum quarter q of the columns, a thread for
+// two rows r and r + 1 (each f from LDS serves two products), reading
+// H[c][r], H[c][r+1] = H[r][c], H[r+1][c]; the four quarters are added in order
+// through LDS.  H comes from the L2 through one CU (256 KiB or
 // 512 KiB a visit), so the loads are what it costs: they go out in chunks of
-// PF columns, one chunk ahead of the sums and the first one before the
-// residual that the solve waits for.  One load a column in the sums' loop,
-// as an earlier form had, left 12 us a visit, of the 1.7 us (FP32) the bytes
-// take.
+// PF columns, one chunk ahead of the sums and the first one before the residual
+// that the solve waits for.  Two buffers are read in turn (copying one to the
+// other would wait for it), and a quarter's bounds and addresses are scalars:
+// with the copy, and tests a lane, a launch took 44 us in FP64 (64^2, W on
+// both levels), 29 (44 x 88, W on one) and 14.3 (48^2, V), 32.6 in FP32 (64^2); now
+// 38, 25, 12.4 and 30.8.  Wider FP32 loads (four rows a lane, halves of the
+// wavefront swapped) gave nothing: there the conversions to FP64 are the bound.
 template <typename T> struct HChunk {
     static constexpr int PF = sizeof(T) == 4 ? 8 : 4;
     T h[PF][2];
 };
-template <typename T> __device__ __forceinline__ void bottom_load(int n, const T *H, int c, HChunk<T> &k)
+struct BotGeo {
+    int n, c0, nq, row;             // this quarter's columns [c0, c0 + nq), this thread's first row
+};
+__device__ __forceinline__ BotGeo bottom_geo(int n)
 {
+    const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 7), m = (n + 3) / 4, c0 = q * m;
+    return {n, c0, min(m, n - c0), 2 * ((int)threadIdx.x & 127)};
+}
+template <typename T> __device__ __forceinline__ void bottom_load(const BotGeo &g, const T *H, int c, HChunk<T> &k)
+{
+    constexpr int PF = HChunk<T>::PF;
     typedef T T2 __attribute__((ext_vector_type(2)));
-    const int r = min(2 * ((int)threadIdx.x & 127), n - 1);
-    const unsigned last = (unsigned)(n - 1) * n;
-    if ((n & 1) == 0) {                                            // rows 2r, 2r + 1 in one aligned load
+    c += g.c0;
+    if ((g.n & 1) == 0) {                                          // rows r, r + 1 in one aligned load
+        const int r = min(g.row, g.n - 2);
 #pragma unroll
-        for (int u = 0; u < HChunk<T>::PF; u++) {
-            const T2 v = *(const T2 *)(H + (min((unsigned)(c + u) * n, last) + (r & ~1)));
+        for (int u = 0; u < PF; u++) {
+            const T2 v = *(const T2 *)(H + (size_t)min(c + u, g.n - 1) * g.n + r);       // past the end: not used
             k.h[u][0] = v.x;
             k.h[u][1] = v.y;
         }
     } else {
-        const int r1 = min(r + 1, n - 1);
+        const int r0 = min(g.row, g.n - 1), r1 = min(g.row + 1, g.n - 1);
 #pragma unroll
-        for (int u = 0; u < HChunk<T>::PF; u++) {
-            const unsigned o = min((unsigned)(c + u) * n, last);      // past the end: a value that is not used
-            k.h[u][0] = H[o + r];
-            k.h[u][1] = H[o + r1];
+        for (int u = 0; u < PF; u++) {
+            const T *p = H + (size_t)min(c + u, g.n - 1) * g.n;
+            k.h[u][0] = p[r0];
+            k.h[u][1] = p[r1];
         }
     }
 }
 // v - h f: fused where the product is exact in FP64 (FP32 entries), which rounds alike
 __device__ __forceinline__ double bottom_acc(float h, double f, double v) { return __builtin_fma(-(double)h, f, v); }
 __device__ __forceinline__ double bottom_acc(double h, double f, double v) { return v - h * f; }
-__device__ __forceinline__ int bottom_col0(int n) { return (threadIdx.x >> 7) * ((n + 3) / 4); }
+// columns c .. c + PF - 1 of the quarter
+template <typename T>
+__device__ __forceinline__ void bottom_add(const BotGeo &g, const HChunk<T> &k, const double *f, int c, double &v0, double &v1)
+{
+    constexpr int PF = HChunk<T>::PF;
+    f += c;
+    if (c + PF <= g.nq) {
+#pragma unroll
+        for (int u = 0; u < PF; u++) {
+            v0 = bottom_acc(k.h[u][0], f[u], v0);
+            v1 = bottom_acc(k.h[u][1], f[u], v1);
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < PF; u++)
+            if (c + u < g.nq) {
+                v0 = bottom_acc(k.h[u][0], f[u], v0);
+                v1 = bottom_acc(k.h[u][1], f[u], v1);
+            }
+    }
+}
 
 template <typename T>
 __device__ __forceinline__ void bottom_solve(int n, const T *H, HChunk<T> &k, const double *bf, double *part, T *X)
 {
     static_assert(CT == 2 * PVK_MG_BOTTOM, "four quarters of the bottom's columns, two rows a thread");
     constexpr int PF = HChunk<T>::PF;
-    const int r = 2 * (threadIdx.x & 127), q = threadIdx.x >> 7, c0 = bottom_col0(n), nq = min((n + 3) / 4, n - c0);
+    const BotGeo g = bottom_geo(n);
+    const int r = g.row, q = threadIdx.x >> 7;
+    const double *f = bf + g.c0;
     double v0 = 0.0, v1 = 0.0;
-    for (int c = 0; c < nq; c += PF) {
-        HChunk<T> nx;
-        bottom_load(n, H, c0 + c + PF, nx);
-        const double *f = bf + c0 + c;
-        if (c + PF <= nq) {
-#pragma unroll
-            for (int u = 0; u < PF; u++) {
-                v0 = bottom_acc(k.h[u][0], f[u], v0);
-                v1 = bottom_acc(k.h[u][1], f[u], v1);
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < PF; u++)
-                if (c + u < nq) {
-                    v0 = bottom_acc(k.h[u][0], f[u], v0);
-                    v1 = bottom_acc(k.h[u][1], f[u], v1);
-                }
-        }
-        k = nx;
+    for (int c = 0; c < g.nq; c += 2 * PF) {
+        HChunk<T> k2;
+        bottom_load(g, H, c + PF, k2);
+        bottom_add(g, k, f, c, v0, v1);
+        if (c + 2 * PF < g.nq) bottom_load(g, H, c + 2 * PF, k);
+        if (c + PF < g.nq) bottom_add(g, k2, f, c + PF, v0, v1);
     }
     if (q > 0) {
         part[(q - 1) * PVK_MG_BOTTOM + r] = v0;
@@ -1065,7 +1086,7 @@ __device__ __forceinline__ void cycle_level(const pvk_mg &m, CState<T, NL> &S, B
         }
         if constexpr (BOT) {
             const int n = S.g[NL].nx * S.g[NL].ny;
-            bottom_load(n, (const T *)m.H, bottom_col0(n), S.h);
+            bottom_load(bottom_geo(n), (const T *)m.H, 0, S.h);
         }
         restrict_res<K, BOT>(g, x, k, S.bf);
         cycle<K + 1>(m, S);
@@ -1144,7 +1165,7 @@ __global__ void __launch_bounds__(CT) k_mg_coarse(pvk_mg m, pvk_scal *sc, pvk_pc
         blk_place(S.g[2], S.k2);
         blk_faces(lev<T>(m.L[m.c0 + 2]), S.k2);
     }
-    if constexpr (NL == 0) bottom_load(nbot, (const T *)m.H, bottom_col0(nbot), S.h);
+    if constexpr (NL == 0) bottom_load(bottom_geo(nbot), (const T *)m.H, 0, S.h);
     if (sc->p_done) return;
     if (check && mg_stop_test(sc, w, n, tol, maxit, S.bf + (NL > 0 ? 0 : MG_BF))) return;
     if constexpr (NL > 0) blk_diag<true>(S.g[0].ny, S.k0);
