@@ -148,15 +148,15 @@ typedef struct pvk_mcg {             /* momentum Jacobi-PCG, [0] = u, [1] = v */
 /* Learned preconditioner network (csrc/pv_cnn.hip): parameters, Adam state
  * and the activation / gradient tensors of the largest batch seen so far. */
 #define PVK_CNN_NPARAM 38177
-#define PVK_CNN_RSPLIT 32                /* row groups of the gradient reduction */
+#define PVK_CNN_PSTRIDE 38208            /* floats a row of gradient partials */
+#define PVK_CNN_ROWS 1024                /* rows of them at most (one a workgroup of the backward kernels) */
 typedef struct pvk_cnn {
     float *w, *g, *m, *v;            /* FP32 parameters, gradient, Adam moments */
     unsigned short *wb, *wt;         /* BF16 32 -> 32 weights: forward, flipped transpose */
     unsigned short *act[5];          /* BF16 NHWC activations of layers 1..5 */
     unsigned short *gz[2];           /* BF16 NHWC gradients w.r.t. pre-activations */
     float *gout;                     /* dLoss / d out */
-    float *part, *lpart;             /* per-block partials: gradients, loss */
-    float *rpart;                    /* PVK_CNN_RSPLIT x 9248 row-group sums of part */
+    float *part, *lpart;             /* per-block partials: gradients (PVK_CNN_PSTRIDE a row), loss */
     size_t cap_pix;                  /* B * H * W the tensors hold */
 } pvk_cnn;
 

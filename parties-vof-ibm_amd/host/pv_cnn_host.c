@@ -40,7 +40,7 @@ void pv_cnn_free(pv_bag *b)
     hipFree(c->wb); hipFree(c->wt);
     for (k = 0; k < 5; k++) hipFree(c->act[k]);
     hipFree(c->gz[0]); hipFree(c->gz[1]);
-    hipFree(c->gout); hipFree(c->part); hipFree(c->lpart); hipFree(c->rpart);
+    hipFree(c->gout); hipFree(c->part); hipFree(c->lpart);
     hipFree(b->cnn_io);
     memset(c, 0, sizeof *c);
     b->cnn_io = NULL;
@@ -60,12 +60,11 @@ static int cnn_reserve(pv_bag *b, size_t npix)
     c->gout = c->part = c->lpart = NULL;
     c->gz[0] = c->gz[1] = NULL;
     c->cap_pix = 0;
-    if (!c->rpart) HIPCHK(hipMalloc((void **)&c->rpart, (size_t)PVK_CNN_RSPLIT * 9248 * sizeof(float)));
     for (k = 0; k < 5; k++) HIPCHK(hipMalloc((void **)&c->act[k], act));
     HIPCHK(hipMalloc((void **)&c->gz[0], act));
     HIPCHK(hipMalloc((void **)&c->gz[1], act));
     HIPCHK(hipMalloc((void **)&c->gout, npix * sizeof(float)));
-    HIPCHK(hipMalloc((void **)&c->part, tiles * 9248 * sizeof(float)));
+    HIPCHK(hipMalloc((void **)&c->part, (tiles < PVK_CNN_ROWS ? tiles : PVK_CNN_ROWS) * PVK_CNN_PSTRIDE * sizeof(float)));
     HIPCHK(hipMalloc((void **)&c->lpart, tiles * sizeof(float)));
     c->cap_pix = npix;
     return PV_OK;

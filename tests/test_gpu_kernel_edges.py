@@ -6,6 +6,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import cnn_ref
 import mg_ref
 import oracle_lib
 import pvof
@@ -254,3 +255,34 @@ def test_fused_boundary_fill(lib, nx, ny):
     s.call("Pressure_apply_BCs", pvof.F["P"])
     for f, a in got.items():
         assert np.array_equal(s.get(f), a), f
+
+
+# one tile, a row of tiles
+@pytest.mark.parametrize("shape", [(1, 16, 16), (3, 16, 48)])
+@pytest.mark.parametrize("px", [0, 1])
+def test_network_gradient_small(lib, shape, px):
+    """The smallest batches: the loss is a mean, so four copies of a batch have
+    its gradient, summed over other workgroups (a power of two, so the BF16
+    gradients scale without rounding); FP32 sums, 1e-5."""
+    net = pvof.Network(pvof.Solver(pvof.config1_params(NXM=32, NYM=64), lib), seed=7)
+    net.set_params(cnn_ref.init_params(5).astype(np.float32))
+    rng = np.random.default_rng(sum(shape) + px)
+    x, tgt = rng.standard_normal(shape + (3,)).astype(np.float32), rng.standard_normal(shape).astype(np.float32)
+    one, four = (net.eval(np.concatenate([x] * k), np.concatenate([tgt] * k), px=px, border=3, want_grad=True)[2].astype(np.float64)
+                 for k in (1, 4))
+    for a, b in [(0, 896)] + [(896 + k * 9248, 896 + (k + 1) * 9248) for k in range(4)] + [(37888, 38177)]:
+        assert 0 < np.linalg.norm(one[a:b] - four[a:b]) + np.linalg.norm(one[a:b])
+        assert np.linalg.norm(one[a:b] - four[a:b]) < 1e-5 * np.linalg.norm(one[a:b]), a
+
+
+def test_network_gradient_many_tiles(lib):
+    """More tiles than rows of partials (1030 of 1024): workgroups with two
+    tiles.  The loss is a mean, so the gradient of the batch is the mean of
+    its halves' gradients; FP32 sums of 264000 pixels, 1e-5."""
+    net = pvof.Network(pvof.Solver(pvof.config1_params(NXM=32, NYM=64), lib), seed=7)
+    net.set_params(cnn_ref.init_params(6).astype(np.float32))
+    rng = np.random.default_rng(9)
+    x, tgt = rng.standard_normal((1030, 16, 16, 3)).astype(np.float32), rng.standard_normal((1030, 16, 16)).astype(np.float32)
+    g = [net.eval(x[s], tgt[s], px=0, border=3, want_grad=True)[2].astype(np.float64)
+         for s in (slice(None), slice(0, 515), slice(515, None))]
+    assert np.linalg.norm(g[0] - 0.5 * (g[1] + g[2])) < 1e-5 * np.linalg.norm(g[0])
