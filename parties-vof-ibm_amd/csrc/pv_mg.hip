@@ -63,7 +63,7 @@ template <typename T> __device__ __forceinline__ T fget(const Lev<T> &L, const d
     return r0 ? (T)r0[(ptrdiff_t)j * p0 + i] : ld(L.f, L.pitch, i, j);
 }
 
-// stop test of CG iteration n on the <r, r> partials (as k_transpose):
+// stop test of CG iteration n on the <r, r> partials (as k_tri_cols):
 // n = -1 sets the reference norm, n = -2 keeps it (warm restart).  The
 // partials of r_{n+1} come from the level-0 pre-smoothing (rrt, per tile)
 // when it forms r_{n+1}, else from the start or update kernels (rr, per row).
@@ -540,26 +540,141 @@ __global__ void __launch_bounds__(NTH) k_mg_faces0(Lev<double> L, Lev<float> C)
 // (P G P)_rc = G_rc - m_r - m_c + mean of the m, m the column means (the row
 // means of a symmetric G), in the cycle's type.
 #define BW 64
-// NX: the largest band this instantiation takes.  NX = 16 (bottoms up to 16
-// wide, all the common sizes) uses a padded layout: row stride 17 and 16 zero
-// rows after the last, so every loop below runs its full, compile-time
-// length with no bounds tests (entries past the band stay zero through the
-// factorisation); wider bottoms use stride nx + 1 and tested bounds.
-template <int NX> struct BandLayout {
-    static constexpr bool PAD = (NX == 16);
-    __device__ static int stride(int nx) { return PAD ? NX + 1 : nx + 1; }
-    __device__ static int rows(int nb) { return PAD ? nb + NX : nb; }
-};
+// Bottoms at most 16 wide (all the common sizes; a window of 16 x 16 fits the
+// registers of a wavefront, a wider one does not) go to k_mg_bottom_factor16 and
+// k_mg_bottom_cols16, whose band is padded: row stride 17 and 16 zero rows
+// after the last, so every loop runs its full, compile-time length with no
+// bounds tests (entries past the band stay zero through the factorisation).
+#define BK 16
+#define BKT 256
+
+// lane moves within a quad, compile-time pattern
+template <int CTRL> __device__ __forceinline__ double quad_move(double v)
+{
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+#define QUAD_ALL(k) ((k) * 0x55)           // lane k of the quad to all four
+#define QUAD_UP 0x90                       // lane g takes lane g - 1 (lane 0 its own)
+#define QUAD_X1 0xB1                       // lane g takes lane g ^ 1
+#define QUAD_X2 0x4E                       // lane g takes lane g ^ 2
+
+__device__ __forceinline__ double read_lane(double v, int lane)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// Right-looking band Cholesky of a bottom at most 16 wide, the trailing 16 x 16
+// window in the registers of one wavefront: lane 4 (r % 16) + g holds row r's
+// columns c with c % 4 = g, one register for each c % 16 / 4.  Row k + 16 takes
+// row k's place in step k; its entry in column k is untouched until then and
+// comes separately.  A step (unrolled 16 times, so registers and lanes are
+// compile-time): the unscaled column k goes round through LDS while 1 / sqrt of
+// the pivot is formed, then each lane updates its four entries; the next pivot
+// needs no LDS (its row's own factor, squared).  Bound by these two chains, 0.16
+// us a step.  One wavefront on the band in LDS, the pivot, the column and
+// the updated entries read and written there in each step, took 87 us for 16 x
+// 16 and 51 for 12 x 12; 41 and 24 here.
+template <typename T> __global__ void __launch_bounds__(BKT) k_mg_bottom_factor16(Lev<T> B, double *Lg, double *dinv)
+{
+    constexpr int W = BK + 1;
+    extern __shared__ double in[];         // in[r BK + c % 4 * 4 + c % 16 / 4] = M[r][c], r - 16 < c <= r
+    const int nx = B.nx, ny = B.ny, nb = nx * ny, p = B.pitch, t = threadIdx.x;
+    const int nbp = (nb + BK - 1) / BK * BK, RP = nbp + BK + 1;    // rows past nb: those of the identity
+    double *in16 = in + (size_t)RP * BK, *col = in16 + RP;         // M[r][r - 16]; the column of a step
+    for (int q = t; q < RP * W; q += BKT) in[q] = 0.0;
+    __syncthreads();
+    // row r's diagonal and its couplings to the columns before it: the west
+    // neighbour, the periodic east neighbour (of i = nx - 1) and the south one
+    for (int r = t; r < nb; r += BKT) {
+        const int j = r / nx, i = r - j * nx;
+        const int ie = (i + 1 == nx) ? 0 : i + 1, iw = (i == 0) ? nx - 1 : i - 1;
+        const double ce = ld(B.bx, p, i, j), cw = ld(B.bx, p, iw, j);
+        const double cn = (j + 1 < ny) ? (double)ld(B.by, p, i, j) : 0.0;
+        const double cs = (j > 0) ? (double)ld(B.by, p, i, j - 1) : 0.0;
+        double dg = ce + cw + cn + cs;
+        if (ie == i) dg -= ce;             // nx = 1: the periodic image is the cell itself
+        if (iw == i) dg -= cw;
+        if (r == 0) dg += dg;              // grounding: the (0, 0) entry doubled
+        auto entry = [&](int d) -> double & {
+            const int c = (r - d) & (BK - 1);
+            return (d == BK) ? in16[r] : in[r * BK + (c & 3) * 4 + (c >> 2)];
+        };
+        entry(0) = dg;
+        if (iw < i) entry(i - iw) -= cw;
+        if (ie < i) entry(i - ie) -= ce;
+        if (j > 0) entry(nx) -= cs;
+    }
+    for (int r = nb + t; r < nbp; r += BKT) in[r * BK + (r & 3) * 4 + ((r & (BK - 1)) >> 2)] = 1.0;
+    // the couplings in the padded band that no step writes
+    for (int q = t; q < (nbp + BK) * W; q += BKT) {
+        const int r = q / W, c = r - (q - r * W);
+        if (c < 0 || c >= nbp) Lg[q] = 0.0;
+    }
+    __syncthreads();
+    if (t >= 64) return;
+    const int row = t >> 2, g = t & 3;
+    double A[4], nA[4], n16;
+#pragma unroll
+    for (int u = 0; u < 4; u++) A[u] = in[row * BK + g * 4 + u];
+#pragma unroll
+    for (int u = 0; u < 4; u++) nA[u] = in[BK * BK + g * 4 + u];
+    n16 = in16[BK];
+    double piv = read_lane(A[0], 0);
+    // lanes g = 0 store their row's factor, at row * W + (row - k), lane 1
+    // stores 1 / L[k][k] (L[k][k] itself is not used)
+    const bool keep = (g == 0);
+    int off = keep ? row * W + row : (int)(dinv - Lg);
+    const int wrap = keep ? BK * (W + 1) : 0, next = keep ? -1 : 1;
+    for (int kb = 0; kb < nbp; kb += BK) {
+#pragma unroll
+        for (int s = 0; s < BK; s++) {
+            const int k = kb + s;
+            const double As = (row == s) ? n16 : A[s >> 2];      // column k, in lanes g = k % 4
+            if (g == (s & 3)) col[(row & 3) * 4 + (row >> 2)] = As;
+            __builtin_amdgcn_wave_barrier();
+            double cj[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) cj[u] = col[g * 4 + u];
+            const double c = ((s & 3) == 0) ? quad_move<QUAD_ALL(0)>(As) : ((s & 3) == 1) ? quad_move<QUAD_ALL(1)>(As)
+                           : ((s & 3) == 2) ? quad_move<QUAD_ALL(2)>(As) : quad_move<QUAD_ALL(3)>(As);
+            if (row == s) {
+                off += wrap;
+#pragma unroll
+                for (int u = 0; u < 4; u++) A[u] = nA[u];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) nA[u] = in[(k + BK + 1) * BK + g * 4 + u];
+            n16 = in16[k + BK + 1];
+            __builtin_amdgcn_wave_barrier();
+            // 1 / sqrt(piv): the hardware estimate (about 23 bits) and two Newton
+            // steps (quadratic: to FP64 rounding), far shorter a chain than an
+            // IEEE sqrt and divide; L[k][k] = piv / sqrt(piv)
+            double inv = __builtin_amdgcn_rsq(piv);
+            inv = inv * (1.5 - 0.5 * piv * inv * inv);
+            inv = inv * (1.5 - 0.5 * piv * inv * inv);
+            const double li = c * inv;
+            constexpr int N = BK - 1;
+            piv = read_lane(A[((s + 1) & N) >> 2] - li * li, 4 * ((s + 1) & N) + ((s + 1) & 3));
+#pragma unroll
+            for (int u = 0; u < 4; u++) A[u] = A[u] - li * (cj[u] * inv);  // M[i][j] -= L[i][k] L[j][k]
+            const double out = keep ? li : inv;
+            if (keep || t == 1) *(double *)((char *)Lg + (unsigned)off * 8u) = out;
+            off += next;
+        }
+    }
+}
 
 template <typename T, int NX> __global__ void __launch_bounds__(BW) k_mg_bottom_factor(Lev<T> B, double *Lg, double *dinv)
 {
-    using BL = BandLayout<NX>;
     constexpr int TRI_PER_LANE = (NX * (NX + 1) / 2 + BW - 1) / BW;
     extern __shared__ double lb[];         // lb[r W + d] = M[r][r - d] (L after the factorisation)
     const int nx = B.nx, ny = B.ny, nb = nx * ny, p = B.pitch, t = threadIdx.x;
-    const int W = BL::stride(nx), RP = BL::rows(nb), nbw = BL::PAD ? NX : nx;
-    const int ntri = nbw * (nbw + 1) / 2;
-    // this lane's pairs (i, j), 1 <= j <= i <= nbw, of the trailing update:
+    const int W = nx + 1;
+    const int ntri = nx * (nx + 1) / 2;
+    // this lane's pairs (i, j), 1 <= j <= i <= nx, of the trailing update:
     // q = t + BW u in the order (1,1), (2,1), (2,2), (3,1), ...
     int ti[TRI_PER_LANE], tj[TRI_PER_LANE];
 #pragma unroll
@@ -567,10 +682,10 @@ template <typename T, int NX> __global__ void __launch_bounds__(BW) k_mg_bottom_
         const int q = t + BW * u;
         int i = 1, base = 0;
         while (base + i <= q) { base += i; i++; }
-        ti[u] = (q < ntri) ? i : nbw + 1;                // nbw + 1: never active
+        ti[u] = (q < ntri) ? i : nx + 1;                 // nx + 1: never active
         tj[u] = q - base + 1;
     }
-    for (int q = t; q < RP * W; q += BW) lb[q] = 0.0;
+    for (int q = t; q < nb * W; q += BW) lb[q] = 0.0;
     __syncthreads();
     // row r's diagonal and its couplings to the columns before it: the west
     // neighbour, the periodic east neighbour (of i = nx - 1) and the south one
@@ -590,8 +705,7 @@ template <typename T, int NX> __global__ void __launch_bounds__(BW) k_mg_bottom_
         if (j > 0) lb[r * W + nx] -= cs;
     }
     __syncthreads();
-    // right-looking band Cholesky (padded: the steps touch the zero rows past
-    // nb and the zero entries past the band, which stay zero).  The block is
+    // right-looking band Cholesky.  The block is
     // one wavefront, whose LDS accesses complete in program order, so a step
     // needs no workgroup barrier: it reads the pivot, column k (unscaled) and
     // its pairs' entries, then writes L[k][k], the scaled column and the
@@ -600,7 +714,7 @@ template <typename T, int NX> __global__ void __launch_bounds__(BW) k_mg_bottom_
     // the next step's reads come after these writes.  The wave barriers keep
     // the compiler from moving LDS accesses across steps.
     for (int k = 0; k < nb; k++) {
-        const int m = BL::PAD ? NX : min(nx, nb - 1 - k);
+        const int m = min(nx, nb - 1 - k);
         const double piv = lb[k * W];
         const double ck = (t >= 1 && t <= m) ? lb[(k + t) * W + t] : 0.0;
         double mi[TRI_PER_LANE], mj[TRI_PER_LANE], mij[TRI_PER_LANE];
@@ -635,7 +749,7 @@ template <typename T, int NX> __global__ void __launch_bounds__(BW) k_mg_bottom_
         __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
-    for (int q = t; q < RP * W; q += BW) Lg[q] = lb[q];
+    for (int q = t; q < nb * W; q += BW) Lg[q] = lb[q];
 }
 
 // sum over d = 2 .. NX of a[d] w[d - 1] as a pairwise tree: these terms do
@@ -661,18 +775,16 @@ template <int NX>
 __global__ void __launch_bounds__(BW) k_mg_bottom_cols(int nx, int nb, int cpb, const double *Lg, const double *dinv,
                                                        double *G, double *cm)
 {
-    using BL = BandLayout<NX>;
     extern __shared__ double sm[];
-    const int W = BL::stride(nx), RP = BL::rows(nb), t = threadIdx.x;
-    double *lb = sm, *di = sm + (size_t)RP * W, *y = di + nb;    // y[r cpb + lane]
-    for (int q = t; q < RP * W; q += BW) lb[q] = Lg[q];
+    const int W = nx + 1, t = threadIdx.x;
+    double *lb = sm, *di = sm + (size_t)nb * W, *y = di + nb;    // y[r cpb + lane]
+    for (int q = t; q < nb * W; q += BW) lb[q] = Lg[q];
     for (int q = t; q < nb; q += BW) di[q] = dinv[q];
     __syncthreads();
     const int c = blockIdx.x * cpb + t;
     if (t >= cpb || c >= nb) return;
-    // a band entry, 0 past the band or past the last row (no test when padded)
+    // a band entry, 0 past the band or past the last row
     auto band = [&](int row, int d) -> double {
-        if (BL::PAD) return lb[row * W + d];
         return (d <= nx && row < nb) ? lb[row * W + d] : 0.0;
     };
     double w[NX], a[NX + 1], an[NX + 1];
@@ -723,83 +835,92 @@ __global__ void __launch_bounds__(BW) k_mg_bottom_cols(int nx, int nb, int cpb, 
     cm[c] = s / nb;
 }
 
-// The padded (16-wide) form of k_mg_bottom_cols: the row loop is unrolled by
-// 16, so the window of the last 16 values is a ring indexed by row % 16 at
-// compile time (no register moves per step) and the band rows alternate
-// between two register sets; rows are taken up to a multiple of 16, past nb
-// the band and 1 / diag are zero, so those rows yield zero.
-__global__ void __launch_bounds__(BW) k_mg_bottom_cols16(int nb, int cpb, const double *Lg, const double *dinv,
-                                                         double *G, double *cm)
+// The columns of bottoms at most 16 wide, 16 a block.  A quad of lanes shares a
+// column: lane g forms the products with the values 4 g + 1 .. 4 g + 4 rows
+// back (its window x, a ring of four at compile-time places, the row loop
+// unrolled by 16; a value goes from lane to lane as it ages), the pairwise
+// tree of band_sum ends in two moves within the quad, and all four lanes form
+// the new value, so only one product and two adds of a step wait on the step
+// before.  Rows are taken up to a multiple of 16, past nb the band and 1 / diag
+// are zero, so those rows yield zero.  Three wavefronts only help to stage the
+// band and to store the columns.  With a lane a column, all 16 products in
+// it and 17 LDS reads a row, 94 us for 16 x 16 and 45 for 12 x 12; 53 and 31 here.
+#define BYP (BK + 1)                       // pitch of y: no bank conflicts down a column
+__global__ void __launch_bounds__(BKT) k_mg_bottom_cols16(int nb, const double *Lg, const double *dinv, double *G,
+                                                          double *cm)
 {
-    constexpr int K = 16, W = K + 1;
+    constexpr int W = BK + 1;
     extern __shared__ double sm[];
-    const int t = threadIdx.x, nbp = (nb + K - 1) / K * K, RP = nbp + K;
-    double *lb = sm, *di = sm + (size_t)RP * W, *y = di + RP;    // y[r cpb + lane]
-    for (int q = t; q < RP * W; q += BW) lb[q] = (q < (nb + K) * W) ? Lg[q] : 0.0;
-    for (int q = t; q < RP; q += BW) di[q] = (q < nb) ? dinv[q] : 0.0;
+    const int t = threadIdx.x, nbp = (nb + BK - 1) / BK * BK, RP = nbp + BK, c0 = blockIdx.x * BK;
+    double *lb = sm, *di = sm + (size_t)RP * W, *y = di + RP;    // y[r BYP + column]
+#pragma unroll 6
+    for (int q = t; q < RP * W; q += BKT) lb[q] = (q < (nb + BK) * W) ? Lg[q] : 0.0;
+    for (int q = t; q < RP; q += BKT) di[q] = (q < nb) ? dinv[q] : 0.0;
     __syncthreads();
-    const int c = blockIdx.x * cpb + t;
-    if (t >= cpb || c >= nb) return;
-    double w[K], a0[W], a1[W];
-    // L y = e_c, from the first row of this block's columns (y is zero
-    // before its column): w[r % K] = y_r, a[d] = L[r][r - d], a[0] = 1 / L[r][r]
-    const int r0 = (blockIdx.x * cpb) / K * K;
+    if (t < 64) {
+        const int cc = t >> 2, g = t & 3, c = c0 + cc;
+        double x[4] = {0.0, 0.0, 0.0, 0.0}, a[2][4], d[2], v = 0.0;
+        // one row: sum, new value; xs the slot of the value before, m-th back in slot ord(m)
+        auto step = [&](const double (&A)[4], double D, double e, double &x0, double x1, double x2, double x3) {
+            const double o = quad_move<QUAD_UP>(x0);             // the value 4 g + 1 rows back, g > 0
+            double p0 = A[0] * o, p2 = A[2] * x2;
+            if (g == 0) p0 = 0.0;
+            p0 += A[1] * x1;
+            p2 += A[3] * x3;
+            p0 += p2;
+            p0 += quad_move<QUAD_X1>(p0);
+            p0 += quad_move<QUAD_X2>(p0);
+            const double a1 = quad_move<QUAD_ALL(0)>(A[0]), w0 = v;
+            x0 = (g == 0) ? w0 : o;
+            v = (e - (p0 + a1 * w0)) * D;
+        };
+        // L y = e_c, from the first row of this block's columns (y is zero
+        // before its column): A[m] = L[r][r - 4 g - 1 - m]
+        auto row_f = [&](double (&A)[4], double &D, int r) {
 #pragma unroll
-    for (int q = 0; q < K; q++) w[q] = 0.0;
+            for (int m = 0; m < 4; m++) A[m] = lb[r * W + 4 * g + 1 + m];
+            D = di[r];
+        };
+        row_f(a[0], d[0], c0);
+        for (int rb = c0; rb < nbp; rb += BK) {
 #pragma unroll
-    for (int d = 0; d < W; d++) a0[d] = (d == 0) ? di[r0] : lb[r0 * W + d];
-    for (int rb = r0; rb < nbp; rb += K) {
+            for (int s = 0; s < BK; s++) {
+                const int r = rb + s;
+                row_f(a[(s + 1) & 1], d[(s + 1) & 1], r + 1);
+                step(a[s & 1], d[s & 1], (r == c) ? 1.0 : 0.0, x[(s + 3) & 3], x[(s + 2) & 3], x[(s + 1) & 3], x[s & 3]);
+                if (g == 0) y[r * BYP + cc] = v;
+            }
+        }
+        // L^T g = y in place, from the last row: A[m] = L[r + 4 g + 1 + m][r]
+        auto row_b = [&](double (&A)[4], double &D, int r) {
 #pragma unroll
-        for (int s2 = 0; s2 < K; s2++) {
-            const int r = rb + s2;
-            double *a = (s2 & 1) ? a1 : a0, *an = (s2 & 1) ? a0 : a1;
+            for (int m = 0; m < 4; m++) A[m] = lb[r * W + (4 * g + 1 + m) * (W + 1)];
+            D = di[r];
+        };
+        v = 0.0;
 #pragma unroll
-            for (int d = 0; d < W; d++) an[d] = (d == 0) ? di[r + 1] : lb[(r + 1) * W + d];
-            double p[K];
+        for (int q = 0; q < 4; q++) x[q] = 0.0;
+        row_b(a[0], d[0], nbp - 1);
+        for (int rb = nbp - BK; rb >= 0; rb -= BK) {
 #pragma unroll
-            for (int d = 0; d < K; d++) p[d] = (d >= 1) ? a[d + 1] * w[(s2 - d - 1 + 2 * K) % K] : 0.0;
-#pragma unroll
-            for (int h = 1; h < K; h <<= 1)
-#pragma unroll
-                for (int d = 0; d + h < K; d += 2 * h) p[d] += p[d + h];
-            const double v = ((r == c ? 1.0 : 0.0) - (p[0] + a[1] * w[(s2 - 1 + K) % K])) * a[0];
-            w[s2] = v;
-            y[r * cpb + t] = v;
+            for (int q = 0; q < BK; q++) {
+                const int s = BK - 1 - q, r = rb + s;
+                row_b(a[(q + 1) & 1], d[(q + 1) & 1], max(r - 1, 0));
+                const double yr = (rb >= c0) ? y[r * BYP + cc] : 0.0;
+                step(a[q & 1], d[q & 1], yr, x[(s + 1) & 3], x[(s + 2) & 3], x[(s + 3) & 3], x[s & 3]);
+                if (g == 0) y[r * BYP + cc] = v;
+            }
         }
     }
-    // L^T g = y in place, from the last row: w[r % K] = g_r, a[d] = L[r + d][r]
-#pragma unroll
-    for (int q = 0; q < K; q++) w[q] = 0.0;
-#pragma unroll
-    for (int d = 0; d < W; d++) a0[d] = (d == 0) ? di[nbp - 1] : lb[(nbp - 1 + d) * W + d];
-    for (int rb = nbp - K; rb >= 0; rb -= K) {
-#pragma unroll
-        for (int s2 = K - 1; s2 >= 0; s2--) {
-            const int r = rb + s2;
-            double *a = ((K - 1 - s2) & 1) ? a1 : a0, *an = ((K - 1 - s2) & 1) ? a0 : a1;
-            const int rp = (r > 0) ? r - 1 : 0;
-#pragma unroll
-            for (int d = 0; d < W; d++) an[d] = (d == 0) ? di[rp] : lb[(rp + d) * W + d];
-            const double yr = (r >= r0) ? y[r * cpb + t] : 0.0;
-            double p[K];
-#pragma unroll
-            for (int d = 0; d < K; d++) p[d] = (d >= 1) ? a[d + 1] * w[(s2 + d + 1) % K] : 0.0;
-#pragma unroll
-            for (int h = 1; h < K; h <<= 1)
-#pragma unroll
-                for (int d = 0; d + h < K; d += 2 * h) p[d] += p[d + h];
-            const double v = (yr - (p[0] + a[1] * w[(s2 + 1) % K])) * a[0];
-            w[s2] = v;
-            y[r * cpb + t] = v;
-        }
+    __syncthreads();
+    for (int u = t >> 6; u < BK; u += BKT / 64)
+        if (c0 + u < nb)
+            for (int r = t & 63; r < nb; r += 64) G[(size_t)(c0 + u) * nb + r] = y[r * BYP + u];
+    if (t < BK && c0 + t < nb) {
+        double sum = 0.0;
+        for (int r = 0; r < nb; r++) sum += y[r * BYP + t];
+        cm[c0 + t] = sum / nb;
     }
-    double sum = 0.0;
-    for (int r = 0; r < nb; r++) {
-        const double g = y[r * cpb + t];
-        G[(size_t)c * nb + r] = g;
-        sum += g;
-    }
-    cm[c] = sum / nb;
 }
 
 template <typename T> __global__ void __launch_bounds__(NTH) k_mg_bottom_proj(int nb, const double *G, const double *cm, T *H)
@@ -834,7 +955,8 @@ template <typename T> __global__ void __launch_bounds__(NTH) k_mg_bottom_proj(in
 // Reading the level descriptors (with their pointers) from LDS instead, as
 // an earlier form did, made every access a flat one, and each pass reloaded
 // the coefficients: at 1024^2 (64^2, 32^2 and the 16^2 bottom, W on both,
-// FP32) 53.5 us a launch against 33 now; FP64, V at 96^2, 26 against 15.
+// FP32) 53.5 us a launch, FP64, V at 96^2, 26; with registers 33 and 15, and
+// with the bottom solve's bounds scalar and its chunks read in turn 28 and 12.4.
 // ---------------------------------------------------------------------------
 #define CT 512
 static_assert(PVK_MG_LDS_CELLS <= 8 * CT, "level c0 has at most two 2 x 2 blocks a thread");
@@ -1297,7 +1419,7 @@ extern "C" int pvk_mg_nrz(const pvk_mg *m)
 
 // the bottom matrix of a solve: G column by column, then P G P.  Above 64 KiB
 // of LDS (bottoms wider than 16 columns) the factorisation kernel must be
-// allowed it, raised once per device under a lock as for k_mg_coarse.
+// allowed it.
 // above 64 KiB of dynamic LDS a kernel must be allowed it (gfx950: up to 160
 // KiB per workgroup); raised once per device and kernel, under a lock
 static void allow_lds(const void *k, int slot)
@@ -1319,23 +1441,21 @@ static void allow_lds(const void *k, int slot)
 template <typename T> static void bottom_setup(const pvk_mg *m, hipStream_t s)
 {
     const pvk_mglev &Lb = m->L[m->nlev - 1];
-    const int nx = Lb.nx, nb = nx * Lb.ny, pad = (nx <= 16);
-    const size_t W = pad ? 17 : (size_t)nx + 1, RP = pad ? (size_t)nb + 16 : (size_t)nb;
-    const size_t band = sizeof(double) * RP * W, budget = 160 * 1024;
-    int cpb = BW;                                   // columns per block: as many as LDS holds
-    while (cpb > 1 && band + sizeof(double) * (size_t)nb * (cpb + 1) > budget) cpb >>= 1;
-    const size_t need_cols = band + sizeof(double) * (size_t)nb * (cpb + 1);
+    const int nx = Lb.nx, nb = nx * Lb.ny;
     double *dinv = m->Lb + (size_t)PVK_MG_BOTTOM * (PVK_MG_BOTTOM_NX + 1);
-    if (pad) {
-        hipLaunchKernelGGL((k_mg_bottom_factor<T, 16>), dim3(1), dim3(BW), band, s, lev<T>(Lb), m->Lb, dinv);
-        const size_t nbp = ((size_t)nb + 15) / 16 * 16;
-        int cp = BW;
-        while (cp > 1 && sizeof(double) * ((nbp + 16) * 18 + nbp * cp) > budget) cp >>= 1;
-        const size_t need16 = sizeof(double) * ((nbp + 16) * 18 + nbp * cp);
-        if (need16 > 65536) allow_lds((const void *)k_mg_bottom_cols16, 2);
-        hipLaunchKernelGGL(k_mg_bottom_cols16, dim3((nb + cp - 1) / cp), dim3(BW), need16, s, nb, cp,
+    if (nx <= BK) {
+        const size_t nbp = ((size_t)nb + BK - 1) / BK * BK;
+        const size_t fac = sizeof(double) * ((nbp + BK + 1) * (BK + 1) + BK);
+        const size_t cols = sizeof(double) * ((nbp + BK) * (BK + 2) + nbp * BYP);
+        hipLaunchKernelGGL(k_mg_bottom_factor16<T>, dim3(1), dim3(BKT), fac, s, lev<T>(Lb), m->Lb, dinv);
+        if (cols > 65536) allow_lds((const void *)k_mg_bottom_cols16, 2);
+        hipLaunchKernelGGL(k_mg_bottom_cols16, dim3((unsigned)(nbp / BK)), dim3(BKT), cols, s, nb,
                            (const double *)m->Lb, (const double *)dinv, m->G, m->cm);
     } else {
+        const size_t band = sizeof(double) * (size_t)nb * (nx + 1), budget = 160 * 1024;
+        int cpb = BW;                               // columns per block: as many as LDS holds
+        while (cpb > 1 && band + sizeof(double) * (size_t)nb * (cpb + 1) > budget) cpb >>= 1;
+        const size_t need_cols = band + sizeof(double) * (size_t)nb * (cpb + 1);
         if (band > 65536) allow_lds((const void *)k_mg_bottom_factor<T, PVK_MG_BOTTOM_NX>, sizeof(T) == 4 ? 0 : 1);
         hipLaunchKernelGGL((k_mg_bottom_factor<T, PVK_MG_BOTTOM_NX>), dim3(1), dim3(BW), band, s, lev<T>(Lb), m->Lb,
                            dinv);

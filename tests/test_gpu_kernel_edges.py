@@ -64,6 +64,28 @@ def test_in_workgroup_levels(lib, nx, ny, nu, w, fp32):
     assert relerr(z, zr) < (1e-5 if fp32 else 1e-11)
 
 
+# the grid is the bottom itself: full 16 x 16, rows no multiple of 16 (odd
+# widths, 255 and 247 of 256 cells), the fewest cells and columns, and two
+# wider than 16 (the other factorisation); a second density on the same handle
+@pytest.mark.parametrize("nx,ny", [(16, 16), (15, 17), (13, 19), (9, 28), (8, 8), (10, 25), (17, 15), (32, 8)])
+@pytest.mark.parametrize("fp32", [0, 1])
+def test_bottom_inverse(lib, nx, ny, fp32):
+    p = params(nx, ny)
+    s = pvof.Solver(p, lib)
+    s.check(lib.pv_set_mg_precision(s.h, fp32))
+    for seed in (1, 2):
+        rho = mg_ref.bubbles(nx, ny, seed=seed, nb=4)
+        f = np.random.default_rng(seed).standard_normal((ny, nx))
+        f -= f.mean()
+        s.set("RHO", canonical(p, rho))
+        s.set("P_RES", canonical(p, f))
+        s.call("mg_vcycle_apply")
+        z = s.get("SCRATCH0")[regions(p)["cell"]]
+        lv, G = mg_ref.build(*mg_ref.faces(rho, float(nx * nx), float(nx * nx)))
+        assert len(lv) == 1
+        assert relerr(z, mg_ref.vcycle(lv, G, f, 2)) < (1e-5 if fp32 else 1e-11)
+
+
 # one row of a buffer's worth left over, exactly one buffer (2048-value rows,
 # 128 of them), one row more, and many buffers
 @pytest.mark.parametrize("nx,ny", [(8, 8), (1000, 300), (2041, 121), (2041, 122), (3001, 700)])
