@@ -837,13 +837,130 @@ __global__ void __launch_bounds__(NTH) k_mcg_update_pc(pvk_grid g, pvk_scal *sc,
     if (!START) block_store_partial(a1, w.rr[c], m.band, sh);
 }
 
+// The same on bands of two rows, both rows of a chunk of columns at once.  Row
+// by row, a band comes back to the rows it shares (with its own other row and
+// with the next bands) half a launch later, when half of what the launch
+// moves, twice an L2 at 1024^2, has gone by: r, A d and the diagonal came
+// from HBM twice.  The second row's terms of the sums wait in registers until
+// the first row is through (KC chunks at most: rows up to KC NTH cells), so the
+// sums keep their order.  23.3 -> 18.1 us at 1024^2 and 118 -> 103 at 2048^2 (402
+// MB, 3.9 TB/s); the start 18.5 -> 15.1 and 98 -> 94.
+template <bool START, int KC>
+__global__ void __launch_bounds__(NTH) k_mcg_update_pc2(pvk_grid g, pvk_scal *sc, pvk_mcg w, int n)
+{
+    __shared__ double sh[NTH];
+    __shared__ double sq[2][2][NTH + 2];
+    const mom_band m = mom_locate(g, w);
+    const int c = m.comp, t = threadIdx.x;
+    if (!START && sc->m_done[c]) return;
+    const int P = g.P, NXM = g.NXM, NYM = g.NYM;
+    const double *rold = (n & 1) ? w.r2[c] : w.r[c];
+    double *rnew = (n & 1) ? w.r[c] : w.r2[c], *z = START ? w.d[c][0] : w.z[c];
+    const float *Ad = w.Adf[c], *dg = w.dgf[c];
+    const bool two = m.j0 + 1 < m.j1;
+    struct cell { double r; float a, d; };
+    cell v[4], e;                                       // rows j0 - 1 .. j0 + 2; the column beside the chunk
+    float cf[2][4];
+    auto get = [&](cell &q, int i, int j) {
+        q.r = AT(rold, i, j);
+        if (!START) q.a = AT(Ad, i, j);
+        q.d = AT(dg, i, j);
+    };
+    auto load = [&](int cb) {
+        const int nc = min(NTH, NXM - cb), i = m.i0 + cb + min(t, nc - 1);
+#pragma unroll
+        for (int a = 0; a < 4; a++) get(v[a], i, min(max(m.j0 - 1 + a, m.jlo), NYM - 1));
+        if (t < 4) {                                    // thread 2 a + side: row j0 + a, west or east
+            const int ie = m.i0 + cb + ((t & 1) ? nc : -1);
+            get(e, c ? wrapc(ie, NXM) : wrapu(ie, NXM), min(m.j0 + (t >> 1), NYM - 1));
+        }
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) cf[a][q] = AT(w.cf[c][1 + q], i, min(m.j0 + a, NYM - 1));
+    };
+    load(0);
+    const double alpha = START ? 0.0 : mom_alpha(sc, w, m, n, sh);
+    auto rv = [&](const cell &q) { return START ? q.r : q.r - alpha * (double)q.a; };
+    auto quo = [&](const cell &q) { return rv(q) / mom_D(q.d); };
+    double a0 = 0.0, a1 = 0.0, p0[KC], p1[KC];
+#pragma unroll
+    for (int k = 0; k < KC; k++) {
+        const int cb = k * NTH, par = k & 1;
+        p0[k] = p1[k] = 0.0;
+        if (cb < NXM) {
+            const int nc = min(NTH, NXM - cb), i = m.i0 + cb + t;
+            double q[4], r[2], D[2];
+            float cc[2][4];
+#pragma unroll
+            for (int a = 0; a < 4; a++) q[a] = quo(v[a]);
+#pragma unroll
+            for (int a = 0; a < 2; a++) {
+                r[a] = rv(v[a + 1]);
+                D[a] = mom_D(v[a + 1].d);
+                if (t < nc) sq[par][a][t + 1] = q[a + 1];
+#pragma unroll
+                for (int u = 0; u < 4; u++) cc[a][u] = cf[a][u];
+            }
+            if (t < 4) sq[par][t >> 1][(t & 1) ? nc + 1 : 0] = quo(e);
+            if (cb + NTH < NXM) load(cb + NTH);
+            lds_barrier();
+            if (t < nc) {
+#pragma unroll
+                for (int a = 0; a < 2; a++) {
+                    const int j = m.j0 + a;
+                    double s = r[a];
+                    s += (double)cc[a][0] * sq[par][a][t + 2];
+                    s += (double)cc[a][1] * sq[par][a][t];
+                    if (j + 1 < NYM) s += (double)cc[a][2] * q[a + 2];
+                    if (j - 1 >= m.jlo) s += (double)cc[a][3] * q[a];
+                    const double zz = s / D[a];
+                    if (a == 0 || two) {
+                        if (!START) AT(rnew, i, j) = r[a];
+                        AT(z, i, j) = zz;
+                        if (a == 0) {
+                            a0 += r[a] * zz;
+                            a1 += r[a] * r[a];
+                        } else {
+                            p0[k] = r[a] * zz;
+                            p1[k] = r[a] * r[a];
+                        }
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < KC; k++) {
+        a0 += p0[k];
+        a1 += p1[k];
+    }
+    block_store_partial(a0, w.rz[c][START ? 0 : (n + 1) & 1], m.band, sh);
+    if (!START) block_store_partial(a1, w.rr[c], m.band, sh);
+}
+
+// Two rows a band (the default) and at most eight chunks of terms to hold in
+// registers (90 in all for four, 104 for eight; 128 keep four blocks on a CU):
+// chunk by chunk; other bands and wider grids row by row.
+template <bool START>
+static void mcg_update_pc(const pvk_grid *g, pvk_scal *sc, const pvk_mcg *w, int n, hipStream_t s)
+{
+    const dim3 gr(w->nb[0] + w->nb[1]);
+    if (w->band == 2 && g->NXM <= 4 * NTH)
+        hipLaunchKernelGGL((k_mcg_update_pc2<START, 4>), gr, dim3(NTH), 0, s, *g, sc, *w, n);
+    else if (w->band == 2 && g->NXM <= 8 * NTH)
+        hipLaunchKernelGGL((k_mcg_update_pc2<START, 8>), gr, dim3(NTH), 0, s, *g, sc, *w, n);
+    else
+        hipLaunchKernelGGL(k_mcg_update_pc<START>, gr, dim3(NTH), 0, s, *g, sc, *w, n);
+}
+
 extern "C" void pvk_mcg_init(const pvk_grid *g, const pvk_phys *ph, int stage, pvk_scal *sc, const pvk_mcg *w,
                              hipStream_t s)
 {
     const dim3 gr(w->nb[0] + w->nb[1]);
     if (ph->precision) {
         hipLaunchKernelGGL(k_mcg_init<float>, gr, dim3(NTH), 0, s, *g, *ph, stage, sc, *w);
-        if (w->pc) hipLaunchKernelGGL(k_mcg_update_pc<true>, gr, dim3(NTH), 0, s, *g, sc, *w, 0);
+        if (w->pc) mcg_update_pc<true>(g, sc, w, 0, s);
     } else
         hipLaunchKernelGGL(k_mcg_init<double>, gr, dim3(NTH), 0, s, *g, *ph, stage, sc, *w);
 }
@@ -870,7 +987,7 @@ extern "C" void pvk_mcg_iter(const pvk_grid *g, const pvk_phys *ph, pvk_scal *sc
     } else if (!ph->precision)
         hipLaunchKernelGGL(k_mcg_update<double>, gr, dim3(NTH), 0, s, *g, sc, *w, n);
     else if (w->pc)                                  // the polynomial preconditioner: FP32 form only
-        hipLaunchKernelGGL(k_mcg_update_pc<false>, gr, dim3(NTH), 0, s, *g, sc, *w, n);
+        mcg_update_pc<false>(g, sc, w, n, s);
     else
         hipLaunchKernelGGL(k_mcg_update<float>, gr, dim3(NTH), 0, s, *g, sc, *w, n);
 }

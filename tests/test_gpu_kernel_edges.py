@@ -173,6 +173,14 @@ def test_momentum_cg(lib, nx, ny, rows, form):
             assert relerr(s.get(f)[R[c]], o.get(f)[R[c]]) < tol, (f, relerr(s.get(f)[R[c]], o.get(f)[R[c]]))
 
 
+# two rows a band chunk by chunk: four chunks short of full, full, one column
+# over (the form that holds eight), eight full, one over (row by row); bands of
+# one row left over in u or v
+@pytest.mark.parametrize("nx,ny", [(1023, 9), (1024, 8), (1025, 9), (2048, 8), (2049, 9)])
+def test_momentum_preconditioner_chunks(lib, nx, ny):
+    test_momentum_cg(lib, nx, ny, 2, "mixed_pc")
+
+
 # tiled levels: narrower than a tile, the halo going round more than once
 # (16 x 1024), tiles of 32 x 8 with a part left over (200 x 56), of 32 x 16 with
 # one in both directions (400 x 40), and of 64 x 16 down to 32 x 16 (1056 x 64:
