@@ -27,7 +27,7 @@ timed live with HIP events on the library's stream (every timer_period-th
 launch) over a separate run of kernel_steps steps of the same configuration,
 so that the event records do not perturb the timed run.  The multigrid's
 one-workgroup coarse kernel (MG_COARSE in kernels) can take more time; it
-runs on one CU, bound by its workgroup barriers rather than by HBM, so it has
+runs on one CU, bound by its instruction issue rather than by HBM, so it has
 no byte count and no roofline.
 The cpu_baseline block times the CPU oracle (serial C restatement of the
 reference algorithm) on a bounded sample of the same workload.
@@ -52,10 +52,11 @@ TIMERS = ["CH_APPLY", "CH_UPDATE", "MOM_APPLY", "MOM_UPDATE", "P_APPLY", "P_UPDA
           "MG_PRE0", "MG_COARSE", "MG_POST0"]
 # algorithmic HBM bytes per cell and launch (each distinct array read or
 # written once; stencil neighbours come from cache); MOM_* per velocity
-# component (a launch carries u and v together)
+# component (a launch carries u and v together; the operator kernel also
+# makes the x step); P_APPLY / P_UPDATE here the Jacobi-PCG's two kernels
 BYTES_PER_CELL = {
-    "CH_APPLY": 32, "CH_UPDATE": 48, "MOM_APPLY": 56, "MOM_UPDATE": 56,
-    "P_APPLY": 24, "P_UPDATE": 48, "P_DUPDATE": 24,
+    "CH_APPLY": 32, "CH_UPDATE": 48, "MOM_APPLY": 72, "MOM_UPDATE": 40,
+    "P_APPLY": 48, "P_UPDATE": 64, "P_DUPDATE": 24,
     "FFT_ROWS_FWD": 16, "FFT_COLS": 16, "FFT_ROWS_INV": 24,
     "CH_RHS": 56, "MOM_TERMS": 88, "P_TRANSPOSE": 16,
 }
@@ -63,22 +64,23 @@ BYTES_PER_CELL = {
 # new direction (z, d_old, faces -> d, Ad) and the forward x-FFT (-> spectrum)
 BYTES_PER_CELL_FFT = dict(BYTES_PER_CELL, P_APPLY=48, P_UPDATE=56)
 # MG-PCG: the same direction kernel; the level-0 pre-smoothing also does the
-# CG step (r_n, A d, d, phi, faces -> r_{n+1}, phi, pre-smoothed x, coarse f)
-# and correction + post-smoothing (x, coarse x, r, faces -> z).  P_UPDATE is
+# CG step (r_n, A d, d, phi, faces -> r_{n+1}, phi, the red half of the
+# pre-smoothed x, coarse f) and correction + post-smoothing (that half, coarse
+# x, r, faces -> z).  P_UPDATE is
 # the separate step kernel of grids without tiled levels.
-BYTES_PER_CELL_MG = dict(BYTES_PER_CELL, P_APPLY=48, P_UPDATE=48, MG_PRE0=74, MG_POST0=42)
+BYTES_PER_CELL_MG = dict(BYTES_PER_CELL, P_APPLY=48, P_UPDATE=48, MG_PRE0=70, MG_POST0=38)
 # the FP32 V-cycle (mixed precision): FP32 faces and pre-smoothed x, FP64 r,
 # A d, d, phi and z
-BYTES_PER_CELL_MG32 = dict(BYTES_PER_CELL_MG, MG_PRE0=61, MG_POST0=29)
+BYTES_PER_CELL_MG32 = dict(BYTES_PER_CELL_MG, MG_PRE0=59, MG_POST0=27)
 # per pressure iteration, all of its kernels (MG: level 0 + 1/3 of the level-0
 # smoothing bytes, without the CG step, for the coarser levels)
-BYTES_PER_ITER = {"fft": 144, "mg": 189, "mg32": 155, "jacobi": 112}
+BYTES_PER_ITER = {"fft": 144, "mg": 179, "mg32": 149, "jacobi": 112}
 # HBM bytes per launch measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE on
 # the 1024^2 MG-PCG mixed form (FETCH_SIZE scaled by 2.0, WRITE_SIZE by 1.0:
 # the factors a 256 MiB device copy gives in runs of its own); the summary is
 # profiles/mg_pcg_mixed_1024_pmc_traffic.md
-TRAFFIC_MB_MG32_1024 = {"MG_PRE0": 66.5, "MG_POST0": 32.0, "P_APPLY": 51.5,
-                        "MOM_APPLY": 114.6, "MOM_UPDATE": 226.0, "CH_RHS": 68.8, "MOM_TERMS": 111.0}
+TRAFFIC_MB_MG32_1024 = {"MG_PRE0": 64.2, "MG_POST0": 29.7, "P_APPLY": 51.5,
+                        "MOM_APPLY": 141.0, "MOM_UPDATE": 105.5, "CH_RHS": 68.6, "MOM_TERMS": 111.0}
 SEED = 20261202
 # the headline metric: the timed form is the learned-start mixed form, the plain
 # FP64 path is reported beside it (compare.plain_fp64), the dominant kernel's
@@ -101,11 +103,11 @@ def workload_params(n=1024, solver=pvof.PV_PSOLVE_FFT_PCG, precision=pvof.PV_PRE
 
 def step_bytes_per_cell(st, family, mixed=False, mom_pc=0):
     """Algorithmic bytes per cell for one RK3 step from the solver counts
-    (fixed 563 B per substep + 88 per biharmonic, 136 per momentum (140 in the
-    mixed form, whose operator kernel reads five FP32 coefficients instead of
-    rho and mu; 16 more with the polynomial preconditioner) and BYTES_PER_ITER
+    (fixed 563 B per substep + 88 per biharmonic, 112 per momentum (96 in the
+    mixed form, whose operator kernel reads five FP32 coefficients and writes
+    A d in FP32; 16 more with the polynomial preconditioner) and BYTES_PER_ITER
     per pressure iteration)."""
-    total, mom = 0, (140 if mixed else 136) + (16 if mom_pc else 0)
+    total, mom = 0, (96 if mixed else 112) + (16 if mom_pc and mixed else 0)
     for k in range(3):
         total += 563 + 88 * st["n_ch"][k] + mom * (st["n_u"][k] + st["n_v"][k]) + BYTES_PER_ITER[family] * st["n_p"][k]
     return total
@@ -232,14 +234,14 @@ def run(lib, args, solver, precision, steps, warmup, F, net_params=None, timers=
            "mg32": BYTES_PER_CELL_MG32}[fam]
     cells = p.NXM * p.NYM
     if precision == "mixed":
-        # the FP32 operator reads r, diag, d_old and five FP32 coefficients per
-        # component (formed by the start kernel) instead of rho and mu
-        bpc = dict(bpc, MOM_APPLY=60)
+        # the FP32 operator reads z, d_old, x and five FP32 coefficients per
+        # component (formed by the start kernel) and writes d, x and A d
+        # (FP32); the update reads r, A d and the FP32 diagonal
+        bpc = dict(bpc, MOM_APPLY=64, MOM_UPDATE=32)
         if o["mom_pc"]:
-            # polynomial preconditioner: the operator reads z instead of r and
-            # diag; the update also reads diag and four coefficients and
-            # writes r_{n+1} and z
-            bpc = dict(bpc, MOM_APPLY=52, MOM_UPDATE=80)
+            # polynomial preconditioner: the update also reads four
+            # coefficients; r_{n+1} and z are written
+            bpc = dict(bpc, MOM_UPDATE=48)
     if not any(sum(st["n_ch"]) for st in stats):
         # spectral CH start: the CH CG launches only take the stop test (no cell work)
         bpc = {k: v for k, v in bpc.items() if k not in ("CH_APPLY", "CH_UPDATE")}

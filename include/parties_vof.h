@@ -50,7 +50,7 @@ extern "C" {
                                     counterpart in the reference; needs a trained network) */
 #define PV_PSOLVE_LEARNED_FCG 3  /* learned warm start + learned-preconditioned flexible
                                     CG, falling back to FFT-PCG when the residual stalls */
-#define PV_PSOLVE_FFT_PCG    1   /* PCG preconditioned by the FFT-x/Thomas-y solve
+#define PV_PSOLVE_FFT_PCG    1   /* PCG preconditioned by the FFT-x/tridiagonal-y solve
                                     of psolve_fft.c:1536-1802, relative-residual stop */
 #define PV_PSOLVE_MG_PCG     4   /* the same CG, start, gauge and stop test, preconditioned
                                     by one geometric multigrid V-cycle on the variable face
@@ -230,7 +230,7 @@ int pv_Pressure_compute_velocity_divergence(pv_bag *bag, double *div_max);   /* 
  * (for tests of the preconditioner as a linear operator). */
 int pv_mg_vcycle_apply(pv_bag *bag);
 /* Constant-coefficient Poisson solve, FFT in x (R2HC, 1/NXM scale, modified
- * wavenumbers) and Thomas in y with the (0,0) mode pinned at j = 0:
+ * wavenumbers) and tridiagonal in y with the (0,0) mode pinned at j = 0:
  * lsolver/psolve_fft.c:17-207, :467-591, :1536-1802 (z of length 1). */
 int pv_Pressure_solve_fft(pv_bag *bag, int rhs_field, int out_field);
 
@@ -327,11 +327,11 @@ int pv_batch_autotune_mg(pv_batch *bt, int *wlevels, int *sweeps);
  * tiled levels. */
 int pv_set_momentum_rows(pv_bag *bag, int rows);
 int pv_set_mg_tile0(pv_bag *bag, int shape);
-/* Shape of the FFT preconditioner's y tridiagonal solves (partitioned
- * Thomas): rows per thread's segment, 1..16 (0 = 8), and columns per block,
+/* Shape of the FFT preconditioner's y tridiagonal solves (two first-order
+ * recurrences, their carries combined by a scan): rows per thread's segment, 1..16 (0 = 8), and columns per block,
  * a power of two <= 64 (0 = 2, or more where a block would hold less than a
  * wavefront; halved while a block would exceed 512 threads).  Changes the order of the arithmetic
- * (the separators' reduced system), so results differ at rounding level. */
+ * (where the carries are combined), so results differ at rounding level. */
 int pv_set_fft_tri_shape(pv_bag *bag, int rows, int cols);
 int pv_autotune_tiles(pv_bag *bag, int *mom_rows, int *mg_tile0);
 

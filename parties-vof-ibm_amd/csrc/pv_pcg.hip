@@ -3,15 +3,16 @@
 // (operator of lsolver/psolve_cg.c:302-344), preconditioned by the
 // constant-coefficient FFT-x / DCT-y solve.
 //
-// One iteration = six launches and no one-block kernels:
+// One iteration = four launches and no one-block kernels:
 //   K1 k_pcg_apply      d_n = z + beta d_{n-1} on the fly (double-buffered d),
 //                       Ad = A d_n, partials <d, Ad>           (row bands)
 //   K2 k_pcg_update_fwd alpha; phi += alpha d; r -= alpha Ad; partials <r,r>;
 //                       forward real FFT of the new r rows    (R rows per block)
-//   K3 k_transpose      stop test from <r,r>; spec -> specT   (32 x 32 tiles)
-//   K4 k_dct_rows       DCT-II, divide by lambda, DCT-III along y (rows of specT)
-//   K5 k_transpose      specT -> spec
+//   K4 k_tri_cols       stop test from <r,r>; the y solves in place on the
+//                       columns of the spectrum                (columns)
 //   K6 k_ifft_rows_dot  z = inverse real FFT; partials <r, z>
+// The Cahn-Hilliard solve's spectral start replaces K4 by K3 k_transpose,
+// k_dct_rows (DCT-II, divide, DCT-III along y) and K5 k_transpose.
 // Scalars are never stored by one block and read by others in the same
 // kernel: every block re-adds the few hundred partials of the previous
 // kernel in the same fixed order, so all blocks see bit-identical alpha,
