@@ -203,7 +203,8 @@ __global__ void __launch_bounds__(NTH, 4) k_pcg_apply(pvk_grid g, pvk_scal *sc, 
 // took 19.6 us and the inverse one 13.7 at 1024^2 (13.4 and 10.9 at 128 x 256);
 // now 15.0 and 8.7 (7.9 and 5.3).  One wavefront a block against 256 threads
 // (NT / T rows): 15.0 and 8.7 against 15.8 and 9.4 at 1024^2, 14.1 and 9.5
-// against 15.0 and 11.6 at 768 x 491, 7.9 and 5.3 against 9.9 and 7.0 at 128 x 256.
+// against 15.0 and 11.6 at 768 x 491 (12.9 and 8.2 since the index arithmetic
+// there is shifts), 7.9 and 5.3 against 9.9 and 7.0 at 128 x 256.
 #define RU 8
 #define TWK 8                    // twiddle pairs a thread stages: M <= 8 NT
 typedef double v2d __attribute__((ext_vector_type(2)));

@@ -127,6 +127,14 @@ def test_fft_rows_and_columns(lib, nx, ny):
     assert relerr(got, ref) < 1e-10
 
 
+# rows of 2^a 3^b whose passes differ: one, two, three and four radix-3 passes, the
+# power-of-two part ending with radix 8 alone (48, 144, 432, 1296), 4 (192, 576) or 2
+# (96, 288, 864), and with a second radix-8 pass before them (3072, 768)
+@pytest.mark.parametrize("nx", [48, 144, 432, 1296, 192, 576, 96, 288, 864, 768, 3072])
+def test_fft_mixed_radix_rows(lib, nx):
+    test_fft_rows_and_columns(lib, nx, 24)
+
+
 # columns: less than a chunk of 256, one short of one, exactly one, one over,
 # two and a remainder; rows: every remainder of the bands of 1, 2 and 4 rows
 # of u (NYM rows) and v (NYM - 1)
