@@ -125,7 +125,9 @@ void pv_host_metrics_free(pv_metrics *m)
 /* handle                                                              */
 /* ------------------------------------------------------------------ */
 
-#define OFF0 13                     /* (OFF0 + 3) % 16 == 0: column 0 on 128 B */
+#define OFF0 13                     /* (OFF0 + 3) % 16 == 0: column 0 on 128 B, in each field of the
+                                       slab, since a field is whole lines of 16 doubles: the row
+                                       transforms and the multigrid read pairs of doubles from there */
 
 static double *fld(pv_bag *b, int f) { return b->f[f]; }
 
@@ -203,7 +205,7 @@ static int create_on_device(pv_bag *b, const pv_params *prm)
     b->NXM = prm->NXM; b->NYM = prm->NYM;
     b->NXT = prm->NXM + 7; b->NYT = prm->NYM + 7;
     b->P = ((b->NXT + 15) / 16) * 16;
-    b->alloc_elems = (size_t)OFF0 + (size_t)b->P * (size_t)b->NYT + 16;
+    b->alloc_elems = ((size_t)OFF0 + (size_t)b->P * (size_t)b->NYT + 16 + 15) / 16 * 16;
     bytes = b->alloc_elems * sizeof(double) * PV_FI_END;
     if (hipMalloc((void **)&b->slabmem, bytes) != hipSuccess) {
         b->slabmem = NULL;

@@ -1,0 +1,108 @@
+/*
+ * handle_check.c -- what a handle asks of the device, checked without one.
+ * The HIP calls of libparties_vof.so resolve to the functions below: device
+ * memory is host memory, kernels are counted and not run.  Modes:
+ *   layout NX NY    offsets of the arrays the kernels read in pairs of doubles
+ */
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+#include "../../parties-vof-ibm_amd/host/pv_host.h"
+
+/* ---- the runtime's part ---- */
+#define NBLOCK 256
+static struct { char *p; size_t n; } block[NBLOCK];
+static int nblock;
+
+hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
+hipError_t hipSetDevice(int d) { (void)d; return hipSuccess; }
+hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
+hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int d)
+{
+    (void)d;
+    memset(p, 0, sizeof *p);
+    strcpy(p->gcnArchName, "gfx950");
+    return hipSuccess;
+}
+hipError_t hipGetLastError(void) { return hipSuccess; }
+const char *hipGetErrorString(hipError_t e) { (void)e; return "none"; }
+
+hipError_t hipMalloc(void **p, size_t n)
+{
+    if (nblock == NBLOCK || posix_memalign(p, 4096, n ? n : 1)) return hipErrorOutOfMemory;
+    block[nblock].p = (char *)*p;
+    block[nblock++].n = n;
+    return hipSuccess;
+}
+hipError_t hipFree(void *p)
+{
+    int k;
+    for (k = 0; k < nblock; k++)
+        if (block[k].p == (char *)p) block[k] = block[--nblock];
+    free(p);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; *p = malloc(n); return *p ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipMemset(void *p, int v, size_t n) { memset(p, v, n); return hipSuccess; }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { (void)k; memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st)
+{
+    (void)st;
+    return hipMemcpy(d, s, n, k);
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned flags) { (void)flags; *s = (hipStream_t)malloc(1); return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { free(s); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; return hipSuccess; }
+
+static struct { dim3 g, b; size_t lds; hipStream_t s; } cfg;
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s)
+{
+    cfg.g = g; cfg.b = b; cfg.lds = lds; cfg.s = s;
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t *s)
+{
+    *g = cfg.g; *b = cfg.b; *lds = cfg.lds; *s = cfg.s;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t lds, hipStream_t s)
+{
+    (void)f; (void)g; (void)b; (void)args; (void)lds; (void)s;
+    return hipSuccess;
+}
+
+/* ---- the checks ---- */
+static pv_bag *create(int nx, int ny)
+{
+    pv_params p;
+    pv_bag *b;
+    pv_params_default(&p);
+    p.NXM = nx;
+    p.NYM = ny;
+    p.ymax = (double)ny / nx;
+    if (pv_create(&p, 0, &b)) { fprintf(stderr, "%s\n", pv_last_error()); exit(1); }
+    return b;
+}
+
+static unsigned past(const void *p, unsigned n) { return (unsigned)((size_t)p % n); }
+
+static int layout(int nx, int ny)
+{
+    pv_bag *b = create(nx, ny);
+    unsigned worst = 0;
+    int k;
+    for (k = 0; k < PV_FI_END; k++)
+        if (past(b->f[k], 128) > worst) worst = past(b->f[k], 128);
+    printf("field %u\n", worst);
+    if (b->fft.ok) printf("rtx %u\nwx %u\n", past(b->fft.rtx, 16), past(b->fft.wx, 16));
+    if (b->mg_ok) printf("r2 %u\n", past(b->mgw.r2, 16));
+    pv_destroy(b);
+    return 0;
+}
+
+int main(int argc, char **argv)
+{
+    if (argc == 4 && !strcmp(argv[1], "layout")) return layout(atoi(argv[2]), atoi(argv[3]));
+    return 2;
+}

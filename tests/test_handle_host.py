@@ -1,0 +1,37 @@
+"""What a handle asks of the device, checked on the CPU: the library's HIP
+calls go to the stand-ins of tests/host/handle_check.c, which run no kernels."""
+import os
+import subprocess
+
+import pytest
+
+import pvof
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PKG = os.path.join(os.path.dirname(HERE), "parties-vof-ibm_amd")
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    pvof.load_lib()                                   # builds it if nothing is there
+    out, so = str(tmp_path_factory.mktemp("handle") / "handle_check"), os.path.join(PKG, "_build")
+    subprocess.run(["gcc", "-O1", "-std=gnu99", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-rdynamic", "-o", out,
+                    os.path.join(HERE, "host", "handle_check.c"), "-L" + so, "-lparties_vof", "-Wl,-rpath," + so,
+                    "-Wl,-rpath-link,/opt/rocm/lib", "-Wl,--allow-shlib-undefined"], check=True, capture_output=True)
+    return out
+
+
+def check(exe, *args):
+    r = subprocess.run([exe] + [str(a) for a in args], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stderr
+    return {k: int(v) for k, v in (line.split() for line in r.stdout.splitlines())}
+
+
+# odd and even numbers of rows, pitches of an odd and an even number of lines
+SIZES = [(8, 8), (96, 96), (768, 491), (88, 56), (64, 33), (9, 13), (256, 128)]
+
+
+@pytest.mark.parametrize("nx,ny", SIZES)
+def test_fields_start_on_a_line(exe, nx, ny):
+    """Cell (0, 0) of every field, which kernels read in pairs of doubles."""
+    assert check(exe, "layout", nx, ny)["field"] == 0
