@@ -609,7 +609,7 @@ int pv_fft_create(pv_bag *b)
 {
     const double PI_ = 3.14159265358979323846;
     int nx = b->NXM, ny = b->NYM, lx = ilog2_exact(nx), ly = ilog2_exact(ny), k;
-    size_t n_rtx, n_rty, n_dct, n_wx, n_wy, total;
+    size_t n_rtx, n_rty, n_dct, n_ly, n_wx, n_wy, total;
     double *h, *d, *q;
     double idx2, idy2;
     memset(&b->fft, 0, sizeof b->fft);
@@ -625,8 +625,9 @@ int pv_fft_create(pv_bag *b)
     b->fft.logmy = (ly >= 3) ? ly - 1 : 0;
     n_rtx = 2 * (size_t)(nx / 2 + 1); n_rty = 2 * (size_t)(ny / 2 + 1);
     n_dct = 2 * (size_t)ny;
+    n_ly = (size_t)ny + (ny & 1);          /* even, so that wx, read in pairs of doubles, starts on one */
     n_wx = 2 * (size_t)(nx / 2); n_wy = 2 * (size_t)(ny / 2);
-    total = n_rtx + n_rty + n_dct + nx + ny + n_wx + n_wy + 4 * (size_t)nx;
+    total = n_rtx + n_rty + n_dct + nx + n_ly + n_wx + n_wy + 4 * (size_t)nx;
     h = (double *)calloc(total, sizeof(double));
     if (!h) return pv_set_error(PV_ENOMEM, "FFT table allocation failed");
     q = h;
@@ -646,7 +647,7 @@ int pv_fft_create(pv_bag *b)
     }
     q += nx;
     for (k = 0; k < ny; k++) q[k] = 2.0 * (1 - cos(PI_ * k / ny)) * idy2;
-    q += ny;
+    q += n_ly;
     /* Stockham twiddles of the half-length complex transforms */
     for (k = 0; k < nx / 2; k++) { double a = 2.0 * PI_ * k / (nx / 2); q[2 * k] = cos(a); q[2 * k + 1] = -sin(a); }
     q += n_wx;
@@ -718,7 +719,7 @@ int pv_fft_create(pv_bag *b)
     b->fft.rty = q; q += n_rty;
     b->fft.dcty = q; q += n_dct;
     b->fft.lamx = q; q += nx;
-    b->fft.lamy = q; q += ny;
+    b->fft.lamy = q; q += n_ly;
     b->fft.wx = q; q += n_wx;
     b->fft.wy = q; q += n_wy;
     b->fft.tri_q = q; q += nx;

@@ -35,3 +35,10 @@ SIZES = [(8, 8), (96, 96), (768, 491), (88, 56), (64, 33), (9, 13), (256, 128)]
 def test_fields_start_on_a_line(exe, nx, ny):
     """Cell (0, 0) of every field, which kernels read in pairs of doubles."""
     assert check(exe, "layout", nx, ny)["field"] == 0
+
+
+@pytest.mark.parametrize("nx,ny", [s for s in SIZES if s[0] % 16 == 0])
+def test_row_tables_start_on_a_pair(exe, nx, ny):
+    """Cosines and twiddles of the row transforms, read in pairs of doubles."""
+    got = check(exe, "layout", nx, ny)
+    assert got["rtx"] == 0 and got["wx"] == 0
