@@ -102,7 +102,8 @@ template <typename T> struct Blk {
 };
 
 // Two values of a row from column 2 I on, in one load: a smoothing level's
-// width and pitch are even and its arrays start on two values.
+// width and pitch are even and its arrays, like the CG's fields, start on two
+// values (pv_create, pv_mg_create).
 template <typename T> __device__ __forceinline__ void ld2(const T *a, int pitch, int i, int j, T &v0, T &v1)
 {
     typedef T T2 __attribute__((ext_vector_type(2)));

@@ -28,7 +28,7 @@ int pv_mg_create(pv_bag *b)
     pvk_mg *m = &b->mg, *mf = &b->mgf;
     int lx[PVK_MG_MAXLEV], ly[PVK_MG_MAXLEV], nl = 1, c0, l, nrz, nx = b->NXM, ny = b->NYM;
     size_t cells = 0, total, totalf, nc0 = (size_t)nx * ny;
-    double *q;
+    double *q, *r2;
     float *qf;
     memset(m, 0, sizeof *m);
     memset(mf, 0, sizeof *mf);
@@ -91,7 +91,11 @@ int pv_mg_create(pv_bag *b)
     m->L[0].f = b->f[PV_F_P_RES];
     m->L[0].bx = b->f[PV_FI_PBX];
     m->L[0].by = b->f[PV_FI_PBY];
+    /* the two arrays of whole lines first: they start on a line, while the
+     * arrays after an odd bottom do not even start on a pair of doubles, which
+     * is how the level-0 kernels read them */
     m->L[0].xp = q; q += (size_t)b->g.P * ny;
+    r2 = q; q += (size_t)b->g.P * ny;
     for (l = 1; l < nl; l++) {
         size_t n = (size_t)lx[l] * ly[l];
         m->L[l].x = q; q += n;
@@ -146,7 +150,7 @@ int pv_mg_create(pv_bag *b)
         w->sad = q; q += ny;
         w->rz[0] = q; q += nrz;
         w->rz[1] = q; q += nrz;
-        w->r2 = q; q += (size_t)b->g.P * ny;     /* r_1, r_3, ...: pitch P like r */
+        w->r2 = r2;                              /* r_1, r_3, ...: pitch P like r */
         w->rrt = q; q += nrz;
         nrz = pvk_mg_nrz(m);                     /* the tiles in use */
         w->nrrt = (c0 > 0) ? nrz : 0;

@@ -96,7 +96,24 @@ static int layout(int nx, int ny)
         if (past(b->f[k], 128) > worst) worst = past(b->f[k], 128);
     printf("field %u\n", worst);
     if (b->fft.ok) printf("rtx %u\nwx %u\n", past(b->fft.rtx, 16), past(b->fft.wx, 16));
-    if (b->mg_ok) printf("r2 %u\n", past(b->mgw.r2, 16));
+    if (b->mg_ok) {
+        /* both hierarchies: the smoothing levels' arrays, the bottom matrix (read in pairs where its
+         * size is even), the other residual */
+        unsigned lev = 0, h = 0;
+        for (k = 0; k < 2; k++) {
+            const pvk_mg *m = k ? &b->mgf : &b->mg;
+            const unsigned n = k ? 8 : 16;
+            const pvk_mglev *e = &m->L[m->nlev - 1];
+            int l, q;
+            for (l = 0; l + 1 < m->nlev; l++) {
+                const void *a[5] = { m->L[l].x, m->L[l].f, m->L[l].bx, m->L[l].by, m->L[l].xp };
+                for (q = 0; q < 5; q++) lev += past(a[q], n);
+                lev += (m->L[l].pitch & 1) + (m->L[l].nx & 1);
+            }
+            if (e->nx * e->ny % 2 == 0) h += past(m->H, n);
+        }
+        printf("level %u\nH %u\nr2 %u\n", lev, h, past(b->mgw.r2, 16));
+    }
     pv_destroy(b);
     return 0;
 }

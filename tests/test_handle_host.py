@@ -42,3 +42,11 @@ def test_row_tables_start_on_a_pair(exe, nx, ny):
     """Cosines and twiddles of the row transforms, read in pairs of doubles."""
     got = check(exe, "layout", nx, ny)
     assert got["rtx"] == 0 and got["wx"] == 0
+
+
+# bottoms of an even number of cells and of an odd one (88 x 56 -> 11 x 7, 18 x 26 -> 9 x 13), the grid
+# itself the bottom, and three levels above it
+@pytest.mark.parametrize("nx,ny", [(8, 8), (13, 15), (18, 26), (88, 56), (96, 96), (176, 112), (512, 256)])
+def test_multigrid_arrays_start_on_a_pair(exe, nx, ny):
+    got = check(exe, "layout", nx, ny)
+    assert got["level"] == 0 and got["H"] == 0 and got["r2"] == 0
