@@ -253,6 +253,8 @@ void pvk_div_finalize(const pvk_grid *g, pvk_scal *sc, const pvk_red *rd, hipStr
  * and the six per-iteration stages; n = -1 preconditions the start residual */
 /* threads a block of the row kernels has for rows of N values: T = N / 16 of them a row */
 int  pvk_fft_row_threads(int N);
+/* lets them have the LDS that rows of N values take, on the current device */
+void pvk_fft_row_allow(int N);
 void pvk_pcg_start(const pvk_grid *g, const pvk_fft *F, pvk_scal *sc, const pvk_pcg *w, double tol,
                    hipStream_t s);
 void pvk_pcg_stage(const pvk_grid *g, const pvk_fft *F, pvk_scal *sc, const pvk_pcg *w, int stage, int n,

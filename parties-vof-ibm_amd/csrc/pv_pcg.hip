@@ -21,6 +21,7 @@
 // can be formed from gamma_n and gamma_{n-1}.
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include <mutex>
 #include "pv_kernels.h"
 #include "pv_block.h"
 #include "pv_fftk.h"
@@ -858,6 +859,26 @@ static size_t lds_row(int R, int N)
 #define FWD_WARM(P2, NT) k_pcg_update_fwd<P2, NT, ROW_WARM>
 #define FWD_PLAIN(P2, NT) k_pcg_update_fwd<P2, NT, ROW_PLAIN>
 #define INV_DOT(P2, NT) k_ifft_rows_dot<P2, NT>
+
+// Rows of 3888 and 4096 take more than 64 KiB of dynamic LDS (the padding; up
+// to 68 KiB), which a kernel must be allowed (gfx950: up to 160 KiB a
+// workgroup): their forms are, on the current device, when a handle of that
+// length is made.  A refusal leaves the launch to report the error.
+extern "C" void pvk_fft_row_allow(int N)
+{
+    static std::mutex mu;                // handles may be made by several host threads
+    const void *const k[] = {(const void *)FWD_STEP(true, 256),   (const void *)FWD_STEP(false, 256),
+                             (const void *)FWD_START(true, 256),  (const void *)FWD_START(false, 256),
+                             (const void *)FWD_WARM(true, 256),   (const void *)FWD_WARM(false, 256),
+                             (const void *)FWD_PLAIN(true, 256),  (const void *)FWD_PLAIN(false, 256),
+                             (const void *)(INV_DOT(true, 256)),  (const void *)(INV_DOT(false, 256))};
+    if (lds_row(pvk_fft_row_threads(N) / (N / 16), N) <= 65536) return;
+    std::lock_guard<std::mutex> lk(mu);
+    for (const void *f : k)
+        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+            (void)hipGetLastError();
+}
+
 #define ROWS(KERNEL, N)                                                                                                    \
     do {                                                                                                                   \
         const int nt = pvk_fft_row_threads(g->NXM), nrow = (g->NYM + w->rrow - 1) / w->rrow;                               \

@@ -614,8 +614,8 @@ int pv_fft_create(pv_bag *b)
     double idx2, idy2;
     memset(&b->fft, 0, sizeof b->fft);
     b->fftmem = NULL;
-    /* FFT-PCG unavailable for this size: one row of N/2 complex doubles and
-     * its twiddles must fit the LDS budget of the row transforms (N <= 4096) */
+    /* FFT-PCG unavailable for this size: a block of the row transforms has a
+     * thread for each 16 values of a row and at most 256 of them (N <= 4096) */
     if (!xlen_ok(nx) || nx > 4096 || ny < 8 || ny > 8192) return PV_OK;
     b->fft.mx = nx / 2;
     b->fft.pow2x = (lx >= 4);
@@ -689,6 +689,7 @@ int pv_fft_create(pv_bag *b)
         int band = (ny >= 512) ? 2 : 1, rrow, rdct, nband, nrow, np;
         double *pm;
         rrow = pvk_fft_row_threads(nx) / (nx / 16);
+        pvk_fft_row_allow(nx);
         rdct = 256 / ((ny / 2 >= 8) ? ny / 16 : 1);
         nband = (ny + band - 1) / band;
         nrow = (ny + rrow - 1) / rrow;

@@ -3,6 +3,8 @@
  * The HIP calls of libparties_vof.so resolve to the functions below: device
  * memory is host memory, kernels are counted and not run.  Modes:
  *   layout NX NY    offsets of the arrays the kernels read in pairs of doubles
+ *   lds NX NY       launches of the FFT solves with more than 64 KiB of dynamic
+ *                   LDS, and those of them whose kernel was not allowed it
  */
 #include <stdio.h>
 #include <stdlib.h>
@@ -66,9 +68,24 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t 
     *g = cfg.g; *b = cfg.b; *lds = cfg.lds; *s = cfg.s;
     return hipSuccess;
 }
+static struct { const void *f; size_t lds; } allowed[NBLOCK];
+static int nallowed, nlarge, nrefused;
+hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute a, int v)
+{
+    if (a != hipFuncAttributeMaxDynamicSharedMemorySize || nallowed == NBLOCK) return hipErrorInvalidValue;
+    allowed[nallowed].f = f;
+    allowed[nallowed++].lds = (size_t)v;
+    return hipSuccess;
+}
 hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t lds, hipStream_t s)
 {
-    (void)f; (void)g; (void)b; (void)args; (void)lds; (void)s;
+    (void)g; (void)b; (void)args; (void)s;
+    if (lds > 65536) {
+        int k, ok = 0;
+        for (k = 0; k < nallowed; k++) ok |= allowed[k].f == f && allowed[k].lds >= lds;
+        nlarge++;
+        nrefused += !ok;
+    }
     return hipSuccess;
 }
 
@@ -81,6 +98,7 @@ static pv_bag *create(int nx, int ny)
     p.NXM = nx;
     p.NYM = ny;
     p.ymax = (double)ny / nx;
+    p.p_max_iter = 2;
     if (pv_create(&p, 0, &b)) { fprintf(stderr, "%s\n", pv_last_error()); exit(1); }
     return b;
 }
@@ -118,8 +136,20 @@ static int layout(int nx, int ny)
     return 0;
 }
 
+static int lds(int nx, int ny)
+{
+    pv_bag *b = create(nx, ny);
+    if (pv_Pressure_solve_fft(b, PV_F_SCRATCH0, PV_F_SCRATCH1)) { fprintf(stderr, "%s\n", pv_last_error()); return 1; }
+    pv_set_pressure_solver(b, PV_PSOLVE_FFT_PCG);
+    pv_Pressure_solve_cg(b, NULL);       /* start and two iterations; no kernel ran, so it did not stop */
+    printf("large %d\nrefused %d\n", nlarge, nrefused);
+    pv_destroy(b);
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
     if (argc == 4 && !strcmp(argv[1], "layout")) return layout(atoi(argv[2]), atoi(argv[3]));
+    if (argc == 4 && !strcmp(argv[1], "lds")) return lds(atoi(argv[2]), atoi(argv[3]));
     return 2;
 }

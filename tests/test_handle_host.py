@@ -50,3 +50,11 @@ def test_row_tables_start_on_a_pair(exe, nx, ny):
 def test_multigrid_arrays_start_on_a_pair(exe, nx, ny):
     got = check(exe, "layout", nx, ny)
     assert got["level"] == 0 and got["H"] == 0 and got["r2"] == 0
+
+
+# the longest rows (powers of two and 2^a 3^b), whose padded transforms take more than 64 KiB, and the
+# longest that do not
+@pytest.mark.parametrize("nx,large", [(4096, 1), (3888, 1), (3456, 0), (2048, 0), (16, 0)])
+def test_row_transforms_are_allowed_their_lds(exe, nx, large):
+    got = check(exe, "lds", nx, 9)
+    assert (got["large"] > 0) == bool(large) and got["refused"] == 0
