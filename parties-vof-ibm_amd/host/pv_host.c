@@ -438,6 +438,7 @@ int pv_set_field(pv_bag *b, int f, const double *host)
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(b->xfer_ev[k], b->stream));
     }
+    HIPCHK(hipStreamSynchronize(b->stream));     /* the field is set, and its errors are this call's */
     return PV_OK;
 }
 

@@ -5,6 +5,8 @@
  *   layout NX NY    offsets of the arrays the kernels read in pairs of doubles
  *   lds NX NY       launches of the FFT solves with more than 64 KiB of dynamic
  *                   LDS, and those of them whose kernel was not allowed it
+ *   transfers NX NY work still queued when a transfer of a field returns, for a
+ *                   host array and for a device array; what the latter carried
  */
 #include <stdio.h>
 #include <stdlib.h>
@@ -48,6 +50,33 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; *p =
 hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 hipError_t hipMemset(void *p, int v, size_t n) { memset(p, v, n); return hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { (void)k; memcpy(d, s, n); return hipSuccess; }
+/* work queued on the one stream and work known to be finished */
+static long queued, finished;
+hipError_t hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, hipMemcpyKind k, hipStream_t st)
+{
+    size_t j;
+    (void)k; (void)st;
+    for (j = 0; j < h; j++) memcpy((char *)d + j * dp, (const char *)s + j * sp, w);
+    queued++;
+    return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
+{
+    int k;
+    memset(a, 0, sizeof *a);
+    a->type = hipMemoryTypeUnregistered;
+    for (k = 0; k < nblock; k++)
+        if ((char *)p >= block[k].p && (char *)p < block[k].p + block[k].n) a->type = hipMemoryTypeDevice;
+    return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned flags) { (void)flags; *e = (hipEvent_t)calloc(1, sizeof(long)); return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { free(e); return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { (void)s; *(long *)e = queued; return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t e)
+{
+    if (*(long *)e > finished) finished = *(long *)e;
+    return hipSuccess;
+}
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st)
 {
     (void)st;
@@ -55,7 +84,7 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hip
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned flags) { (void)flags; *s = (hipStream_t)malloc(1); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { free(s); return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) { (void)s; finished = queued; return hipSuccess; }
 
 static struct { dim3 g, b; size_t lds; hipStream_t s; } cfg;
 hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s)
@@ -86,6 +115,7 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t ld
         nlarge++;
         nrefused += !ok;
     }
+    queued++;
     return hipSuccess;
 }
 
@@ -147,9 +177,33 @@ static int lds(int nx, int ny)
     return 0;
 }
 
+static int transfers(int nx, int ny)
+{
+    pv_bag *b = create(nx, ny);
+    const size_t n = (size_t)(nx + 7) * (ny + 7);
+    double *h = (double *)calloc(n, sizeof(double)), *d, *e;
+    size_t k, wrong = 0;
+    hipMalloc((void **)&d, n * sizeof(double));
+    hipMalloc((void **)&e, n * sizeof(double));
+    for (k = 0; k < n; k++) { d[k] = (double)k; e[k] = -1.0; }
+    if (pv_set_field(b, PV_F_U, h)) return 1;
+    printf("set %ld\n", queued - finished);
+    if (pv_get_field(b, PV_F_U, h)) return 1;
+    printf("get %ld\n", queued - finished);
+    if (pv_set_field(b, PV_F_V, d)) return 1;
+    printf("device_set %ld\n", queued - finished);
+    if (pv_get_field(b, PV_F_V, e)) return 1;
+    printf("device_get %ld\n", queued - finished);
+    for (k = 0; k < n; k++) wrong += e[k] != d[k];
+    printf("wrong %zu\n", wrong);
+    pv_destroy(b);
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
     if (argc == 4 && !strcmp(argv[1], "layout")) return layout(atoi(argv[2]), atoi(argv[3]));
     if (argc == 4 && !strcmp(argv[1], "lds")) return lds(atoi(argv[2]), atoi(argv[3]));
+    if (argc == 4 && !strcmp(argv[1], "transfers")) return transfers(atoi(argv[2]), atoi(argv[3]));
     return 2;
 }

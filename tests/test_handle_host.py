@@ -58,3 +58,12 @@ def test_multigrid_arrays_start_on_a_pair(exe, nx, ny):
 def test_row_transforms_are_allowed_their_lds(exe, nx, large):
     got = check(exe, "lds", nx, 9)
     assert (got["large"] > 0) == bool(large) and got["refused"] == 0
+
+
+# part of one staging buffer, several
+@pytest.mark.parametrize("nx,ny", [(8, 8), (1000, 700)])
+def test_transfers_are_complete_on_return(exe, nx, ny):
+    """Setting and reading a field leave nothing queued, whether the array is
+    on the host (staged) or on the device (a strided copy)."""
+    got = check(exe, "transfers", nx, ny)
+    assert got == dict(set=0, get=0, device_set=0, device_get=0, wrong=0)
