@@ -147,7 +147,8 @@ int pv_get_params(const pv_bag *bag, pv_params *out);   /* derived values filled
 
 /* H2D / D2H of one field in canonical layout ((NYM+7)*(NXM+7) doubles).
  * Stand-in for Resume_h5_data / Output_h5_data (IO/Resume.c:341, IO/Output.c:277).
- * Complete when they return. */
+ * Complete when they return.  The first one pins host memory for the handle,
+ * until pv_destroy: twice a field or 4 MiB, whichever is less. */
 int pv_set_field(pv_bag *bag, int field, const double *host);
 int pv_get_field(pv_bag *bag, int field, double *host);
 int pv_fill_field(pv_bag *bag, int field, double value);

@@ -6,7 +6,8 @@
  *   lds NX NY       launches of the FFT solves with more than 64 KiB of dynamic
  *                   LDS, and those of them whose kernel was not allowed it
  *   transfers NX NY work still queued when a transfer of a field returns, for a
- *                   host array and for a device array; what the latter carried
+ *                   host array and for a device array; what the latter carried;
+ *                   bytes of host memory pinned for them
  */
 #include <stdio.h>
 #include <stdlib.h>
@@ -46,7 +47,14 @@ hipError_t hipFree(void *p)
     free(p);
     return hipSuccess;
 }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; *p = malloc(n); return *p ? hipSuccess : hipErrorOutOfMemory; }
+static size_t pinned;
+hipError_t hipHostMalloc(void **p, size_t n, unsigned flags)
+{
+    (void)flags;
+    pinned += n;
+    *p = malloc(n);
+    return *p ? hipSuccess : hipErrorOutOfMemory;
+}
 hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 hipError_t hipMemset(void *p, int v, size_t n) { memset(p, v, n); return hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { (void)k; memcpy(d, s, n); return hipSuccess; }
@@ -182,6 +190,7 @@ static int transfers(int nx, int ny)
     pv_bag *b = create(nx, ny);
     const size_t n = (size_t)(nx + 7) * (ny + 7);
     double *h = (double *)calloc(n, sizeof(double)), *d, *e;
+    const size_t pinned0 = pinned;
     size_t k, wrong = 0;
     hipMalloc((void **)&d, n * sizeof(double));
     hipMalloc((void **)&e, n * sizeof(double));
@@ -190,6 +199,7 @@ static int transfers(int nx, int ny)
     printf("set %ld\n", queued - finished);
     if (pv_get_field(b, PV_F_U, h)) return 1;
     printf("get %ld\n", queued - finished);
+    printf("pinned %zu\n", pinned - pinned0);
     if (pv_set_field(b, PV_F_V, d)) return 1;
     printf("device_set %ld\n", queued - finished);
     if (pv_get_field(b, PV_F_V, e)) return 1;

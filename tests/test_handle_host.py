@@ -66,4 +66,11 @@ def test_transfers_are_complete_on_return(exe, nx, ny):
     """Setting and reading a field leave nothing queued, whether the array is
     on the host (staged) or on the device (a strided copy)."""
     got = check(exe, "transfers", nx, ny)
+    got.pop("pinned")
     assert got == dict(set=0, get=0, device_set=0, device_get=0, wrong=0)
+
+
+@pytest.mark.parametrize("nx,ny", [(8, 8), (96, 96), (505, 505), (1000, 700)])
+def test_transfers_pin_no_more_than_they_stage(exe, nx, ny):
+    """Two buffers of a field, or of 2 MiB where a field is larger."""
+    assert check(exe, "transfers", nx, ny)["pinned"] <= 2 * min(8 * (nx + 7) * (ny + 7), 2 << 20)
