@@ -56,8 +56,8 @@ TIMERS = ["CH_APPLY", "CH_UPDATE", "MOM_APPLY", "MOM_UPDATE", "P_APPLY", "P_UPDA
 # makes the x step); P_APPLY / P_UPDATE here the Jacobi-PCG's two kernels
 BYTES_PER_CELL = {
     "CH_APPLY": 32, "CH_UPDATE": 48, "MOM_APPLY": 72, "MOM_UPDATE": 40,
-    "P_APPLY": 48, "P_UPDATE": 64, "P_DUPDATE": 24,
-    "FFT_ROWS_FWD": 16, "FFT_COLS": 16, "FFT_ROWS_INV": 24,
+    "P_APPLY": 48, "P_UPDATE": 64,
+    "FFT_COLS": 16, "FFT_ROWS_INV": 24,
     "CH_RHS": 56, "MOM_TERMS": 88, "P_TRANSPOSE": 16,
 }
 # the fused FFT-PCG kernels behind the P_APPLY / P_UPDATE timers also form the

@@ -244,19 +244,19 @@ int pv_Pressure_solve_fft(pv_bag *bag, int rhs_field, int out_field);
 enum pv_timer {
     PV_T_CH_APPLY = 0,     /* biharmonic operator + <p,Ap>       */
     PV_T_CH_UPDATE,        /* x, r update + <r,r>                */
-    PV_T_MOM_APPLY,        /* momentum operator + <d,Ad>         */
-    PV_T_MOM_UPDATE,       /* x, r update + two sums             */
-    PV_T_P_APPLY,          /* pressure operator + <d,Ad>         */
-    PV_T_P_UPDATE,         /* phi, r update + sums               */
-    PV_T_P_DUPDATE,        /* d = z + beta d                     */
-    PV_T_FFT_ROWS_FWD,     /* forward real FFT of rows           */
-    PV_T_FFT_COLS,         /* DCT-II / scale / DCT-III of columns */
+    PV_T_MOM_APPLY,        /* momentum direction, operator, <d,Ad>; x of the iteration before */
+    PV_T_MOM_UPDATE,       /* r update, z + two sums             */
+    PV_T_P_APPLY,          /* pressure direction, operator + <d,Ad> */
+    PV_T_P_UPDATE,         /* phi, r update + sums (Jacobi: and z; FFT: and the forward real FFT of the rows) */
+    PV_T_P_DUPDATE,        /* not recorded: P_APPLY forms the direction (number kept) */
+    PV_T_FFT_ROWS_FWD,     /* not recorded: part of P_UPDATE (number kept) */
+    PV_T_FFT_COLS,         /* y solves; CH start: DCT-II / divide / DCT-III of columns */
     PV_T_FFT_ROWS_INV,     /* inverse real FFT + <r,z>           */
     PV_T_CH_RHS,           /* fused explicit CH right-hand side  */
     PV_T_MOM_TERMS,        /* fused momentum right-hand side     */
-    PV_T_P_TRANSPOSE,      /* spectrum transposes of the FFT-PCG */
+    PV_T_P_TRANSPOSE,      /* spectrum transposes of the CH start */
     PV_T_MG_PRE0,          /* multigrid pre-smoothing + restriction, level 0 */
-    PV_T_MG_COARSE,        /* multigrid levels 1 .. (both ways)  */
+    PV_T_MG_COARSE,        /* multigrid levels 1 .. (both ways), the in-workgroup ones among them */
     PV_T_MG_POST0,         /* correction + post-smoothing + <r,z>, level 0 */
     PV_NTIMERS
 };
