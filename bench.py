@@ -26,9 +26,9 @@ algorithmic byte count per cell) with the largest share of device time,
 timed live with HIP events on the library's stream (every timer_period-th
 launch) over a separate run of kernel_steps steps of the same configuration,
 so that the event records do not perturb the timed run.  The multigrid's
-one-workgroup coarse kernel (MG_COARSE in kernels) can take more time; it
-runs on one CU, bound by its instruction issue rather than by HBM, so it has
-no byte count and no roofline.
+coarse part (MG_COARSE in kernels: the tiled levels below level 0 and the
+one-workgroup kernel) can take more time; what bounds it is latency, the
+one-workgroup kernel's on one CU, so it has no byte count and no roofline.
 The cpu_baseline block times the CPU oracle (serial C restatement of the
 reference algorithm) on a bounded sample of the same workload.
 """
@@ -79,8 +79,8 @@ BYTES_PER_ITER = {"fft": 144, "mg": 179, "mg32": 149, "jacobi": 112}
 # the 1024^2 MG-PCG mixed form (FETCH_SIZE scaled by 2.0, WRITE_SIZE by 1.0:
 # the factors a 256 MiB device copy gives in runs of its own); the summary is
 # profiles/mg_pcg_mixed_1024_pmc_traffic.md
-TRAFFIC_MB_MG32_1024 = {"MG_PRE0": 64.2, "MG_POST0": 29.7, "P_APPLY": 51.5,
-                        "MOM_APPLY": 141.0, "MOM_UPDATE": 105.5, "CH_RHS": 68.6, "MOM_TERMS": 111.0}
+TRAFFIC_MB_MG32_1024 = {"MG_PRE0": 63.7, "MG_POST0": 29.6, "P_APPLY": 51.0,
+                        "MOM_APPLY": 139.9, "MOM_UPDATE": 104.8, "CH_RHS": 68.2, "MOM_TERMS": 104.7}
 SEED = 20261202
 # the headline metric: the timed form is the learned-start mixed form, the plain
 # FP64 path is reported beside it (compare.plain_fp64), the dominant kernel's

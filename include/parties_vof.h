@@ -55,9 +55,9 @@ extern "C" {
 #define PV_PSOLVE_MG_PCG     4   /* the same CG, start, gauge and stop test, preconditioned
                                     by one geometric multigrid V-cycle on the variable face
                                     coefficients (no counterpart in the reference): NXM and
-                                    NYM must halve together down to <= 1024 cells; halving
+                                    NYM must halve together down to <= 4096 cells; halving
                                     goes on while both are even, to a last level of at most
-                                    64 cells */
+                                    256 cells and 64 columns */
 #define PV_PSOLVE_LEARNED_MG 5   /* MG-PCG from the learned network's warm start, kept
                                     only when its energy is below the cold start's */
 
@@ -330,10 +330,11 @@ int pv_batch_autotune_mg(pv_batch *bt, int *wlevels, int *sweeps);
 int pv_set_momentum_rows(pv_bag *bag, int rows);
 int pv_set_mg_tile0(pv_bag *bag, int shape);
 /* Shape of the FFT preconditioner's y tridiagonal solves (two first-order
- * recurrences, their carries combined by a scan): rows per thread's segment, 1..16 (0 = 8), and columns per block,
- * a power of two <= 64 (0 = 2, or more where a block would hold less than a
- * wavefront; halved while a block would exceed 512 threads).  Changes the order of the arithmetic
- * (where the carries are combined), so results differ at rounding level. */
+ * recurrences, their carries combined by a scan): rows per thread's segment,
+ * 1..16 (0 = 8), and columns per block, a power of two <= 64 (0 = 2, or more
+ * where a block would hold less than a wavefront; halved while a block would
+ * exceed 512 threads).  Changes the order of the arithmetic (where the carries
+ * are combined), so results differ at rounding level. */
 int pv_set_fft_tri_shape(pv_bag *bag, int rows, int cols);
 int pv_autotune_tiles(pv_bag *bag, int *mom_rows, int *mg_tile0);
 

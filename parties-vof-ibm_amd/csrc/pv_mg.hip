@@ -236,11 +236,11 @@ __device__ __forceinline__ void blk_residual(int hx, const T *x, const Blk<T> &k
 // the residual needs) holds exactly what sweeping the whole level would give.
 //
 // A thread owns one 2 x 2 block of the extended tile, two on the widest tile.
-// What bounds these kernels on large levels is instruction issue.  With a
+// What bounded these kernels on large levels was instruction issue.  With a
 // thread a cell (half the lanes idle in each half-sweep, four LDS reads an
 // update, five loads, a column modulo and a position a cell) a launch took,
 // pre and post, FP32, 21.7 and 15.4 us at 1024^2, 75 and 33 at 2048^2; with
-// blocks 14.7 and 10.9, 58 and 26: the rate of the memory they touch (62 and
+// blocks 14.0 and 10.5, 58 and 26: the rate of the memory they touch (62 and
 // 27 MB at 1024^2) within a factor of two, at 2048^2 4.2 TB/s.
 // ---------------------------------------------------------------------------
 template <int NU, int SH> struct MgTile {
@@ -942,8 +942,11 @@ template <typename T> __global__ void __launch_bounds__(NTH) k_mg_bottom_proj(in
 
 // ---------------------------------------------------------------------------
 // Levels c0 .. nlev-1 in one workgroup.  The kernel runs on one CU, so its
-// time is a chain of barrier-separated half-sweeps; what a half-sweep costs
-// is instruction issue and LDS round trips.
+// time is a chain of barrier-separated half-sweeps and bottom visits, and it
+// is bound by their latency: at 1024^2 (64^2, 32^2 and the 16^2 bottom, W on
+// both, FP32) a wavefront spends 53 % of its time waiting for the L2, LDS or a
+// barrier, 16 % for an issue slot and 31 % on an instruction, a SIMD's vector
+// unit is busy for 30 % (FP64, V at 96^2: 64, 14, 22 and 26 %).
 //
 // A thread owns 2 x 2 blocks of cells (one coarse cell each): two blocks of
 // level c0, one of each level below.  It keeps their faces, 1 / diagonal, f
@@ -955,9 +958,8 @@ template <typename T> __global__ void __launch_bounds__(NTH) k_mg_bottom_proj(in
 // offset from the one dynamic array, so the accesses are LDS instructions.
 // Reading the level descriptors (with their pointers) from LDS instead, as
 // an earlier form did, made every access a flat one, and each pass reloaded
-// the coefficients: at 1024^2 (64^2, 32^2 and the 16^2 bottom, W on both,
-// FP32) 53.5 us a launch, FP64, V at 96^2, 26; with registers 33 and 15, and
-// with the bottom solve's bounds scalar and its chunks read in turn 28 and 12.4.
+// the coefficients: at 1024^2 as above 53.4 us a launch, FP64, V at 96^2, 26;
+// now 33.3 and 13.8 (kernel traces of whole runs).
 // ---------------------------------------------------------------------------
 #define CT 512
 static_assert(PVK_MG_LDS_CELLS <= 8 * CT, "level c0 has at most two 2 x 2 blocks a thread");
@@ -1072,10 +1074,11 @@ __device__ __forceinline__ void restrict_res(const CGeo &g, T *x, const Blk<T> (
 // PF columns, one chunk ahead of the sums and the first one before the residual
 // that the solve waits for.  Two buffers are read in turn (copying one to the
 // other would wait for it), and a quarter's bounds and addresses are scalars:
-// with the copy, and tests a lane, a launch took 44 us in FP64 (64^2, W on
-// both levels), 29 (44 x 88, W on one) and 14.3 (48^2, V), 32.6 in FP32 (64^2); now
-// 38, 25, 12.4 and 30.8.  Wider FP32 loads (four rows a lane, halves of the
-// wavefront swapped) gave nothing: there the conversions to FP64 are the bound.
+// launched alone, back to back (faster than in a run, where other kernels come
+// between), with the copy, and tests a lane, a launch took 44 us in FP64 (64^2,
+// W on both levels), 29 (44 x 88, W on one) and 14.3 (48^2, V), 32.6 in FP32
+// (64^2), and 38, 25, 12.4 and 30.8 without.  Wider FP32 loads (four rows a
+// lane, halves of the wavefront swapped) gave nothing.
 template <typename T> struct HChunk {
     static constexpr int PF = sizeof(T) == 4 ? 8 : 4;
     T h[PF][2];
@@ -1418,9 +1421,6 @@ extern "C" int pvk_mg_nrz(const pvk_mg *m)
     return (int)(gr.x * gr.y);
 }
 
-// the bottom matrix of a solve: G column by column, then P G P.  Above 64 KiB
-// of LDS (bottoms wider than 16 columns) the factorisation kernel must be
-// allowed it.
 // above 64 KiB of dynamic LDS a kernel must be allowed it (gfx950: up to 160
 // KiB per workgroup); raised once per device and kernel, under a lock
 static void allow_lds(const void *k, int slot)

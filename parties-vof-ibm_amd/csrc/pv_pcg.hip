@@ -106,7 +106,7 @@ __global__ void __launch_bounds__(NTH) k_pcg_faces(pvk_grid g, pvk_pcg w)
 // columns of the three rows are loaded ahead of the sums that give beta (all
 // blocks of a grid this size run at once, so nothing else covers them); its
 // row's east and west values go through LDS.  Bound by memory, 48 bytes a
-// cell: 11.9 us at 1024^2 (50 MB; 14.9 with every stencil
+// cell: 11.2 us at 1024^2 (50 MB; 14.9 with every stencil
 // value formed from its own loads after the sums), 50 at 2048^2 (73), 6.6 at
 // 768 x 491 (10.6).
 // ---------------------------------------------------------------------------
@@ -202,7 +202,7 @@ __global__ void __launch_bounds__(NTH, 4) k_pcg_apply(pvk_grid g, pvk_scal *sc, 
 // the twiddles staged one by one and the split table read where it is used, a
 // chain of ~12 us of memory latency whatever the grid, the forward kernel
 // took 19.6 us and the inverse one 13.7 at 1024^2 (13.4 and 10.9 at 128 x 256);
-// now 15.0 and 8.7 (7.9 and 5.3).  One wavefront a block against 256 threads
+// now 14.2 and 8.3 (7.9 and 5.3).  One wavefront a block against 256 threads
 // (NT / T rows): 15.0 and 8.7 against 15.8 and 9.4 at 1024^2, 14.1 and 9.5
 // against 15.0 and 11.6 at 768 x 491 (12.9 and 8.2 since the index arithmetic
 // there is shifts), 7.9 and 5.3 against 9.9 and 7.0 at 128 x 256.
@@ -558,8 +558,8 @@ __global__ void __launch_bounds__(NTH) k_dct_rows(pvk_grid g, pvk_fft F, pvk_sca
 // with powers of q.  q, K, q^N and 1 / (1 - q^{2N}) are tables (per column), so
 // the kernel has no division; the elimination it replaces (partitioned
 // Thomas, a pivot division a row and a cyclic reduction of the separators
-// with two divisions a step) took 16.6 us at 1024^2 against 10.6 now, and 13.2
-// at 768 x 491 against 8.7.
+// with two divisions a step) took 16.6 us at 1024^2 against 10.2 now, and 13.2
+// at 768 x 491 against 7.7.
 // Column 0 (m = 0, row 0 replaced by the pin x_0 = 0) is two running sums:
 // x_{j+1} - x_j = -sum_{i > j} f_i / c.  With mean removal (the PCG's
 // pseudo-inverse) it is shifted to zero mean afterwards.  In the PCG this

@@ -394,7 +394,7 @@ static int check_field(pv_bag *b, int f)
  * pitched field straight into host memory (or unpacks them from it) while the
  * host copies the other buffer from or to the caller's array.  A strided copy between the field and pageable memory,
  * which this replaces, pins the caller's pages: 8.5 MB (1024^2) took 7.7 ms
- * down and 9.6 ms up; staged it takes 0.34 and 0.27 ms. */
+ * down and 9.6 ms up; staged it takes 0.37 and 0.28 ms. */
 #define PV_XFER_BYTES ((size_t)2 << 20)
 
 /* the next buffer (of rows rows), free to be written by the host or the GPU */
@@ -568,9 +568,10 @@ static int xlen_ok(int n)
  * row; 0 = 8) and cols columns per block (a power of two; 0 = 2, or more
  * where a block would hold less than a wavefront; halved while the block
  * would exceed 512 threads).  Short segments and many blocks (512 at 1024
- * columns) are near the fastest at every size tried: 10.2 us at 1024^2 (9.9 for
- * 16 rows and 4 columns, 14.7 for 8 and 1, 12.2 for 4 and 4), 8.3 us at 768 x
- * 491 (7.9, 9.1, 9.9) and 6.0 us at 128 x 256 (6.5, 6.3, 7.3).
+ * columns) are near the fastest at every size tried: between events, which add
+ * half a microsecond, 10.7 us at 1024^2 (10.1 for 16 rows and 4 columns, 11.1
+ * for 16 and 2, 12.3 for 16 and 8), 8.3 us at 768 x 491 (8.1, 8.1, 9.2), 9.3 at
+ * 512 x 1024 (9.5, 8.9, 11.8) and 6.3 at 128 x 256 (6.7, 7.1, 7.1).
  * The blocks of one XCD take neighbouring columns, so each row's cache lines
  * come from HBM once per XCD.  Nonzero if no shape fits. */
 static int tri_shape(pv_bag *b, int rows, int cols)
